@@ -30,7 +30,8 @@
 // a bounded number of polls backs that up, after which every wavefront leaves and the call
 // reports an error.  Early pivots of a column
 // overlap with the tail of the columns before it, which is where a banded factor, whose
-// columns form one long dependency chain, gets its parallelism from.
+// columns form one long dependency chain, gets its parallelism from.  Factors that stay within a
+// narrow band have a kernel of their own (lu_band_kernel, below).
 #include "nm_common.hpp"
 #include "nm_scan.hpp"
 
@@ -214,7 +215,8 @@ constexpr int64_t kLuSpinLimit = 1 << 24;  // polls of one dependency flag, with
 struct LuFlow {
     int64_t *below;  // [cols] position of the column's first entry below the diagonal
     int32_t *done;   // [cols] 0 = pending, 1 = the column holds its final values
-    int32_t *ctl;    // [0] next ticket, [1] failure, [2] columns finished
+    int32_t *ctl;    // [0] next ticket, [1] failure, [2] columns finished, [3] the band kernel made the factors,
+                     // [4] reach above the diagonal, [5] below it, [6] columns that do not name their predecessor
 };
 
 size_t flow_layout(int64_t cols, void *base, LuFlow *F) {
@@ -247,17 +249,41 @@ struct OwnColumn {
     }
 };
 
-// below[k] = position of the first entry of column k with a row index > k.
-__global__ void lu_below_kernel(int64_t cols, const int64_t *__restrict__ indices,
-                                const int64_t *__restrict__ indptr, int64_t *__restrict__ below) {
+// below[k] = position of the first entry of column k with a row index > k.  Also what the choice of
+// the numeric kernel depends on: ctl[4] / ctl[5] = entries the widest column reaches above / below its
+// diagonal, ctl[6] = columns that do not name the column before them.
+__global__ __launch_bounds__(kBlock) void lu_below_kernel(int64_t cols, const int64_t *__restrict__ indices,
+                                                          const int64_t *__restrict__ indptr,
+                                                          int64_t *__restrict__ below, int32_t *ctl) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    int32_t up = 0, down = 0, breaks = 0;
     for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < cols; k += stride) {
-        int64_t lo = indptr[k], hi = indptr[k + 1];
+        const int64_t pb = indptr[k], pe = indptr[k + 1];
+        int64_t lo = pb, hi = pe;
         while (lo < hi) {
             const int64_t mid = (lo + hi) >> 1;
             if (indices[mid] <= k) lo = mid + 1; else hi = mid;
         }
         below[k] = lo;
+        if (pe > pb) {
+            const int64_t first = indices[pb], last = indices[pe - 1];
+            if (first < k) up = max(up, (int32_t)(k - first));
+            if (last > k) down = max(down, (int32_t)(last - k));
+        }
+        int64_t q = lo - 1;                        // last entry on or above the diagonal
+        if (q >= pb && indices[q] == k) --q;
+        if (k > 0 && !(q >= pb && indices[q] == k - 1)) ++breaks;
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        up = max(up, __shfl_xor(up, off, nm::kWave));
+        down = max(down, __shfl_xor(down, off, nm::kWave));
+        breaks += __shfl_xor(breaks, off, nm::kWave);
+    }
+    if ((threadIdx.x & 63) == 0) {
+        if (up) atomicMax(ctl + 4, up);
+        if (down) atomicMax(ctl + 5, down);
+        if (breaks) atomicAdd(ctl + 6, breaks);
     }
 }
 
@@ -415,6 +441,7 @@ __global__ __launch_bounds__(kLuFlowBlock) void lu_flow_kernel(int64_t cols, con
     __shared__ int32_t s_ready[kLuWavesPerBlock];
     __shared__ int32_t s_ticket, s_abort;
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (ctl[3] != 0) return;   // lu_band_kernel, earlier on the stream, has made the factors
     for (;;) {
         // one ticket per workgroup and batch of consecutive columns, one column per wavefront
         if (threadIdx.x == 0) {
@@ -444,6 +471,420 @@ __global__ __launch_bounds__(kLuFlowBlock) void lu_flow_kernel(int64_t cols, con
         }
         __syncthreads();   // the batch's columns in LDS have no readers left
     }
+}
+
+// ---- banded factors --------------------------------------------------------------
+//
+// A factor whose entries stay near the diagonal is ONE chain of columns: column k + 1 needs column k,
+// and lu_flow_kernel pays a hand-over between wavefronts, workgroups or compute units (1.4 us) for
+// every link of it whatever the width of the band.  Here one workgroup keeps the part of the matrix
+// that is still to be updated in registers and eliminates column by column (right-looking): every
+// entry receives the same products in the same ascending order of pivots, so the factors are the
+// serial ones bit for bit.
+//   * Wavefront v owns the columns j = v mod 16, CS of them at a time; its lanes are rows: row i sits
+//     in lane i mod 64 of register i / 64 mod RL, a ring of 64 RL rows.  At step k the last row of any
+//     column at hand is below k + 16 CS + bl <= k + 64 RL, so a place of the ring means one row.
+//   * Step k: the multipliers of column k come through LDS; the pivot row's entries are in the
+//     wavefront's own registers (one lane of each column) and become scalars.  The owner of column
+//     k + 1 updates that column first, divides it and hands its multipliers on before it turns to
+//     its other columns; the others wait for the column's number in LDS, not for a barrier.
+//   * Only products of two STORED entries are subtracted (a bit per row and column, read with the
+//     pivot row; a ballot per column of multipliers): a zero or infinite pivot spreads exactly as far
+//     as in the serial loop.
+//   * A finished column is written out, and the wavefront's next one, requested a round of sixteen
+//     steps earlier, takes its place, in the two steps after, when nobody waits for this wavefront.
+// 64 x 64 five-point grid in fp64 (4096 columns, reach 64 either way): 5.57 -> 2.41 ms, 0.59 us a column.
+// Bound by what the SIMDs issue: 240 vector instructions per step and SIMD, three quarters of the
+// time; the chain alone (LDS trip, update, division, LDS trip) would be 0.34 us.  Eight wavefronts of
+// nine columns: 2.84 ms; a barrier a step instead of the numbers in LDS: 4.6 ms; without the raised
+// priority of the wavefronts whose turn is near: 2.75 ms; the owner putting off the update before its
+// turn as well: 2.65 ms.
+#define NM_INLINE __attribute__((always_inline))   // (lambdas over register arrays)
+constexpr int kBandWaves = 16;
+constexpr int kBandMaxRl = 3;
+// More breaks in the chain (columns that do not name their predecessor) than this and the matrix may
+// be made of three independent blocks or more, which lu_flow_kernel works on side by side: it takes
+// 0.75 us a column of ONE block where the reach is 1 and 1.3 us where it is 60, this kernel 0.27 and
+// 0.50 us whatever the blocks.
+constexpr int kBandMaxBreaks = 1;
+
+// Multipliers are kept for as many columns as there are wavefronts: who publishes column c has seen
+// every other wavefront publish one of the fifteen columns before it, and each read the multipliers
+// of column c - 16 before it did.
+constexpr int kBandDepth = kBandWaves;
+
+struct BandShared {
+    double l[kBandDepth][64 * kBandMaxRl];              // multipliers of a column, by ring position (T at the front)
+    uint64_t head[kBandDepth][kBandMaxRl + 1];          // which of them are stored entries, whose they are (written last)
+    double value[kBandWaves][64 * kBandMaxRl];          // columns on their way into the registers
+    int32_t entry[kBandWaves][64 * kBandMaxRl];
+};
+
+// w -= l * u on the active lanes for every place S of a register whose bit of `stored` is set; products and
+// differences are rounded on their own.  In assembler because the compiler turned the choice per
+// column into selects, branches or copies of every column (a step 1.5 to 4 times as long).  The
+// inner places are mostly all stored and then go without a choice; the first (finished for a step
+// out of eight) and the last (mostly outside the band) are chosen by the execution mask.
+#define NM_BAND_M64(i, t) "v_mul_f64 %[t" #t "], %[l], %[u" #i "]\n\t"
+#define NM_BAND_M32(i, t) "v_mul_f32 %[t" #t "], %[u" #i "], %[l]\n\t"
+#define NM_BAND_D64(i, t) "v_add_f64 %[w" #i "], %[w" #i "], -%[t" #t "]\n\t"
+#define NM_BAND_D32(i, t) "v_sub_f32 %[w" #i "], %[w" #i "], %[t" #t "]\n\t"
+#define NM_BAND_IF(i) "s_bitcmp1_b32 %[stored], %[S]+" #i "\n\ts_cselect_b64 exec, %[sv], 0\n\t"
+#define NM_BAND_P64(i, t) NM_BAND_IF(i) NM_BAND_D64(i, t)
+#define NM_BAND_P32(i, t) NM_BAND_IF(i) NM_BAND_D32(i, t)
+// (E: all lanes again before the next products)
+#define NM_BAND_SEQ2(M, D, E) M(0, 0) M(1, 1) D(0, 0) D(1, 1)
+#define NM_BAND_SEQ3(M, D, E) M(0, 0) M(1, 1) M(2, 2) D(0, 0) D(1, 1) D(2, 2)
+#define NM_BAND_SEQ4(M, D, E) M(0, 0) M(1, 1) M(2, 2) M(3, 3) D(0, 0) D(1, 1) D(2, 2) D(3, 3)
+#define NM_BAND_ALL_LANES "s_mov_b64 exec, %[sv]\n\t"
+#define NM_BAND_TEXT(SEQ, M, D, P)                                                                                   \
+    "s_bfe_u32 %[bits], %[stored], %[field]\n\ts_cmp_eq_u32 %[bits], %[whole]\n\ts_cbranch_scc0 .Lpick_%=\n\t" SEQ(M, D, )  \
+    "s_branch .Ldone_%=\n.Lpick_%=:\n\ts_mov_b64 %[sv], exec\n\t" SEQ(M, P, NM_BAND_ALL_LANES) NM_BAND_ALL_LANES ".Ldone_%=:"
+#define NM_BAND_W(i) [w##i] "+v"(W[S + i][q])
+#define NM_BAND_U(i) [u##i] "s"(u[S + i])
+#define NM_BAND_LIST2(X) X(0), X(1)
+#define NM_BAND_LIST3(X) NM_BAND_LIST2(X), X(2)
+#define NM_BAND_LIST4(X) NM_BAND_LIST3(X), X(3)
+#define NM_BAND_CASE(N)                                                                                              \
+    if constexpr (CS - 2 == N) {                                                                                     \
+        if constexpr (sizeof(T) == 8)                                                                                \
+            NM_BAND_ASM_(NM_BAND_TEXT(NM_BAND_SEQ##N, NM_BAND_M64, NM_BAND_D64, NM_BAND_P64), N);                    \
+        else                                                                                                         \
+            NM_BAND_ASM_(NM_BAND_TEXT(NM_BAND_SEQ##N, NM_BAND_M32, NM_BAND_D32, NM_BAND_P32), N);                    \
+    }
+#define NM_BAND_ASM_(TEXT, N)                                                                                        \
+    asm volatile(TEXT : NM_BAND_LIST##N(NM_BAND_W), [t0] "=&v"(t0), [t1] "=&v"(t1), [t2] "=&v"(t2), [t3] "=&v"(t3),  \
+                 [sv] "=&s"(sv), [bits] "=&s"(bits) : [l] "v"(l), [stored] "s"(stored), [S] "n"(S),                  \
+                 [field] "n"(S | N << 16), [whole] "n"((1 << N) - 1), NM_BAND_LIST##N(NM_BAND_U) : "scc")
+// the places 1 .. CS - 2
+template <int CS, typename T, int RL>
+__device__ __forceinline__ void band_inner(T l, uint32_t stored, const T (&u)[CS], T (&W)[CS][RL], int q) {
+    constexpr int S = 1;
+    uint64_t sv;
+    uint32_t bits;
+    T t0, t1, t2, t3;
+    NM_BAND_CASE(2)
+    NM_BAND_CASE(3)
+    NM_BAND_CASE(4)
+}
+// the two outer places, bits 0 and 1 of `stored`
+template <typename T>
+__device__ __forceinline__ void band_outer(T l, uint32_t stored, T u0, T u1, T &w0, T &w1) {
+    uint64_t sv;
+    T t0, t1;
+    constexpr int S = 0;
+    if constexpr (sizeof(T) == 8)
+        asm volatile("s_mov_b64 %[sv], exec\n\t" NM_BAND_SEQ2(NM_BAND_M64, NM_BAND_P64, ) "s_mov_b64 exec, %[sv]"
+                     : [w0] "+v"(w0), [w1] "+v"(w1), [t0] "=&v"(t0), [t1] "=&v"(t1), [sv] "=&s"(sv)
+                     : [l] "v"(l), [stored] "s"(stored), [S] "n"(S), [u0] "s"(u0), [u1] "s"(u1) : "scc");
+    else
+        asm volatile("s_mov_b64 %[sv], exec\n\t" NM_BAND_SEQ2(NM_BAND_M32, NM_BAND_P32, ) "s_mov_b64 exec, %[sv]"
+                     : [w0] "+v"(w0), [w1] "+v"(w1), [t0] "=&v"(t0), [t1] "=&v"(t1), [sv] "=&s"(sv)
+                     : [l] "v"(l), [stored] "s"(stored), [S] "n"(S), [u0] "s"(u0), [u1] "s"(u1) : "scc");
+}
+
+// LDS accesses that stay in program order (no waits between them).
+template <typename V> __device__ __forceinline__ V lds_get(V *p) {
+    asm volatile("" ::: "memory");
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+template <typename V> __device__ __forceinline__ void lds_put(V *p, V v) {
+    asm volatile("" ::: "memory");
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+template <typename T, int RL, int CS>
+__device__ __forceinline__ void lu_band(int32_t n, int bl, const int64_t *__restrict__ indices,
+                                        const int64_t *__restrict__ indptr, T *values, BandShared &sh) {
+    constexpr int R = 64 * RL;
+    const int lane = threadIdx.x & 63, v = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    T W[CS][RL];              // the wavefront's columns
+    uint32_t pos[CS];         // entry number inside the column of each of this lane's rows, a byte each; 0xff: not stored
+    uint32_t has[RL];         // bit S: this lane's row of the register is stored in column S and not finished
+    T fetched[RL];            // the next column: entry e = lane + 64 q
+    int32_t fetched_row[RL];
+    int32_t fetched_len = 0;
+    int64_t base[CS], fetched_b = 0, staged_b = 0;   // where a column starts in the arrays: of the columns, of the
+                                                     // one requested, of the one in LDS
+    int64_t next_b, next_e;   // place of the column after that in the arrays
+    int32_t next_col = 0;
+
+    // (vector loads: a scalar load would be waited for with the next access to LDS, microseconds later)
+    int32_t zero = 0;
+    asm volatile("" : "+v"(zero));
+    auto pointers = [&](int32_t col) NM_INLINE {
+        const int32_t at = min(col, n - 1) + zero;
+        next_b = indptr[at];
+        next_e = indptr[at + 1];
+        next_col = col;
+    };
+    // Requests the column that `pointers` looked up last: unconditional loads (clamped to an entry
+    // that exists), so that nothing waits for them before `stage` does.
+    auto fetch = [&]() NM_INLINE {
+        fetched_len = next_col < n ? (int32_t)(next_e - next_b) : 0;
+        fetched_b = next_b;
+#pragma unroll
+        for (int q = 0; q < RL; ++q) {
+            const int64_t t = max(min(next_b + q * 64 + lane, next_e - 1), (int64_t)0);
+            fetched_row[q] = reinterpret_cast<const int32_t *>(indices)[2 * t];   // (low half: rows fit 31 bits)
+            fetched[q] = values[t];
+        }
+    };
+    T *s_value = reinterpret_cast<T *>(sh.value[v]);
+    int32_t *s_entry = sh.entry[v];
+    auto stage = [&]() NM_INLINE {
+        staged_b = fetched_b;
+#pragma unroll
+        for (int q = 0; q < RL; ++q) s_entry[q * 64 + lane] = -1;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+        for (int q = 0; q < RL; ++q)
+            if (q * 64 + lane < fetched_len) {
+                const uint32_t at = (uint32_t)fetched_row[q] % (uint32_t)R;
+                s_value[at] = fetched[q];
+                s_entry[at] = q * 64 + lane;
+            }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    };
+    // the column in LDS takes the last place
+    auto unstage = [&]() NM_INLINE {
+        constexpr int S = CS - 1;
+        base[S] = staged_b;
+        pos[S] = 0;
+#pragma unroll
+        for (int q = 0; q < RL; ++q) {
+            const int32_t e = s_entry[q * 64 + lane];
+            W[S][q] = e >= 0 ? s_value[q * 64 + lane] : T(0);
+            pos[S] |= (uint32_t)(e >= 0 ? e : 0xff) << (8 * q);
+            has[q] |= e >= 0 ? 1u << S : 0u;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    };
+    // the columns move up, so that the next one to finish is always in place 0
+    auto shift = [&]() NM_INLINE {
+#pragma unroll
+        for (int S = 0; S + 1 < CS; ++S) {
+            pos[S] = pos[S + 1];
+            base[S] = base[S + 1];
+#pragma unroll
+            for (int q = 0; q < RL; ++q) W[S][q] = W[S + 1][q];
+        }
+#pragma unroll
+        for (int q = 0; q < RL; ++q) has[q] >>= 1;
+    };
+    // f(constant q) for the register that holds ring position p
+    auto by_ring = [&](int p, auto f) NM_INLINE {
+        if (RL == 1 || p < 64)
+            f(std::integral_constant<int, 0>{});
+        else if (RL == 2 || p < 128)
+            f(std::integral_constant<int, RL < 2 ? 0 : 1>{});
+        else
+            f(std::integral_constant<int, RL - 1>{});
+    };
+    // which of this lane's rows are stored below the diagonal (ring position p) of the column in place 0
+    bool below[RL];
+    uint64_t below_mask[RL];
+    bool has_diagonal = false;
+    auto look_below = [&](int p) NM_INLINE {
+#pragma unroll
+        for (int q = 0; q < RL; ++q) {
+            int delta = q * 64 + lane - p;
+            if (delta < 0) delta += R;
+            below[q] = delta >= 1 && delta <= bl && (has[q] & 1u) != 0;
+            below_mask[q] = __ballot(below[q]);
+        }
+        by_ring(p, [&](auto q) NM_INLINE { has_diagonal = (nm::read_lane((int)has[q], p & 63) & 1) != 0; });
+    };
+    // Divides column c, in place 0 (diagonal at ring position p), and leaves its multipliers for everybody.
+    // A wavefront's LDS accesses are carried out in order: who sees the column's number sees them.
+    auto finish = [&](int32_t c, int p) NM_INLINE {
+        const int buffer = c % kBandDepth;
+        T *s_l = reinterpret_cast<T *>(sh.l[buffer]);
+        if (has_diagonal) {
+            T d = T(0);
+            by_ring(p, [&](auto q) NM_INLINE { d = nm::read_lane(W[0][q], p & 63); });
+#pragma unroll
+            for (int q = 0; q < RL; ++q) {
+                const T quot = W[0][q] / d;
+                W[0][q] = below[q] ? quot : W[0][q];
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < RL; ++q) lds_put(s_l + q * 64 + lane, W[0][q]);
+        if (lane == 0) {
+#pragma unroll
+            for (int q = 0; q < RL; ++q) lds_put(&sh.head[buffer][q], below_mask[q]);
+            lds_put(reinterpret_cast<int32_t *>(&sh.head[buffer][kBandMaxRl]), c);
+        }
+#pragma unroll
+        for (int q = 0; q < RL; ++q) has[q] &= ~1u;
+    };
+    auto write_out = [&]() NM_INLINE {
+#pragma unroll
+        for (int q = 0; q < RL; ++q) {
+            const uint32_t e = pos[0] >> (8 * q) & 0xffu;
+            if (e != 0xffu) values[base[0] + e] = W[0][q];
+        }
+    };
+
+#pragma unroll
+    for (int q = 0; q < RL; ++q) has[q] = 0;
+#pragma unroll
+    for (int S = 0; S < CS; ++S) {
+        pos[S] = ~0u;
+        base[S] = 0;
+#pragma unroll
+        for (int q = 0; q < RL; ++q) W[S][q] = T(0);
+    }
+    pointers(v);
+#pragma unroll 1
+    for (int S = 0; S < CS; ++S) {
+        fetch();
+        pointers(v + kBandWaves * (S + 1));
+        stage();
+        shift();
+        unstage();
+    }
+    int32_t ahead = v + kBandWaves * CS;        // column `next_b` belongs to
+    if (threadIdx.x < kBandDepth) sh.head[threadIdx.x][kBandMaxRl] = ~0ull;
+    __syncthreads();
+    int p = 0;                                  // ring position of row k
+    auto next = [&](int p) NM_INLINE { return p + 1 == R ? 0 : p + 1; };
+    // the multipliers of column k into l, their mask into m; HURRY: asks for everything every time
+    auto receive = [&](int32_t k, T (&l)[RL], uint64_t (&m)[RL], auto HURRY) NM_INLINE {
+        const int buffer = k & (kBandDepth - 1);
+        T *s_l = reinterpret_cast<T *>(sh.l[buffer]);
+        int32_t *s_column = reinterpret_cast<int32_t *>(&sh.head[buffer][kBandMaxRl]);
+        auto read = [&]() NM_INLINE {
+            const int32_t there = lds_get(s_column);
+            uint64_t w[RL];
+#pragma unroll
+            for (int q = 0; q < RL; ++q) w[q] = lds_get(&sh.head[buffer][q]);
+#pragma unroll
+            for (int q = 0; q < RL; ++q) l[q] = lds_get(s_l + q * 64 + lane);
+#pragma unroll
+            for (int q = 0; q < RL; ++q)
+                m[q] = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(w[q] >> 32)) << 32 |
+                       (uint32_t)__builtin_amdgcn_readfirstlane((int)w[q]);
+            return __builtin_amdgcn_readfirstlane(there) == k;
+        };
+        if constexpr (HURRY) {
+            while (!read()) {}
+        } else if (__builtin_expect(!read(), 0)) {
+            while (__builtin_amdgcn_readfirstlane(lds_get(s_column)) != k) __builtin_amdgcn_s_sleep(1);
+            read();
+        }
+    };
+    // the column whose multipliers are l applied to the columns of this wavefront; OWN: but not to place 0
+    auto apply = [&](const T (&l)[RL], const uint64_t (&m)[RL], const T (&u)[CS], uint32_t stored, auto OWN) NM_INLINE {
+        stored = (uint32_t)__builtin_amdgcn_readfirstlane((int)stored);
+        const uint32_t first = OWN ? 0u : stored & 1u;
+        const uint32_t outer = (uint32_t)__builtin_amdgcn_readfirstlane((int)(first | stored >> (CS - 1) << 1));
+#pragma unroll
+        for (int q = 0; q < RL; ++q)
+            if (__builtin_amdgcn_inverse_ballot_w64(m[q])) {
+                band_inner<CS>(l[q], stored, u, W, q);
+                band_outer(l[q], outer, u[0], u[CS - 1], W[0][q], W[CS - 1][q]);
+            }
+    };
+    // the entries of the row at ring position p in this wavefront's columns, and which of them are stored
+    auto row = [&](int p, T (&u)[CS]) NM_INLINE {
+        uint32_t stored = 0;
+        by_ring(p, [&](auto q) NM_INLINE {
+            stored = (uint32_t)nm::read_lane((int)has[q], p & 63);
+            nm::static_for<CS>([&](auto S) NM_INLINE { u[S] = nm::read_lane(W[S][q], p & 63); });
+        });
+        return stored;
+    };
+    constexpr std::true_type yes;
+    constexpr std::false_type no;
+    auto step = [&](int32_t k) NM_INLINE {
+        T l[RL], u[CS];
+        uint64_t m[RL];
+        const uint32_t stored = row(p, u);
+        receive(k, l, m, no);
+        apply(l, m, u, stored, no);
+        p = next(p);
+    };
+    auto update_first = [&](const T (&l)[RL], const uint64_t (&m)[RL], T u0, uint32_t stored) NM_INLINE {
+        if ((uint32_t)__builtin_amdgcn_readfirstlane((int)stored) & 1u) {
+#pragma unroll
+            for (int q = 0; q < RL; ++q)
+                if (__builtin_amdgcn_inverse_ballot_w64(m[q])) {
+                    const T prod = l[q] * u0;
+                    W[0][q] = W[0][q] - prod;
+                }
+        }
+    };
+    // Step c - 1: column c is finished and handed on before the wavefront turns to its other columns.
+    auto own = [&](int32_t c) NM_INLINE {
+        T l[RL], u[CS];
+        uint64_t m[RL];
+        uint32_t stored = 0;
+        const int p1 = c >= 1 ? next(p) : p;    // row c
+        look_below(p1);
+        if (c >= 1) {
+            stored = row(p, u);
+            receive(c - 1, l, m, yes);
+            __builtin_amdgcn_s_setprio(3);
+            update_first(l, m, u[0], stored);
+        }
+        finish(c, p1);
+        __builtin_amdgcn_s_setprio(0);
+        if (c >= 1) apply(l, m, u, stored, yes);
+        p = p1;
+    };
+    // Sixteen steps a round: the wavefront finishes its column c, writes it out at step c, puts the column
+    // that waits in LDS in its place at step c + 1 and requests the next one, which has the rest of the
+    // round to arrive.
+#pragma unroll 1
+    for (int32_t c = v - kBandWaves; c < n; c += kBandWaves) {
+        int32_t k = 0;
+        if (c >= 0) {
+            own(c);
+#pragma unroll 1
+            for (k = c; k < min(c + 2, n); ++k) {
+                step(k);
+                if (k == c) {
+                    write_out();
+                    shift();
+                } else {
+                    unstage();
+                }
+            }
+        }
+        fetch();
+        ahead += kBandWaves;
+        pointers(ahead);
+        // a wavefront goes before the others of its SIMD as the step at which everybody waits for it comes up
+#pragma unroll 1
+        for (; k < min(c + kBandWaves - 1, n); ++k) {
+            if (k == c + kBandWaves - 8) __builtin_amdgcn_s_setprio(1);
+            if (k == c + kBandWaves - 4) __builtin_amdgcn_s_setprio(2);
+            step(k);
+        }
+        stage();
+    }
+}
+
+template <typename T>
+__global__ __launch_bounds__(kBandWaves * 64) void lu_band_kernel(int32_t n, const int64_t *__restrict__ indices,
+                                                                  const int64_t *__restrict__ indptr, T *values,
+                                                                  int32_t *ctl) {
+    __shared__ BandShared sh;
+    const int bu = ctl[4], bl = ctl[5];
+    if (ctl[6] > kBandMaxBreaks || n >= 1 << 30 || indptr[n] == 0) return;   // lu_flow_kernel's
+    // The smallest set of registers that holds the band: the ring (above), and room for bu + 4 columns, as
+    // a column is in place two steps after its predecessor is done.  us a column, fp64, this kernel
+    // and lu_flow_kernel: reach 28 0.27 and 1.24, reach 60 0.50 and 1.30, reach 76 0.61 and 2.2, reach
+    // 92 0.70 and 2.2.
+    auto fits = [&](int rl, int cs) { return bu + 4 <= kBandWaves * cs && bl + kBandWaves * cs <= 64 * rl; };
+    if (fits(1, 2)) lu_band<T, 1, 2>(n, bl, indices, indptr, values, sh);
+    else if (fits(2, 4)) lu_band<T, 2, 4>(n, bl, indices, indptr, values, sh);
+    else if (fits(3, 5)) lu_band<T, 3, 5>(n, bl, indices, indptr, values, sh);
+    else if (fits(3, 6)) lu_band<T, 3, 6>(n, bl, indices, indptr, values, sh);
+    else return;
+    if (threadIdx.x == 0) ctl[3] = 1;
 }
 
 int check_rows(int64_t rows) {
@@ -556,8 +997,20 @@ extern "C" int nm_splu_numeric(nm_dtype dt, int64_t cols, void *Mt_data, const i
     {
         int64_t g = nm::ceil_div(cols, kBlock);
         hipLaunchKernelGGL(lu_below_kernel, dim3((unsigned)(g > 65536 ? 65536 : g)), dim3(kBlock), 0, s, cols,
-                           Mt_indices, Mt_indptr, F.below);
+                           Mt_indices, Mt_indptr, F.below, F.ctl);
         NM_LAUNCH_CHECK("lu_below_kernel");
+    }
+    // Whether the factors are a band is known on the device only: the band kernel leaves at once
+    // where they are not, lu_flow_kernel where the band kernel has made them.  (A caller that bounds
+    // the polls asks for the kernel that polls.)
+    if (poll_limit <= 0) {
+        if (dt == NM_F32)
+            hipLaunchKernelGGL(lu_band_kernel<float>, dim3(1), dim3(kBandWaves * 64), 0, s, (int32_t)cols, Mt_indices,
+                               Mt_indptr, (float *)Mt_data, F.ctl);
+        else
+            hipLaunchKernelGGL(lu_band_kernel<double>, dim3(1), dim3(kBandWaves * 64), 0, s, (int32_t)cols, Mt_indices,
+                               Mt_indptr, (double *)Mt_data, F.ctl);
+        NM_LAUNCH_CHECK("lu_band_kernel");
     }
     int64_t grid = nm::ceil_div(cols, kLuWavesPerBlock);
     if (grid > 1024) grid = 1024;

@@ -217,3 +217,62 @@ def test_pattern_scratch_is_bounded(dev):
     diag_pos = p[:-1] + (np.arange(n) > 0)
     assert np.array_equal(got[diag_pos], u)
     assert np.array_equal(got[p[1:-1]], lo[1:])
+
+
+def _banded(n, below, above, dtype, seed, holes=0.0):
+    """Dense band (a chain of columns), `holes` of the entries off the three middle diagonals left out."""
+    rng = np.random.default_rng(seed)
+    i, j = np.indices((n, n))
+    off = j - i
+    keep = (off >= -below) & (off <= above) & ((np.abs(off) <= 1) | (rng.random((n, n)) >= holes))
+    a = np.where(keep, rng.uniform(-1, 1, (n, n)), 0.0)
+    a[np.arange(n), np.arange(n)] = (below + above + 1) * rng.uniform(1, 2, n)
+    r, c = np.nonzero(keep)
+    p = np.zeros(n + 1, np.int64)
+    np.cumsum(np.bincount(r, minlength=n), out=p[1:])
+    return a[r, c].astype(dtype), c.astype(np.int64), p
+
+
+# reaches at the edges of the band kernel's register sets (32, 64, 112, 96 below and 28, 60, 76, 92 above the
+# diagonal), sizes that are no multiples of a round of sixteen columns, one of them below sixteen
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n, below, above", [(5, 1, 1), (16, 3, 1), (33, 1, 14), (130, 28, 28), (131, 29, 29), (150, 32, 28),
+                                             (150, 33, 28), (190, 60, 60), (190, 61, 61), (210, 64, 60), (210, 65, 60),
+                                             (230, 76, 76), (231, 77, 77), (290, 112, 76), (290, 113, 76),
+                                             (260, 92, 92), (261, 96, 92), (261, 97, 92), (262, 93, 93), (100, 5, 28), (300, 2, 92)])
+def test_banded_factors_match_the_oracle_bit_for_bit(dev, dtype, n, below, above):
+    ext = numml_amd.load_compiled()
+    for holes in (0.0, 0.6):
+        print("case band", n, below, above, holes, dtype.__name__, flush=True)
+        d, i, p = _banded(n, below, above, dtype, n + below, holes)
+        out, want = ext.splu(n, n, *to_dev(dev, d, i, p)), oracle.splu(n, n, d, i, p)
+        for got, ref, what in zip(out, want, NAMES):
+            assert_same(host(got), ref, f"{n} {below} {above} {holes} {what}")
+
+
+@pytest.mark.parametrize("special", ["zero pivot", "negative zeros", "infinity", "two blocks", "three blocks"])
+def test_banded_factors_of_unusual_matrices(dev, special):
+    # what a zero pivot makes of its column, and what -0.0 and inf in A become, reaches stored entries only
+    n, w = 100, 20
+    d, i, p = _banded(n, w, w, np.float64, 5, 0.5)
+    r = np.repeat(np.arange(n), np.diff(p))
+    if special == "zero pivot":
+        d[(r == 0) & (i == 0)] = 0.0
+    elif special == "negative zeros":
+        d[(np.arange(d.size) % 3 == 0) & (r != i)] = -0.0
+    elif special == "infinity":
+        d[(r == 40) & (i == 41)] = np.inf
+    else:
+        cut = [50] if special == "two blocks" else [33, 66]
+        block = np.searchsorted(cut, np.arange(n), side="right")
+        keep = block[r] == block[i]
+        d, i, r = d[keep], i[keep], r[keep]
+        p = np.concatenate(([0], np.cumsum(np.bincount(r, minlength=n)))).astype(np.int64)
+    got = numml_amd.load_compiled().splu(n, n, *to_dev(dev, d, i, p))
+    want = oracle.splu(n, n, d, i, p)
+    for g, ref, what in zip(got, want, NAMES):
+        g = host(g)
+        assert_same(g, ref, f"{special} {what}")
+        if g.dtype == np.float64:
+            ok = ~np.isnan(ref)
+            assert np.array_equal(np.signbit(g[ok]), np.signbit(ref[ok])), f"{special} {what}: signs of zeros"
