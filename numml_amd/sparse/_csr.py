@@ -27,6 +27,13 @@ def _type_error(kind_a, a, kind_b, b):
     return RuntimeError(f"{kind_a} should be same data type, got {a.type()} and {b.type()}, respectively.")
 
 
+# Functions that return structure beside values switch off autograd's materialised gradients: it would
+# fill an int64 tensor of zeros for every structure tensor of the result before each backward pass (128^3
+# seven-point A A: 77 us of 675).  A gradient of the values that is missing still counts as zeros.
+def _grad_or_zeros(grad, pattern, dtype):
+    return torch.zeros(pattern.shape, dtype=dtype, device=pattern.device) if grad is None else grad
+
+
 class spgemv(torch.autograd.Function):
     """y = A x with gradients for A's stored values and x (numml/sparse/_csr.py:102-133)."""
 
@@ -87,6 +94,7 @@ class spgemm(torch.autograd.Function):
                               C_indices, C_indptr)
         ctx.A_shape, ctx.B_shape = A_shape, B_shape
         ctx.mark_non_differentiable(C_indices, C_indptr)
+        ctx.set_materialize_grads(False)
         return (A_shape[0], B_shape[1]), C_data, C_indices, C_indptr
 
     @staticmethod
@@ -94,7 +102,7 @@ class spgemm(torch.autograd.Function):
         (A_data, A_indices, A_indptr, B_data, B_indices, B_indptr,
          C_indices, C_indptr) = ctx.saved_tensors
         grad_A, grad_B = _ext.spgemm_backward(
-            grad_C_data, C_indices, C_indptr,
+            _grad_or_zeros(grad_C_data, C_indices, A_data.dtype), C_indices, C_indptr,
             ctx.A_shape[0], ctx.A_shape[1], A_data, A_indices, A_indptr,
             ctx.B_shape[0], ctx.B_shape[1], B_data, B_indices, B_indptr)
         return None, grad_A, None, None, None, grad_B, None, None
@@ -110,19 +118,22 @@ class sptranspose(torch.autograd.Function):
         At_data, At_indices, At_indptr, At_to_A_idx = _ext.csr_transpose_forward(
             A_shape[0], A_shape[1], A_data, A_indices, A_indptr)
         ctx.save_for_backward(At_to_A_idx)
+        ctx.dtype = A_data.dtype
         ctx.mark_non_differentiable(At_indices, At_indptr)
+        ctx.set_materialize_grads(False)
         return tuple(A_shape[::-1]), At_data, At_indices, At_indptr
 
     @staticmethod
     def backward(ctx, _g_shape, grad_At_data, _g_indices, _g_indptr):
         (At_to_A_idx,) = ctx.saved_tensors
+        grad_At_data = _grad_or_zeros(grad_At_data, At_to_A_idx, ctx.dtype)
         return None, _ext.csr_transpose_backward(grad_At_data, At_to_A_idx), None, None
 
 
 class splincomb(torch.autograd.Function):
     """C = alpha A + beta B; returns ``(C_data, C_indices, C_indptr)``.  The scalars
-    get sum(A.data) and sum(B.data) as their gradients, as in the reference
-    (numml/sparse/_csr.py:187-231)."""
+    get sum(A.data) and sum(B.data) as their gradients where they ask for one, as in the
+    reference (numml/sparse/_csr.py:187-231)."""
 
     @staticmethod
     def forward(ctx, shape, alpha, A_data, A_col_ind, A_rowptr, beta, B_data, B_col_ind, B_rowptr):
@@ -134,6 +145,7 @@ class splincomb(torch.autograd.Function):
                               C_col_ind, C_rowptr)
         ctx.shape = shape
         ctx.mark_non_differentiable(C_col_ind, C_rowptr)
+        ctx.set_materialize_grads(False)
         return C_data, C_col_ind, C_rowptr
 
     @staticmethod
@@ -142,9 +154,10 @@ class splincomb(torch.autograd.Function):
          C_col_ind, C_rowptr) = ctx.saved_tensors
         grad_A, grad_B = _ext.splincomb_backward(
             ctx.shape[0], ctx.shape[1], alpha, A_data, A_col_ind, A_rowptr, beta, B_data, B_col_ind, B_rowptr,
-            grad_C_data, C_col_ind, C_rowptr)
-        return (None, torch.sum(A_data).to(alpha.device), grad_A, None, None,
-                torch.sum(B_data).to(beta.device), grad_B, None, None)
+            _grad_or_zeros(grad_C_data, C_col_ind, A_data.dtype), C_col_ind, C_rowptr)
+        grad_alpha = torch.sum(A_data).to(alpha.device) if ctx.needs_input_grad[1] else None
+        grad_beta = torch.sum(B_data).to(beta.device) if ctx.needs_input_grad[5] else None
+        return None, grad_alpha, grad_A, None, None, grad_beta, grad_B, None, None
 
 
 def _reduction(forward_name, backward_name, doc):
