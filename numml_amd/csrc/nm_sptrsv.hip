@@ -741,19 +741,24 @@ __global__ void gather_ell_kernel(int64_t rows, int pre, const T *__restrict__ d
                                   const int32_t *__restrict__ dsrc, const int32_t *__restrict__ diag,
                                   double *__restrict__ ell_coef, double *__restrict__ rb,
                                   int32_t *__restrict__ status, unsigned long long *__restrict__ cells,
-                                  int64_t cell_words) {
+                                  int64_t cell_words, unsigned long long *__restrict__ xs, int32_t f0, int32_t f1) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (tid == 0) status[0] = 0;   // first kernel of the solve
+    // slots [f0, f1): taken by sptrsv_flow_kernel, which reads no operands from here
+    for (int64_t q = f0 + tid; q < f1; q += stride) xs[q] = ~0ull;
+    const int64_t skip = f1 - f0;
+    rows -= skip;
     // the mailbox of the launches that several workgroups share: empty before the solve starts
     for (int64_t i = tid; i < cell_words; i += stride) cells[i] = 0ull;
     for (int64_t i = tid; i < rows * pre; i += stride) {
-        const int64_t q = i / pre;
-        const int e = (int)(i - q * pre);
+        const int64_t k = i / pre, q = k < f0 ? k : k + skip;
+        const int e = (int)(i - k * pre);
         const int32_t lo = dptr[q], n = dptr[q + 1] - lo;
-        ell_coef[i] = e < n ? (double)data[dsrc[lo + e]] : 0.;
+        ell_coef[q * pre + e] = e < n ? (double)data[dsrc[lo + e]] : 0.;
     }
-    for (int64_t q = tid; q < rows; q += stride) {
+    for (int64_t k = tid; k < rows; k += stride) {
+        const int64_t q = k < f0 ? k : k + skip;
         const int32_t d = diag[q];
         rb[2 * q] = (double)b[order[q]];
         rb[2 * q + 1] = d >= 0 ? (double)data[d] : 0.;
@@ -1427,6 +1432,151 @@ __global__ __launch_bounds__(kBlock) void sptrsv_level_group_kernel(SolveArgs a,
     }
 }
 
+// ---- stretches of wide levels: one launch, values handed over row by row ------------
+//
+// A level of thousands of rows is a few microseconds of work for the chip, and a stretch of such
+// levels used to be a launch each (3.5 us apart, whatever their width).  Here ONE launch takes the
+// whole stretch: tiles of 64 consecutive slots, in the order of the solve, are dealt to the
+// launch's wavefronts in turn, and a row starts when the rows it needs are solved, not when
+// their level is.  The running solution xs is its own mailbox: its slots in the stretch hold
+// kUnsolved until a row's value is stored there (agent scope, one 64-bit word that is never
+// torn, so there is no flag and no fence), and a lane polls the slots of its dependencies, all of
+// them at once.  A lane stores its value inside the polling loop, so rows of one tile may wait
+// for each other.  The operands come straight from the caller's arrays through three stages, each
+// requested a tile ahead of the next, so no pass gathers them into level order beforehand.
+//
+// What bounds it: the hand-over, ~0.6 us from a store to a polling load on another compute unit,
+// plus a poll's own round trip, per level.  The launch has about four tiles in flight per tile of
+// the widest level, which is what the request stages need; more only poll.  97 x 89 x 101
+// seven-point triangle, fp32 (285 levels of up to 4500 rows): see flow_stretch.
+//
+// A wavefront waits for tiles before its own only, and all workgroups are resident (a launch has
+// at most one per compute unit), so the waits end; as a backstop a wavefront that has polled
+// `poll_limit` times for one tile raises the status word, every wavefront leaves when it
+// sees that, and the solve hands out NaN.
+constexpr unsigned long long kUnsolved = ~0ull;   // a NaN; a result with these bits is stored as the default NaN
+constexpr int kFlowMaxGroups = 256;
+constexpr int64_t kFlowMinLevels = 4, kFlowMeanWidth = 16384;   // see flow_stretch
+
+template <typename T> struct FlowArgs {
+    const T *data, *b;
+    const int32_t *order, *dptr, *dslot, *dsrc, *diag;
+    unsigned long long *xs;
+    int32_t *status;
+    int32_t q0, q1;   // the stretch's slots
+    int down;         // walked from the last slot to the first
+    int unit;
+    int64_t poll_limit;
+};
+
+template <typename T, int PRE>
+__global__ __launch_bounds__(kBlock) void sptrsv_flow_kernel(FlowArgs<T> f) {
+    struct Range { int32_t q, lo, n, row, diag; bool live; };
+    struct Source { int32_t q, n; bool live; int32_t ds[PRE], src[PRE]; T bv, dv; };
+    struct Operands { int32_t q, n; bool live; int32_t ds[PRE]; T v[PRE], bv, dv; };
+    const int lane = (int)threadIdx.x & 63;
+    // neighbouring tiles on different compute units
+    const int waves = (int)gridDim.x * (kBlock / 64);
+    const int wave = (int)(threadIdx.x >> 6) * (int)gridDim.x + (int)blockIdx.x;
+    const int64_t m = f.q1 - f.q0;
+    // (indices are clamped to slots and entries that exist, so that every request is unconditional)
+    auto range = [&](int64_t tile) {
+        Range r;
+        const int64_t at = tile * 64 + lane;
+        r.live = at < m;
+        r.q = !r.live ? f.q0 : f.down ? (int32_t)(f.q1 - 1 - at) : (int32_t)(f.q0 + at);
+        r.lo = f.dptr[r.q];
+        r.n = f.dptr[r.q + 1] - r.lo;
+        r.row = f.order[r.q];
+        r.diag = f.diag[r.q];
+        return r;
+    };
+    auto source = [&](const Range &r) {
+        Source s;
+        s.q = r.q;
+        s.n = r.n;
+        s.live = r.live;
+#pragma unroll
+        for (int e = 0; e < PRE; ++e) {
+            const int32_t at = e < r.n ? r.lo + e : 0;
+            s.ds[e] = f.dslot[at];
+            s.src[e] = f.dsrc[at];
+        }
+        s.bv = f.b[r.row];
+        s.dv = r.diag >= 0 ? f.data[r.diag] : (T)0;
+        return s;
+    };
+    auto operands = [&](const Source &s) {
+        Operands o;
+        o.q = s.q;
+        o.n = s.n;
+        o.live = s.live;
+#pragma unroll
+        for (int e = 0; e < PRE; ++e) {
+            o.ds[e] = s.ds[e];
+            o.v[e] = f.data[s.src[e]];
+        }
+        o.bv = s.bv;
+        o.dv = s.dv;
+        return o;
+    };
+    const int64_t tiles = (m + 63) / 64;
+    Range r = range(wave);
+    Source s = source(r);
+    r = range((int64_t)wave + waves);
+    Operands o = operands(s);
+    s = source(r);
+    r = range((int64_t)wave + 2 * (int64_t)waves);
+    int64_t polls = f.poll_limit < 0 ? -1 : 0;
+    for (int64_t tile = wave; tile < tiles; tile += waves) {
+        const Operands cur = o;
+        o = operands(s);
+        s = source(r);
+        r = range(tile + 3 * (int64_t)waves);
+        bool pending = cur.live;
+        unsigned need = pending ? (1u << (cur.n < PRE ? cur.n : PRE)) - 1u : 0u;
+        double x[PRE];
+#pragma unroll
+        for (int e = 0; e < PRE; ++e) x[e] = 0.;
+        while (true) {
+            unsigned long long got[PRE];
+#pragma unroll
+            for (int e = 0; e < PRE; ++e)
+                if (need >> e & 1u)
+                    got[e] = __hip_atomic_load(f.xs + cur.ds[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+            for (int e = 0; e < PRE; ++e)
+                // (a row of an earlier launch is solved whatever its bits)
+                if ((need >> e & 1u) && (got[e] != kUnsolved || cur.ds[e] < f.q0 || cur.ds[e] >= f.q1)) {
+                    x[e] = __longlong_as_double((long long)got[e]);
+                    need &= ~(1u << e);
+                }
+            if (pending && need == 0) {
+                double acc = 0.;
+#pragma unroll
+                for (int e = 0; e < PRE; ++e)
+                    if (e < cur.n) acc += (double)cur.v[e] * x[e];
+                double xi = (double)cur.bv - acc;
+                if (!f.unit) xi /= (double)cur.dv;
+                unsigned long long bits = (unsigned long long)__double_as_longlong(xi);
+                if (bits == kUnsolved) bits = 0x7ff8000000000000ull;
+                __hip_atomic_store(f.xs + cur.q, bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                pending = false;
+            }
+            if (!__any(pending)) break;
+            ++polls;
+            if (polls > f.poll_limit) {
+                if (lane == 0) __hip_atomic_store(f.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                return;
+            }
+            if ((polls & 1023) == 0 &&
+                __hip_atomic_load(f.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)
+                return;
+        }
+        if (f.poll_limit >= 0) polls = 0;
+    }
+}
+
 // ---- chains: runs of levels of one row each -----------------------------------
 //
 // A banded factor, a bidiagonal or a tridiagonal triangle is one long chain: every level has
@@ -1910,6 +2060,35 @@ __global__ void unslot_kernel(int64_t n, const int32_t *__restrict__ order, cons
         x[order[q]] = (T)(failed ? nan : xs[q]);
 }
 
+// A launch whose levels go one by one to a grid each (unless sptrsv_flow_kernel takes them).
+bool by_level(const nm_sptrsv_plan *p, int dirn, bool teams, const nm_sptrsv_plan::Launch &L) {
+    return L.wide || (L.run && !(teams && p->ell_pre[dirn] > 0 && L.team[dirn].P > 1));
+}
+
+// The longest stretch [*a, *b) of consecutive launches that go level by level, where
+// sptrsv_flow_kernel is the better way: rows of at most 8 dependencies, several levels, and levels
+// that are not so wide that a launch each is no matter.
+void flow_stretch(const nm_sptrsv_plan *p, int dirn, int *a, int *b) {
+    *a = *b = 0;
+    if (p->ell_pre[dirn] == 0 || p->nnz == 0) return;
+    const int n = (int)p->launches.size();
+    int64_t best = 0;
+    for (int i = 0; i < n;) {
+        int j = i;
+        while (j < n && p->launches[j].chain[dirn] == 0 && by_level(p, dirn, true, p->launches[j])) ++j;
+        if (j > i) {
+            const int64_t levels = p->launches[j - 1].l1 - p->launches[i].l0;
+            const int64_t slots = p->launches[j - 1].q1 - p->launches[i].q0;
+            if (levels >= kFlowMinLevels && slots <= levels * kFlowMeanWidth && levels > best) {
+                best = levels;
+                *a = i;
+                *b = j;
+            }
+        }
+        i = j > i ? j : i + 1;
+    }
+}
+
 template <typename T>
 int solve_typed(const nm_sptrsv_plan *p, int transposed, const void *data, int unit, const void *b, void *x,
                 void *work, hipStream_t s) {
@@ -1922,9 +2101,11 @@ int solve_typed(const nm_sptrsv_plan *p, int transposed, const void *data, int u
     a.unit = unit;
     bool any_wide = false;
     const bool teams = g_team_enabled.load();
-    for (const auto &L : p->launches)
-        any_wide = any_wide || L.wide ||
-                   (L.run && !(teams && p->ell_pre[transposed ? 1 : 0] > 0 && L.team[transposed ? 1 : 0].P > 1));
+    // the launches [flow_a, flow_b) that one sptrsv_flow_kernel takes
+    int flow_a = 0, flow_b = 0;
+    if (teams) flow_stretch(p, transposed ? 1 : 0, &flow_a, &flow_b);
+    for (int li = 0; li < (int)p->launches.size(); ++li)
+        any_wide = any_wide || ((li < flow_a || li >= flow_b) && by_level(p, transposed ? 1 : 0, teams, p->launches[li]));
     if (any_wide || p->ell_pre[transposed ? 1 : 0] == 0) {   // the range-based arrays have readers
         int64_t m = p->nnz > p->rows ? p->nnz : p->rows;
         int64_t grid = nm::ceil_div(m, kBlock);
@@ -1939,19 +2120,36 @@ int solve_typed(const nm_sptrsv_plan *p, int transposed, const void *data, int u
     const int pre = p->ell_pre[dirn];
     EllArgs ea{p->level_ptr, P.dptr, P.dslot, P.lvl_sig, reinterpret_cast<const uint16_t *>(P.ell_ds), a.w.ell_coef,
                a.w.rb, a.w.xs, unit};
+    const int32_t flow_q0 = flow_b > flow_a ? p->launches[flow_a].q0 : 0;
+    const int32_t flow_q1 = flow_b > flow_a ? p->launches[flow_b - 1].q1 : 0;
     if (pre > 0) {
         int64_t grid = nm::ceil_div(p->rows * pre, kBlock);
         if (grid > 65536) grid = 65536;
         const T *dat = p->nnz > 0 ? (const T *)data : (const T *)b;
         hipLaunchKernelGGL(gather_ell_kernel<T>, dim3((unsigned)grid), dim3(kBlock), 0, s, p->rows, pre, dat,
                            (const T *)b, p->order, P.dptr, P.dsrc, P.diag, a.w.ell_coef, a.w.rb, a.w.status,
-                           a.w.cells, (int64_t)2 * p->team_cells[dirn]);
+                           a.w.cells, (int64_t)2 * p->team_cells[dirn], reinterpret_cast<unsigned long long *>(a.w.xs),
+                           flow_q0, flow_q1);
         NM_LAUNCH_CHECK("gather_ell_kernel");
     }
     const int n = (int)p->launches.size();
     for (int li = 0; li < n; ++li) {
-        const auto &L = p->launches[transposed ? n - 1 - li : li];
-        if (L.chain[dirn] != 0) {
+        const int at = transposed ? n - 1 - li : li;
+        const auto &L = p->launches[at];
+        if (at >= flow_a && at < flow_b) {
+            if (at != (transposed ? flow_b - 1 : flow_a)) continue;
+            FlowArgs<T> f{(const T *)data, (const T *)b, p->order, P.dptr, P.dslot, P.dsrc, P.diag,
+                          reinterpret_cast<unsigned long long *>(a.w.xs), a.w.status, flow_q0, flow_q1,
+                          transposed ? 1 : 0, unit, g_sig_poll_limit.load()};
+            int32_t widest = 0;
+            for (int j = flow_a; j < flow_b; ++j) widest = widest > p->launches[j].width ? widest : p->launches[j].width;
+            int64_t groups = nm::ceil_div((int64_t)widest, (int64_t)64);
+            const dim3 fg((unsigned)(groups > kFlowMaxGroups ? kFlowMaxGroups : groups));
+            if (pre == 2) hipLaunchKernelGGL((sptrsv_flow_kernel<T, 2>), fg, dim3(kBlock), 0, s, f);
+            else if (pre == 4) hipLaunchKernelGGL((sptrsv_flow_kernel<T, 4>), fg, dim3(kBlock), 0, s, f);
+            else hipLaunchKernelGGL((sptrsv_flow_kernel<T, 8>), fg, dim3(kBlock), 0, s, f);
+            NM_LAUNCH_CHECK("sptrsv_flow_kernel");
+        } else if (L.chain[dirn] != 0) {
             // one wavefront walks the run of one-row levels; `ell_coef` and `rb` are free for it
             // (a direction that has chains does not use the fixed-width layout)
             ChainArgs c;
@@ -1985,7 +2183,7 @@ int solve_typed(const nm_sptrsv_plan *p, int transposed, const void *data, int u
                 else hipLaunchKernelGGL((sptrsv_chain_kernel<false, false>), dim3(1), dim3(64), 0, s, c);
             }
             NM_LAUNCH_CHECK("sptrsv_chain_kernel");
-        } else if (L.wide || (L.run && !(teams && pre > 0 && L.team[dirn].P > 1))) {
+        } else if (by_level(p, dirn, teams, L)) {
             // a grid launch per level (a run without a team: its levels one after the other)
             const int G = L.group[dirn] > 0 ? L.group[dirn] : 1;
             const int nl = L.l1 - L.l0;
