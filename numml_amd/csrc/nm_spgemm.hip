@@ -3,12 +3,14 @@
 // Forward, two phases around the caller's allocation of C:
 //   symbolic: rows of A are binned by an upper bound on their products
 //             (sum of the lengths of the B rows they touch).  A group of lanes
-//             (8, 64 or 256, by bin) inserts the row's column indices into a
-//             hash set in LDS and counts the distinct ones; an exclusive scan
-//             of the counts is C_indptr.
+//             (8 or 16, by bin) or a workgroup (longer rows) inserts the row's
+//             column indices into a hash set in LDS and counts the distinct
+//             ones; an exclusive scan of the counts is C_indptr.
 //   numeric : rows are re-binned by their exact length.  The group accumulates
 //             (column, value) pairs in an LDS hash table, walking A's row
-//             entry by entry and B's row across the lanes, so every output
+//             entry by entry and B's row across the lanes (a workgroup deals
+//             the products of a longer row to its threads and lets those that
+//             meet in an entry take turns), so every output
 //             entry receives its products in the order of A's row -- the
 //             order of the serial SMMP loop (cpp/sparse_csr_cpu.cpp:182-212) --
 //             and then writes the table out ranked by column, so C's rows are
@@ -40,8 +42,8 @@ using nm::kWave;
 
 constexpr int32_t kEmpty = -1;
 constexpr int kBlock = 256;
-constexpr int kBins = 8;
-constexpr int kBinStart = 8, kBinCursor = 20, kBinInts = 32;   // layout of the bins array, see Work
+constexpr int kBins = 10;
+constexpr int kBinStart = 10, kBinCursor = 21, kBinInts = 32;   // layout of the bins array, see Work
 // Workgroups (and dense accumulator slices of B_cols entries each) of the spill path: as many as
 // fit a fixed budget of scratch, between 8 and 64.
 constexpr int64_t kSpillBudgetBytes = int64_t(192) << 20;
@@ -57,16 +59,16 @@ constexpr int kAhead = 8;            // B rows whose first columns a group reque
 #endif
 
 // bin upper limits (inclusive); the last bin takes the rest and spills
-constexpr int32_t kSymLimit[7] = {64, 128, 256, 512, 1024, 2048, 8192};     // on the product bound
-constexpr int32_t kNumLimit[7] = {32, 64, 128, 256, 512, 1024, 4096};       // on the exact row length
+constexpr int32_t kSymLimit[kBins - 1] = {64, 128, 256, 512, 1024, 2048, 8192, 24576, 24576};   // on the product bound
+// on the exact row length; the last one is what a whole CU's LDS holds (kRowLimitMost below)
+constexpr int32_t kNumLimit[kBins - 2] = {32, 64, 128, 256, 512, 1024, 2048, 4096};
 // lanes per row and table sizes per bin.  The kernels wait on memory (A's row, the bounds of its B
 // rows, the B rows: a chain of round trips per row) and LDS decides how many rows a CU has in
 // flight, so rows get the smallest table that holds them at half load.
-constexpr int kGroup0 = 8, kGroup1 = 16, kGroup2 = 16, kGroup3 = 64, kGroup4 = 64, kGroup5 = 256, kGroup6 = 256;
-constexpr int kSymTable0 = 128, kSymTable1 = 256, kSymTable2 = 512, kSymTable3 = 1024, kSymTable4 = 2048,
-              kSymTable5 = 4096, kSymTable6 = 16384;
-constexpr int kNumTable0 = 64, kNumTable1 = 128, kNumTable2 = 256, kNumTable3 = 512, kNumTable4 = 1024,
-              kNumTable5 = 2048, kNumTable6 = 8192;
+// (Bins 0 to 2; longer rows get a workgroup each, see SetShape and RowShape.)
+constexpr int kGroup0 = 8, kGroup1 = 16, kGroup2 = 16;
+constexpr int kSymTable0 = 128, kSymTable1 = 256, kSymTable2 = 512;
+constexpr int kNumTable0 = 64, kNumTable1 = 128, kNumTable2 = 256;
 
 constexpr int kMergeCap = 8;                  // longest A row and B row of the merge path
 constexpr int32_t kColEnd = 0x7fffffff;       // past-the-end column of a staged B row
@@ -114,20 +116,8 @@ template <int TABLE> __device__ __forceinline__ uint32_t first_slot(int32_t key)
 }
 
 template <int G> __device__ __forceinline__ void group_sync() {
-    if (G > kWave) __syncthreads();
-    else __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-}
-
-// Sum over a group of G lanes (G <= 64: shuffles; G == blockDim: via LDS).
-template <int G> __device__ __forceinline__ int group_total(int v, int *s_red) {
-    if (G <= kWave) return nm::group_sum<G>(v);
-    v = nm::wave_sum(v);
-    if ((threadIdx.x & (kWave - 1)) == 0) s_red[threadIdx.x / kWave] = v;
-    __syncthreads();
-    int t = 0;
-    for (int w = 0; w < G / kWave; ++w) t += s_red[w];
-    __syncthreads();
-    return t;
+    static_assert(G <= kWave, "a group is part of a wavefront");
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
 }
 
 // ---- binning ---------------------------------------------------------------
@@ -736,8 +726,7 @@ __global__ __launch_bounds__(kBlock) void symbolic_hash_kernel(
     // bank space; without the pad they would all map slot t to the same LDS bank
     constexpr int STRIDE = TABLE + (GPB > 1 ? kTablePad : 0);
     __shared__ __align__(16) int32_t s_keys[GPB * STRIDE];
-    __shared__ int s_red[kBlock / kWave];
-    const int gl = threadIdx.x % G, gi = G >= kWave ? __builtin_amdgcn_readfirstlane(threadIdx.x / G) : threadIdx.x / G;
+    const int gl = threadIdx.x % G, gi = threadIdx.x / G;
     int32_t *tab = s_keys + gi * STRIDE;
     const int32_t b0 = bins[kBinStart + bin], b1 = bins[kBinStart + bin + 1];
     for (int32_t idx0 = b0 + blockIdx.x * GPB; idx0 < b1; idx0 += gridDim.x * GPB) {
@@ -758,26 +747,22 @@ __global__ __launch_bounds__(kBlock) void symbolic_hash_kernel(
         };
         {
             // Latency-lean walk: each lane fetches one entry of A's row together with the
-            // bounds of the B row it names; the first S columns of up to kAhead B rows are
-            // then requested back to back before any of them is inserted.  A group wider than
-            // a wavefront gives each of its wavefronts its own 64 entries of A's row (the
-            // order of insertion does not matter for the count).
-            constexpr int S = G < kWave ? G : kWave;
+            // bounds of the B row it names; the first G columns of up to kAhead B rows are
+            // then requested back to back before any of them is inserted.
             // A group of 16 lanes takes TWO rows of B per step, eight lanes each: the rows these bins
             // see are mostly shorter than eight entries (stencil powers), and insertion into a set
             // has no order to keep, so the second half of the group need not idle.
-            constexpr int W = G == 16 ? 8 : S, NSUB = S / W;
-            const int sl = gl & (S - 1), sub = G > kWave ? __builtin_amdgcn_readfirstlane(gl / S) : 0;
-            const int hl = sl & (W - 1), half = sl / W;
-            const int gbase = (threadIdx.x & (kWave - 1)) & ~(S - 1);
+            constexpr int W = G == 16 ? 8 : G, NSUB = G / W;
+            const int hl = gl & (W - 1), half = gl / W;
+            const int gbase = (threadIdx.x & (kWave - 1)) & ~(G - 1);
             row = live ? perm[idx] : 0;
             const int64_t ab = live ? A_indptr[row] : 0, ae = live ? A_indptr[row + 1] : 0;
-            for (int64_t a0 = ab + sub * S; a0 < ae; a0 += G) {
-                const int64_t my_ai = a0 + sl;
+            for (int64_t a0 = ab; a0 < ae; a0 += G) {
+                const int64_t my_ai = a0 + gl;
                 const bool mine = my_ai < ae;
                 const int64_t my_j = mine ? A_indices[my_ai] : 0;
                 const int64_t my_bb = mine ? B_indptr[my_j] : 0, my_be = mine ? B_indptr[my_j + 1] : 0;
-                const int nb = (int)(ae - a0 < S ? ae - a0 : S);
+                const int nb = (int)(ae - a0 < G ? ae - a0 : G);
                 if constexpr (G == 16) {
                     // the group is one DPP row: entries 2 u and 2 u + 1 of A's row reach the two halves
                     // by row broadcasts instead of shuffles through the LDS crossbar, and the bounds of a
@@ -832,11 +817,121 @@ __global__ __launch_bounds__(kBlock) void symbolic_hash_kernel(
                 }
             }
         }
-        cnt = group_total<G>(cnt, s_red);
+        cnt = nm::group_sum<G>(cnt);
         if (live && gl == 0) C_count[row] = cnt;
         group_sync<G>();
     }
 }
+
+// Exclusive sum over the workgroup's threads; `total` gets the sum.  s_wave: one word per wavefront.
+template <int TPB, typename V> __device__ __forceinline__ V row_scan(V v, V *s_wave, V &total) {
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    V incl = v;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+        const V up = __shfl_up(incl, off, kWave);
+        if (lane >= off) incl += up;
+    }
+    if constexpr (TPB == kWave) {
+        total = __shfl(incl, kWave - 1, kWave);
+        return incl - v;
+    } else {
+        __syncthreads();   // (the words may still be read from the last use)
+        if (lane == kWave - 1) s_wave[wave] = incl;
+        __syncthreads();
+        V before = 0, all = 0;
+#pragma unroll
+        for (int w = 0; w < TPB / kWave; ++w) {
+            const V t = s_wave[w];
+            if (w < wave) before += t;
+            all += t;
+        }
+        total = all;
+        return before + incl - v;
+    }
+}
+
+// Rows of many products: one row per workgroup, its products numbered through and dealt to the
+// threads by number (see numeric_row_kernel); a set has no order to keep, so there are no turns.
+// Bound by the row's chain of round trips (A's row, the bounds of B's rows, their columns).  A
+// 150 000-row power-law graph squared (mean 8, rows up to 1000, 10 M products), by product bound, against
+// groups of 64 and 256 lanes that took B's rows one by one: 257-512 43 -> 22 us, 513-1024 70 -> 29,
+// 1025-2048 51 -> 20, 2049-8192 106 -> 44, more (a marker per column in global memory) 94 -> 17.  Groups
+// of 16 lanes with their tables side by side stay ahead below 256 products (46 us for 129-256).
+template <int TPB_, int SLOTS_> struct SetShape {
+    static constexpr int TPB = TPB_, SLOTS = SLOTS_, BATCH = TPB < 512 ? TPB : 512, UNROLL = 4;
+    static constexpr size_t at_row = 8 * (BATCH + 2), at_wave = at_row + 8 * BATCH, at_key = at_wave + 8 * (TPB / kWave) + 16;
+    static constexpr size_t lds = at_key + 4 * SLOTS;
+    static_assert(lds <= 160 * 1024, "a CU's LDS");
+};
+template <typename S>
+__global__ __launch_bounds__(S::TPB) void symbolic_row_kernel(
+    int bin, const int32_t *__restrict__ bins, const int32_t *__restrict__ perm,
+    const int64_t *__restrict__ A_indices, const int64_t *__restrict__ A_indptr,
+    const int64_t *__restrict__ B_indices, const int64_t *__restrict__ B_indptr, int32_t *__restrict__ C_count) {
+    constexpr int TPB = S::TPB, SLOTS = S::SLOTS, BATCH = S::BATCH, U = S::UNROLL;
+    extern __shared__ __align__(16) unsigned char s_raw[];
+    int64_t *s_off = reinterpret_cast<int64_t *>(s_raw);               // number of an entry's first product
+    int64_t *s_row = reinterpret_cast<int64_t *>(s_raw + S::at_row);   // start of its row of B, less that number
+    int64_t *s_wave = reinterpret_cast<int64_t *>(s_raw + S::at_wave);
+    int32_t *tab = reinterpret_cast<int32_t *>(s_raw + S::at_key);
+    const int tid = threadIdx.x;
+    const int32_t b0 = bins[kBinStart + bin], b1 = bins[kBinStart + bin + 1];
+    for (int32_t idx = b0 + (int32_t)blockIdx.x; idx < b1; idx += (int32_t)gridDim.x) {
+        const int64_t row = perm[idx];
+        const int64_t ab = A_indptr[row], ae = A_indptr[row + 1];
+        for (int t = tid; t < SLOTS; t += TPB) tab[t] = kEmpty;
+        int cnt = 0;
+        for (int64_t a0 = ab; a0 < ae; a0 += BATCH) {
+            const bool mine = tid < BATCH && a0 + tid < ae;
+            const int64_t j = mine ? A_indices[a0 + tid] : 0;
+            const int64_t bb = mine ? B_indptr[j] : 0, be = mine ? B_indptr[j + 1] : 0;
+            int64_t total;
+            const int64_t off = row_scan<TPB, int64_t>(be - bb, s_wave, total);
+            __syncthreads();   // the last batch's products are done with the lists
+            if (tid < BATCH) {
+                s_off[tid] = off;   // (threads past the row's end: the total)
+                s_row[tid] = bb - off;
+            }
+            __syncthreads();
+            for (int64_t p0 = 0; p0 < total; p0 += TPB * U) {
+                int32_t key[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const int64_t p = p0 + u * TPB + tid;
+                    const bool have = p < total;
+                    const int64_t at = have ? p : 0;
+                    int e = 0;   // the last entry whose first product is not behind this one
+#pragma unroll
+                    for (int step = BATCH / 2; step > 0; step >>= 1)
+                        if (s_off[e + step] <= at) e += step;
+                    key[u] = (int32_t)B_indices[s_row[e] + at];
+                    if (!have) key[u] = kEmpty;
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    if (key[u] == kEmpty) continue;
+                    uint32_t h = __umulhi((uint32_t)key[u] * 0x9E3779B1u, (uint32_t)SLOTS);
+                    int32_t old = atomicCAS(&tab[h], kEmpty, key[u]);
+                    while (old != kEmpty && old != key[u]) {
+                        h = h + 1 == SLOTS ? 0 : h + 1;
+                        old = atomicCAS(&tab[h], kEmpty, key[u]);
+                    }
+                    cnt += old == kEmpty;
+                }
+            }
+        }
+        int all;
+        row_scan<TPB, int>(cnt, reinterpret_cast<int *>(s_wave), all);
+        if (tid == 0) C_count[row] = all;
+        __syncthreads();
+    }
+}
+using SetShape3 = SetShape<64, 768>;      // up to 512 products
+using SetShape4 = SetShape<64, 1536>;     // up to 1024
+using SetShape5 = SetShape<256, 3072>;    // up to 2048
+using SetShape6 = SetShape<512, 10240>;   // up to 8192
+using SetShape7 = SetShape<1024, 32768>;  // up to 24576
 
 // Spill path: distinct columns counted with a stamped dense marker per workgroup.
 __global__ __launch_bounds__(kSpillBlock) void symbolic_spill_kernel(
@@ -888,18 +983,16 @@ __global__ __launch_bounds__(kBlock) void numeric_hash_kernel(
     extern __shared__ __align__(16) unsigned char s_raw[];
     T *s_vals = reinterpret_cast<T *>(s_raw);
     int32_t *s_keys = reinterpret_cast<int32_t *>(s_raw + sizeof(T) * GPB * STRIDE);
-    const int gl = threadIdx.x % G, gi = G >= kWave ? __builtin_amdgcn_readfirstlane(threadIdx.x / G) : threadIdx.x / G;
+    const int gl = threadIdx.x % G, gi = threadIdx.x / G;
     int32_t *tab = s_keys + gi * STRIDE;
     T *val = s_vals + gi * STRIDE;
     // compacted (column, slot) lists used to order the row on the way out.  The groups that share
     // a wavefront keep them where the key table was (its keys are in registers by then): LDS per
     // row is what decides how many rows a CU has in flight.
     constexpr int CSTRIDE = TABLE / 2 + 4;
-    constexpr bool ALIAS = G <= kWave;
-    static_assert(!ALIAS || (CSTRIDE + TABLE / 4 <= TABLE && TABLE <= 65536), "the lists fit the key table");
-    int32_t *ck = ALIAS ? tab : s_keys + GPB * STRIDE + gi * 2 * CSTRIDE;
-    int32_t *cs = ck + CSTRIDE;
-    uint16_t *cs16 = reinterpret_cast<uint16_t *>(cs);
+    static_assert(CSTRIDE + TABLE / 4 <= TABLE && TABLE <= 65536, "the lists fit the key table");
+    int32_t *ck = tab;
+    uint16_t *cs16 = reinterpret_cast<uint16_t *>(ck + CSTRIDE);
     const int32_t b0 = bins[kBinStart + bin], b1 = bins[kBinStart + bin + 1];
     for (int32_t idx0 = b0 + blockIdx.x * GPB; idx0 < b1; idx0 += gridDim.x * GPB) {
         const int32_t idx = idx0 + gi;
@@ -920,7 +1013,7 @@ __global__ __launch_bounds__(kBlock) void numeric_hash_kernel(
             const T cur = val[h];
             val[h] = old == kEmpty ? prod : cur + prod;
         };
-        if (G <= kWave) {
+        {
             // Same latency-lean walk as the symbolic phase; entries of A's row are still
             // applied one after the other, so every output entry gets its products in
             // the order of A's row.
@@ -1001,100 +1094,9 @@ __global__ __launch_bounds__(kBlock) void numeric_hash_kernel(
                     }
                 }
             }
-        } else if (live) {
-            // One row per workgroup.  Every lane fetches one entry of A's row and the bounds of
-            // the B row it names into LDS (the compaction lists are free until the row is
-            // complete); the entries are then applied in order, the first G columns of kAhead
-            // B rows being requested before the first of them is added.
-            static_assert(G <= kWave || 2 * CSTRIDE * 4 >= G * (16 + (int)sizeof(T)), "staging area");
-            int64_t *s_bb = reinterpret_cast<int64_t *>(ck), *s_be = s_bb + G;
-            T *s_a = reinterpret_cast<T *>(s_be + G);
-            row = perm[idx];
-            const int64_t ab = A_indptr[row], ae = A_indptr[row + 1];
-            for (int64_t a0 = ab; a0 < ae; a0 += G) {
-                const int64_t my_ai = a0 + gl < ae ? a0 + gl : ab;
-                const int64_t my_j = A_indices[my_ai];
-                s_a[gl] = A_data[my_ai];
-                s_bb[gl] = B_indptr[my_j];
-                s_be[gl] = B_indptr[my_j + 1];
-                __syncthreads();
-                const int nb = (int)(ae - a0 < G ? ae - a0 : G);
-                for (int e0 = 0; e0 < nb; e0 += kAhead) {
-                    int32_t pk[kAhead];
-                    T pv[kAhead], as[kAhead];
-                    int64_t bbs[kAhead], bes[kAhead];
-#pragma unroll
-                    for (int u = 0; u < kAhead; ++u) {
-                        const int src = e0 + u < nb ? e0 + u : e0;
-                        bbs[u] = s_bb[src];
-                        bes[u] = s_be[src];
-                        as[u] = s_a[src];
-                        const int64_t kk = bbs[u] + gl;
-                        const bool ok = e0 + u < nb && kk < bes[u];
-                        pk[u] = ok ? (int32_t)B_indices[kk] : kEmpty;
-                        pv[u] = ok ? B_data[kk] : T(0);
-                    }
-#pragma unroll
-                    for (int u = 0; u < kAhead; ++u) {
-                        if (e0 + u >= nb) break;
-                        if (pk[u] != kEmpty) add(pk[u], as[u] * pv[u]);
-                        for (int64_t kk = bbs[u] + G + gl; kk < bes[u]; kk += G)
-                            add((int32_t)B_indices[kk], as[u] * B_data[kk]);
-                        __syncthreads();  // the next entry of A's row adds after this one
-                    }
-                }
-            }
         }
-        if (G > kWave) __syncthreads();
         // Output in ascending column order.
-        if constexpr (G > kWave) {
-            // One row per workgroup, up to TABLE / 2 entries: the occupied slots are compacted
-            // into a list of (column, slot) words, the list is padded to a power of two and
-            // sorted by a bitonic network in LDS, and the row is written out in order.  (Ranking
-            // every entry against the whole list, as the narrow groups do, grows with the square
-            // of the row and took most of this kernel's time on rows of thousands of entries.)
-            unsigned long long *list = reinterpret_cast<unsigned long long *>(ck);
-            int *scr = reinterpret_cast<int *>(cs);
-            int mine = 0;
-            for (int t = gl; t < TABLE; t += G) mine += tab[t] != kEmpty;
-            scr[gl] = mine;
-            __syncthreads();
-            int pos = 0, c = 0;
-            for (int l2 = 0; l2 < G; ++l2) {
-                const int v = scr[l2];
-                if (l2 < gl) pos += v;
-                c += v;
-            }
-            __syncthreads();
-            for (int t = gl; t < TABLE; t += G) {
-                const int32_t key = tab[t];
-                if (key != kEmpty) list[pos++] = ((unsigned long long)(uint32_t)key << 32) | (uint32_t)t;
-            }
-            int P = 2 * kWave;
-            while (P < c) P <<= 1;
-            for (int t = c + gl; t < P; t += G) list[t] = ~0ull;
-            __syncthreads();
-            for (int k = 2; k <= P; k <<= 1) {
-                for (int j = k >> 1; j > 0; j >>= 1) {
-                    for (int t = gl; t < P / 2; t += G) {
-                        const int i = ((t & ~(j - 1)) << 1) | (t & (j - 1)), l = i | j;
-                        const unsigned long long x = list[i], y = list[l];
-                        if ((x > y) == ((i & k) == 0)) { list[i] = y; list[l] = x; }
-                    }
-                    // a wavefront's pairs stay inside its own 128 words while j <= 64
-                    if (j > kWave) __syncthreads(); else group_sync<kWave>();
-                }
-                if (k >= 2 * kWave) __syncthreads();
-            }
-            if (live) {
-                const int64_t base = C_indptr[row];
-                for (int e = gl; e < c; e += G) {
-                    const unsigned long long w = list[e];
-                    C_indices[base + e] = (int64_t)(w >> 32);
-                    C_data[base + e] = val[(uint32_t)w];
-                }
-            }
-        } else {
+        {
             // The occupied slots are compacted into a dense list, then every entry is ranked
             // against that list only (its rank is its position in the row).  Rows fill at most
             // half of their table, so this is a fraction of the compares a rank over the whole
@@ -1145,6 +1147,237 @@ __global__ __launch_bounds__(kBlock) void numeric_hash_kernel(
         group_sync<G>();
     }
 }
+
+// ---- numeric, rows of more than 128 entries -------------------------------------------
+//
+// One row of C per workgroup.  The row's products are numbered in the order of A's row (and of
+// B's rows inside it) and dealt to the threads by number, so the lanes are busy whatever the
+// lengths of B's rows are; applied entry by entry of A's row, a row of B of eight entries kept
+// eight of 256 lanes busy behind a barrier and a memory round trip each.  A product finds or
+// claims its column's slot of the table in LDS; products of one chunk that meet in a slot take
+// turns in the order of their numbers (every round the lowest one in each slot adds), so an entry
+// of C still receives its products in the order of A's row, from +0.0.
+// The row is then ordered by counting its columns into buckets of equal width between its first
+// and last column and ranking each against its bucket, out of registers.
+// Bound by the row's chain of round trips and the barriers of the turns.  A 150 000-row power-law
+// graph squared (mean 8, rows up to 1000, fp32), by length of C's row, against groups of 64 and 256
+// lanes that applied A's entries one by one and ordered the row by ranks or a bitonic network:
+// 129-256 60 -> 33 us, 257-512 127 -> 39, 513-1024 136 -> 40, 1025-4096 806 -> 110, more (dense
+// accumulators in global memory) 854 -> 75.
+template <typename T_, int TPB_, int SLOTS_, int LIMIT_, int UNROLL_> struct RowShape {
+    using T = T_;
+    static constexpr int TPB = TPB_, SLOTS = SLOTS_, LIMIT = LIMIT_, UNROLL = UNROLL_;
+    static constexpr int BATCH = TPB < 512 ? TPB : 512;                      // entries of A's row at a time
+    static constexpr int TURNS = TPB < 1024 ? (TPB == kWave ? 512 : 1024) : 1024;   // turn words, by slot
+    static constexpr int BUCKETS = TPB == kWave ? 256 : SLOTS < 4096 ? 1024 : 4096;
+    static constexpr int PER = (SLOTS + TPB - 1) / TPB;                      // slots a thread reads out
+    static constexpr size_t at_off = sizeof(T) * SLOTS, at_row = at_off + 8 * (BATCH + 2), at_a = at_row + 8 * BATCH,
+                            at_key = at_a + sizeof(T) * BATCH, at_turn = at_key + 4 * SLOTS,
+                            end_sum = at_turn + 4 * TURNS;
+    static constexpr size_t at_count = sizeof(T) * LIMIT, at_list = at_count + 4 * (BUCKETS + 2),
+                            end_sort = at_list + 4 * LIMIT;
+    static constexpr size_t at_red = ((end_sum > end_sort ? end_sum : end_sort) + 15) / 16 * 16;
+    static constexpr size_t lds = at_red + 8 * (TPB / kWave) + 4 * 8;
+    static_assert(lds <= 160 * 1024, "a CU's LDS");
+    static_assert(LIMIT < SLOTS && (TURNS & (TURNS - 1)) == 0 && SLOTS % 2 == 0 && LIMIT % 2 == 0, "tables");
+};
+
+template <typename S>
+__global__ __launch_bounds__(S::TPB) void numeric_row_kernel(
+    int bin, const int32_t *__restrict__ bins, const int32_t *__restrict__ perm,
+    const typename S::T *__restrict__ A_data, const int64_t *__restrict__ A_indices,
+    const int64_t *__restrict__ A_indptr, const typename S::T *__restrict__ B_data,
+    const int64_t *__restrict__ B_indices, const int64_t *__restrict__ B_indptr,
+    const int64_t *__restrict__ C_indptr, int64_t *__restrict__ C_indices, typename S::T *__restrict__ C_data) {
+    using T = typename S::T;
+    constexpr int TPB = S::TPB, SLOTS = S::SLOTS, BATCH = S::BATCH, U = S::UNROLL, PER = S::PER;
+    extern __shared__ __align__(16) unsigned char s_raw[];
+    T *val = reinterpret_cast<T *>(s_raw);
+    int64_t *s_off = reinterpret_cast<int64_t *>(s_raw + S::at_off);   // number of an entry's first product
+    int64_t *s_row = reinterpret_cast<int64_t *>(s_raw + S::at_row);   // start of its row of B, less that number
+    T *s_a = reinterpret_cast<T *>(s_raw + S::at_a);
+    int32_t *tab = reinterpret_cast<int32_t *>(s_raw + S::at_key);
+    uint32_t *turn = reinterpret_cast<uint32_t *>(s_raw + S::at_turn);
+    int32_t *count = reinterpret_cast<int32_t *>(s_raw + S::at_count);
+    int32_t *list = reinterpret_cast<int32_t *>(s_raw + S::at_list);
+    int64_t *s_wave = reinterpret_cast<int64_t *>(s_raw + S::at_red);
+    int32_t *s_flag = reinterpret_cast<int32_t *>(s_raw + S::at_red + 8 * (TPB / kWave));   // [0, 3) more, [3] first, [4] last column
+    const int tid = threadIdx.x;
+    const int32_t b0 = bins[kBinStart + bin], b1 = bins[kBinStart + bin + 1];
+    for (int32_t idx = b0 + (int32_t)blockIdx.x; idx < b1; idx += (int32_t)gridDim.x) {
+        const int64_t row = perm[idx];
+        const int64_t ab = A_indptr[row], ae = A_indptr[row + 1];
+        for (int t = tid; t < SLOTS; t += TPB) {
+            tab[t] = kEmpty;
+            val[t] = T(0);
+        }
+        for (int t = tid; t < S::TURNS; t += TPB) turn[t] = 0;
+        if (tid < 3) s_flag[tid] = 0;
+        if (tid == 3) s_flag[3] = 0x7fffffff;
+        if (tid == 4) s_flag[4] = -1;
+        uint32_t round = 0;
+        int32_t first = 0x7fffffff, last = -1;
+        for (int64_t a0 = ab; a0 < ae; a0 += BATCH) {
+            const bool mine = tid < BATCH && a0 + tid < ae;
+            const int64_t j = mine ? A_indices[a0 + tid] : 0;
+            const T a = mine ? A_data[a0 + tid] : T(0);
+            const int64_t bb = mine ? B_indptr[j] : 0, be = mine ? B_indptr[j + 1] : 0;
+            int64_t total;
+            const int64_t off = row_scan<TPB, int64_t>(be - bb, s_wave, total);
+            __syncthreads();   // the last batch's products are done with the lists
+            if (tid < BATCH) {
+                s_off[tid] = off;   // (threads past the row's end: the total)
+                s_row[tid] = bb - off;
+                s_a[tid] = a;
+            }
+            __syncthreads();
+            for (int64_t p0 = 0; p0 < total; p0 += TPB * U) {
+                int32_t key[U];
+                T prod[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const int64_t p = p0 + u * TPB + tid;
+                    const bool have = p < total;
+                    const int64_t at = have ? p : 0;
+                    int e = 0;   // the last entry whose first product is not behind this one
+#pragma unroll
+                    for (int step = BATCH / 2; step > 0; step >>= 1)
+                        if (s_off[e + step] <= at) e += step;
+                    const int64_t kk = s_row[e] + at;
+                    key[u] = (int32_t)B_indices[kk];
+                    prod[u] = s_a[e] * B_data[kk];
+                    if (!have) key[u] = kEmpty;
+                }
+                int slot[U] = {};
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    if (key[u] == kEmpty) continue;
+                    first = min(first, key[u]);
+                    last = max(last, key[u]);
+                    uint32_t h = __umulhi((uint32_t)key[u] * 0x9E3779B1u, (uint32_t)SLOTS);
+                    int32_t old = atomicCAS(&tab[h], kEmpty, key[u]);
+                    while (old != kEmpty && old != key[u]) {
+                        h = h + 1 == SLOTS ? 0 : h + 1;
+                        old = atomicCAS(&tab[h], kEmpty, key[u]);
+                    }
+                    slot[u] = (int)h;
+                }
+                // Turns.  A word of `turn` holds the latest round it was asked for and, of the threads
+                // that asked, the lowest: a later round's words are larger than an earlier one's, so
+                // nothing is reset in between.  (Slots that share a word only wait for each other.)
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    if (p0 + u * TPB >= total) break;
+                    bool waits = key[u] != kEmpty;
+                    bool more;
+                    do {
+                        if (++round == (1u << 22)) {   // 10 bits below hold the thread
+                            __syncthreads();
+                            for (int t = tid; t < S::TURNS; t += TPB) turn[t] = 0;
+                            round = 1;
+                            __syncthreads();
+                        }
+                        const int now = round % 3, next = (round + 1) % 3;
+                        uint32_t *word = turn + (slot[u] & (S::TURNS - 1));
+                        const uint32_t asked = round << 10 | (uint32_t)(TPB - 1 - tid);
+                        if (waits) atomicMax(word, asked);
+                        if (TPB > kWave && tid == 0) s_flag[next] = 0;
+                        __syncthreads();
+                        if (waits && *word == asked) {
+                            val[slot[u]] += prod[u];
+                            waits = false;
+                        }
+                        if constexpr (TPB > kWave) {
+                            if (waits) s_flag[now] = 1;
+                            __syncthreads();
+                            more = s_flag[now] != 0;
+                        } else {
+                            more = __ballot(waits) != 0;
+                        }
+                    } while (more);
+                }
+            }
+        }
+        // ---- the row in ascending order of its columns ----
+        if (last >= 0) {
+            atomicMin(&s_flag[3], first);
+            atomicMax(&s_flag[4], last);
+        }
+        int32_t key[PER], rank[PER];
+        T sum[PER];
+#pragma unroll
+        for (int q = 0; q < PER; ++q) {
+            const int t = tid + q * TPB;
+            key[q] = t < SLOTS ? tab[t] : kEmpty;
+            sum[q] = t < SLOTS ? val[t] : T(0);
+        }
+        __syncthreads();   // the table's memory is free from here on
+        const int32_t low = s_flag[3];
+        const uint32_t width = s_flag[4] >= low ? (uint32_t)(s_flag[4] - low) : 0;
+        constexpr int BITS = __builtin_ctz(S::BUCKETS);
+        const int need = 32 - __clz(width | 1), shift = need > BITS ? need - BITS : 0;
+        for (int t = tid; t < S::BUCKETS; t += TPB) count[t] = 0;
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < PER; ++q)
+            rank[q] = key[q] != kEmpty ? atomicAdd(&count[(uint32_t)(key[q] - low) >> shift], 1) : 0;
+        __syncthreads();
+        {
+            constexpr int RUN = S::BUCKETS / TPB;
+            int c[RUN], mine = 0, all;
+#pragma unroll
+            for (int q = 0; q < RUN; ++q) {
+                c[q] = count[tid * RUN + q];
+                mine += c[q];
+            }
+            int run = row_scan<TPB, int>(mine, reinterpret_cast<int *>(s_wave), all);
+#pragma unroll
+            for (int q = 0; q < RUN; ++q) {
+                count[tid * RUN + q] = run;
+                run += c[q];
+            }
+            if (tid == 0) count[S::BUCKETS] = all;
+        }
+        __syncthreads();
+        const int n = count[S::BUCKETS];
+#pragma unroll
+        for (int q = 0; q < PER; ++q)
+            if (key[q] != kEmpty) list[count[(uint32_t)(key[q] - low) >> shift] + rank[q]] = key[q];
+        __syncthreads();
+        int32_t *sorted = reinterpret_cast<int32_t *>(s_raw);
+#pragma unroll
+        for (int q = 0; q < PER; ++q) {
+            if (key[q] == kEmpty) continue;
+            const uint32_t b = (uint32_t)(key[q] - low) >> shift;
+            const int lo = count[b], hi = count[b + 1];
+            int r = lo;
+            for (int t = lo; t < hi; ++t) r += list[t] < key[q];
+            rank[q] = r;
+            sorted[r] = key[q];
+        }
+        __syncthreads();
+        const int64_t base = C_indptr[row];
+        for (int t = tid; t < n; t += TPB) C_indices[base + t] = (int64_t)sorted[t];
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < PER; ++q)
+            if (key[q] != kEmpty) val[rank[q]] = sum[q];
+        __syncthreads();
+        for (int t = tid; t < n; t += TPB) C_data[base + t] = val[t];
+        __syncthreads();
+    }
+}
+
+// The shapes: LDS decides how many rows a CU has in flight, so a row gets the smallest table that
+// holds its bin at three quarters load; the last one takes the LDS of a whole CU.
+template <typename T> using RowShape3 = RowShape<T, 64, 384, 256, 2>;
+template <typename T> using RowShape4 = RowShape<T, 64, 704, 512, 2>;
+template <typename T> using RowShape5 = RowShape<T, 256, 1408, 1024, 2>;
+template <typename T> using RowShape6 = RowShape<T, 512, 2816, 2048, 4>;
+template <typename T> using RowShape7 = RowShape<T, 1024, 5632, 4096, 4>;
+constexpr int32_t kRowLimitMost32 = 16384, kRowLimitMost64 = 10880;
+template <typename T>
+using RowShape8 = RowShape<T, 1024, sizeof(T) == 4 ? 18176 : 12224, sizeof(T) == 4 ? kRowLimitMost32 : kRowLimitMost64, 4>;
 
 // Spill path: dense accumulator slice per workgroup, emitted by a scan of the
 // touched column range (ascending by construction).
@@ -1501,12 +1734,8 @@ int launch_numeric(const Work &w, int64_t B_cols, const void *A_data, const int6
     auto hashed = [&](auto group, auto table, int bin, unsigned grid) -> int {
         constexpr int G = decltype(group)::value, TABLE = decltype(table)::value;
         auto k = numeric_hash_kernel<T, G, TABLE>;
-        // tables (values + keys), padded apart when groups share a workgroup, and the two compaction lists
-        // (narrow groups keep the lists where the key table was)
-        const size_t lds = (kBlock / G) * (per * (TABLE + (G < kBlock ? kTablePad : 0)) + (G > kWave ? 4 * (TABLE + 8) : 0));
-        if (lds > 64 * 1024)
-            NM_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(k),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        const size_t lds = (kBlock / G) * per * (TABLE + kTablePad);   // tables (values + keys), padded apart
+        static_assert((kBlock / G) * per * (TABLE + kTablePad) <= 64 * 1024, "no attribute asked for");
         hipLaunchKernelGGL(k, dim3(grid), dim3(kBlock), lds, s, bin, w.bins, w.perm, Ad, A_indices, A_indptr, Bd,
                            B_indices, B_indptr, C_indptr, C_indices, Cd);
         NM_LAUNCH_CHECK("numeric_hash_kernel");
@@ -1516,10 +1745,23 @@ int launch_numeric(const Work &w, int64_t B_cols, const void *A_data, const int6
     if (int rc = hashed(integral_constant<int, kGroup0>{}, integral_constant<int, kNumTable0>{}, 0, kPersistGrid)) return rc;
     if (int rc = hashed(integral_constant<int, kGroup1>{}, integral_constant<int, kNumTable1>{}, 1, kPersistGrid)) return rc;
     if (int rc = hashed(integral_constant<int, kGroup2>{}, integral_constant<int, kNumTable2>{}, 2, kPersistGrid)) return rc;
-    if (int rc = hashed(integral_constant<int, kGroup3>{}, integral_constant<int, kNumTable3>{}, 3, kPersistGrid)) return rc;
-    if (int rc = hashed(integral_constant<int, kGroup4>{}, integral_constant<int, kNumTable4>{}, 4, kPersistGrid)) return rc;
-    if (int rc = hashed(integral_constant<int, kGroup5>{}, integral_constant<int, kNumTable5>{}, 5, kPersistGrid)) return rc;
-    if (int rc = hashed(integral_constant<int, kGroup6>{}, integral_constant<int, kNumTable6>{}, 6, 1024)) return rc;
+    auto rows = [&](auto shape, int bin, unsigned grid) -> int {
+        using S = decltype(shape);
+        auto k = numeric_row_kernel<S>;
+        if (S::lds > 64 * 1024)
+            NM_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(k),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::lds));
+        hipLaunchKernelGGL(k, dim3(grid), dim3(S::TPB), S::lds, s, bin, w.bins, w.perm, Ad, A_indices, A_indptr, Bd,
+                           B_indices, B_indptr, C_indptr, C_indices, Cd);
+        NM_LAUNCH_CHECK("numeric_row_kernel");
+        return NM_OK;
+    };
+    if (int rc = rows(RowShape3<T>{}, 3, 2 * kPersistGrid)) return rc;
+    if (int rc = rows(RowShape4<T>{}, 4, 2 * kPersistGrid)) return rc;
+    if (int rc = rows(RowShape5<T>{}, 5, kPersistGrid)) return rc;
+    if (int rc = rows(RowShape6<T>{}, 6, 2048)) return rc;
+    if (int rc = rows(RowShape7<T>{}, 7, 1024)) return rc;
+    if (int rc = rows(RowShape8<T>{}, 8, 512)) return rc;
     hipLaunchKernelGGL(numeric_spill_kernel<T>, dim3(spill_groups(B_cols)), dim3(kSpillBlock), 0, s, w.bins, w.perm,
                        B_cols, Ad, A_indices, A_indptr, Bd, B_indices, B_indptr, C_indptr, C_indices, Cd, w.mark,
                        w.acc);
@@ -1613,15 +1855,24 @@ int symbolic_phase(int64_t A_rows, int64_t A_cols, int64_t B_cols, const int64_t
                        w.perm, A_indices, A_indptr, B_indices, B_indptr, w.count);
     hipLaunchKernelGGL((symbolic_hash_kernel<kGroup2, kSymTable2>), dim3(kPersistGrid), dim3(kBlock), 0, s, 2, w.bins,
                        w.perm, A_indices, A_indptr, B_indices, B_indptr, w.count);
-    hipLaunchKernelGGL((symbolic_hash_kernel<kGroup3, kSymTable3>), dim3(kPersistGrid), dim3(kBlock), 0, s, 3, w.bins,
-                       w.perm, A_indices, A_indptr, B_indices, B_indptr, w.count);
-    hipLaunchKernelGGL((symbolic_hash_kernel<kGroup4, kSymTable4>), dim3(kPersistGrid), dim3(kBlock), 0, s, 4, w.bins,
-                       w.perm, A_indices, A_indptr, B_indices, B_indptr, w.count);
-    hipLaunchKernelGGL((symbolic_hash_kernel<kGroup5, kSymTable5>), dim3(kPersistGrid), dim3(kBlock), 0, s, 5, w.bins,
-                       w.perm, A_indices, A_indptr, B_indices, B_indptr, w.count);
-    hipLaunchKernelGGL((symbolic_hash_kernel<kGroup6, kSymTable6>), dim3(1024), dim3(kBlock), 0, s, 6, w.bins, w.perm,
-                       A_indices, A_indptr, B_indices, B_indptr, w.count);
     NM_LAUNCH_CHECK("symbolic_hash_kernel");
+    auto sets = [&](auto shape, int bin, unsigned grid) -> int {
+        using S = decltype(shape);
+        auto k = symbolic_row_kernel<S>;
+        if (S::lds > 64 * 1024)
+            NM_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(k),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::lds));
+        hipLaunchKernelGGL(k, dim3(grid), dim3(S::TPB), S::lds, s, bin, w.bins, w.perm, A_indices, A_indptr,
+                           B_indices, B_indptr, w.count);
+        NM_LAUNCH_CHECK("symbolic_row_kernel");
+        return NM_OK;
+    };
+    if (int rc = sets(SetShape3{}, 3, 2 * kPersistGrid)) return rc;
+    if (int rc = sets(SetShape4{}, 4, 2 * kPersistGrid)) return rc;
+    if (int rc = sets(SetShape5{}, 5, kPersistGrid)) return rc;
+    if (int rc = sets(SetShape6{}, 6, 1024)) return rc;
+    if (int rc = sets(SetShape7{}, 7, 512)) return rc;
+    // (bins 7 and 8 share a limit: nothing is in bin 8)
     hipLaunchKernelGGL(symbolic_spill_kernel, dim3(spill_groups(B_cols)), dim3(kSpillBlock), 0, s, w.bins, w.perm, B_cols,
                        A_indices, A_indptr, B_indices, B_indptr, w.mark, w.count);
     NM_LAUNCH_CHECK("symbolic_spill_kernel");
@@ -1724,7 +1975,10 @@ extern "C" int nm_spgemm_numeric(nm_dtype dt, int64_t A_rows, int64_t A_cols, in
     if (hashed) {
         hipLaunchKernelGGL(row_length_kernel, dim3((unsigned)grid), dim3(kBlock), 0, s, A_rows, C_indptr, w.key);
         NM_LAUNCH_CHECK("row_length_kernel");
-        if (int rc = bin_rows(A_rows, kNumLimit, w, s)) return rc;
+        int32_t limit[kBins - 1];
+        for (int q = 0; q < kBins - 2; ++q) limit[q] = kNumLimit[q];
+        limit[kBins - 2] = dt == NM_F32 ? kRowLimitMost32 : kRowLimitMost64;
+        if (int rc = bin_rows(A_rows, limit, w, s)) return rc;
     }
     const int64_t nbatch = nm::xcd_padded(nm::ceil_div(A_rows, kMergeRows));
     // (every row on the hash path: the merge kernel would look at each row's key and leave)

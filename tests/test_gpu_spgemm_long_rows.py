@@ -1,0 +1,92 @@
+"""Products whose rows leave the narrow hash tables: lengths on both sides of every table's limit,
+columns in which many products meet, rows of B from empty to thousands of entries, columns packed
+together and far apart.  Sums keep the order of A's row, so everything is compared bit for bit
+against the serial loop, except rows longer than any table (added with atomics) and the gradient
+of B (atomics): a sum of m products in any order is off by at most m * eps * sum |products|, and the
+parity bound of the suite is above that for the lengths here."""
+import numpy as np
+import pytest
+
+import oracle
+from numml_amd import generators as G
+from numml_amd import numml_torch_cpp as ext
+from util import assert_close, assert_same, host, randn, to_dev
+
+pytestmark = pytest.mark.gpu
+DTYPES = [np.float32, np.float64]
+
+
+def _csr(rows, cols, seed, dtype):
+    indptr = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int64)
+    indices = np.concatenate([np.asarray(r, np.int64) for r in rows] + [np.zeros(0, np.int64)])
+    return randn(seed, indices.size, dtype), indices, indptr, (len(rows), cols)
+
+
+def _lengths(lengths, spread, hub, dtype):
+    """Row i of C has lengths[i] entries: B's row k holds column (k + 1) * spread and, with `hub`,
+    column 0 in every third row, so that many products of a row meet there."""
+    K = max(lengths)
+    B = [([0] if hub and k % 3 == 0 else []) + [(k + 1) * spread] for k in range(K)]
+    rng = np.random.default_rng(len(lengths) + spread)
+    A = [np.sort(rng.choice(K, n - 1, replace=False)) if hub else np.arange(n) for n in lengths]
+    return _csr(A, K, 1, dtype), _csr(B, (K + 1) * spread, 2, dtype)
+
+
+def _blocks(dtype):
+    """B's rows are runs of 0, 1, 300 and 5000 columns that overlap; columns packed in one corner
+    with a single one far away."""
+    cols = 3_000_000
+    B = []
+    for k in range(400):
+        n = (0, 1, 300, 7)[k % 4] if k != 203 else 5000
+        B.append(np.arange(k * 11, k * 11 + n))
+    B[5] = np.concatenate([B[5], [cols - 1]])
+    rng = np.random.default_rng(3)
+    A = [np.arange(400), np.arange(0, 400, 2), np.arange(2, 400, 4), np.arange(0, 400, 4), np.arange(5, 60),
+         np.sort(rng.choice(400, 130, replace=False)), [203], []]
+    return _csr(A, 400, 4, dtype), _csr(B, cols, 5, dtype)
+
+
+def _check(dev, a, b, dtype, exact=True):
+    (ad, ai, ap, (ar, ac)), (bd, bi, bp, (br, bc)) = a, b
+    Cd_ref, Ci_ref, Cp_ref = oracle.spgemm_forward(ar, ac, ad, ai, ap, br, bc, bd, bi, bp)
+    gC = randn(9, Cd_ref.shape[0], dtype)
+    gA_ref, gB_ref = oracle.spgemm_backward(gC, Ci_ref, Cp_ref, ar, ac, ad, ai, ap, br, bc, bd, bi, bp)
+    AD, AI, AP, BD, BI, BP, GC = to_dev(dev, ad, ai, ap, bd, bi, bp, gC)
+    Cd, Ci, Cp = ext.spgemm_forward(ar, ac, AD, AI, AP, br, bc, BD, BI, BP)
+    assert_same(host(Cp), Cp_ref, "C_indptr")
+    assert_same(host(Ci), Ci_ref, "C_indices")
+    (assert_same if exact else assert_close)(host(Cd), Cd_ref, "C_data")
+    for mode in ("planned", "atomic"):
+        old_mode, ext.BACKWARD_MODE = ext.BACKWARD_MODE, mode
+        try:
+            gA, gB = ext.spgemm_backward(GC, Ci, Cp, ar, ac, AD, AI, AP, br, bc, BD, BI, BP)
+        finally:
+            ext.BACKWARD_MODE = old_mode
+        assert_same(host(gA), gA_ref, f"grad_A ({mode})")
+        assert_close(host(gB), gB_ref, f"grad_B ({mode})")
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("hub", [False, True])
+@pytest.mark.parametrize("spread", [1, 37])
+def test_rows_at_the_limits_of_the_tables(dev, dtype, hub, spread):
+    lengths = [n + d for n in (64, 128, 256, 512, 1024, 2048, 4096) for d in (0, 1)]
+    _check(dev, *_lengths(lengths + lengths[::-1], spread, hub, dtype), dtype)
+
+
+@pytest.mark.parametrize("dtype,most", [(np.float32, 16384), (np.float64, 10880)])
+def test_rows_at_the_limit_of_a_compute_unit(dev, dtype, most):
+    _check(dev, *_lengths([most, most - 1, 8192], 3, False, dtype), dtype)
+    _check(dev, *_lengths([most + 1, 5000], 3, False, dtype), dtype, exact=False)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_rows_of_runs_and_of_packed_columns(dev, dtype):
+    _check(dev, *_blocks(dtype), dtype)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_two_hop_graph(dev, dtype):
+    a = G.powerlaw(6000, 6000, 60000, max_deg=1500, seed=7, dtype=dtype)
+    _check(dev, a, a, dtype)
