@@ -1467,22 +1467,18 @@ __global__ __launch_bounds__(kSpillBlock) void numeric_spill_kernel(
 // gC[i,c] * B[k,c] are then added lane by lane in ascending column order --
 // the order of the reference's merge -- which keeps grad_A bit-identical.
 //
-// Rows of C longer than kBwdStage go to a second kernel in which a whole
-// workgroup owns the row: its 32 groups share out the entries of A's row, whole
-// wavefronts take the entries whose row of B is long, and the row of C is staged
-// in LDS -- columns and gradient up to kBwdLongCap entries; columns only beyond
-// that (every stride-th column past kBwdHugeCap entries: the last steps of the
-// search then read global memory).
-// Left to one group of eight lanes, a row with thousands of products and a
-// global-memory search per product set the time of the whole launch.
+// Rows of C longer than kBwdStage get a workgroup each, of 64, 256 or 1024 threads by length.  The
+// row's products are numbered through in the order of A's row and dealt to the threads by number
+// (as in numeric_row_kernel), each looks its column up in the row of C in LDS, and the thread of an
+// entry of A adds the entry's products from LDS in order.  Of a row longer than LDS holds, every
+// stride-th column is staged: the last steps of the search then read global memory.
+// Bound by the row's chain of round trips, the searches in LDS and the atomic adds of the gradient of B.  A
+// 150 000-row power-law graph squared (mean 8, rows up to 1000, fp32), by length of C's row, against
+// one workgroup of 256 threads whose groups of eight lanes took A's entries one by one: 65-2048 617 -> 224 us
+// (65-512 107, 513-2048 117), more 679 -> 261 (2049-4096 73, above 188).
 constexpr int kBwdG = 8;
 constexpr int kBwdStage = 64;
-constexpr int kBwdLong = kBwdStage;
-constexpr int kBwdLongCap = 2048;     // rows up to this long: columns and gradient in LDS
-constexpr int kBwdHugeCap = 14336;    // longer rows: columns only
 constexpr int kBwdLongChunk = 256;   // rows a workgroup of the long-row kernel looks through at a time, at most
-constexpr int kBwdWide = 64;         // rows of B longer than this are walked by a whole wavefront ...
-constexpr int kBwdWideCap = 1024;    // ... up to this many per row of A (the rest stay with their group)
 
 // What lane E of every eight consecutive lanes holds, handed to all eight (ds_swizzle in bit mode:
 // lane = (lane & 0x18) | E inside each half of the wavefront; no address to compute).
@@ -1585,129 +1581,159 @@ __global__ __launch_bounds__(kBlock) void spgemm_bwd_kernel(
     }
 }
 
-template <typename T, int CAP, bool STAGE_G>
-__global__ __launch_bounds__(kBlock) void spgemm_bwd_long_kernel(
-    int64_t A_rows, int chunk, int64_t longer_than, int64_t up_to, const T *__restrict__ gC, const int64_t *__restrict__ C_indices,
-    const int64_t *__restrict__ C_indptr, const T *__restrict__ A_data,
-    const int64_t *__restrict__ A_indices, const int64_t *__restrict__ A_indptr,
-    const T *__restrict__ B_data, const int64_t *__restrict__ B_indices,
-    const int64_t *__restrict__ B_indptr, T *__restrict__ grad_A, T *__restrict__ grad_B) {
-    constexpr int G = kBwdG, GROUPS = kBlock / G;
-    __shared__ T cg[STAGE_G ? CAP : 1];
-    __shared__ int32_t ci[CAP];
-    __shared__ int s_long[kBwdLongChunk];
-    __shared__ int s_wide[kBwdWideCap];
-    __shared__ int s_n, s_nw;
-    const int gl = threadIdx.x % G, gi = threadIdx.x / G;
-    const int gbase = (threadIdx.x & (kWave - 1)) & ~(G - 1);
-    const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+template <typename T_, int TPB_, int CAP_, int UNROLL_> struct BackShape {
+    using T = T_;
+    static constexpr int TPB = TPB_, CAP = CAP_, UNROLL = UNROLL_, BATCH = TPB < 512 ? TPB : 512;
+    static constexpr int STEP = TPB * UNROLL;                                  // products at a time
+    static constexpr size_t at_prod = sizeof(T) * CAP, at_off = at_prod + sizeof(T) * STEP,
+                            at_row = at_off + 8 * (BATCH + 2), at_a = at_row + 8 * BATCH,
+                            at_wave = at_a + 8 * BATCH, at_col = at_wave + 8 * (TPB / kWave) + 16,
+                            at_long = at_col + 4 * CAP;
+    static constexpr size_t lds = at_long + 4 * (kBwdLongChunk + 2);
+    static_assert(lds <= 160 * 1024, "a CU's LDS");
+    static_assert((CAP * sizeof(T)) % 8 == 0 && (STEP * sizeof(T)) % 8 == 0, "64-bit words behind the values");
+};
+
+template <typename S>
+__global__ __launch_bounds__(S::TPB) void spgemm_bwd_long_kernel(
+    int64_t A_rows, int chunk, int64_t longer_than, int64_t up_to, const typename S::T *__restrict__ gC,
+    const int64_t *__restrict__ C_indices, const int64_t *__restrict__ C_indptr,
+    const typename S::T *__restrict__ A_data, const int64_t *__restrict__ A_indices,
+    const int64_t *__restrict__ A_indptr, const typename S::T *__restrict__ B_data,
+    const int64_t *__restrict__ B_indices, const int64_t *__restrict__ B_indptr,
+    typename S::T *__restrict__ grad_A, typename S::T *__restrict__ grad_B) {
+    using T = typename S::T;
+    constexpr int TPB = S::TPB, CAP = S::CAP, BATCH = S::BATCH, U = S::UNROLL, STEP = S::STEP;
+    extern __shared__ __align__(16) unsigned char s_raw[];
+    T *cg = reinterpret_cast<T *>(s_raw);
+    T *s_prod = reinterpret_cast<T *>(s_raw + S::at_prod);
+    int64_t *s_off = reinterpret_cast<int64_t *>(s_raw + S::at_off);   // number of an entry's first product
+    int64_t *s_row = reinterpret_cast<int64_t *>(s_raw + S::at_row);   // start of its row of B, less that number
+    T *s_a = reinterpret_cast<T *>(s_raw + S::at_a);
+    int64_t *s_wave = reinterpret_cast<int64_t *>(s_raw + S::at_wave);
+    int32_t *ci = reinterpret_cast<int32_t *>(s_raw + S::at_col);
+    int32_t *s_long = reinterpret_cast<int32_t *>(s_raw + S::at_long);
+    int32_t *s_n = s_long + kBwdLongChunk;
+    const int tid = threadIdx.x;
     for (int64_t r0 = (int64_t)blockIdx.x * chunk; r0 < A_rows; r0 += (int64_t)gridDim.x * chunk) {
         // the long rows among this chunk of rows (mostly there are none)
-        const int64_t r = r0 + threadIdx.x;
-        bool is_long = false;
-        if ((int)threadIdx.x < chunk && r < A_rows) {
+        if (tid == 0) *s_n = 0;
+        __syncthreads();
+        for (int t = tid; t < chunk; t += TPB) {
+            const int64_t r = r0 + t;
+            if (r >= A_rows) continue;
             const int64_t len = C_indptr[r + 1] - C_indptr[r];
-            is_long = len > longer_than && len <= up_to;
+            if (len > longer_than && len <= up_to) s_long[atomicAdd(s_n, 1)] = t;
         }
-        if (!__syncthreads_or(is_long)) continue;
-        if (threadIdx.x == 0) s_n = 0;
         __syncthreads();
-        if (is_long) s_long[atomicAdd(&s_n, 1)] = threadIdx.x;
-        __syncthreads();
-        const int n = s_n;
+        const int n = *s_n;
         for (int q = 0; q < n; ++q) {
             const int64_t i = r0 + s_long[q];
-            const int64_t cb = C_indptr[i], ce = C_indptr[i + 1], clen = ce - cb;
+            const int64_t cb = C_indptr[i], clen = C_indptr[i + 1] - cb;
             const int64_t stride = (clen + CAP - 1) / CAP;
             const int ns = (int)((clen + stride - 1) / stride);
             const bool whole = stride == 1;
-            for (int t = threadIdx.x; t < ns; t += kBlock) {
+            for (int t = tid; t < ns; t += TPB) {
                 ci[t] = (int32_t)C_indices[cb + t * stride];
-                if (STAGE_G) cg[t] = gC[cb + t];   // STAGE_G kernels only get rows of at most CAP entries
+                if (whole) cg[t] = gC[cb + t];
             }
-            if (threadIdx.x == 0) s_nw = 0;
-            __syncthreads();
-            // One entry (i,k) of A: W lanes (lane wl of them, the first being lane wbase of the
-            // wavefront) walk row k of B; returns sum_c gC[i,c] * B[k,c] added in ascending c.
-            auto entry = [&](auto width, int wl, int wbase, int64_t bb, int64_t be, T a) -> T {
-                constexpr int W = decltype(width)::value;
-                T acc = 0;
-                for (int64_t kk0 = bb; kk0 < be; kk0 += W) {
-                    const int64_t kk = kk0 + wl;
-                    const bool have = kk < be;
-                    const int64_t c = have ? B_indices[kk] : -1;
-                    const T bval = have ? B_data[kk] : T(0);
-                    int l = 0, h = ns;
-                    while (l < h) {
-                        const int mid = (l + h) >> 1;
-                        if ((int64_t)ci[mid] < c) l = mid + 1; else h = mid;
-                    }
-                    bool hit;
-                    T g = 0;
-                    if (whole) {
-                        hit = have && l < ns && (int64_t)ci[l] == c;
-                        if (hit) g = STAGE_G ? cg[l] : gC[cb + l];
-                    } else {
-                        // sample l is the first one not below c: the column, if present, sits
-                        // after sample l - 1 and no later than sample l
-                        int64_t lo = l == 0 ? 0 : (int64_t)(l - 1) * stride + 1;
-                        int64_t hi = (int64_t)l * stride < clen ? (int64_t)l * stride : clen;
-                        if (!have) hi = lo;
-                        while (lo < hi) {
-                            const int64_t mid = (lo + hi) >> 1;
-                            if (C_indices[cb + mid] < c) lo = mid + 1; else hi = mid;
-                        }
-                        hit = have && lo < clen && C_indices[cb + lo] == c;
-                        if (hit) g = gC[cb + lo];
-                    }
-                    if (hit && grad_B) nm::atomic_add(grad_B + kk, a * g);
-                    const T prod = hit ? g * bval : T(0);
-                    // ordered sum over the lanes = ascending column
-                    const int cnt = (int)(be - kk0 < W ? be - kk0 : W);
-                    for (int l2 = 0; l2 < cnt; ++l2) {
-                        const T pl = __shfl(prod, wbase + l2, kWave);
-                        const int hl = __shfl((int)hit, wbase + l2, kWave);
-                        if (hl) acc += pl;
-                    }
-                }
-                return acc;
-            };
+            const int top = 1 << (31 - __clz(ns));   // the first step of a search through ns columns
             const int64_t ab = A_indptr[i], ae = A_indptr[i + 1];
-            // entries of A's row per group and pass: as few as keeps all groups busy
-            const int64_t even = (ae - ab + GROUPS - 1) / GROUPS;
-            const int per = (int)(even < 1 ? 1 : (even > G ? G : even));
-            for (int64_t a0 = ab + gi * per; a0 < ae; a0 += GROUPS * per) {
-                const int64_t my_ai = a0 + gl;
-                const bool mine = gl < per && my_ai < ae;
-                const int64_t my_k = mine ? A_indices[my_ai] : 0;
-                const T my_a = (mine && grad_B) ? A_data[my_ai] : T(0);
-                const int64_t my_bb = mine ? B_indptr[my_k] : 0, my_be = mine ? B_indptr[my_k + 1] : 0;
-                // entries whose row of B is long are set aside for a whole wavefront
-                bool later = false;
-                if (mine && my_be - my_bb > kBwdWide) {
-                    const int slot = atomicAdd(&s_nw, 1);
-                    later = slot < kBwdWideCap;
-                    if (later) s_wide[slot] = (int)(my_ai - ab);
+            for (int64_t a0 = ab; a0 < ae; a0 += BATCH) {
+                const bool mine = tid < BATCH && a0 + tid < ae;
+                const int64_t j = mine ? A_indices[a0 + tid] : 0;
+                const T a = mine && grad_B ? A_data[a0 + tid] : T(0);
+                const int64_t bb = mine ? B_indptr[j] : 0, be = mine ? B_indptr[j + 1] : 0;
+                int64_t total;
+                const int64_t off = row_scan<TPB, int64_t>(be - bb, s_wave, total), end = off + (be - bb);
+                if (tid < BATCH) {
+                    s_off[tid] = off;   // (threads past the row's end: the total)
+                    s_row[tid] = bb - off;
+                    s_a[tid] = a;
                 }
-                const int nb = (int)(ae - a0 < per ? ae - a0 : per);
-                T my_acc = 0;
-                for (int e = 0; e < nb; ++e) {
-                    if (__shfl((int)later, gbase + e, kWave)) continue;
-                    const int64_t bb = __shfl(my_bb, gbase + e, kWave), be = __shfl(my_be, gbase + e, kWave);
-                    const T a = __shfl(my_a, gbase + e, kWave);
-                    const T acc = entry(std::integral_constant<int, G>{}, gl, gbase, bb, be, a);
-                    if (gl == e) my_acc = acc;
+                __syncthreads();
+                T acc = 0;
+                for (int64_t p0 = 0; p0 < total; p0 += STEP) {
+                    int64_t kk[U], c[U];
+                    T b[U], av[U];
+                    int l[U];
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        const int64_t p = p0 + u * TPB + tid;
+                        const bool have = p < total;
+                        const int64_t at = have ? p : 0;
+                        int e = 0;   // the last entry whose first product is not behind this one
+#pragma unroll
+                        for (int step = BATCH / 2; step > 0; step >>= 1)
+                            if (s_off[e + step] <= at) e += step;
+                        kk[u] = s_row[e] + at;
+                        av[u] = s_a[e];
+                        c[u] = B_indices[kk[u]];
+                        b[u] = grad_A ? B_data[kk[u]] : T(0);
+                        if (!have) c[u] = -1;
+                        l[u] = 0;
+                    }
+                    // the number of staged columns below c
+                    for (int step = top; step > 0; step >>= 1)
+#pragma unroll
+                        for (int u = 0; u < U; ++u)
+                            if (l[u] + step <= ns && (int64_t)ci[l[u] + step - 1] < c[u]) l[u] += step;
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        bool hit;
+                        T g = 0;
+                        if (whole) {
+                            hit = l[u] < ns && (int64_t)ci[l[u]] == c[u];
+                            if (hit) g = cg[l[u]];
+                        } else {
+                            // sample l is the first one not below c: the column, if present, sits
+                            // after sample l - 1 and no later than sample l
+                            int64_t lo = l[u] == 0 ? 0 : (int64_t)(l[u] - 1) * stride + 1;
+                            int64_t hi = (int64_t)l[u] * stride < clen ? (int64_t)l[u] * stride : clen;
+                            if (c[u] < 0) hi = lo;
+                            while (lo < hi) {
+                                const int64_t mid = (lo + hi) >> 1;
+                                if (C_indices[cb + mid] < c[u]) lo = mid + 1; else hi = mid;
+                            }
+                            hit = c[u] >= 0 && lo < clen && C_indices[cb + lo] == c[u];
+                            if (hit) g = gC[cb + lo];
+                        }
+                        if (hit && grad_B) nm::atomic_add(grad_B + kk[u], av[u] * g);
+                        s_prod[u * TPB + tid] = hit ? g * b[u] : T(0);
+                    }
+                    if (!grad_A) continue;
+                    __syncthreads();
+                    // an entry's thread adds its products in ascending column (a product that is missing
+                    // is +0.0, which changes no sum that began at +0.0)
+                    if (off < p0 + STEP && end > p0) {
+                        int t = off > p0 ? (int)(off - p0) : 0;
+                        const int t1 = end - p0 < STEP ? (int)(end - p0) : STEP;
+                        // (eight are on their way while eight are added: one after the other, a row of B of
+                        // a thousand entries was a thousand trips to LDS)
+                        constexpr int W = 8;
+                        if (t + W <= t1) {
+                            T x[W];
+#pragma unroll
+                            for (int w = 0; w < W; ++w) x[w] = s_prod[t + w];
+                            for (t += W; t + W <= t1; t += W) {
+                                T y[W];
+#pragma unroll
+                                for (int w = 0; w < W; ++w) y[w] = s_prod[t + w];
+#pragma unroll
+                                for (int w = 0; w < W; ++w) {
+                                    acc += x[w];
+                                    x[w] = y[w];
+                                }
+                            }
+#pragma unroll
+                            for (int w = 0; w < W; ++w) acc += x[w];
+                        }
+                        for (; t < t1; ++t) acc += s_prod[t];
+                    }
+                    __syncthreads();
                 }
-                if (mine && !later && grad_A) grad_A[my_ai] = my_acc;
-            }
-            __syncthreads();
-            const int nw = s_nw < kBwdWideCap ? s_nw : kBwdWideCap;
-            for (int d = wave; d < nw; d += kBlock / kWave) {
-                const int64_t ai = ab + s_wide[d];
-                const int64_t k = A_indices[ai];
-                const T a = grad_B ? A_data[ai] : T(0);
-                const T acc = entry(std::integral_constant<int, kWave>{}, lane, 0, B_indptr[k], B_indptr[k + 1], a);
-                if (lane == 0 && grad_A) grad_A[ai] = acc;
+                if (mine && grad_A) grad_A[a0 + tid] = acc;
+                __syncthreads();   // (the lists are this batch's until here)
             }
             __syncthreads();
         }
@@ -2049,27 +2075,37 @@ extern "C" int nm_spgemm_backward(nm_dtype dt, int64_t A_rows, int64_t A_nnz, in
                            (const double *)B_data, B_indices, B_indptr, (double *)grad_A, (double *)grad_B);
     NM_LAUNCH_CHECK("spgemm_bwd_kernel");
     // A workgroup works off the long rows of its chunk one after the other, so a chunk is sized
-    // for at least ~4096 of them over the matrix (8 rows or more; 256 at the sizes where the pass
-    // over the row lengths is itself worth keeping short).
-    int chunk = kBwdLongChunk;
-    while (chunk > 8 && A_rows / chunk < 4096) chunk /= 2;
-    grid = nm::ceil_div(A_rows, chunk);
-    if (grid > 4096) grid = 4096;
-    const int64_t none = INT64_MAX;
-#define NM_BWD_LONG(T)                                                                                          \
-    do {                                                                                                        \
-        hipLaunchKernelGGL((spgemm_bwd_long_kernel<T, kBwdLongCap, true>), dim3((unsigned)grid), dim3(kBlock),  \
-                           0, s, A_rows, chunk, (int64_t)kBwdLong, (int64_t)kBwdLongCap, (const T *)gC, C_indices,\
-                           C_indptr, (const T *)A_data, A_indices, A_indptr, (const T *)B_data, B_indices,      \
-                           B_indptr, (T *)grad_A, (T *)grad_B);                                                 \
-        hipLaunchKernelGGL((spgemm_bwd_long_kernel<T, kBwdHugeCap, false>), dim3((unsigned)grid), dim3(kBlock), \
-                           0, s, A_rows, chunk, (int64_t)kBwdLongCap, none, (const T *)gC, C_indices, C_indptr, \
-                           (const T *)A_data, A_indices, A_indptr, (const T *)B_data, B_indices, B_indptr,      \
-                           (T *)grad_A, (T *)grad_B);                                                           \
-    } while (0)
-    if (dt == NM_F32) NM_BWD_LONG(float);
-    else NM_BWD_LONG(double);
-#undef NM_BWD_LONG
-    NM_LAUNCH_CHECK("spgemm_bwd_long_kernel");
+    // for `groups` of them or more over the matrix: as many as spread the rows, and fewer where a workgroup
+    // takes a CU's LDS and those that find nothing pass through one at a time (half as many of the
+    // largest: 196 against 188 us).  The limits between the shapes follow from LDS: 512 columns with
+    // their gradients leave room for 10 to 14 rows in a CU, 4096 for two; (2049-4096 and the rest in one shape:
+    // 256 us, in two 73 + 188).
+    auto longer = [&](auto shape, int groups, int64_t longer_than, int64_t up_to) -> int {
+        using S = decltype(shape);
+        using T = typename S::T;
+        int chunk = kBwdLongChunk;
+        while (chunk > 4 && A_rows / chunk < groups) chunk /= 2;
+        int64_t most = nm::ceil_div(A_rows, chunk);
+        if (most > 2 * groups) most = 2 * groups;
+        auto k = spgemm_bwd_long_kernel<S>;
+        if (S::lds > 64 * 1024)
+            NM_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(k),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::lds));
+        hipLaunchKernelGGL(k, dim3((unsigned)most), dim3(S::TPB), S::lds, s, A_rows, chunk, longer_than, up_to,
+                           (const T *)gC, C_indices, C_indptr, (const T *)A_data, A_indices, A_indptr,
+                           (const T *)B_data, B_indices, B_indptr, (T *)grad_A, (T *)grad_B);
+        NM_LAUNCH_CHECK("spgemm_bwd_long_kernel");
+        return NM_OK;
+    };
+    auto all = [&](auto value, auto most) -> int {
+        using T = decltype(value);
+        if (int rc = longer(BackShape<T, 64, 512, 4>{}, 16384, kBwdStage, 512)) return rc;
+        if (int rc = longer(BackShape<T, 256, 2048, 4>{}, 4096, 512, 2048)) return rc;
+        if (int rc = longer(BackShape<T, 512, 4096, 4>{}, 4096, 2048, 4096)) return rc;
+        return longer(BackShape<T, 1024, decltype(most)::value, 4>{}, 2048, 4096, INT64_MAX);
+    };
+    if (int rc = dt == NM_F32 ? all(0.0f, std::integral_constant<int, 14336>{})
+                              : all(0.0, std::integral_constant<int, 8192>{}))
+        return rc;
     return NM_OK;
 }
