@@ -1662,27 +1662,46 @@ __global__ void chain_check_kernel(int32_t nlevels, int dirn, const int32_t *__r
 // Per call and launch, one lane per row of the chain: the part of the row's sum that does not
 // wait for the chain, the reciprocal of its diagonal, and its coefficients on the chain in
 // the layout the chain kernel streams (the wide layout is cleared before this runs).
+// Bound by the lane's round trips: eight dependencies are requested before the first is looked at,
+// and a workgroup is one wavefront, so that the rows of a short chain are spread over the chip (4096
+// rows of a band of 64: 52 - 66 us one by one in workgroups of four wavefronts, 17 - 37 us now).
+constexpr int kChainAhead = 8;
 template <bool BAND>
-__global__ void chain_prepare_kernel(ChainArgs c) {
+__global__ __launch_bounds__(64) void chain_prepare_kernel(ChainArgs c) {
     const int32_t t = (int32_t)(blockIdx.x * blockDim.x + threadIdx.x);
     if (t >= c.m) return;
     const int32_t q = chain_slot(c, t);
+    const double d = c.unit ? 1. : c.dg[q];
     double acc = 0., only = 0.;
-    for (int32_t at = c.dptr[q]; at < c.dptr[q + 1]; ++at) {
-        const int32_t ds = c.dslot[at];
-        const double v = c.coef[at];
-        if (ds < c.q0 || ds >= c.q1) {
-            acc += v * c.xs[ds];
-        } else if (BAND) {
-            const int32_t k = chain_pos(c, ds);
-            c.band[(size_t)(k + 1) * 64 + (t & 63)] = v;
-            atomicOr(c.has + k + 1, 1ull << (t & 63));
-        } else {
-            only = v;
+    const int32_t end = c.dptr[q + 1];
+    for (int32_t at0 = c.dptr[q]; at0 < end; at0 += kChainAhead) {
+        int32_t ds[kChainAhead];
+        double v[kChainAhead], x[kChainAhead];
+#pragma unroll
+        for (int u = 0; u < kChainAhead; ++u) {
+            const int32_t at = min(at0 + u, end - 1);
+            ds[u] = c.dslot[at];
+            v[u] = c.coef[at];
+        }
+        // (a solution inside the launch does not exist yet: the load is skipped, not its result)
+#pragma unroll
+        for (int u = 0; u < kChainAhead; ++u) x[u] = ds[u] < c.q0 || ds[u] >= c.q1 ? c.xs[ds[u]] : 0.;
+#pragma unroll
+        for (int u = 0; u < kChainAhead; ++u) {
+            if (at0 + u >= end) break;
+            if (ds[u] < c.q0 || ds[u] >= c.q1) {
+                acc += v[u] * x[u];
+            } else if (BAND) {
+                const int32_t k = chain_pos(c, ds[u]);
+                c.band[(size_t)(k + 1) * 64 + (t & 63)] = v[u];
+                atomicOr(c.has + k + 1, 1ull << (t & 63));
+            } else {
+                only = v[u];
+            }
         }
     }
     c.sum0[q] = acc;
-    c.recip[q] = c.unit ? 1. : 1. / c.dg[q];
+    c.recip[q] = c.unit ? 1. : 1. / d;
     if (!BAND) c.band[t] = only;
 }
 
@@ -2170,15 +2189,15 @@ int solve_typed(const nm_sptrsv_plan *p, int transposed, const void *data, int u
             const int64_t m64 = (int64_t)nm::ceil_div((int64_t)c.m, 64) * 64;
             const bool wide_chain = L.chain[dirn] == 64;
             c.has = reinterpret_cast<unsigned long long *>(c.band + (m64 + 64) * 64);
-            const unsigned pgrid = (unsigned)nm::ceil_div((int64_t)c.m, kBlock);
+            const unsigned pgrid = (unsigned)nm::ceil_div((int64_t)c.m, 64);
             if (wide_chain) {
                 if (int rc = nm::fill_async(c.band, chain_doubles(c.m, 64), 0., s)) return rc;
-                hipLaunchKernelGGL(chain_prepare_kernel<true>, dim3(pgrid), dim3(kBlock), 0, s, c);
+                hipLaunchKernelGGL(chain_prepare_kernel<true>, dim3(pgrid), dim3(64), 0, s, c);
                 if (unit) hipLaunchKernelGGL((sptrsv_chain_kernel<true, true>), dim3(1), dim3(64), 0, s, c);
                 else hipLaunchKernelGGL((sptrsv_chain_kernel<true, false>), dim3(1), dim3(64), 0, s, c);
             } else {
                 if (int rc = nm::fill_async(c.band + c.m, m64 + 64 - c.m, 0., s)) return rc;
-                hipLaunchKernelGGL(chain_prepare_kernel<false>, dim3(pgrid), dim3(kBlock), 0, s, c);
+                hipLaunchKernelGGL(chain_prepare_kernel<false>, dim3(pgrid), dim3(64), 0, s, c);
                 if (unit) hipLaunchKernelGGL((sptrsv_chain_kernel<false, true>), dim3(1), dim3(64), 0, s, c);
                 else hipLaunchKernelGGL((sptrsv_chain_kernel<false, false>), dim3(1), dim3(64), 0, s, c);
             }
