@@ -1448,7 +1448,7 @@ __global__ __launch_bounds__(kBlock) void sptrsv_level_group_kernel(SolveArgs a,
 // What bounds it: the hand-over, ~0.6 us from a store to a polling load on another compute unit,
 // plus a poll's own round trip, per level.  The launch has about four tiles in flight per tile of
 // the widest level, which is what the request stages need; more only poll.  97 x 89 x 101
-// seven-point triangle, fp32 (285 levels of up to 4500 rows): see flow_stretch.
+// seven-point triangle, fp32 (285 levels of up to 4500 rows): 325 us, 763 with a launch per level.
 //
 // A wavefront waits for tiles before its own only, and all workgroups are resident (a launch has
 // at most one per compute unit), so the waits end; as a backstop a wavefront that has polled
@@ -1456,7 +1456,7 @@ __global__ __launch_bounds__(kBlock) void sptrsv_level_group_kernel(SolveArgs a,
 // sees that, and the solve hands out NaN.
 constexpr unsigned long long kUnsolved = ~0ull;   // a NaN; a result with these bits is stored as the default NaN
 constexpr int kFlowMaxGroups = 256;
-constexpr int64_t kFlowMinLevels = 4, kFlowMeanWidth = 16384;   // see flow_stretch
+constexpr int64_t kFlowMinLevels = 2;   // see flow_stretch
 
 template <typename T> struct FlowArgs {
     const T *data, *b;
@@ -2085,8 +2085,12 @@ bool by_level(const nm_sptrsv_plan *p, int dirn, bool teams, const nm_sptrsv_pla
 }
 
 // The longest stretch [*a, *b) of consecutive launches that go level by level, where
-// sptrsv_flow_kernel is the better way: rows of at most 8 dependencies, several levels, and levels
-// that are not so wide that a launch each is no matter.
+// sptrsv_flow_kernel is the better way: rows of at most 8 dependencies and two levels or more,
+// however wide.  fp32, three dependencies a row, a launch per level against one for the stretch: 2 levels
+// of 2000 rows 21 and 15 us, 2 of 1 M 90 and 55 (110 and 76 with dependencies all over the level
+// before), 8 of 250 000 137 and 60, 8 of 1 M 565 and 222; seven-point triangles of 200^3 (13 400 rows a
+// level) 0.92 ms now, of 256^3 (21 900) 4.94 and 1.43 ms, of 300^3 (30 100) 7.30 and 2.14 ms.  Two
+// workgroups per compute unit instead of one: 300^3 2.40 ms, 8 of 1 M 171 us, 356 instead of 336 far apart.
 void flow_stretch(const nm_sptrsv_plan *p, int dirn, int *a, int *b) {
     *a = *b = 0;
     if (p->ell_pre[dirn] == 0 || p->nnz == 0) return;
@@ -2097,8 +2101,7 @@ void flow_stretch(const nm_sptrsv_plan *p, int dirn, int *a, int *b) {
         while (j < n && p->launches[j].chain[dirn] == 0 && by_level(p, dirn, true, p->launches[j])) ++j;
         if (j > i) {
             const int64_t levels = p->launches[j - 1].l1 - p->launches[i].l0;
-            const int64_t slots = p->launches[j - 1].q1 - p->launches[i].q0;
-            if (levels >= kFlowMinLevels && slots <= levels * kFlowMeanWidth && levels > best) {
+            if (levels >= kFlowMinLevels && levels > best) {
                 best = levels;
                 *a = i;
                 *b = j;

@@ -86,9 +86,10 @@ def test_grids(dev, dtype, dims, lower, unit):
     _compare(dev, *_grid(dims, dtype, lower, 1), dtype, lower, unit)
 
 
-# layers at the edges of what goes level by level (1024 rows, 4 levels), of tiles (64 rows) and of the
+# layers at the edges of what goes level by level (1024 rows, 2 levels), of tiles (64 rows) and of the
 # operand widths (2, 4, 8 dependencies; 9 take the other way)
-@pytest.mark.parametrize("width, layers, deps", [(1025, 4, 1), (1025, 3, 2), (1087, 9, 2), (4097, 6, 3), (5000, 5, 4),
+@pytest.mark.parametrize("width, layers, deps", [(1025, 4, 1), (1025, 3, 2), (1025, 2, 1), (30000, 2, 4),
+                                                 (40000, 4, 8), (1087, 9, 2), (4097, 6, 3), (5000, 5, 4),
                                                  (1100, 12, 5), (6001, 7, 8), (4200, 6, 9), (70000, 5, 3), (1500, 40, 4)])
 @pytest.mark.parametrize("lower", [True, False])
 def test_layers(dev, width, layers, deps, lower):
