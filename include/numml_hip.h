@@ -498,10 +498,13 @@ int nm_sptrsv_solve(const nm_sptrsv_plan *plan, nm_dtype dt, int transposed,
  * workgroups (nm_sptrsv_plan_shared_launches; each takes up to 256 rows of every level and
  * receives the few values it needs from the others through device memory, running a
  * few levels behind the workgroup it receives from) are taken by one workgroup
- * instead.  Results are the same bits either way.
- * All waiting is for rows of lower levels, by wavefronts of workgroups that are all
- * resident (a shared launch needs as many free compute units as it has workgroups),
- * so the waits end; `poll_limit` bounds the polls of one wait all the same (0: the
+ * instead, and a stretch of wider levels, otherwise one launch whose rows wait for each
+ * other, gets a launch per level.  Results are the same bits either way.
+ * Bit 2 (for tests): the launch of a stretch of wide levels has more workgroups than the
+ * device runs at once.
+ * All waiting is for rows of lower levels.  A shared launch needs as many free compute
+ * units as it has workgroups, at most sixteen; a stretch of wide levels is solved by
+ * whatever part of its launch runs.  So the waits end; `poll_limit` bounds the polls of one wait all the same (0: the
  * default of 2^22, seconds; negative: give up at once, for tests): when it is
  * exceeded the waiting stops for good and x comes back as NaN throughout.
  * Process-wide; takes effect with the next solve. */

@@ -20,12 +20,13 @@
 // an LDS read instead of an L2 round trip).  A chip-wide pass first gathers
 // this call's coefficients, diagonal and right-hand side into level-major
 // order (as doubles), so the workgroup reads contiguous streams only, two and
-// one level ahead through a register pipeline.  A level wider than 1024 rows gets a grid launch of its own.
-// Where the plan finds it possible, a run of levels wider than 256 rows is shared by up
-// to four workgroups that pass the few values they need from each other through device
+// one level ahead through a register pipeline.  Wider levels go to one launch for the longest
+// stretch of them, in which rows wait for rows (sptrsv_flow_kernel), and to a grid launch each
+// elsewhere.  Where the plan finds it possible, a run of levels wider than 256 rows is shared by
+// up to sixteen workgroups that pass the few values they need from each other through device
 // memory (sptrsv_team_kernel).  Stream order is the only synchronisation between launches;
-// inside a shared launch a workgroup waits for values of lower levels only, all its
-// workgroups are resident, and every wait is bounded (a solve that gives up returns NaN).
+// inside a shared launch a workgroup waits for values of lower levels only, all its (at most
+// sixteen) workgroups are resident, and every wait is bounded (a solve that gives up returns NaN).
 //
 // A row is one lane; sums run in double, in the walk order of the serial
 // CPU loop (cpp/sparse_csr_cpu.cpp:672-718: ascending for a lower triangle,
@@ -159,6 +160,7 @@ std::atomic<bool> g_sig_enabled{[] {
     const char *e = std::getenv("NUMML_AMD_SPTRSV_SIGNALLING");   // "1": neighbours signal
     return e && e[0] == '1';
 }()};
+std::atomic<bool> g_flow_crowd{false};   // sptrsv_flow_kernel with kFlowCrowd workgroups
 
 struct Layout {
     nm::TPlan t;
@@ -1446,17 +1448,27 @@ __global__ __launch_bounds__(kBlock) void sptrsv_level_group_kernel(SolveArgs a,
 // requested a tile ahead of the next, so no pass gathers them into level order beforehand.
 //
 // What bounds it: the hand-over, ~0.6 us from a store to a polling load on another compute unit,
-// plus a poll's own round trip, per level.  The launch has about four tiles in flight per tile of
-// the widest level, which is what the request stages need; more only poll.  97 x 89 x 101
-// seven-point triangle, fp32 (285 levels of up to 4500 rows): 325 us, 763 with a launch per level.
+// plus a poll's own round trip, per level.  Up to levels of 16384 rows the launch has about four tiles in
+// flight per tile of the widest level, which is what the request stages need (more only poll); wider
+// levels keep 1024 wavefronts busy without running ahead.  97 x 89 x 101 seven-point triangle, fp32
+// (285 levels of up to 4500 rows): 325 us, 763 with a launch per level.
 //
-// A wavefront waits for tiles before its own only, and all workgroups are resident (a launch has
-// at most one per compute unit), so the waits end; as a backstop a wavefront that has polled
-// `poll_limit` times for one tile raises the status word, every wavefront leaves when it
+// The tiles are dealt by number, so a wavefront may wait for one of a workgroup that has not started
+// (compute units masked, or taken by other solves on other streams).  It does not wait for ever:
+// a lane that has polled for long (`help`) follows its unsolved dependencies to a row that has
+// none and solves that row itself.  Whoever solves a row stores the same bits, and a lane's
+// search waits for nobody, so the launch ends whatever part of it is on the chip.  (Drawing tiles from a
+// counter ends as surely and costs every launch: 12 ns a draw, 300^3 2.14 -> 5.6 ms with a tile a
+// draw, 3.8 with two, 97 x 89 x 101 325 -> 348 and 574 us.)  As a backstop a wavefront that has
+// polled `poll_limit` times for one tile raises the status word, every wavefront leaves when it
 // sees that, and the solve hands out NaN.
 constexpr unsigned long long kUnsolved = ~0ull;   // a NaN; a result with these bits is stored as the default NaN
 constexpr int kFlowMaxGroups = 256;
+constexpr int kFlowCrowd = 4096;   // more workgroups than the chip holds at once (a test's)
 constexpr int64_t kFlowMinLevels = 2;   // see flow_stretch
+// Polls for one tile (0.7 us each) before a wavefront helps: more than waiting for rows that are being worked on
+// takes; and once it had to, until it got through some tiles without.
+constexpr int kFlowPatience = 256, kFlowImpatience = 16;
 
 template <typename T> struct FlowArgs {
     const T *data, *b;
@@ -1520,6 +1532,38 @@ __global__ __launch_bounds__(kBlock) void sptrsv_flow_kernel(FlowArgs<T> f) {
         o.dv = s.dv;
         return o;
     };
+    auto look = [&](int32_t q) {
+        return __hip_atomic_load(f.xs + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    // (a row of an earlier launch is solved whatever its bits)
+    auto solved = [&](int32_t q, unsigned long long bits) { return bits != kUnsolved || q < f.q0 || q >= f.q1; };
+    auto store = [&](int32_t q, double rhs, double acc, T diag) {
+        double xi = rhs - acc;
+        if (!f.unit) xi /= (double)diag;
+        unsigned long long bits = (unsigned long long)__double_as_longlong(xi);
+        if (bits == kUnsolved) bits = 0x7ff8000000000000ull;
+        __hip_atomic_store(f.xs + q, bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    // Solves a row that row q, not solved, waits for directly or through others (or q itself).
+    auto help = [&](int32_t q) {
+        while (true) {
+            const int32_t end = f.dptr[q + 1];
+            int32_t at = f.dptr[q], waits_for = -1;
+            double acc = 0.;
+            for (; at < end && waits_for < 0; ++at) {
+                const int32_t ds = f.dslot[at];
+                const unsigned long long got = look(ds);
+                if (solved(ds, got)) acc += (double)f.data[f.dsrc[at]] * __longlong_as_double((long long)got);
+                else waits_for = ds;
+            }
+            if (waits_for < 0) {
+                const int32_t diag = f.diag[q];
+                store(q, (double)f.b[f.order[q]], acc, diag >= 0 ? f.data[diag] : (T)0);
+                return;
+            }
+            q = waits_for;
+        }
+    };
     const int64_t tiles = (m + 63) / 64;
     Range r = range(wave);
     Source s = source(r);
@@ -1528,6 +1572,7 @@ __global__ __launch_bounds__(kBlock) void sptrsv_flow_kernel(FlowArgs<T> f) {
     s = source(r);
     r = range((int64_t)wave + 2 * (int64_t)waves);
     int64_t polls = f.poll_limit < 0 ? -1 : 0;
+    int patience = kFlowPatience;
     for (int64_t tile = wave; tile < tiles; tile += waves) {
         const Operands cur = o;
         o = operands(s);
@@ -1538,16 +1583,15 @@ __global__ __launch_bounds__(kBlock) void sptrsv_flow_kernel(FlowArgs<T> f) {
         double x[PRE];
 #pragma unroll
         for (int e = 0; e < PRE; ++e) x[e] = 0.;
+        int waited = 0;
         while (true) {
             unsigned long long got[PRE];
 #pragma unroll
             for (int e = 0; e < PRE; ++e)
-                if (need >> e & 1u)
-                    got[e] = __hip_atomic_load(f.xs + cur.ds[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (need >> e & 1u) got[e] = look(cur.ds[e]);
 #pragma unroll
             for (int e = 0; e < PRE; ++e)
-                // (a row of an earlier launch is solved whatever its bits)
-                if ((need >> e & 1u) && (got[e] != kUnsolved || cur.ds[e] < f.q0 || cur.ds[e] >= f.q1)) {
+                if ((need >> e & 1u) && solved(cur.ds[e], got[e])) {
                     x[e] = __longlong_as_double((long long)got[e]);
                     need &= ~(1u << e);
                 }
@@ -1556,11 +1600,7 @@ __global__ __launch_bounds__(kBlock) void sptrsv_flow_kernel(FlowArgs<T> f) {
 #pragma unroll
                 for (int e = 0; e < PRE; ++e)
                     if (e < cur.n) acc += (double)cur.v[e] * x[e];
-                double xi = (double)cur.bv - acc;
-                if (!f.unit) xi /= (double)cur.dv;
-                unsigned long long bits = (unsigned long long)__double_as_longlong(xi);
-                if (bits == kUnsolved) bits = 0x7ff8000000000000ull;
-                __hip_atomic_store(f.xs + cur.q, bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                store(cur.q, (double)cur.bv, acc, cur.dv);
                 pending = false;
             }
             if (!__any(pending)) break;
@@ -1572,8 +1612,14 @@ __global__ __launch_bounds__(kBlock) void sptrsv_flow_kernel(FlowArgs<T> f) {
             if ((polls & 1023) == 0 &&
                 __hip_atomic_load(f.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)
                 return;
+            if (++waited == patience) {
+                if (pending) help(cur.q);
+                waited = 0;
+                patience = kFlowImpatience;
+            }
         }
         if (f.poll_limit >= 0) polls = 0;
+        if (patience < kFlowPatience) ++patience;
     }
 }
 
@@ -2166,7 +2212,9 @@ int solve_typed(const nm_sptrsv_plan *p, int transposed, const void *data, int u
             int32_t widest = 0;
             for (int j = flow_a; j < flow_b; ++j) widest = widest > p->launches[j].width ? widest : p->launches[j].width;
             int64_t groups = nm::ceil_div((int64_t)widest, (int64_t)64);
-            const dim3 fg((unsigned)(groups > kFlowMaxGroups ? kFlowMaxGroups : groups));
+            if (groups > kFlowMaxGroups) groups = kFlowMaxGroups;
+            if (g_flow_crowd.load()) groups = kFlowCrowd;
+            const dim3 fg((unsigned)groups);
             if (pre == 2) hipLaunchKernelGGL((sptrsv_flow_kernel<T, 2>), fg, dim3(kBlock), 0, s, f);
             else if (pre == 4) hipLaunchKernelGGL((sptrsv_flow_kernel<T, 4>), fg, dim3(kBlock), 0, s, f);
             else hipLaunchKernelGGL((sptrsv_flow_kernel<T, 8>), fg, dim3(kBlock), 0, s, f);
@@ -2923,10 +2971,12 @@ extern "C" int nm_sptrsv_solve_static(const nm_sptrsv_plan *plan, nm_dtype dt, i
 //   signalling   bit 0: wavefronts of a workgroup signal their neighbours, where no row depends on
 //                a row more than one wavefront away, instead of meeting at a barrier after every
 //                level (default off); bit 1: launches that the plan would share among several
-//                workgroups are taken by one (default: shared).
+//                workgroups are taken by one, wide levels by a launch each (default: shared); bit 2
+//                (tests): a stretch of wide levels is launched with more workgroups than can run at once.
 extern "C" int nm_sptrsv_configure(int64_t poll_limit, int signalling) {
     g_sig_poll_limit.store(poll_limit == 0 ? int64_t(1) << 22 : poll_limit);
     g_sig_enabled.store((signalling & 1) != 0);
     g_team_enabled.store((signalling & 2) == 0);
+    g_flow_crowd.store((signalling & 4) != 0);
     return NM_OK;
 }

@@ -136,3 +136,43 @@ def test_in_a_graph(dev):
         want = ext.sptrsv_forward(n, n, D, I, P, True, False, b)
         torch.cuda.synchronize()
         assert torch.equal(x, want)
+
+
+# one workgroup in two of such a launch starts when another has ended; the wavefronts that wait for its rows
+# have to solve these themselves (dependencies of one row: 1, 3 and up to 8)
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("deps, lower", [(1, True), (3, False), (8, True)])
+def test_more_workgroups_than_run_at_once(dev, dtype, deps, lower):
+    print("case", deps, lower, dtype.__name__, flush=True)
+    d, i, p, n = _layers(20000, 20, deps, dtype, lower, deps)
+    b, g = randn(5, n, dtype), randn(6, n, dtype)
+    D, I, P, Bv, Gv = to_dev(dev, d, i, p, b, g)
+    x_ref = oracle.sptrsv_forward(n, n, d, i, p, lower, False, b)
+    ext = numml_amd.load_compiled()
+    try:
+        assert _lib.lib().nm_sptrsv_configure(0, 4) == 0
+        x = ext.sptrsv_forward(n, n, D, I, P, lower, False, Bv)
+        grads = ext.sptrsv_backward(Gv, x, n, n, D, I, P, lower, False, Bv)
+        torch.cuda.synchronize()
+    finally:
+        assert _lib.lib().nm_sptrsv_configure(0, 0) == 0
+    assert_same(host(x), x_ref, "x")
+    for got, ref in zip(grads, oracle.sptrsv_backward(g, x_ref, n, n, d, i, p, lower, False, b)):
+        assert_same(host(got), ref, "gradient")
+
+
+def test_on_four_streams_at_once(dev):
+    d, i, p, n = _layers(20000, 20, 8, np.float64, True, 11)
+    ext = numml_amd.load_compiled()
+    D, I, P = to_dev(dev, d, i, p)
+    bs = to_dev(dev, *(randn(20 + k, n, np.float64) for k in range(4)))
+    want = [ext.sptrsv_forward(n, n, D, I, P, True, False, b) for b in bs]
+    torch.cuda.synchronize()
+    streams, got = [torch.cuda.Stream() for _ in bs], []
+    for _ in range(3):
+        for b, s in zip(bs, streams):
+            with torch.cuda.stream(s):
+                got.append(ext.sptrsv_forward(n, n, D, I, P, True, False, b))
+    torch.cuda.synchronize()
+    for k, x in enumerate(got):
+        assert torch.equal(x, want[k % 4])
