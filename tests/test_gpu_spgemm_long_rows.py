@@ -6,6 +6,7 @@ of B (atomics): a sum of m products in any order is off by at most m * eps * sum
 parity bound of the suite is above that for the lengths here."""
 import numpy as np
 import pytest
+import torch
 
 import oracle
 from numml_amd import generators as G
@@ -90,3 +91,44 @@ def test_rows_of_runs_and_of_packed_columns(dev, dtype):
 def test_two_hop_graph(dev, dtype):
     a = G.powerlaw(6000, 6000, 60000, max_deg=1500, seed=7, dtype=dtype)
     _check(dev, a, a, dtype)
+
+
+def _packed(lengths, cols, dtype):
+    """Rows of C of about the given lengths: a run of columns somewhere, and the last column of all."""
+    B = [np.arange(8 * k, 8 * k + 8) for k in range(4096)] + [[cols - 1]]
+    rng = np.random.default_rng(6)
+    A = [np.append(np.arange(s, s + (n - 1) // 8), 4096) for n in lengths for s in [int(rng.integers(0, 4096 - n // 8))]]
+    return _csr(A, 4097, 6, dtype), _csr(B, cols, 7, dtype)
+
+
+# a row in every shape of workgroup, nearly all of its columns in one bucket
+@pytest.mark.parametrize("dtype,most", [(np.float32, 16384), (np.float64, 10880)])
+@pytest.mark.parametrize("cols", [40_000, 20_000_000])
+def test_a_column_far_from_the_others(dev, dtype, most, cols):
+    _check(dev, *_packed([137, 200, 250, 264, 500, 520, 1000, 1024, 1032, 2000, 2050, 4000, 4100, 8200, most - 8, most],
+                         cols, dtype), dtype)
+
+
+def _time(dev, a, b):
+    (ad, ai, ap, (ar, ac)), (bd, bi, bp, (br, bc)) = a, b
+    AD, AI, AP, BD, BI, BP = to_dev(dev, ad, ai, ap, bd, bi, bp)
+    best = float("inf")
+    for _ in range(6):
+        t0, t1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        torch.cuda.synchronize()
+        t0.record()
+        ext.spgemm_forward(ar, ac, AD, AI, AP, br, bc, BD, BI, BP)
+        t1.record()
+        torch.cuda.synchronize()
+        best = min(best, t0.elapsed_time(t1))
+    return best
+
+
+def test_the_time_of_packed_columns(dev):
+    # a compare for every pair of columns took 13 times as long as columns that are spread out; sorting them 1.2
+    rng = np.random.default_rng(8)
+    spread = [np.sort(rng.choice(1_000_000, 8, replace=False)) for _ in range(4096)]
+    A = [np.sort(rng.choice(4096, 500, replace=False)) for _ in range(300)]
+    even = _time(dev, _csr(A, 4096, 1, np.float32), _csr(spread, 1_000_000, 2, np.float32))
+    packed = _time(dev, *_packed([4000] * 300, 20_000_000, np.float32))
+    assert packed < 4 * even, (packed, even)
