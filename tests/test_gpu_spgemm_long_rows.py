@@ -132,3 +132,29 @@ def test_the_time_of_packed_columns(dev):
     even = _time(dev, _csr(A, 4096, 1, np.float32), _csr(spread, 1_000_000, 2, np.float32))
     packed = _time(dev, *_packed([4000] * 300, 20_000_000, np.float32))
     assert packed < 4 * even, (packed, even)
+
+
+def _hub(dtype, hub):
+    """Two products per entry of A; with `hub` one of them in column 0, else all in columns of their own."""
+    rng = np.random.default_rng(9)
+    A = [np.sort(rng.choice(20_000, 4000, replace=False)) for _ in range(300)]
+    B = [[0 if hub else 2 * k + 1, 2 * k + 2] for k in range(20_000)]
+    return _csr(A, 20_000, 1, dtype), _csr(B, 40_001, 2, dtype)
+
+
+def test_the_time_of_a_full_column(dev):
+    # a turn of 1024 threads for every product in the full column took 8 times as long as products that do not meet, now 1.6
+    even, full = _time(dev, *_hub(np.float64, False)), _time(dev, *_hub(np.float64, True))
+    assert full < 4 * even, (full, even)
+
+
+# products that meet in a few columns: 2 to 1000 of one chunk in a slot, several such slots among others, next to
+# columns that nothing else adds to, in every shape of workgroup
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("hubs", [1, 3, 40, 300])
+def test_products_that_meet(dev, dtype, hubs):
+    rng = np.random.default_rng(hubs)
+    K = 3000
+    B = [np.unique(np.append(rng.integers(0, hubs, rng.integers(1, 4)), [hubs + k, hubs + K + k])) for k in range(K)]
+    A = [np.sort(rng.choice(K, n, replace=False)) for n in (60, 70, 120, 200, 250, 400, 500, 900, 1000, 1900, 2047, K)]
+    _check(dev, _csr(A, K, 1, dtype), _csr(B, hubs + 2 * K, 2, dtype), dtype)
