@@ -1556,18 +1556,18 @@ __global__ __launch_bounds__(kSpillBlock) void numeric_spill_kernel(
 // gC[i,c] * B[k,c] are then added lane by lane in ascending column order --
 // the order of the reference's merge -- which keeps grad_A bit-identical.
 //
-// Rows of C longer than kBwdStage get a workgroup each, of 64, 256 or 1024 threads by length.  The
-// row's products are numbered through in the order of A's row and dealt to the threads by number
-// (as in numeric_row_kernel), each looks its column up in the row of C in LDS, and the thread of an
-// entry of A adds the entry's products from LDS in order.  Of a row longer than LDS holds, every
-// stride-th column is staged: the last steps of the search then read global memory.
+// Rows of C longer than kBwdStage get a wavefront (up to 512 entries) or a workgroup each, of 256 (up
+// to 2048) or 1024 threads.  The row's products are numbered through in the order of A's row and
+// dealt to the threads by number (as in numeric_row_kernel), each looks its column up in the row of
+// C in LDS, and the thread of an entry of A adds the entry's products from LDS in order.  Of a row
+// longer than LDS holds, every stride-th column is staged: the last steps of the search then read
+// global memory.
 // Bound by the row's chain of round trips, the searches in LDS and the atomic adds of the gradient of B.  A
-// 150 000-row power-law graph squared (mean 8, rows up to 1000, fp32), by length of C's row, against
-// one workgroup of 256 threads whose groups of eight lanes took A's entries one by one: 65-2048 617 -> 224 us
-// (65-512 107, 513-2048 117), more 679 -> 261 (2049-4096 73, above 188).
+// 150 000-row power-law graph squared (mean 8, rows up to 1000, fp32), kernels of the rows of 65-2048 and of
+// more entries, against one workgroup of 256 threads whose groups of eight lanes took A's entries
+// one by one: 617 -> 208 us, 679 -> 223 us.
 constexpr int kBwdG = 8;
 constexpr int kBwdStage = 64;
-constexpr int kBwdLongChunk = 256;   // rows a workgroup of the long-row kernel looks through at a time, at most
 
 // What lane E of every eight consecutive lanes holds, handed to all eight (ds_swizzle in bit mode:
 // lane = (lane & 0x18) | E inside each half of the wavefront; no address to compute).
@@ -1670,30 +1670,45 @@ __global__ __launch_bounds__(kBlock) void spgemm_bwd_kernel(
     }
 }
 
+// Threads that work on a row: a wavefront or a workgroup.
+template <int TPB> __device__ __forceinline__ void row_sync() {
+    if constexpr (TPB == kWave) group_sync<kWave>();
+    else __syncthreads();
+}
+
+template <typename T> struct BackArgs {
+    int64_t A_rows;
+    int piece;   // rows a workgroup looks at side by side, see back_row
+    const T *gC;
+    const int64_t *C_indices, *C_indptr;
+    const T *A_data;
+    const int64_t *A_indices, *A_indptr;
+    const T *B_data;
+    const int64_t *B_indices, *B_indptr;
+    T *grad_A, *grad_B;
+};
+
 template <typename T_, int TPB_, int CAP_, int UNROLL_> struct BackShape {
     using T = T_;
     static constexpr int TPB = TPB_, CAP = CAP_, UNROLL = UNROLL_, BATCH = TPB < 512 ? TPB : 512;
     static constexpr int STEP = TPB * UNROLL;                                  // products at a time
     static constexpr size_t at_prod = sizeof(T) * CAP, at_off = at_prod + sizeof(T) * STEP,
                             at_row = at_off + 8 * (BATCH + 2), at_a = at_row + 8 * BATCH,
-                            at_wave = at_a + 8 * BATCH, at_col = at_wave + 8 * (TPB / kWave) + 16,
-                            at_long = at_col + 4 * CAP;
-    static constexpr size_t lds = at_long + 4 * (kBwdLongChunk + 2);
-    static_assert(lds <= 160 * 1024, "a CU's LDS");
+                            at_wave = at_a + 8 * BATCH, at_col = at_wave + 8 * (TPB / kWave) + 16;
+    static constexpr size_t lds = (at_col + 4 * CAP + 15) / 16 * 16;
     static_assert((CAP * sizeof(T)) % 8 == 0 && (STEP * sizeof(T)) % 8 == 0, "64-bit words behind the values");
 };
 
+// Row i by the threads of shape S, the first of them `tid` 0, in the S::lds bytes at s_raw.
 template <typename S>
-__global__ __launch_bounds__(S::TPB) void spgemm_bwd_long_kernel(
-    int64_t A_rows, int chunk, int64_t longer_than, int64_t up_to, const typename S::T *__restrict__ gC,
-    const int64_t *__restrict__ C_indices, const int64_t *__restrict__ C_indptr,
-    const typename S::T *__restrict__ A_data, const int64_t *__restrict__ A_indices,
-    const int64_t *__restrict__ A_indptr, const typename S::T *__restrict__ B_data,
-    const int64_t *__restrict__ B_indices, const int64_t *__restrict__ B_indptr,
-    typename S::T *__restrict__ grad_A, typename S::T *__restrict__ grad_B) {
+__device__ __forceinline__ void back_one_row(const BackArgs<typename S::T> &g, int64_t i, int tid, unsigned char *s_raw) {
     using T = typename S::T;
     constexpr int TPB = S::TPB, CAP = S::CAP, BATCH = S::BATCH, U = S::UNROLL, STEP = S::STEP;
-    extern __shared__ __align__(16) unsigned char s_raw[];
+    const T *__restrict__ gC = g.gC, *__restrict__ A_data = g.A_data, *__restrict__ B_data = g.B_data;
+    const int64_t *__restrict__ C_indices = g.C_indices, *__restrict__ C_indptr = g.C_indptr;
+    const int64_t *__restrict__ A_indices = g.A_indices, *__restrict__ A_indptr = g.A_indptr;
+    const int64_t *__restrict__ B_indices = g.B_indices, *__restrict__ B_indptr = g.B_indptr;
+    T *__restrict__ grad_A = g.grad_A, *__restrict__ grad_B = g.grad_B;
     T *cg = reinterpret_cast<T *>(s_raw);
     T *s_prod = reinterpret_cast<T *>(s_raw + S::at_prod);
     int64_t *s_off = reinterpret_cast<int64_t *>(s_raw + S::at_off);   // number of an entry's first product
@@ -1701,131 +1716,182 @@ __global__ __launch_bounds__(S::TPB) void spgemm_bwd_long_kernel(
     T *s_a = reinterpret_cast<T *>(s_raw + S::at_a);
     int64_t *s_wave = reinterpret_cast<int64_t *>(s_raw + S::at_wave);
     int32_t *ci = reinterpret_cast<int32_t *>(s_raw + S::at_col);
-    int32_t *s_long = reinterpret_cast<int32_t *>(s_raw + S::at_long);
-    int32_t *s_n = s_long + kBwdLongChunk;
+    const int64_t cb = C_indptr[i], clen = C_indptr[i + 1] - cb;
+    const int64_t stride = (clen + CAP - 1) / CAP;
+    const int ns = (int)((clen + stride - 1) / stride);
+    const bool whole = stride == 1;
+    for (int t = tid; t < ns; t += TPB) {
+        ci[t] = (int32_t)C_indices[cb + t * stride];
+        if (whole) cg[t] = gC[cb + t];
+    }
+    const int top = 1 << (31 - __clz(ns));   // the first step of a search through ns columns
+    const int64_t ab = A_indptr[i], ae = A_indptr[i + 1];
+    for (int64_t a0 = ab; a0 < ae; a0 += BATCH) {
+        const bool mine = tid < BATCH && a0 + tid < ae;
+        const int64_t j = mine ? A_indices[a0 + tid] : 0;
+        const T a = mine && grad_B ? A_data[a0 + tid] : T(0);
+        const int64_t bb = mine ? B_indptr[j] : 0, be = mine ? B_indptr[j + 1] : 0;
+        int64_t total;
+        const int64_t off = row_scan<TPB, int64_t>(be - bb, s_wave, total), end = off + (be - bb);
+        if (tid < BATCH) {
+            s_off[tid] = off;   // (threads past the row's end: the total)
+            s_row[tid] = bb - off;
+            s_a[tid] = a;
+        }
+        row_sync<TPB>();
+        T acc = 0;
+        for (int64_t p0 = 0; p0 < total; p0 += STEP) {
+            int64_t kk[U], c[U];
+            T b[U], av[U];
+            int l[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int64_t p = p0 + u * TPB + tid;
+                const bool have = p < total;
+                const int64_t at = have ? p : 0;
+                int e = 0;   // the last entry whose first product is not behind this one
+#pragma unroll
+                for (int step = BATCH / 2; step > 0; step >>= 1)
+                    if (s_off[e + step] <= at) e += step;
+                kk[u] = s_row[e] + at;
+                av[u] = s_a[e];
+                c[u] = B_indices[kk[u]];
+                b[u] = grad_A ? B_data[kk[u]] : T(0);
+                if (!have) c[u] = -1;
+                l[u] = 0;
+            }
+            // the number of staged columns below c
+            for (int step = top; step > 0; step >>= 1)
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    if (l[u] + step <= ns && (int64_t)ci[l[u] + step - 1] < c[u]) l[u] += step;
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                bool hit;
+                T g = 0;
+                if (whole) {
+                    hit = l[u] < ns && (int64_t)ci[l[u]] == c[u];
+                    if (hit) g = cg[l[u]];
+                } else {
+                    // sample l is the first one not below c: the column, if present, sits
+                    // after sample l - 1 and no later than sample l
+                    int64_t lo = l[u] == 0 ? 0 : (int64_t)(l[u] - 1) * stride + 1;
+                    int64_t hi = (int64_t)l[u] * stride < clen ? (int64_t)l[u] * stride : clen;
+                    if (c[u] < 0) hi = lo;
+                    while (lo < hi) {
+                        const int64_t mid = (lo + hi) >> 1;
+                        if (C_indices[cb + mid] < c[u]) lo = mid + 1; else hi = mid;
+                    }
+                    hit = c[u] >= 0 && lo < clen && C_indices[cb + lo] == c[u];
+                    if (hit) g = gC[cb + lo];
+                }
+                if (hit && grad_B) nm::atomic_add(grad_B + kk[u], av[u] * g);
+                s_prod[u * TPB + tid] = hit ? g * b[u] : T(0);
+            }
+            if (!grad_A) continue;
+            row_sync<TPB>();
+            // an entry's thread adds its products in ascending column (a product that is missing
+            // is +0.0, which changes no sum that began at +0.0)
+            if (off < p0 + STEP && end > p0) {
+                int t = off > p0 ? (int)(off - p0) : 0;
+                const int t1 = end - p0 < STEP ? (int)(end - p0) : STEP;
+                // (eight are on their way while eight are added: one after the other, a row of B of
+                // a thousand entries was a thousand trips to LDS)
+                constexpr int W = 8;
+                if (t + W <= t1) {
+                    T x[W];
+#pragma unroll
+                    for (int w = 0; w < W; ++w) x[w] = s_prod[t + w];
+                    for (t += W; t + W <= t1; t += W) {
+                        T y[W];
+#pragma unroll
+                        for (int w = 0; w < W; ++w) y[w] = s_prod[t + w];
+#pragma unroll
+                        for (int w = 0; w < W; ++w) {
+                            acc += x[w];
+                            x[w] = y[w];
+                        }
+                    }
+#pragma unroll
+                    for (int w = 0; w < W; ++w) acc += x[w];
+                }
+                for (; t < t1; ++t) acc += s_prod[t];
+            }
+            row_sync<TPB>();
+        }
+        if (mine && grad_A) grad_A[a0 + tid] = acc;
+        row_sync<TPB>();   // (the lists are this batch's until here)
+    }
+    row_sync<TPB>();
+}
+
+// A workgroup looks through its rows for the long ones, a thread a row.  Rows next to each other are often alike,
+// so they are dealt in pieces of up to eight (a cache line of the row pointer) in turn: the row of thread t in the
+// workgroup's `turn`-th look, or past the last one.
+__device__ __forceinline__ int64_t back_row(int64_t turn, int t, int threads, int piece) {
+    return ((turn * (threads / piece) + t / piece) * (int64_t)gridDim.x + blockIdx.x) * piece + t % piece;
+}
+
+// Rows of C of kBwdStage + 1 to 512 entries, a wavefront each, and of up to 2048, the workgroup's.
+constexpr int kBackMid = 256;
+constexpr int64_t kBackWave = 512, kBackGroup = 2048;
+template <typename T> using BackMidRow = BackShape<T, kBackMid, kBackGroup, 4>;
+template <typename T> using BackWaveRow = BackShape<T, kWave, kBackWave, 4>;
+template <typename T>
+constexpr size_t kBackMidLds = BackMidRow<T>::lds > kBackMid / kWave * BackWaveRow<T>::lds ? BackMidRow<T>::lds
+                                                                                          : kBackMid / kWave * BackWaveRow<T>::lds;
+
+template <typename T> __global__ __launch_bounds__(kBackMid) void spgemm_bwd_mid_kernel(BackArgs<T> g) {
+    extern __shared__ __align__(16) unsigned char s_raw[];
+    __shared__ uint8_t s_of_wave[kBackMid], s_of_group[kBackMid];
+    __shared__ int s_n[3];   // rows in the two lists, next of the first
+    static_assert(kBackMid <= 256, "a thread's number fits a byte");
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    for (int64_t turn = 0; back_row(turn, 0, kBackMid, g.piece) < g.A_rows; ++turn) {
+        const int64_t r = back_row(turn, tid, kBackMid, g.piece);
+        const int64_t len = r < g.A_rows ? g.C_indptr[r + 1] - g.C_indptr[r] : 0;
+        const bool of_wave = len > kBwdStage && len <= kBackWave, of_group = len > kBackWave && len <= kBackGroup;
+        if (!__syncthreads_or(of_wave || of_group)) continue;
+        if (tid < 3) s_n[tid] = 0;
+        __syncthreads();
+        if (of_wave) s_of_wave[atomicAdd(&s_n[0], 1)] = (uint8_t)tid;
+        if (of_group) s_of_group[atomicAdd(&s_n[1], 1)] = (uint8_t)tid;
+        __syncthreads();
+        const int waves = s_n[0], groups = s_n[1];
+        for (int q = 0; q < groups; ++q)
+            back_one_row<BackMidRow<T>>(g, back_row(turn, s_of_group[q], kBackMid, g.piece), tid, s_raw);
+        while (true) {
+            int q = 0;
+            if (lane == 0) q = atomicAdd(&s_n[2], 1);
+            q = __builtin_amdgcn_readfirstlane(q);
+            if (q >= waves) break;
+            back_one_row<BackWaveRow<T>>(g, back_row(turn, s_of_wave[q], kBackMid, g.piece), lane,
+                                         s_raw + wave * BackWaveRow<T>::lds);
+        }
+        __syncthreads();
+    }
+}
+
+// Longer rows, one at a time by a workgroup that takes a CU's LDS.
+template <typename T> using BackLongRow = BackShape<T, 1024, sizeof(T) == 4 ? 14336 : 8192, 4>;
+template <typename T> __global__ __launch_bounds__(1024) void spgemm_bwd_long_kernel(BackArgs<T> g) {
+    extern __shared__ __align__(16) unsigned char s_raw[];
+    __shared__ uint16_t s_long[1024];
+    __shared__ int s_n;
+    static_assert(BackLongRow<T>::lds + sizeof(s_long) + 16 <= 160 * 1024, "a CU's LDS");
     const int tid = threadIdx.x;
-    for (int64_t r0 = (int64_t)blockIdx.x * chunk; r0 < A_rows; r0 += (int64_t)gridDim.x * chunk) {
-        // the long rows among this chunk of rows (mostly there are none)
-        if (tid == 0) *s_n = 0;
+    for (int64_t turn = 0; back_row(turn, 0, 1024, g.piece) < g.A_rows; ++turn) {
+        const int64_t r = back_row(turn, tid, 1024, g.piece);
+        const bool is_long = r < g.A_rows && g.C_indptr[r + 1] - g.C_indptr[r] > kBackGroup;
+        if (!__syncthreads_or(is_long)) continue;
+        if (tid == 0) s_n = 0;
         __syncthreads();
-        for (int t = tid; t < chunk; t += TPB) {
-            const int64_t r = r0 + t;
-            if (r >= A_rows) continue;
-            const int64_t len = C_indptr[r + 1] - C_indptr[r];
-            if (len > longer_than && len <= up_to) s_long[atomicAdd(s_n, 1)] = t;
-        }
+        if (is_long) s_long[atomicAdd(&s_n, 1)] = (uint16_t)tid;
         __syncthreads();
-        const int n = *s_n;
-        for (int q = 0; q < n; ++q) {
-            const int64_t i = r0 + s_long[q];
-            const int64_t cb = C_indptr[i], clen = C_indptr[i + 1] - cb;
-            const int64_t stride = (clen + CAP - 1) / CAP;
-            const int ns = (int)((clen + stride - 1) / stride);
-            const bool whole = stride == 1;
-            for (int t = tid; t < ns; t += TPB) {
-                ci[t] = (int32_t)C_indices[cb + t * stride];
-                if (whole) cg[t] = gC[cb + t];
-            }
-            const int top = 1 << (31 - __clz(ns));   // the first step of a search through ns columns
-            const int64_t ab = A_indptr[i], ae = A_indptr[i + 1];
-            for (int64_t a0 = ab; a0 < ae; a0 += BATCH) {
-                const bool mine = tid < BATCH && a0 + tid < ae;
-                const int64_t j = mine ? A_indices[a0 + tid] : 0;
-                const T a = mine && grad_B ? A_data[a0 + tid] : T(0);
-                const int64_t bb = mine ? B_indptr[j] : 0, be = mine ? B_indptr[j + 1] : 0;
-                int64_t total;
-                const int64_t off = row_scan<TPB, int64_t>(be - bb, s_wave, total), end = off + (be - bb);
-                if (tid < BATCH) {
-                    s_off[tid] = off;   // (threads past the row's end: the total)
-                    s_row[tid] = bb - off;
-                    s_a[tid] = a;
-                }
-                __syncthreads();
-                T acc = 0;
-                for (int64_t p0 = 0; p0 < total; p0 += STEP) {
-                    int64_t kk[U], c[U];
-                    T b[U], av[U];
-                    int l[U];
-#pragma unroll
-                    for (int u = 0; u < U; ++u) {
-                        const int64_t p = p0 + u * TPB + tid;
-                        const bool have = p < total;
-                        const int64_t at = have ? p : 0;
-                        int e = 0;   // the last entry whose first product is not behind this one
-#pragma unroll
-                        for (int step = BATCH / 2; step > 0; step >>= 1)
-                            if (s_off[e + step] <= at) e += step;
-                        kk[u] = s_row[e] + at;
-                        av[u] = s_a[e];
-                        c[u] = B_indices[kk[u]];
-                        b[u] = grad_A ? B_data[kk[u]] : T(0);
-                        if (!have) c[u] = -1;
-                        l[u] = 0;
-                    }
-                    // the number of staged columns below c
-                    for (int step = top; step > 0; step >>= 1)
-#pragma unroll
-                        for (int u = 0; u < U; ++u)
-                            if (l[u] + step <= ns && (int64_t)ci[l[u] + step - 1] < c[u]) l[u] += step;
-#pragma unroll
-                    for (int u = 0; u < U; ++u) {
-                        bool hit;
-                        T g = 0;
-                        if (whole) {
-                            hit = l[u] < ns && (int64_t)ci[l[u]] == c[u];
-                            if (hit) g = cg[l[u]];
-                        } else {
-                            // sample l is the first one not below c: the column, if present, sits
-                            // after sample l - 1 and no later than sample l
-                            int64_t lo = l[u] == 0 ? 0 : (int64_t)(l[u] - 1) * stride + 1;
-                            int64_t hi = (int64_t)l[u] * stride < clen ? (int64_t)l[u] * stride : clen;
-                            if (c[u] < 0) hi = lo;
-                            while (lo < hi) {
-                                const int64_t mid = (lo + hi) >> 1;
-                                if (C_indices[cb + mid] < c[u]) lo = mid + 1; else hi = mid;
-                            }
-                            hit = c[u] >= 0 && lo < clen && C_indices[cb + lo] == c[u];
-                            if (hit) g = gC[cb + lo];
-                        }
-                        if (hit && grad_B) nm::atomic_add(grad_B + kk[u], av[u] * g);
-                        s_prod[u * TPB + tid] = hit ? g * b[u] : T(0);
-                    }
-                    if (!grad_A) continue;
-                    __syncthreads();
-                    // an entry's thread adds its products in ascending column (a product that is missing
-                    // is +0.0, which changes no sum that began at +0.0)
-                    if (off < p0 + STEP && end > p0) {
-                        int t = off > p0 ? (int)(off - p0) : 0;
-                        const int t1 = end - p0 < STEP ? (int)(end - p0) : STEP;
-                        // (eight are on their way while eight are added: one after the other, a row of B of
-                        // a thousand entries was a thousand trips to LDS)
-                        constexpr int W = 8;
-                        if (t + W <= t1) {
-                            T x[W];
-#pragma unroll
-                            for (int w = 0; w < W; ++w) x[w] = s_prod[t + w];
-                            for (t += W; t + W <= t1; t += W) {
-                                T y[W];
-#pragma unroll
-                                for (int w = 0; w < W; ++w) y[w] = s_prod[t + w];
-#pragma unroll
-                                for (int w = 0; w < W; ++w) {
-                                    acc += x[w];
-                                    x[w] = y[w];
-                                }
-                            }
-#pragma unroll
-                            for (int w = 0; w < W; ++w) acc += x[w];
-                        }
-                        for (; t < t1; ++t) acc += s_prod[t];
-                    }
-                    __syncthreads();
-                }
-                if (mine && grad_A) grad_A[a0 + tid] = acc;
-                __syncthreads();   // (the lists are this batch's until here)
-            }
-            __syncthreads();
-        }
+        const int n = s_n;
+        for (int q = 0; q < n; ++q)
+            back_one_row<BackLongRow<T>>(g, back_row(turn, s_long[q], 1024, g.piece), tid, s_raw);
+        __syncthreads();
     }
 }
 
@@ -2163,38 +2229,34 @@ extern "C" int nm_spgemm_backward(nm_dtype dt, int64_t A_rows, int64_t A_nnz, in
                            (const double *)gC, C_indices, C_indptr, (const double *)A_data, A_indices, A_indptr,
                            (const double *)B_data, B_indices, B_indptr, (double *)grad_A, (double *)grad_B);
     NM_LAUNCH_CHECK("spgemm_bwd_kernel");
-    // A workgroup works off the long rows of its chunk one after the other, so a chunk is sized
-    // for `groups` of them or more over the matrix: as many as spread the rows, and fewer where a workgroup
-    // takes a CU's LDS and those that find nothing pass through one at a time (half as many of the
-    // largest: 196 against 188 us).  The limits between the shapes follow from LDS: 512 columns with
-    // their gradients leave room for 10 to 14 rows in a CU, 4096 for two; (2049-4096 and the rest in one shape:
-    // 256 us, in two 73 + 188).
-    auto longer = [&](auto shape, int groups, int64_t longer_than, int64_t up_to) -> int {
-        using S = decltype(shape);
-        using T = typename S::T;
-        int chunk = kBwdLongChunk;
-        while (chunk > 4 && A_rows / chunk < groups) chunk /= 2;
-        int64_t most = nm::ceil_div(A_rows, chunk);
-        if (most > 2 * groups) most = 2 * groups;
-        auto k = spgemm_bwd_long_kernel<S>;
-        if (S::lds > 64 * 1024)
-            NM_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(k),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::lds));
-        hipLaunchKernelGGL(k, dim3((unsigned)most), dim3(S::TPB), S::lds, s, A_rows, chunk, longer_than, up_to,
-                           (const T *)gC, C_indices, C_indptr, (const T *)A_data, A_indices, A_indptr,
-                           (const T *)B_data, B_indices, B_indptr, (T *)grad_A, (T *)grad_B);
+    // Two launches whether or not there are long rows, which the host does not know: so few workgroups
+    // that finding none is short (a launch of 1024-thread workgroups that take a CU's LDS each: 17 us with
+    // 2800 of them, 4 with 256), so many that long rows find the chip (150 000-row graph: both gradients
+    // 497 us with 1024 workgroups for the longest rows, 546 with 512; 20 000 rows of 600 entries: 685 us
+    // with 4096 of the others, 732 with 2500, 886 with 512).  Both gradients of 5-point 300^2 A A, fp32: 36
+    // us (61 with four launches, one for each shape, of 2800 to 22500 workgroups), 7-point 20^3, fp64: 18 (35).
+    auto groups = [&](int64_t rows_each, int64_t least, int64_t most) {
+        const int64_t n = A_rows / rows_each;
+        return n < least ? least : n > most ? most : n;
+    };
+    auto longer = [&](auto value) -> int {
+        using T = decltype(value);
+        BackArgs<T> g{A_rows, 8, (const T *)gC, C_indices, C_indptr, (const T *)A_data, A_indices, A_indptr,
+                      (const T *)B_data, B_indices, B_indptr, (T *)grad_A, (T *)grad_B};
+        auto launch = [&](auto kernel, int threads, size_t lds, int64_t groups) -> int {
+            for (g.piece = 8; g.piece > 1 && A_rows < groups * g.piece;) g.piece /= 2;
+            const int64_t most = nm::ceil_div(A_rows, g.piece);
+            if (lds > 64 * 1024)
+                NM_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+            hipLaunchKernelGGL(kernel, dim3((unsigned)(most < groups ? most : groups)), dim3(threads), lds, s, g);
+            return NM_OK;
+        };
+        if (int rc = launch(spgemm_bwd_mid_kernel<T>, kBackMid, kBackMidLds<T>, groups(4, 512, 4096))) return rc;
+        NM_LAUNCH_CHECK("spgemm_bwd_mid_kernel");
+        if (int rc = launch(spgemm_bwd_long_kernel<T>, 1024, BackLongRow<T>::lds, groups(128, 256, 1024))) return rc;
         NM_LAUNCH_CHECK("spgemm_bwd_long_kernel");
         return NM_OK;
     };
-    auto all = [&](auto value, auto most) -> int {
-        using T = decltype(value);
-        if (int rc = longer(BackShape<T, 64, 512, 4>{}, 16384, kBwdStage, 512)) return rc;
-        if (int rc = longer(BackShape<T, 256, 2048, 4>{}, 4096, 512, 2048)) return rc;
-        if (int rc = longer(BackShape<T, 512, 4096, 4>{}, 4096, 2048, 4096)) return rc;
-        return longer(BackShape<T, 1024, decltype(most)::value, 4>{}, 2048, 4096, INT64_MAX);
-    };
-    if (int rc = dt == NM_F32 ? all(0.0f, std::integral_constant<int, 14336>{})
-                              : all(0.0, std::integral_constant<int, 8192>{}))
-        return rc;
-    return NM_OK;
+    return dt == NM_F32 ? longer(0.0f) : longer(0.0);
 }

@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 import torch
 
+import numml_amd
 import oracle
 from numml_amd import generators as G
 from numml_amd import numml_torch_cpp as ext
@@ -158,3 +159,61 @@ def test_products_that_meet(dev, dtype, hubs):
     B = [np.unique(np.append(rng.integers(0, hubs, rng.integers(1, 4)), [hubs + k, hubs + K + k])) for k in range(K)]
     A = [np.sort(rng.choice(K, n, replace=False)) for n in (60, 70, 120, 200, 250, 400, 500, 900, 1000, 1900, 2047, K)]
     _check(dev, _csr(A, K, 1, dtype), _csr(B, hubs + 2 * K, 2, dtype), dtype)
+
+
+# the backward's lists of long rows: workgroups that look at 1, 2, 4 or 8 rows side by side, lengths of C's rows at
+# both sides of each list's limits, any order
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("rows", [1, 37, 700, 1500, 3000, 5000, 9001])
+def test_rows_of_all_lengths_in_a_matrix(dev, dtype, rows):
+    rng = np.random.default_rng(rows)
+    lengths = np.where(rng.random(rows) < 0.9, rng.integers(0, 12, rows), 0)
+    special = [64, 65, 512, 513, 2048, 2049, 2500]
+    at = rng.permutation(rows)[:min(rows, 60)]
+    lengths[at] = [special[k % 7] for k in range(at.size)]
+    A = [np.sort(rng.choice(2600, n, replace=False)) for n in lengths]
+    B = [[k] if k % 5 else [k, 2600 + k] for k in range(2600)]
+    _check(dev, _csr(A, 2600, 1, dtype), _csr(B, 5200, 2, dtype), dtype)
+
+
+def test_long_rows_behind_a_million_short_ones(dev):
+    rows, K = 1_300_001, 3000
+    lengths = np.ones(rows, np.int64)
+    long = [3, 1_048_575, 1_048_576, 1_048_577, 1_100_000, 1_299_999, 1_300_000]
+    lengths[long] = [100, 600, 3000, 2049, 513, 65, 2048]
+    indptr = np.concatenate([[0], np.cumsum(lengths)])
+    indices = np.zeros(indptr[-1], np.int64)
+    indices[indptr[:-1]] = np.arange(rows) % K
+    for r in long:
+        indices[indptr[r]:indptr[r + 1]] = np.arange(lengths[r])
+    a = randn(1, indices.size, np.float64), indices, indptr, (rows, K)
+    _check(dev, a, _csr([[k] for k in range(K)], K, 2, np.float64), np.float64)
+
+
+def test_the_time_of_finding_no_long_rows(dev):
+    # both gradients of a stencil's product take as long as the product; with a launch for each of four
+    # shapes of long row that is not there they took 1.7 times as long
+    c = numml_amd.load_compiled()
+    d, i, p, (n, _) = G.poisson2d(300, np.float32)
+    a = to_dev(dev, d, i, p)
+    old = c.backward_mode()
+    c.set_backward_mode("atomic")
+    try:
+        Cd, Ci, Cp = c.spgemm_forward(n, n, *a, n, n, *a)
+        times = []
+        for f in (lambda: c.spgemm_forward(n, n, *a, n, n, *a),
+                  lambda: c.spgemm_backward(Cd, Ci, Cp, n, n, *a, n, n, *a)):
+            best = float("inf")
+            for _ in range(8):
+                t0, t1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+                torch.cuda.synchronize()
+                t0.record()
+                for _ in range(20):
+                    f()
+                t1.record()
+                torch.cuda.synchronize()
+                best = min(best, t0.elapsed_time(t1))
+            times.append(best)
+    finally:
+        c.set_backward_mode(old)
+    assert times[1] < 1.4 * times[0], times
