@@ -59,7 +59,8 @@ constexpr int kAhead = 8;            // B rows whose first columns a group reque
 #endif
 
 // bin upper limits (inclusive); the last bin takes the rest and spills
-constexpr int32_t kSymLimit[kBins - 1] = {64, 128, 256, 512, 1024, 2048, 8192, 24576, 24576};   // on the product bound
+// on the product bound (the symbolic phase has a bin less than the numeric one: the eighth takes no row)
+constexpr int32_t kSymLimit[kBins - 1] = {64, 128, 256, 512, 1024, 2048, 8192, 24576, 24576};
 // on the exact row length; the last one is what a whole CU's LDS holds (kRowLimitMost below)
 constexpr int32_t kNumLimit[kBins - 2] = {32, 64, 128, 256, 512, 1024, 2048, 4096};
 // lanes per row and table sizes per bin.  The kernels wait on memory (A's row, the bounds of its B
@@ -75,10 +76,10 @@ constexpr int32_t kColEnd = 0x7fffffff;       // past-the-end column of a staged
 constexpr int32_t kMergedKey = -1;            // binning key of a row the merge path has taken
 
 struct Work {
-    int32_t *key;      // [rows] binning key (product bound, then exact length)
+    int32_t *key;      // [rows] binning key of the symbolic phase (product bound)
     int32_t *perm;     // [rows] rows grouped by bin
     int32_t *bins;     // [kBinInts]: rows per bin [0, kBins), first row of bin b at kBinStart + b (end at + b + 1), cursor at kBinCursor + b
-    int32_t *count;    // [rows + 1] entries per row of C, before the row pointer is made of them
+    int32_t *count;    // [rows + 1] entries per row of C: the row pointer is made of them, the numeric phase bins by them
     int64_t *scan;     // [tiles + 1] sums of the counts by tile of the row pointer's scan
     int32_t *mark;     // [spill_groups(B_cols) * B_cols]
     double *acc;       // [spill_groups(B_cols) * B_cols]
@@ -396,15 +397,16 @@ __global__ __launch_bounds__(kBlock) void numeric_front_kernel(
     if (it & 7) flush(it & ~7);
 }
 
-// key[i] = C_indptr[i+1] - C_indptr[i], except for rows the merge path has taken
-__global__ void row_length_kernel(int64_t rows, const int64_t *__restrict__ C_indptr,
-                                  int32_t *__restrict__ key) {
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < rows; i += stride)
-        if (key[i] != kMergedKey) key[i] = (int32_t)(C_indptr[i + 1] - C_indptr[i]);
-}
-
-// negative keys (rows taken by the merge path) belong to no bin
+// What the rows are binned by: their key (the symbolic phase), or the length of their row of C, which the
+// symbolic phase has left in `count` (the numeric phase).  Negative keys (rows taken by the merge
+// path) belong to no bin.
+struct RowKeys {
+    const int32_t *key, *count;   // count: null where the key itself is meant
+    __device__ __forceinline__ int32_t operator[](int64_t i) const {
+        const int32_t k = key[i], n = count ? count[i] : k;
+        return k < 0 ? k : n;
+    }
+};
 struct BinLimits { int32_t l[kBins - 1]; };
 __device__ __forceinline__ int bin_of(int32_t k, const BinLimits &lim) {
     if (k < 0) return -1;
@@ -420,7 +422,7 @@ __global__ void bin_clear_kernel(int32_t *bins) {
 
 // Rows per bin.  Each wavefront counts with ballots (one population count per
 // bin) instead of 64 colliding LDS atomics.
-__global__ __launch_bounds__(kBlock) void bin_count_kernel(int64_t rows, const int32_t *__restrict__ key,
+__global__ __launch_bounds__(kBlock) void bin_count_kernel(int64_t rows, RowKeys key,
                                                            BinLimits lim, int32_t *bins) {
     __shared__ int s_cnt[kBins];
     if (threadIdx.x < kBins) s_cnt[threadIdx.x] = 0;
@@ -458,7 +460,7 @@ __global__ void bin_offsets_kernel(int32_t *bins) {
 // and C lines).  A workgroup takes ONE contiguous slice of the rows, counts it, claims its room
 // in every bin with one atomic per bin, and then places the rows: thousands of workgroups claiming
 // room 256 rows at a time queued up on the eight cursors (96 us for 2.1 M rows).
-__global__ __launch_bounds__(kBlock) void bin_scatter_kernel(int64_t rows, const int32_t *__restrict__ key,
+__global__ __launch_bounds__(kBlock) void bin_scatter_kernel(int64_t rows, RowKeys key,
                                                              BinLimits lim, int32_t *bins,
                                                              int32_t *__restrict__ perm) {
     constexpr int kWaves = kBlock / kWave;
@@ -468,16 +470,25 @@ __global__ __launch_bounds__(kBlock) void bin_scatter_kernel(int64_t rows, const
     const int64_t per = ((rows + gridDim.x - 1) / gridDim.x + kBlock - 1) / kBlock * kBlock;   // whole steps
     const int64_t r0 = (int64_t)blockIdx.x * per, r1 = r0 + per < rows ? r0 + per : rows;
     if (r0 >= rows) return;
+    // (where the rows of a wavefront are all of one bin, as a stencil's are, one ballot does for ten: 1 M rows
+    // 21 -> 17 us)
     {   // count the slice
         int mine[kBins] = {};
+        if (lane == 0)
+            for (int q = 0; q < kBins; ++q) s_wave[wave][q] = 0;
         for (int64_t i0 = r0; i0 < r1; i0 += kBlock) {
             const int64_t i = i0 + threadIdx.x;
             const int b = i < r1 ? bin_of(key[i], lim) : -1;
+            const int b0 = __builtin_amdgcn_readfirstlane(b);
+            if (__ballot(b == b0) == ~0ull) {
+                if (lane == 0 && b0 >= 0) s_wave[wave][b0] += kWave;
+                continue;
+            }
 #pragma unroll
             for (int q = 0; q < kBins; ++q) mine[q] += __popcll(__ballot(b == q));
         }
         if (lane == 0)
-            for (int q = 0; q < kBins; ++q) s_wave[wave][q] = mine[q];
+            for (int q = 0; q < kBins; ++q) s_wave[wave][q] += mine[q];
         __syncthreads();
         if (threadIdx.x < kBins) {
             int total = 0;
@@ -490,11 +501,17 @@ __global__ __launch_bounds__(kBlock) void bin_scatter_kernel(int64_t rows, const
         const int64_t i = i0 + threadIdx.x;
         const int b = i < r1 ? bin_of(key[i], lim) : -1;
         int before = 0;   // rows of my bin in lower lanes of my wavefront
+        const int b0 = __builtin_amdgcn_readfirstlane(b);
+        if (__ballot(b == b0) == ~0ull) {
+            before = lane;
+            if (lane < kBins) s_wave[wave][lane] = lane == b0 ? kWave : 0;
+        } else {
 #pragma unroll
-        for (int q = 0; q < kBins; ++q) {
-            const unsigned long long m = __ballot(b == q);
-            if (b == q) before = __popcll(m & ((1ull << lane) - 1ull));
-            if (lane == 0) s_wave[wave][q] = __popcll(m);
+            for (int q = 0; q < kBins; ++q) {
+                const unsigned long long m = __ballot(b == q);
+                if (b == q) before = __popcll(m & ((1ull << lane) - 1ull));
+                if (lane == 0) s_wave[wave][q] = __popcll(m);
+            }
         }
         __syncthreads();
         if (b >= 0) {
@@ -641,7 +658,7 @@ __global__ void summary_out_kernel(const int64_t *__restrict__ summary, volatile
 // work: count, offsets, then rows placed in ascending order inside each bin (ballots, as in the
 // grid-wide kernels).
 constexpr int kBinSmallRows = 4096;
-__global__ __launch_bounds__(1024) void bin_small_kernel(int64_t rows, const int32_t *__restrict__ key,
+__global__ __launch_bounds__(1024) void bin_small_kernel(int64_t rows, RowKeys key,
                                                          BinLimits lim, int32_t *bins,
                                                          int32_t *__restrict__ perm) {
     constexpr int kWaves = 1024 / kWave;
@@ -698,11 +715,11 @@ __global__ __launch_bounds__(1024) void bin_small_kernel(int64_t rows, const int
     if (threadIdx.x < kBins) bins[threadIdx.x] = s_start[threadIdx.x + 1] - s_start[threadIdx.x];
 }
 
-int bin_rows(int64_t rows, const int32_t limit[kBins - 1], const Work &w, hipStream_t s) {
+int bin_rows(int64_t rows, RowKeys key, const int32_t limit[kBins - 1], const Work &w, hipStream_t s) {
     BinLimits lim;
     for (int q = 0; q < kBins - 1; ++q) lim.l[q] = limit[q];
     if (rows <= kBinSmallRows) {
-        hipLaunchKernelGGL(bin_small_kernel, dim3(1), dim3(1024), 0, s, rows, w.key, lim, w.bins, w.perm);
+        hipLaunchKernelGGL(bin_small_kernel, dim3(1), dim3(1024), 0, s, rows, key, lim, w.bins, w.perm);
         NM_LAUNCH_CHECK("bin_small_kernel");
         return NM_OK;
     }
@@ -711,9 +728,9 @@ int bin_rows(int64_t rows, const int32_t limit[kBins - 1], const Work &w, hipStr
     if (grid > 512) grid = 512;
     if (grid < 1) grid = 1;
     hipLaunchKernelGGL(bin_clear_kernel, dim3(1), dim3(64), 0, s, w.bins);
-    hipLaunchKernelGGL(bin_count_kernel, dim3((unsigned)grid), dim3(kBlock), 0, s, rows, w.key, lim, w.bins);
+    hipLaunchKernelGGL(bin_count_kernel, dim3((unsigned)grid), dim3(kBlock), 0, s, rows, key, lim, w.bins);
     hipLaunchKernelGGL(bin_offsets_kernel, dim3(1), dim3(64), 0, s, w.bins);
-    hipLaunchKernelGGL(bin_scatter_kernel, dim3((unsigned)grid), dim3(kBlock), 0, s, rows, w.key, lim, w.bins,
+    hipLaunchKernelGGL(bin_scatter_kernel, dim3((unsigned)grid), dim3(kBlock), 0, s, rows, key, lim, w.bins,
                        w.perm);
     NM_LAUNCH_CHECK("bin kernels");
     return NM_OK;
@@ -857,6 +874,42 @@ template <int TPB, typename V> __device__ __forceinline__ V row_scan(V v, V *s_w
     }
 }
 
+// Spill path: distinct columns counted with a stamped dense marker per workgroup (of the first `groups`).
+__device__ __forceinline__ void symbolic_spill(
+    const int32_t *__restrict__ bins, const int32_t *__restrict__ perm, int64_t B_cols, int groups,
+    const int64_t *__restrict__ A_indices, const int64_t *__restrict__ A_indptr,
+    const int64_t *__restrict__ B_indices, const int64_t *__restrict__ B_indptr, int32_t *mark_all,
+    int32_t *__restrict__ C_count) {
+    __shared__ int s_red[kSpillBlock / kWave];
+    const int32_t b0 = bins[kBinStart + kBins - 1], b1 = bins[kBinStart + kBins];
+    if ((int)blockIdx.x >= groups || b0 + (int32_t)blockIdx.x >= b1) return;
+    int32_t *mark = mark_all + (size_t)blockIdx.x * (B_cols + 1);
+    for (int64_t c = threadIdx.x; c < B_cols; c += kSpillBlock) mark[c] = 0;
+    __syncthreads();
+    const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    for (int32_t idx = b0 + blockIdx.x; idx < b1; idx += groups) {
+        const int64_t row = perm[idx];
+        const int32_t stamp = (int32_t)row + 1;
+        int cnt = 0;
+        const int64_t je = A_indptr[row + 1];
+        for (int64_t jj = A_indptr[row] + wave; jj < je; jj += kSpillBlock / kWave) {
+            const int64_t j = A_indices[jj];
+            const int64_t ke = B_indptr[j + 1];
+            for (int64_t kk = B_indptr[j] + lane; kk < ke; kk += kWave)
+                if (atomicExch(mark + B_indices[kk], stamp) != stamp) ++cnt;
+        }
+        cnt = nm::wave_sum(cnt);
+        if (lane == 0) s_red[wave] = cnt;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            int t = 0;
+            for (int w = 0; w < kSpillBlock / kWave; ++w) t += s_red[w];
+            C_count[row] = t;
+        }
+        __syncthreads();
+    }
+}
+
 // Rows of many products: one row per workgroup, its products numbered through and dealt to the
 // threads by number (see numeric_row_kernel); a set has no order to keep, so there are no turns.
 // Bound by the row's chain of round trips (A's row, the bounds of B's rows, their columns).  A
@@ -864,7 +917,9 @@ template <int TPB, typename V> __device__ __forceinline__ V row_scan(V v, V *s_w
 // groups of 64 and 256 lanes that took B's rows one by one: 257-512 43 -> 22 us, 513-1024 70 -> 29,
 // 1025-2048 51 -> 20, 2049-8192 106 -> 44, more (a marker per column in global memory) 94 -> 17.  Groups
 // of 16 lanes with their tables side by side stay ahead below 256 products (46 us for 129-256).
-template <int TPB_, int SLOTS_> struct SetShape {
+// The launch for the longest rows takes those that spill as well.
+template <int TPB_, int SLOTS_, bool SPILL_ = false> struct SetShape {
+    static constexpr bool SPILL = SPILL_;
     static constexpr int TPB = TPB_, SLOTS = SLOTS_, BATCH = TPB < 512 ? TPB : 512, UNROLL = 4;
     static constexpr size_t at_row = 8 * (BATCH + 2), at_wave = at_row + 8 * BATCH, at_key = at_wave + 8 * (TPB / kWave) + 16;
     static constexpr size_t lds = at_key + 4 * SLOTS;
@@ -874,7 +929,8 @@ template <typename S>
 __global__ __launch_bounds__(S::TPB) void symbolic_row_kernel(
     int bin, const int32_t *__restrict__ bins, const int32_t *__restrict__ perm,
     const int64_t *__restrict__ A_indices, const int64_t *__restrict__ A_indptr,
-    const int64_t *__restrict__ B_indices, const int64_t *__restrict__ B_indptr, int32_t *__restrict__ C_count) {
+    const int64_t *__restrict__ B_indices, const int64_t *__restrict__ B_indptr, int32_t *__restrict__ C_count,
+    int64_t B_cols, int32_t *mark, int spill_groups) {
     constexpr int TPB = S::TPB, SLOTS = S::SLOTS, BATCH = S::BATCH, U = S::UNROLL;
     extern __shared__ __align__(16) unsigned char s_raw[];
     int64_t *s_off = reinterpret_cast<int64_t *>(s_raw);               // number of an entry's first product
@@ -932,48 +988,16 @@ __global__ __launch_bounds__(S::TPB) void symbolic_row_kernel(
         if (tid == 0) C_count[row] = all;
         __syncthreads();
     }
+    if constexpr (S::SPILL) {
+        static_assert(TPB == kSpillBlock && S::lds + 256 <= 160 * 1024, "the spill path's workgroup and LDS");
+        symbolic_spill(bins, perm, B_cols, spill_groups, A_indices, A_indptr, B_indices, B_indptr, mark, C_count);
+    }
 }
 using SetShape3 = SetShape<64, 768>;      // up to 512 products
 using SetShape4 = SetShape<64, 1536>;     // up to 1024
 using SetShape5 = SetShape<256, 3072>;    // up to 2048
 using SetShape6 = SetShape<512, 10240>;   // up to 8192
-using SetShape7 = SetShape<1024, 32768>;  // up to 24576
-
-// Spill path: distinct columns counted with a stamped dense marker per workgroup.
-__global__ __launch_bounds__(kSpillBlock) void symbolic_spill_kernel(
-    const int32_t *__restrict__ bins, const int32_t *__restrict__ perm, int64_t B_cols,
-    const int64_t *__restrict__ A_indices, const int64_t *__restrict__ A_indptr,
-    const int64_t *__restrict__ B_indices, const int64_t *__restrict__ B_indptr, int32_t *mark_all,
-    int32_t *__restrict__ C_count) {
-    __shared__ int s_red[kSpillBlock / kWave];
-    const int32_t b0 = bins[kBinStart + kBins - 1], b1 = bins[kBinStart + kBins];
-    if (b0 + (int32_t)blockIdx.x >= b1) return;
-    int32_t *mark = mark_all + (size_t)blockIdx.x * (B_cols + 1);
-    for (int64_t c = threadIdx.x; c < B_cols; c += kSpillBlock) mark[c] = 0;
-    __syncthreads();
-    const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    for (int32_t idx = b0 + blockIdx.x; idx < b1; idx += gridDim.x) {
-        const int64_t row = perm[idx];
-        const int32_t stamp = (int32_t)row + 1;
-        int cnt = 0;
-        const int64_t je = A_indptr[row + 1];
-        for (int64_t jj = A_indptr[row] + wave; jj < je; jj += kSpillBlock / kWave) {
-            const int64_t j = A_indices[jj];
-            const int64_t ke = B_indptr[j + 1];
-            for (int64_t kk = B_indptr[j] + lane; kk < ke; kk += kWave)
-                if (atomicExch(mark + B_indices[kk], stamp) != stamp) ++cnt;
-        }
-        cnt = nm::wave_sum(cnt);
-        if (lane == 0) s_red[wave] = cnt;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            int t = 0;
-            for (int w = 0; w < kSpillBlock / kWave; ++w) t += s_red[w];
-            C_count[row] = t;
-        }
-        __syncthreads();
-    }
-}
+using SetShape7 = SetShape<1024, 32768, true>;   // up to 24576, and the rest
 
 // ---- numeric -------------------------------------------------------------------
 
@@ -1154,6 +1178,83 @@ __global__ __launch_bounds__(kBlock) void numeric_hash_kernel(
     }
 }
 
+// Spill path: dense accumulator slice per workgroup (of the first `groups`), emitted by a scan of the
+// touched column range (ascending by construction).
+template <typename T>
+__device__ __forceinline__ void numeric_spill(
+    const int32_t *__restrict__ bins, const int32_t *__restrict__ perm, int64_t B_cols, int groups,
+    const T *__restrict__ A_data, const int64_t *__restrict__ A_indices,
+    const int64_t *__restrict__ A_indptr, const T *__restrict__ B_data,
+    const int64_t *__restrict__ B_indices, const int64_t *__restrict__ B_indptr,
+    const int64_t *__restrict__ C_indptr, int64_t *__restrict__ C_indices, T *__restrict__ C_data,
+    int32_t *mark_all, double *acc_all) {
+    __shared__ int64_t s_wave[kSpillBlock / kWave];
+    __shared__ unsigned long long s_lo, s_hi;
+    const int32_t b0 = bins[kBinStart + kBins - 1], b1 = bins[kBinStart + kBins];
+    if ((int)blockIdx.x >= groups || b0 + (int32_t)blockIdx.x >= b1) return;
+    int32_t *mark = mark_all + (size_t)blockIdx.x * (B_cols + 1);
+    T *acc = reinterpret_cast<T *>(acc_all + (size_t)blockIdx.x * (B_cols + 1));
+    for (int64_t c = threadIdx.x; c < B_cols; c += kSpillBlock) { mark[c] = 0; acc[c] = T(0); }
+    __syncthreads();
+    const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    for (int32_t idx = b0 + blockIdx.x; idx < b1; idx += groups) {
+        const int64_t row = perm[idx];
+        const int32_t stamp = -((int32_t)row + 1);
+        if (threadIdx.x == 0) { s_lo = ~0ull; s_hi = 0ull; }
+        __syncthreads();
+        unsigned long long lo = ~0ull, hi = 0ull;
+        const int64_t je = A_indptr[row + 1];
+        for (int64_t jj = A_indptr[row] + wave; jj < je; jj += kSpillBlock / kWave) {
+            const int64_t j = A_indices[jj];
+            const T a = A_data[jj];
+            const int64_t ke = B_indptr[j + 1];
+            for (int64_t kk = B_indptr[j] + lane; kk < ke; kk += kWave) {
+                const unsigned long long c = (unsigned long long)B_indices[kk];
+                nm::atomic_add(acc + c, a * B_data[kk]);
+                mark[c] = stamp;
+                lo = c < lo ? c : lo;
+                hi = c > hi ? c : hi;
+            }
+        }
+        if (lo != ~0ull) { atomicMin(&s_lo, lo); atomicMax(&s_hi, hi); }
+        __syncthreads();
+        const int64_t c_lo = (int64_t)s_lo, c_hi = (int64_t)s_hi;
+        int64_t out = C_indptr[row];
+        if (s_lo != ~0ull) {
+            // Every wavefront takes a contiguous segment of the touched column range: it counts its
+            // hits, the counts are summed over the wavefronts before it, and it then emits its
+            // segment in order.  (A workgroup-wide scan per 1024 columns cost two barriers each.)
+            constexpr int kWaves = kSpillBlock / kWave;
+            const int64_t span = c_hi - c_lo + 1;
+            const int64_t seg = ((span + kWaves - 1) / kWaves + kWave - 1) / kWave * kWave;
+            const int64_t sb = c_lo + wave * seg;
+            const int64_t se = sb + seg < c_hi + 1 ? sb + seg : c_hi + 1;
+            int64_t cnt = 0;
+            for (int64_t c0 = sb; c0 < se; c0 += kWave) {
+                const int64_t c = c0 + lane;
+                cnt += __popcll(__ballot(c < se && mark[c] == stamp));
+            }
+            if (lane == 0) s_wave[wave] = cnt;
+            __syncthreads();
+            for (int w = 0; w < wave; ++w) out += s_wave[w];
+            const unsigned long long below = (1ull << lane) - 1ull;
+            for (int64_t c0 = sb; c0 < se; c0 += kWave) {
+                const int64_t c = c0 + lane;
+                const bool hit = c < se && mark[c] == stamp;
+                const unsigned long long m = __ballot(hit);
+                if (hit) {
+                    const int64_t at = out + __popcll(m & below);
+                    C_indices[at] = c;
+                    C_data[at] = acc[c];
+                    acc[c] = T(0);
+                }
+                out += __popcll(m);
+            }
+        }
+        __syncthreads();
+    }
+}
+
 // ---- numeric, rows of more than 128 entries -------------------------------------------
 //
 // One row of C per workgroup.  The row's products are numbered in the order of A's row (and of
@@ -1177,8 +1278,10 @@ __global__ __launch_bounds__(kBlock) void numeric_hash_kernel(
 // lanes that applied A's entries one by one and ordered the row by ranks or a bitonic network:
 // 129-256 60 -> 33 us, 257-512 127 -> 39, 513-1024 136 -> 40, 1025-4096 806 -> 110, more (dense
 // accumulators in global memory) 854 -> 75.
-template <typename T_, int TPB_, int SLOTS_, int LIMIT_, int UNROLL_> struct RowShape {
+// The launch for the longest rows takes those that spill as well.
+template <typename T_, int TPB_, int SLOTS_, int LIMIT_, int UNROLL_, bool SPILL_ = false> struct RowShape {
     using T = T_;
+    static constexpr bool SPILL = SPILL_;
     static constexpr int TPB = TPB_, SLOTS = SLOTS_, LIMIT = LIMIT_, UNROLL = UNROLL_;
     static constexpr int BATCH = TPB < 512 ? TPB : 512;                      // entries of A's row at a time
     static constexpr int TURNS = TPB < 1024 ? (TPB == kWave ? 512 : 1024) : 1024;   // turn words, by slot
@@ -1208,7 +1311,8 @@ __global__ __launch_bounds__(S::TPB) void numeric_row_kernel(
     const typename S::T *__restrict__ A_data, const int64_t *__restrict__ A_indices,
     const int64_t *__restrict__ A_indptr, const typename S::T *__restrict__ B_data,
     const int64_t *__restrict__ B_indices, const int64_t *__restrict__ B_indptr,
-    const int64_t *__restrict__ C_indptr, int64_t *__restrict__ C_indices, typename S::T *__restrict__ C_data) {
+    const int64_t *__restrict__ C_indptr, int64_t *__restrict__ C_indices, typename S::T *__restrict__ C_data,
+    int64_t B_cols, int32_t *mark, double *acc, int spill_groups) {
     using T = typename S::T;
     constexpr int TPB = S::TPB, SLOTS = S::SLOTS, BATCH = S::BATCH, U = S::UNROLL, PER = S::PER;
     extern __shared__ __align__(16) unsigned char s_raw[];
@@ -1455,6 +1559,11 @@ __global__ __launch_bounds__(S::TPB) void numeric_row_kernel(
         for (int t = tid; t < n; t += TPB) C_data[base + t] = val[t];
         __syncthreads();
     }
+    if constexpr (S::SPILL) {
+        static_assert(TPB == kSpillBlock && S::lds + 256 <= 160 * 1024, "the spill path's workgroup and LDS");
+        numeric_spill<T>(bins, perm, B_cols, spill_groups, A_data, A_indices, A_indptr, B_data, B_indices, B_indptr,
+                         C_indptr, C_indices, C_data, mark, acc);
+    }
 }
 
 // The shapes: LDS decides how many rows a CU has in flight, so a row gets the smallest table that
@@ -1466,84 +1575,7 @@ template <typename T> using RowShape6 = RowShape<T, 512, 2816, 2048, 4>;
 template <typename T> using RowShape7 = RowShape<T, 1024, 5632, 4096, 4>;
 constexpr int32_t kRowLimitMost32 = 16384, kRowLimitMost64 = 10880;
 template <typename T>
-using RowShape8 = RowShape<T, 1024, sizeof(T) == 4 ? 18176 : 12224, sizeof(T) == 4 ? kRowLimitMost32 : kRowLimitMost64, 4>;
-
-// Spill path: dense accumulator slice per workgroup, emitted by a scan of the
-// touched column range (ascending by construction).
-template <typename T>
-__global__ __launch_bounds__(kSpillBlock) void numeric_spill_kernel(
-    const int32_t *__restrict__ bins, const int32_t *__restrict__ perm, int64_t B_cols,
-    const T *__restrict__ A_data, const int64_t *__restrict__ A_indices,
-    const int64_t *__restrict__ A_indptr, const T *__restrict__ B_data,
-    const int64_t *__restrict__ B_indices, const int64_t *__restrict__ B_indptr,
-    const int64_t *__restrict__ C_indptr, int64_t *__restrict__ C_indices, T *__restrict__ C_data,
-    int32_t *mark_all, double *acc_all) {
-    __shared__ int64_t s_wave[kSpillBlock / kWave];
-    __shared__ unsigned long long s_lo, s_hi;
-    const int32_t b0 = bins[kBinStart + kBins - 1], b1 = bins[kBinStart + kBins];
-    if (b0 + (int32_t)blockIdx.x >= b1) return;
-    int32_t *mark = mark_all + (size_t)blockIdx.x * (B_cols + 1);
-    T *acc = reinterpret_cast<T *>(acc_all + (size_t)blockIdx.x * (B_cols + 1));
-    for (int64_t c = threadIdx.x; c < B_cols; c += kSpillBlock) { mark[c] = 0; acc[c] = T(0); }
-    __syncthreads();
-    const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    for (int32_t idx = b0 + blockIdx.x; idx < b1; idx += gridDim.x) {
-        const int64_t row = perm[idx];
-        const int32_t stamp = -((int32_t)row + 1);
-        if (threadIdx.x == 0) { s_lo = ~0ull; s_hi = 0ull; }
-        __syncthreads();
-        unsigned long long lo = ~0ull, hi = 0ull;
-        const int64_t je = A_indptr[row + 1];
-        for (int64_t jj = A_indptr[row] + wave; jj < je; jj += kSpillBlock / kWave) {
-            const int64_t j = A_indices[jj];
-            const T a = A_data[jj];
-            const int64_t ke = B_indptr[j + 1];
-            for (int64_t kk = B_indptr[j] + lane; kk < ke; kk += kWave) {
-                const unsigned long long c = (unsigned long long)B_indices[kk];
-                nm::atomic_add(acc + c, a * B_data[kk]);
-                mark[c] = stamp;
-                lo = c < lo ? c : lo;
-                hi = c > hi ? c : hi;
-            }
-        }
-        if (lo != ~0ull) { atomicMin(&s_lo, lo); atomicMax(&s_hi, hi); }
-        __syncthreads();
-        const int64_t c_lo = (int64_t)s_lo, c_hi = (int64_t)s_hi;
-        int64_t out = C_indptr[row];
-        if (s_lo != ~0ull) {
-            // Every wavefront takes a contiguous segment of the touched column range: it counts its
-            // hits, the counts are summed over the wavefronts before it, and it then emits its
-            // segment in order.  (A workgroup-wide scan per 1024 columns cost two barriers each.)
-            constexpr int kWaves = kSpillBlock / kWave;
-            const int64_t span = c_hi - c_lo + 1;
-            const int64_t seg = ((span + kWaves - 1) / kWaves + kWave - 1) / kWave * kWave;
-            const int64_t sb = c_lo + wave * seg;
-            const int64_t se = sb + seg < c_hi + 1 ? sb + seg : c_hi + 1;
-            int64_t cnt = 0;
-            for (int64_t c0 = sb; c0 < se; c0 += kWave) {
-                const int64_t c = c0 + lane;
-                cnt += __popcll(__ballot(c < se && mark[c] == stamp));
-            }
-            if (lane == 0) s_wave[wave] = cnt;
-            __syncthreads();
-            for (int w = 0; w < wave; ++w) out += s_wave[w];
-            const unsigned long long below = (1ull << lane) - 1ull;
-            for (int64_t c0 = sb; c0 < se; c0 += kWave) {
-                const int64_t c = c0 + lane;
-                const bool hit = c < se && mark[c] == stamp;
-                const unsigned long long m = __ballot(hit);
-                if (hit) {
-                    const int64_t at = out + __popcll(m & below);
-                    C_indices[at] = c;
-                    C_data[at] = acc[c];
-                    acc[c] = T(0);
-                }
-                out += __popcll(m);
-            }
-        }
-        __syncthreads();
-    }
-}
+using RowShape8 = RowShape<T, 1024, sizeof(T) == 4 ? 18176 : 12224, sizeof(T) == 4 ? kRowLimitMost32 : kRowLimitMost64, 4, true>;
 
 // ---- backward --------------------------------------------------------------------
 
@@ -1933,20 +1965,16 @@ int launch_numeric(const Work &w, int64_t B_cols, const void *A_data, const int6
             NM_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(k),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::lds));
         hipLaunchKernelGGL(k, dim3(grid), dim3(S::TPB), S::lds, s, bin, w.bins, w.perm, Ad, A_indices, A_indptr, Bd,
-                           B_indices, B_indptr, C_indptr, C_indices, Cd);
+                           B_indices, B_indptr, C_indptr, C_indices, Cd, B_cols, w.mark, w.acc, spill_groups(B_cols));
         NM_LAUNCH_CHECK("numeric_row_kernel");
         return NM_OK;
     };
-    if (int rc = rows(RowShape3<T>{}, 3, 2 * kPersistGrid)) return rc;
-    if (int rc = rows(RowShape4<T>{}, 4, 2 * kPersistGrid)) return rc;
+    if (int rc = rows(RowShape3<T>{}, 3, kPersistGrid)) return rc;
+    if (int rc = rows(RowShape4<T>{}, 4, kPersistGrid)) return rc;
     if (int rc = rows(RowShape5<T>{}, 5, kPersistGrid)) return rc;
     if (int rc = rows(RowShape6<T>{}, 6, 2048)) return rc;
     if (int rc = rows(RowShape7<T>{}, 7, 1024)) return rc;
     if (int rc = rows(RowShape8<T>{}, 8, 512)) return rc;
-    hipLaunchKernelGGL(numeric_spill_kernel<T>, dim3(spill_groups(B_cols)), dim3(kSpillBlock), 0, s, w.bins, w.perm,
-                       B_cols, Ad, A_indices, A_indptr, Bd, B_indices, B_indptr, C_indptr, C_indices, Cd, w.mark,
-                       w.acc);
-    NM_LAUNCH_CHECK("numeric_spill_kernel");
     return NM_OK;
 }
 
@@ -2028,7 +2056,7 @@ int symbolic_phase(int64_t A_rows, int64_t A_cols, int64_t B_cols, const int64_t
         }
     }
     {
-    if (int rc = bin_rows(A_rows, kSymLimit, w, s)) return rc;
+    if (int rc = bin_rows(A_rows, RowKeys{w.key, nullptr}, kSymLimit, w, s)) return rc;
 
     hipLaunchKernelGGL((symbolic_hash_kernel<kGroup0, kSymTable0>), dim3(kPersistGrid), dim3(kBlock), 0, s, 0, w.bins,
                        w.perm, A_indices, A_indptr, B_indices, B_indptr, w.count);
@@ -2044,19 +2072,15 @@ int symbolic_phase(int64_t A_rows, int64_t A_cols, int64_t B_cols, const int64_t
             NM_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(k),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::lds));
         hipLaunchKernelGGL(k, dim3(grid), dim3(S::TPB), S::lds, s, bin, w.bins, w.perm, A_indices, A_indptr,
-                           B_indices, B_indptr, w.count);
+                           B_indices, B_indptr, w.count, B_cols, w.mark, spill_groups(B_cols));
         NM_LAUNCH_CHECK("symbolic_row_kernel");
         return NM_OK;
     };
-    if (int rc = sets(SetShape3{}, 3, 2 * kPersistGrid)) return rc;
-    if (int rc = sets(SetShape4{}, 4, 2 * kPersistGrid)) return rc;
+    if (int rc = sets(SetShape3{}, 3, kPersistGrid)) return rc;
+    if (int rc = sets(SetShape4{}, 4, kPersistGrid)) return rc;
     if (int rc = sets(SetShape5{}, 5, kPersistGrid)) return rc;
     if (int rc = sets(SetShape6{}, 6, 1024)) return rc;
     if (int rc = sets(SetShape7{}, 7, 512)) return rc;
-    // (bins 7 and 8 share a limit: nothing is in bin 8)
-    hipLaunchKernelGGL(symbolic_spill_kernel, dim3(spill_groups(B_cols)), dim3(kSpillBlock), 0, s, w.bins, w.perm, B_cols,
-                       A_indices, A_indptr, B_indices, B_indptr, w.mark, w.count);
-    NM_LAUNCH_CHECK("symbolic_spill_kernel");
     }
     return row_pointer(w.bins, nullptr);
 }
@@ -2148,18 +2172,14 @@ extern "C" int nm_spgemm_numeric(nm_dtype dt, int64_t A_rows, int64_t A_cols, in
         return nm::fail(NM_ERR_WORKSPACE, "workspace of %zu bytes, %zu needed", workspace_bytes, need);
     if (A_rows == 0) return NM_OK;
     hipStream_t s = nm::as_stream(stream);
-    int64_t grid = nm::ceil_div(A_rows, kBlock);
-    if (grid > 65536) grid = 65536;
     // hash_rows == 0 (from nm_spgemm_symbolic_result): every row is one of the merge path's and
     // the binning and the hash launches, a dozen launches that would find nothing to do, are left out
     const bool hashed = hash_rows != 0;
     if (hashed) {
-        hipLaunchKernelGGL(row_length_kernel, dim3((unsigned)grid), dim3(kBlock), 0, s, A_rows, C_indptr, w.key);
-        NM_LAUNCH_CHECK("row_length_kernel");
         int32_t limit[kBins - 1];
         for (int q = 0; q < kBins - 2; ++q) limit[q] = kNumLimit[q];
         limit[kBins - 2] = dt == NM_F32 ? kRowLimitMost32 : kRowLimitMost64;
-        if (int rc = bin_rows(A_rows, limit, w, s)) return rc;
+        if (int rc = bin_rows(A_rows, RowKeys{w.key, w.count}, limit, w, s)) return rc;
     }
     const int64_t nbatch = nm::xcd_padded(nm::ceil_div(A_rows, kMergeRows));
     // (every row on the hash path: the merge kernel would look at each row's key and leave)

@@ -217,3 +217,14 @@ def test_the_time_of_finding_no_long_rows(dev):
     finally:
         c.set_backward_mode(old)
     assert times[1] < 1.4 * times[0], times
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("width, exact", [(300, True), (9000, True), (30_000, False)])
+def test_more_products_than_any_table_holds(dev, dtype, width, exact):
+    # 25 000 to 40 000 products a row, more such rows than there are workgroups with markers for them, beside rows
+    # of every other length; what comes out fits a small table, a large one, or none
+    rng = np.random.default_rng(width)
+    B = [np.unique(rng.integers(0, width, 100)) for _ in range(2000)]
+    A = [np.sort(rng.choice(2000, n, replace=False)) for n in [400, 1, 20, 300, 2, 90] * 24]
+    _check(dev, _csr(A, 2000, 1, dtype), _csr(B, width, 2, dtype), dtype, exact)
