@@ -2856,10 +2856,15 @@ extern "C" int64_t nm_sptrsv_plan_levels(const nm_sptrsv_plan *plan) { return pl
 
 extern "C" int64_t nm_sptrsv_plan_launches(const nm_sptrsv_plan *plan) {
     if (!plan) return -1;
-    // (of the solve with A; a stretch of wide levels that no team shares is launched level by level)
-    int64_t n = 0;
-    for (const auto &L : plan->launches)
-        n += L.run && !(plan->ell_pre[0] > 0 && L.team[0].P > 1) ? L.l1 - L.l0 : 1;
+    // (of the solve with A, as solve_typed issues them)
+    const bool teams = g_team_enabled.load();
+    int flow_a = 0, flow_b = 0;
+    if (teams) flow_stretch(plan, 0, &flow_a, &flow_b);
+    int64_t n = flow_b > flow_a ? 1 : 0;
+    for (int li = 0; li < (int)plan->launches.size(); ++li) {
+        const auto &L = plan->launches[li];
+        if (li < flow_a || li >= flow_b) n += by_level(plan, 0, teams, L) ? L.l1 - L.l0 : 1;
+    }
     return n;
 }
 

@@ -83,7 +83,16 @@ def _compare(dev, d, i, p, n, dtype, lower, unit, b=None):
                                                ((9, 10, 11, 12, 13), True, True), ((70, 64, 33), True, True)])
 def test_grids(dev, dtype, dims, lower, unit):
     print("case", dims, dtype.__name__, flush=True)
-    _compare(dev, *_grid(dims, dtype, lower, 1), dtype, lower, unit)
+    d, i, p, n = _grid(dims, dtype, lower, 1)
+    _compare(dev, d, i, p, n, dtype, lower, unit)
+    ext = numml_amd.load_compiled()
+    I, P = to_dev(dev, i, p)
+    one = ext.sptrsv_schedule(n, I, P, lower)[1]
+    try:
+        assert _lib.lib().nm_sptrsv_configure(0, 2) == 0
+        assert one < ext.sptrsv_schedule(n, I, P, lower)[1] - 4   # the wide levels one by one
+    finally:
+        assert _lib.lib().nm_sptrsv_configure(0, 0) == 0
 
 
 # layers at the edges of what goes level by level (1024 rows, 2 levels), of tiles (64 rows) and of the
@@ -92,9 +101,21 @@ def test_grids(dev, dtype, dims, lower, unit):
                                                  (40000, 4, 8), (1087, 9, 2), (4097, 6, 3), (5000, 5, 4),
                                                  (1100, 12, 5), (6001, 7, 8), (4200, 6, 9), (70000, 5, 3), (1500, 40, 4)])
 @pytest.mark.parametrize("lower", [True, False])
-def test_layers(dev, width, layers, deps, lower):
-    print("case", width, layers, deps, lower, flush=True)
-    _compare(dev, *_layers(width, layers, deps, np.float64, lower, width), np.float64, lower, False)
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_layers(dev, width, layers, deps, lower, dtype):
+    print("case", width, layers, deps, lower, dtype.__name__, flush=True)
+    d, i, p, n = _layers(width, layers, deps, dtype, lower, width)
+    _compare(dev, d, i, p, n, dtype, lower, False)
+    # one launch for all the layers, which is what gives up where waiting is not allowed
+    ext = numml_amd.load_compiled()
+    D, I, P, Bv = to_dev(dev, d, i, p, randn(5, n, dtype))
+    one = deps <= 8
+    assert tuple(ext.sptrsv_schedule(n, I, P, lower)) == (layers, 1 if one else layers)
+    try:
+        assert _lib.lib().nm_sptrsv_configure(-1, 0) == 0
+        assert bool(torch.isnan(ext.sptrsv_forward(n, n, D, I, P, lower, False, Bv)).all()) == one
+    finally:
+        assert _lib.lib().nm_sptrsv_configure(0, 0) == 0
 
 
 def test_not_a_number_and_infinity(dev):
