@@ -1567,7 +1567,8 @@ __global__ __launch_bounds__(S::TPB) void numeric_row_kernel(
 }
 
 // The shapes: LDS decides how many rows a CU has in flight, so a row gets the smallest table that
-// holds its bin at three quarters load; the last one takes the LDS of a whole CU.
+// holds its bin at three quarters load; the last one takes the LDS of a whole CU, at nine tenths, and
+// keeps ten registers (fp64: eleven) of a thread's share of the table in scratch memory.
 template <typename T> using RowShape3 = RowShape<T, 64, 384, 256, 2>;
 template <typename T> using RowShape4 = RowShape<T, 64, 704, 512, 2>;
 template <typename T> using RowShape5 = RowShape<T, 256, 1408, 1024, 2>;

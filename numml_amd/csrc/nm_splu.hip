@@ -31,7 +31,8 @@
 // reports an error.  Early pivots of a column
 // overlap with the tail of the columns before it, which is where a banded factor, whose
 // columns form one long dependency chain, gets its parallelism from.  Factors that stay within a
-// narrow band have a kernel of their own (lu_band_kernel, below).
+// narrow band have a kernel of their own (lu_band_kernel, below): one workgroup, whose wavefronts wait
+// for each other in LDS.  Those waits have no bound: the wavefronts of a workgroup run or none does.
 #include "nm_common.hpp"
 #include "nm_scan.hpp"
 
@@ -532,14 +533,13 @@ struct BandShared {
 #define NM_BAND_IF(i) "s_bitcmp1_b32 %[stored], %[S]+" #i "\n\ts_cselect_b64 exec, %[sv], 0\n\t"
 #define NM_BAND_P64(i, t) NM_BAND_IF(i) NM_BAND_D64(i, t)
 #define NM_BAND_P32(i, t) NM_BAND_IF(i) NM_BAND_D32(i, t)
-// (E: all lanes again before the next products)
-#define NM_BAND_SEQ2(M, D, E) M(0, 0) M(1, 1) D(0, 0) D(1, 1)
-#define NM_BAND_SEQ3(M, D, E) M(0, 0) M(1, 1) M(2, 2) D(0, 0) D(1, 1) D(2, 2)
-#define NM_BAND_SEQ4(M, D, E) M(0, 0) M(1, 1) M(2, 2) M(3, 3) D(0, 0) D(1, 1) D(2, 2) D(3, 3)
+#define NM_BAND_SEQ2(M, D) M(0, 0) M(1, 1) D(0, 0) D(1, 1)
+#define NM_BAND_SEQ3(M, D) M(0, 0) M(1, 1) M(2, 2) D(0, 0) D(1, 1) D(2, 2)
+#define NM_BAND_SEQ4(M, D) M(0, 0) M(1, 1) M(2, 2) M(3, 3) D(0, 0) D(1, 1) D(2, 2) D(3, 3)
 #define NM_BAND_ALL_LANES "s_mov_b64 exec, %[sv]\n\t"
 #define NM_BAND_TEXT(SEQ, M, D, P)                                                                                   \
-    "s_bfe_u32 %[bits], %[stored], %[field]\n\ts_cmp_eq_u32 %[bits], %[whole]\n\ts_cbranch_scc0 .Lpick_%=\n\t" SEQ(M, D, )  \
-    "s_branch .Ldone_%=\n.Lpick_%=:\n\ts_mov_b64 %[sv], exec\n\t" SEQ(M, P, NM_BAND_ALL_LANES) NM_BAND_ALL_LANES ".Ldone_%=:"
+    "s_bfe_u32 %[bits], %[stored], %[field]\n\ts_cmp_eq_u32 %[bits], %[whole]\n\ts_cbranch_scc0 .Lpick_%=\n\t" SEQ(M, D)    \
+    "s_branch .Ldone_%=\n.Lpick_%=:\n\ts_mov_b64 %[sv], exec\n\t" SEQ(M, P) NM_BAND_ALL_LANES ".Ldone_%=:"
 #define NM_BAND_W(i) [w##i] "+v"(W[S + i][q])
 #define NM_BAND_U(i) [u##i] "s"(u[S + i])
 #define NM_BAND_LIST2(X) X(0), X(1)
@@ -574,11 +574,11 @@ __device__ __forceinline__ void band_outer(T l, uint32_t stored, T u0, T u1, T &
     T t0, t1;
     constexpr int S = 0;
     if constexpr (sizeof(T) == 8)
-        asm volatile("s_mov_b64 %[sv], exec\n\t" NM_BAND_SEQ2(NM_BAND_M64, NM_BAND_P64, ) "s_mov_b64 exec, %[sv]"
+        asm volatile("s_mov_b64 %[sv], exec\n\t" NM_BAND_SEQ2(NM_BAND_M64, NM_BAND_P64) "s_mov_b64 exec, %[sv]"
                      : [w0] "+v"(w0), [w1] "+v"(w1), [t0] "=&v"(t0), [t1] "=&v"(t1), [sv] "=&s"(sv)
                      : [l] "v"(l), [stored] "s"(stored), [S] "n"(S), [u0] "s"(u0), [u1] "s"(u1) : "scc");
     else
-        asm volatile("s_mov_b64 %[sv], exec\n\t" NM_BAND_SEQ2(NM_BAND_M32, NM_BAND_P32, ) "s_mov_b64 exec, %[sv]"
+        asm volatile("s_mov_b64 %[sv], exec\n\t" NM_BAND_SEQ2(NM_BAND_M32, NM_BAND_P32) "s_mov_b64 exec, %[sv]"
                      : [w0] "+v"(w0), [w1] "+v"(w1), [t0] "=&v"(t0), [t1] "=&v"(t1), [sv] "=&s"(sv)
                      : [l] "v"(l), [stored] "s"(stored), [S] "n"(S), [u0] "s"(u0), [u1] "s"(u1) : "scc");
 }
