@@ -1276,8 +1276,8 @@ __device__ __forceinline__ void numeric_spill(
 // Bound by the row's chain of round trips and the barriers of the turns.  A 150 000-row power-law
 // graph squared (mean 8, rows up to 1000, fp32), by length of C's row, against groups of 64 and 256
 // lanes that applied A's entries one by one and ordered the row by ranks or a bitonic network:
-// 129-256 60 -> 33 us, 257-512 127 -> 39, 513-1024 136 -> 40, 1025-4096 806 -> 110, more (dense
-// accumulators in global memory) 854 -> 75.
+// 129-256 60 -> 34 us, 257-512 127 -> 40, 513-1024 136 -> 43, 1025-4096 806 -> 108, more (dense
+// accumulators in global memory) 854 -> 78.
 // The launch for the longest rows takes those that spill as well.
 template <typename T_, int TPB_, int SLOTS_, int LIMIT_, int UNROLL_, bool SPILL_ = false> struct RowShape {
     using T = T_;
