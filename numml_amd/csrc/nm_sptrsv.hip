@@ -1459,9 +1459,9 @@ __global__ __launch_bounds__(kBlock) void sptrsv_level_group_kernel(SolveArgs a,
 // none and solves that row itself.  Whoever solves a row stores the same bits, and a lane's
 // search waits for nobody, so the launch ends whatever part of it is on the chip.  (Drawing tiles from a
 // counter ends as surely and costs every launch: 12 ns a draw, 300^3 2.14 -> 5.6 ms with a tile a
-// draw, 3.8 with two, 97 x 89 x 101 325 -> 348 and 574 us.)  As a backstop a wavefront that has
-// polled `poll_limit` times for one tile raises the status word, every wavefront leaves when it
-// sees that, and the solve hands out NaN.
+// draw, 3.8 with two, 97 x 89 x 101 325 -> 348 and 574 us.)  A `poll_limit` below
+// kFlowPatience gives up instead of helping: a wavefront that has polled that often in a row raises the
+// status word and leaves, those that wait for its rows do so in turn, and the solve hands out NaN.
 constexpr unsigned long long kUnsolved = ~0ull;   // a NaN; a result with these bits is stored as the default NaN
 constexpr int kFlowMaxGroups = 256;
 constexpr int kFlowCrowd = 4096;   // more workgroups than the chip holds at once (a test's)
@@ -1571,7 +1571,6 @@ __global__ __launch_bounds__(kBlock) void sptrsv_flow_kernel(FlowArgs<T> f) {
     Operands o = operands(s);
     s = source(r);
     r = range((int64_t)wave + 2 * (int64_t)waves);
-    int64_t polls = f.poll_limit < 0 ? -1 : 0;
     int patience = kFlowPatience;
     for (int64_t tile = wave; tile < tiles; tile += waves) {
         const Operands cur = o;
@@ -1604,21 +1603,16 @@ __global__ __launch_bounds__(kBlock) void sptrsv_flow_kernel(FlowArgs<T> f) {
                 pending = false;
             }
             if (!__any(pending)) break;
-            ++polls;
-            if (polls > f.poll_limit) {
+            if (++waited > f.poll_limit) {
                 if (lane == 0) __hip_atomic_store(f.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 return;
             }
-            if ((polls & 1023) == 0 &&
-                __hip_atomic_load(f.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)
-                return;
-            if (++waited == patience) {
-                if (pending) help(cur.q);
+            if (waited == patience) {
+                if (pending) help(cur.q);   // (some row is solved: the waiting starts anew)
                 waited = 0;
                 patience = kFlowImpatience;
             }
         }
-        if (f.poll_limit >= 0) polls = 0;
         if (patience < kFlowPatience) ++patience;
     }
 }
