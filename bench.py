@@ -961,7 +961,7 @@ class SpSolve(Workload):
         self.dominant_bytes = self.nnz * (s + 8) + 2 * self.nnzM * (s + 8) + 3 * (rows + 1) * 8
         self.bytes_per_step = self.dominant_bytes + 4 * (self.nnzM * (s + 8) + (rows + 1) * 8 + 2 * rows * s) \
             + self.nnz * s
-        self.dominant_name = "splu on a cached pattern: lu_values_kernel, transpose_expand_kernel, lu_flow_kernel, transpose_scatter_kernel"
+        self.dominant_name = "splu on a cached pattern: lu_values_kernel, transpose_expand_kernel, lu_band_kernel, transpose_scatter_kernel"
         self.config = {"workload": f"spsolve_fwd_bwd_f64_poisson2d_{n}", "rows": rows, "nnz": self.nnz,
                        "nnz_LU": self.nnzM, "binding": _binding.name,
                        "pattern": "filled pattern and level schedules cached per structure; a step is what "
