@@ -499,12 +499,14 @@ int nm_sptrsv_solve(const nm_sptrsv_plan *plan, nm_dtype dt, int transposed,
  * receives the few values it needs from the others through device memory, running a
  * few levels behind the workgroup it receives from) are taken by one workgroup
  * instead, and a stretch of wider levels, otherwise one launch whose rows wait for each
- * other, gets a launch per level.  Results are the same bits either way.
+ * other, gets a launch per level; the triangle of a five-point or seven-point matrix, otherwise
+ * solved line by line by one launch (unless bit 0 is set), goes by levels as well.  Results are
+ * the same bits either way.
  * Bit 2 (for tests): the launch of a stretch of wide levels has more workgroups than the
  * device runs at once.
  * All waiting is for rows of lower levels.  A shared launch needs as many free compute
- * units as it has workgroups, at most sixteen; a stretch of wide levels is solved by
- * whatever part of its launch runs.  So the waits end; `poll_limit` bounds the polls of one wait all the same (0: the
+ * units as it has workgroups, at most sixteen; a stretch of wide levels and a grid's lines are
+ * solved by whatever part of their launch runs.  So the waits end; `poll_limit` bounds the polls of one wait all the same (0: the
  * default of 2^22, seconds; negative: give up at once, for tests): when it is
  * exceeded the waiting stops for good and x comes back as NaN throughout.
  * Process-wide; takes effect with the next solve. */

@@ -35,6 +35,8 @@
 // direct solve): there 16 or 64 lanes share a row and add their partial sums
 // across the group, which differs from the serial order by rounding in double.
 //
+// The triangle of a five-point or seven-point matrix goes line by line instead (nm_sptrsv_lines.hpp).
+//
 // Algorithmic HBM bytes of one solve (s = sizeof(value)):
 //   nnz*(s+8) + (rows+1)*8 + 2*rows*s
 #include "nm_common.hpp"
@@ -50,6 +52,8 @@
 #include <vector>
 
 namespace {
+#include "nm_sptrsv_lines.hpp"
+
 struct Packed {        // one solve direction, level-major (all int32, device)
     int32_t *dptr;     // [rows+1] dependency range of slot q
     int32_t *dslot;    // [nnz]    slot of the row a dependency refers to
@@ -58,6 +62,7 @@ struct Packed {        // one solve direction, level-major (all int32, device)
     int32_t *ell_ds;   // [ell_capacity] room for the fixed-width dependency entries: 16 bits each, `pre` per row
     int32_t *lvl_sig;  // [levels] which neighbouring wavefronts the rows of a level wait for (kSigLower | kSigHigher)
     int32_t *team;     // [team_capacity] exchange tables of the launches that several workgroups share
+    int32_t *lines;    // [rows][4] where a grid's lines find their values (lines::plan_kernel)
 };
 // Entries of the fixed-width (ELLPACK) arrays; the layout is used when (rows + kEllPad) * pre
 // fits.  kEllPad slots of padding follow the last row in every array the fixed-width kernel
@@ -121,6 +126,7 @@ struct nm_sptrsv_plan {
     std::vector<Launch> launches;
     int32_t team_cells[2] = {0, 0};   // mailbox cells one solve clears, per direction
     std::vector<int32_t> lp_host;     // level_ptr on the host (the level-by-level launches of a run)
+    lines::Grid grid;                 // length > 0: the triangle of a five-point or seven-point matrix
 };
 
 namespace {
@@ -190,6 +196,7 @@ size_t plan_layout(int64_t rows, int64_t nnz, void *base, Layout *L) {
         l.dir[d].ell_ds = take(ell_capacity(rows, nnz));
         l.dir[d].lvl_sig = take(rows + 1);
         l.dir[d].team = take(team_capacity(rows));
+        l.dir[d].lines = take(4 * rows);
     }
     if (L) *L = l;
     return off;
@@ -2119,6 +2126,11 @@ __global__ void unslot_kernel(int64_t n, const int32_t *__restrict__ order, cons
         x[order[q]] = (T)(failed ? nan : xs[q]);
 }
 
+// A grid's triangle goes line by line (nm_sptrsv_lines.hpp), whatever its sides.
+bool by_lines(const nm_sptrsv_plan *p) {
+    return p->grid.length > 0 && g_team_enabled.load() && !g_sig_enabled.load();
+}
+
 // A launch whose levels go one by one to a grid each (unless sptrsv_flow_kernel takes them).
 bool by_level(const nm_sptrsv_plan *p, int dirn, bool teams, const nm_sptrsv_plan::Launch &L) {
     return L.wide || (L.run && !(teams && p->ell_pre[dirn] > 0 && L.team[dirn].P > 1));
@@ -2163,6 +2175,11 @@ int solve_typed(const nm_sptrsv_plan *p, int transposed, const void *data, int u
     a.unit = unit;
     bool any_wide = false;
     const bool teams = g_team_enabled.load();
+    if (by_lines(p)) {
+        const T *dat = p->nnz > 0 ? (const T *)data : (const T *)b;
+        return lines::solve<T>(p->grid, p->rows, transposed ? p->lower : !p->lower, P.lines, dat, unit, (const T *)b, (T *)x,
+                               a.w.ell_coef, a.w.rb, a.w.coef, a.w.status, g_sig_poll_limit.load(), s);
+    }
     // the launches [flow_a, flow_b) that one sptrsv_flow_kernel takes
     int flow_a = 0, flow_b = 0;
     if (teams) flow_stretch(p, transposed ? 1 : 0, &flow_a, &flow_b);
@@ -2448,7 +2465,11 @@ extern "C" int nm_sptrsv_analyse(int64_t rows, int64_t nnz, const int64_t *indic
         }
     }
 
-    int32_t meta_h[4] = {0, 0, 0, 0};
+    int32_t meta_h[8] = {};
+    if (int rc = nm::fill_async(L.meta + 6, 1, (int32_t)0x7fffffff, s)) return bail(rc);
+    hipLaunchKernelGGL(lines::reach_kernel, dim3((unsigned)(rgrid > 1024 ? 1024 : rgrid)), dim3(kBlock), 0, s, (int32_t)rows,
+                       p->order, p->dir[0].dptr, p->dir[0].dslot, L.meta + 6);
+    if (hipGetLastError() != hipSuccess) return bail(nm::fail(NM_ERR_HIP, "lines::reach_kernel launch failed"));
     if (hipMemcpyAsync(meta_h, L.meta, sizeof(meta_h), hipMemcpyDeviceToHost, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess)
         return bail(nm::fail(NM_ERR_HIP, "reading the level count back failed: %s",
@@ -2458,6 +2479,18 @@ extern "C" int nm_sptrsv_analyse(int64_t rows, int64_t nnz, const int64_t *indic
     p->nlevels = meta_h[0];
     p->max_deps[0] = meta_h[2];
     p->max_deps[1] = meta_h[3];
+    // The lines of a grid: the smallest distance above 1 is a line, the largest a plane.  The per-call
+    // areas (solve_work_layout) hold what the lines need where there are as many entries as rows.
+    lines::Grid grid;
+    if (meta_h[6] == 0x7fffffff || p->max_deps[0] > 3 || p->max_deps[1] > 3 || nnz < rows ||
+        !lines::make_grid(rows, meta_h[6], meta_h[7] > meta_h[6] ? meta_h[7] : 0, &grid) || grid.edges() > nnz)
+        grid = lines::Grid();
+    for (int d = 0; d < 2 && grid.length > 0; ++d) {
+        hipLaunchKernelGGL(lines::plan_kernel, dim3((unsigned)(rgrid > 4096 ? 4096 : rgrid)), dim3(kBlock), 0, s, grid,
+                           (int32_t)rows, d == 0 ? !p->lower : p->lower, p->order, p->dir[d].dptr, p->dir[d].dslot,
+                           p->dir[d].dsrc, p->dir[d].diag, reinterpret_cast<int4 *>(p->dir[d].lines), L.meta + 8);
+        if (hipGetLastError() != hipSuccess) return bail(nm::fail(NM_ERR_HIP, "lines::plan_kernel launch failed"));
+    }
     std::vector<int32_t> lp((size_t)p->nlevels + 1);
     if (hipMemcpyAsync(lp.data(), p->level_ptr, lp.size() * 4, hipMemcpyDeviceToHost, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess)
@@ -2836,12 +2869,13 @@ extern "C" int nm_sptrsv_analyse(int64_t rows, int64_t nnz, const int64_t *indic
                 return bail(nm::fail(NM_ERR_HIP, "uploading the exchange tables failed"));
         }
     }
-    int32_t reach_h[2] = {0, 0};
+    int32_t reach_h[5] = {};
     if (hipMemcpyAsync(reach_h, L.meta + 4, sizeof(reach_h), hipMemcpyDeviceToHost, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess)   // also keeps `level_launch` and `team_tab` alive until their copies are done
         return bail(nm::fail(NM_ERR_HIP, "waiting for the plan to complete failed"));
     p->reach[0] = reach_h[0];
     p->reach[1] = reach_h[1];
+    if (reach_h[4] == 0) p->grid = grid;
     *plan_out = p;
     return NM_OK;
 }
@@ -2850,6 +2884,7 @@ extern "C" int64_t nm_sptrsv_plan_levels(const nm_sptrsv_plan *plan) { return pl
 
 extern "C" int64_t nm_sptrsv_plan_launches(const nm_sptrsv_plan *plan) {
     if (!plan) return -1;
+    if (by_lines(plan)) return 1;
     // (of the solve with A, as solve_typed issues them)
     const bool teams = g_team_enabled.load();
     int flow_a = 0, flow_b = 0;
