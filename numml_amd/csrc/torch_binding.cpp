@@ -19,6 +19,7 @@
 #include <ATen/hip/HIPEvent.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/hip/HIPCachingAllocator.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPGuard.h>
 #include <c10/hip/HIPStream.h>
 
@@ -206,6 +207,11 @@ struct Plan {
     // the first time a policy asks for it
     int32_t info[16] = {0};
     std::atomic<bool> info_loaded{false};
+    // 'T': the content key of the transposed structure, known from the second explicit transpose on
+    // (t_known, t_key under g_plans_mutex)
+    std::atomic<int64_t> transposes{0};
+    bool t_known = false;
+    Key t_key;
     // the stream the plan was built on and the event that marks its completion there
     c10::StreamId build_stream = 0;
     std::unique_ptr<at::cuda::CUDAEvent> ready;
@@ -258,6 +264,27 @@ bool alias_matches(const Alias &al, const Tensor &indices, const Tensor &indptr)
            al.key.device == indices.device().index() && !al.idx_weak.expired() && !al.ptr_weak.expired();
 }
 
+// Notes the content key of a pair of structure tensors.
+void remember_key(const Tensor &indices, const Tensor &indptr, const Key &key) {
+    Alias al{indices.unsafeGetTensorImpl(),
+             indptr.unsafeGetTensorImpl(),
+             WeakImpl(indices.getIntrusivePtr()),
+             WeakImpl(indptr.getIntrusivePtr()),
+             indices.data_ptr(),
+             indptr.data_ptr(),
+             indices._version(),
+             indptr._version(),
+             key};
+    std::lock_guard<std::mutex> lock(g_plans_mutex);
+    // entries of tensors that have died, or that describe these very tensors at an older version
+    g_aliases.remove_if([&](const Alias &o) {
+        return o.idx_weak.expired() || o.ptr_weak.expired() ||
+               (o.idx_impl == al.idx_impl && o.ptr_impl == al.ptr_impl);
+    });
+    g_aliases.push_front(std::move(al));
+    while (g_aliases.size() > kAliasTableSize) g_aliases.pop_back();
+}
+
 // The content key of (indices, indptr): from the alias table, or computed (waits for the stream).
 // With `compute` false a pair of tensors that has not been seen yields false instead.
 bool structure_key(const Tensor &indices, const Tensor &indptr, bool compute, Key *out) {
@@ -283,28 +310,8 @@ bool structure_key(const Tensor &indices, const Tensor &indptr, bool compute, Ke
                             current_stream(dev)),
           "nm_structure_hash");
     g_keys_computed.fetch_add(1, std::memory_order_relaxed);
-    if (!aliased) {
-        *out = Key{h[0], h[1], indices.numel(), indptr.numel(), dev.index()};
-        return true;
-    }
-    Alias al{indices.unsafeGetTensorImpl(),
-             indptr.unsafeGetTensorImpl(),
-             WeakImpl(indices.getIntrusivePtr()),
-             WeakImpl(indptr.getIntrusivePtr()),
-             indices.data_ptr(),
-             indptr.data_ptr(),
-             indices._version(),
-             indptr._version(),
-             Key{h[0], h[1], indices.numel(), indptr.numel(), dev.index()}};
-    *out = al.key;
-    std::lock_guard<std::mutex> lock(g_plans_mutex);
-    // entries of tensors that have died, or that describe these very tensors at an older version
-    g_aliases.remove_if([&](const Alias &o) {
-        return o.idx_weak.expired() || o.ptr_weak.expired() ||
-               (o.idx_impl == al.idx_impl && o.ptr_impl == al.ptr_impl);
-    });
-    g_aliases.push_front(std::move(al));
-    while (g_aliases.size() > kAliasTableSize) g_aliases.pop_back();
+    *out = Key{h[0], h[1], indices.numel(), indptr.numel(), dev.index()};
+    if (aliased) remember_key(indices, indptr, *out);
     return true;
 }
 
@@ -807,6 +814,28 @@ std::vector<Tensor> csr_transpose_forward(int A_rows, int A_columns, Tensor A_da
                                    At_indptr.data_ptr<int64_t>(), At_to_A.data_ptr<int64_t>(),
                                    current_stream(dev)),
           "nm_csr_transpose_forward");
+    // A sum or a product with the transpose has fresh structure tensors on every call, and would merge the
+    // patterns and only then, with a pass over them for their key, find that it has a plan for the
+    // pair: the key is the same every time, so it goes with the plan.
+    if (nnz > 0 && backward_mode_now() != kAtomic && tracked(At_indices) && tracked(At_indptr) &&
+        plan->transposes.fetch_add(1, std::memory_order_relaxed) > 0) {
+        Key key;
+        bool known = false;
+        {
+            std::lock_guard<std::mutex> lock(g_plans_mutex);
+            known = plan->t_known;
+            key = plan->t_key;
+        }
+        if (known) {
+            remember_key(At_indices, At_indptr, key);
+        } else if (c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None) {
+            // (making a key waits for the stream)
+            structure_key(At_indices, At_indptr, true, &key);
+            std::lock_guard<std::mutex> lock(g_plans_mutex);
+            plan->t_key = key;
+            plan->t_known = true;
+        }
+    }
     return {At_data, At_indices, At_indptr, At_to_A};
 }
 
