@@ -250,12 +250,12 @@ struct OwnColumn {
     }
 };
 
-// below[k] = position of the first entry of column k with a row index > k.  Also what the choice of
+// below[k] = position of the first entry of column k with a row index > k; no column is done.  Also what the choice of
 // the numeric kernel depends on: ctl[4] / ctl[5] = entries the widest column reaches above / below its
 // diagonal, ctl[6] = columns that do not name the column before them.
 __global__ __launch_bounds__(kBlock) void lu_below_kernel(int64_t cols, const int64_t *__restrict__ indices,
                                                           const int64_t *__restrict__ indptr,
-                                                          int64_t *__restrict__ below, int32_t *ctl) {
+                                                          int64_t *__restrict__ below, int32_t *__restrict__ done, int32_t *ctl) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     int32_t up = 0, down = 0, breaks = 0;
     for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < cols; k += stride) {
@@ -266,6 +266,7 @@ __global__ __launch_bounds__(kBlock) void lu_below_kernel(int64_t cols, const in
             if (indices[mid] <= k) lo = mid + 1; else hi = mid;
         }
         below[k] = lo;
+        done[k] = 0;
         if (pe > pb) {
             const int64_t first = indices[pb], last = indices[pe - 1];
             if (first < k) up = max(up, (int32_t)(k - first));
@@ -304,8 +305,10 @@ struct LuBatch {
     volatile int32_t *ready;      // [kLuWavesPerBlock] LDS: 0 pending, 1 final values in LDS, 2 final values in global memory only
 };
 
-template <typename T, bool IN_LDS>
-__device__ bool lu_column(int64_t k, int64_t pb, int64_t len, const OwnColumn<T, IN_LDS> &own,
+// RESUME: the rows before `base` of the column are final (lu_band_kernel wrote them), so that pivots there only update
+// the rows from `base` on.
+template <typename T, bool IN_LDS, bool RESUME>
+__device__ bool lu_column(int64_t base, int64_t k, int64_t pb, int64_t len, const OwnColumn<T, IN_LDS> &own,
                           const LuBatch<T> &batch,
                           const int64_t *__restrict__ indices, const int64_t *__restrict__ indptr,
                           const int64_t *__restrict__ below_of, T *values, int32_t *done, int32_t *ctl,
@@ -394,14 +397,14 @@ __device__ bool lu_column(int64_t k, int64_t pb, int64_t len, const OwnColumn<T,
             }
             return __hip_atomic_load(values + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         };
-        if (at_first >= 0) {
+        if (at_first >= 0 && !(RESUME && own.row(at_first) < base)) {
             const T prod = other(t_first) * m_ik;
             own.set(at_first, own.val(at_first) - prod);
         }
         for (int64_t t0 = ls + 64; t0 < ie; t0 += 64) {          // columns with more than 64 entries below
             const int64_t t = t0 + lane;
             const int64_t at = t < ie ? find(e, indices[t]) : (int64_t)-1;
-            if (at >= 0) {
+            if (at >= 0 && !(RESUME && own.row(at) < base)) {
                 const T prod = other(t) * m_ik;
                 own.set(at, own.val(at) - prod);
             }
@@ -428,11 +431,11 @@ __device__ bool lu_column(int64_t k, int64_t pb, int64_t len, const OwnColumn<T,
     return true;
 }
 
-template <typename T>
-__global__ __launch_bounds__(kLuFlowBlock) void lu_flow_kernel(int64_t cols, const int64_t *__restrict__ indices,
-                                                         const int64_t *__restrict__ indptr,
-                                                         const int64_t *__restrict__ below, T *values,
-                                                         int32_t *done, int32_t *ctl, int64_t spin_limit) {
+// Columns are drawn from ctl[0]; RESUME: from ctl[8], where lu_band_kernel has left some.
+template <typename T, bool RESUME>
+__device__ __forceinline__ void lu_flow(int64_t cols, const int64_t *__restrict__ indices, const int64_t *__restrict__ indptr,
+                                        const int64_t *__restrict__ below, T *values, int32_t *done, int32_t *ctl,
+                                        int64_t spin_limit) {
     // dynamic LDS: the batch's columns, values first (8-byte aligned), then rows
     extern __shared__ __align__(16) unsigned char s_columns[];
     T (*s_vals)[kLuCap] = reinterpret_cast<T (*)[kLuCap]>(s_columns);
@@ -442,10 +445,11 @@ __global__ __launch_bounds__(kLuFlowBlock) void lu_flow_kernel(int64_t cols, con
     __shared__ int32_t s_ready[kLuWavesPerBlock];
     __shared__ int32_t s_ticket, s_abort;
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t resume = RESUME ? (int64_t)ctl[7] : 0;
     for (;;) {
         // one ticket per workgroup and batch of consecutive columns, one column per wavefront
         if (threadIdx.x == 0) {
-            s_ticket = atomicAdd(ctl, kLuWavesPerBlock);
+            s_ticket = atomicAdd(ctl + (RESUME ? 8 : 0), kLuWavesPerBlock);
             s_abort = __hip_atomic_load(ctl + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         if (threadIdx.x < kLuWavesPerBlock) s_ready[threadIdx.x] = 0;
@@ -460,11 +464,11 @@ __global__ __launch_bounds__(kLuFlowBlock) void lu_flow_kernel(int64_t cols, con
             bool ok;
             if (len <= kLuCap) {
                 const OwnColumn<T, true> own{s_rows[w], s_vals[w], nullptr, nullptr};
-                ok = lu_column<T, true>(k, pb, len, own, batch, indices, indptr, below, values, done, ctl, spin_limit,
+                ok = lu_column<T, true, RESUME>(resume, k, pb, len, own, batch, indices, indptr, below, values, done, ctl, spin_limit,
                                         lane);
             } else {
                 const OwnColumn<T, false> own{nullptr, nullptr, indices + pb, values + pb};
-                ok = lu_column<T, false>(k, pb, len, own, batch, indices, indptr, below, values, done, ctl, spin_limit,
+                ok = lu_column<T, false, RESUME>(resume, k, pb, len, own, batch, indices, indptr, below, values, done, ctl, spin_limit,
                                          lane);
             }
             if (!ok && lane == 0) atomicExch(ctl + 1, 1);
@@ -473,419 +477,636 @@ __global__ __launch_bounds__(kLuFlowBlock) void lu_flow_kernel(int64_t cols, con
     }
 }
 
+template <typename T>
+__global__ __launch_bounds__(kLuFlowBlock) void lu_flow_kernel(int64_t cols, const int64_t *__restrict__ indices,
+                                                         const int64_t *__restrict__ indptr,
+                                                         const int64_t *__restrict__ below, T *values,
+                                                         int32_t *done, int32_t *ctl, int64_t spin_limit) {
+    if (ctl[7] == 0) lu_flow<T, false>(cols, indices, indptr, below, values, done, ctl, spin_limit);
+    else lu_flow<T, true>(cols, indices, indptr, below, values, done, ctl, spin_limit);
+}
+
 // ---- banded factors --------------------------------------------------------------
 //
 // A factor whose entries stay near the diagonal is ONE chain of columns: column k + 1 needs column k,
 // and lu_flow_kernel pays a hand-over between wavefronts, workgroups or compute units (1.4 us) for
-// every link of it whatever the width of the band.  Here one workgroup keeps the part of the matrix
-// that is still to be updated in registers and eliminates column by column (right-looking): every
-// entry receives the same products in the same ascending order of pivots, so the factors are the
-// serial ones bit for bit.
-//   * Wavefront v owns the columns j = v mod 16, CS of them at a time; its lanes are rows: row i sits
-//     in lane i mod 64 of register i / 64 mod RL, a ring of 64 RL rows.  At step k the last row of any
-//     column at hand is below k + 16 CS + bl <= k + 64 RL, so a place of the ring means one row.
-//   * Step k: the multipliers of column k come through LDS; the pivot row's entries are in the
-//     wavefront's own registers (one lane of each column) and become scalars.  The owner of column
-//     k + 1 updates that column first, divides it and hands its multipliers on before it turns to
-//     its other columns; the others wait for the column's number in LDS, not for a barrier.
-//   * Only products of two STORED entries are subtracted (a bit per row and column, read with the
-//     pivot row; a ballot per column of multipliers): a zero or infinite pivot spreads exactly as far
-//     as in the serial loop.
-//   * A finished column is written out, and the wavefront's next one, requested a round of sixteen
-//     steps earlier, takes its place, in the two steps after, when nobody waits for this wavefront.
-// 64 x 64 five-point grid in fp64 (4096 columns, reach 64 either way): 5.57 -> 2.41 ms, 0.59 us a column.
-// Bound by what the SIMDs issue: 240 vector instructions per step and SIMD, three quarters of the
-// time; the chain alone (LDS trip, update, division, LDS trip) would be 0.34 us.  Eight wavefronts of
-// nine columns: 2.84 ms; a barrier a step instead of the numbers in LDS: 4.6 ms; without the raised
-// priority of the wavefronts whose turn is near: 2.75 ms; the owner putting off the update before its
-// turn as well: 2.65 ms.
+// every link of it whatever the width of the band.  Here one workgroup keeps the window of the matrix that
+// is being worked on in LDS and eliminates it panel by panel of eight columns.  Every entry receives the
+// same products in the same ascending order of pivots, so the factors are the serial ones bit for
+// bit.  The wavefronts have tasks of their own and wait for counts in LDS, never at a barrier:
+//   * wavefronts 0 and 1 factor the panels in turn, rows in lanes, columns in registers: while one divides and
+//     updates inside its panel, the other applies the panel before that one to the next and then each pivot as it comes
+//     out;
+//   * wavefronts 2 and 3 (lanes are columns) finish the panel's eight rows to the right of it, pivot by pivot;
+//   * six wavefronts apply the panel to the rest of the window, eight columns of all its rows at a time;
+//   * wavefronts 14 and 15 bring columns in, 8 and 9 rows, as far ahead as the rings allow, and wavefront 4 writes
+//     what is finished.
+// What bounds it: the chain inside a panel, a division, the broadcast of the row and the update of the next column a
+// pivot (380 cycles), and the last pivot's way to the panel that waits for it (1700 cycles a panel of eight); at a
+// reach of 64 and more the update of the window takes over.  us for 4096 columns with everything around it (a kernel
+// that kept the window in registers and handed every column round by itself took the figure in brackets):
+//   reach      1            8            28           56           64           76           92
+//   fp64  1100 (1166)  1110 (1169)  1105 (1164)  1151 (2070)  1391 (2491)  2214 (2559)  2495 (2942)
+//   fp32  1064 (1162)  1064 (1160)  1055 (1178)  1091 (1780)  1205 (2187)  1481 (2231)  2013 (2375)
+// A 100 x 100 grid in fp32, which did not fit the registers, takes 4.9 ms instead of 25.
+// Entries that the pattern does not have are zeros when they are handed on, whatever a product has left in
+// their places, and a zero takes no part in a sum of finite numbers (no input is -0, a difference is
+// -0 only where one operand was).  A -0 among the inputs, an infinity or a NaN among the factors ends
+// the launch before they are written or used further: lu_flow_kernel goes on at that panel.
 #define NM_INLINE __attribute__((always_inline))   // (lambdas over register arrays)
 constexpr int kBandWaves = 16;
-constexpr int kBandMaxRl = 3;
+constexpr int kBandTrailing = 6;     // wavefronts of the update
+constexpr int kPanel = 8;
+static_assert(kPanel == kLuWavesPerBlock, "lu_flow_kernel goes on at a batch of its own");
+constexpr size_t kBandLds = 160 * 1024;
 // More breaks in the chain (columns that do not name their predecessor) than this and the matrix may
-// be made of three independent blocks or more, which lu_flow_kernel works on side by side: it takes
-// 0.75 us a column of ONE block where the reach is 1 and 1.3 us where it is 60, this kernel 0.27 and
-// 0.50 us whatever the blocks.
+// be made of three independent blocks or more, which lu_flow_kernel works on side by side.
 constexpr int kBandMaxBreaks = 1;
 
-// Multipliers are kept for as many columns as there are wavefronts: who publishes column c has seen
-// every other wavefront publish one of the fifteen columns before it, and each read the multipliers
-// of column c - 16 before it did.
-constexpr int kBandDepth = kBandWaves;
-
-struct BandShared {
-    double l[kBandDepth][64 * kBandMaxRl];              // multipliers of a column, by ring position (T at the front)
-    uint64_t head[kBandDepth][kBandMaxRl + 1];          // which of them are stored entries, whose they are (written last)
-    double value[kBandWaves][64 * kBandMaxRl];          // columns on their way into the registers
-    int32_t entry[kBandWaves][64 * kBandMaxRl];
+enum BandCount : int {
+    kPivots,                     // pivots whose multipliers are there
+    kRows0, kRows1,              // rows of U that are there, of the first 64 columns right of the panel and of the rest
+    kColumns0, kColumns1, kIn0, kIn1,   // panels whose new columns / rows are in the window (kLoaded: all four)
+    kWritten,                    // panels written
+    kGoodPanel0, kGoodPanel1,    // panels found finite, by the wavefront that factors them
+    kGoodRows0, kGoodRows1,
+    kStop,                       // somebody found one that is not
+    kNegativeZero,
+    kTrailing0 = 16,             // per wavefront: panels applied to the rest of the window
+    kBandCounts = kTrailing0 + kBandTrailing
 };
+constexpr int32_t kBandNever = 0x40000000;
+constexpr int kLoaded = kColumns0, kLoaders = 4;
 
-// w -= l * u on the active lanes for every place S of a register whose bit of `stored` is set; products and
-// differences are rounded on their own.  In assembler because the compiler turned the choice per
-// column into selects, branches or copies of every column (a step 1.5 to 4 times as long).  The
-// inner places are mostly all stored and then go without a choice; the first (finished for a step
-// out of eight) and the last (mostly outside the band) are chosen by the execution mask.
-#define NM_BAND_M64(i, t) "v_mul_f64 %[t" #t "], %[l], %[u" #i "]\n\t"
-#define NM_BAND_M32(i, t) "v_mul_f32 %[t" #t "], %[u" #i "], %[l]\n\t"
-#define NM_BAND_D64(i, t) "v_add_f64 %[w" #i "], %[w" #i "], -%[t" #t "]\n\t"
-#define NM_BAND_D32(i, t) "v_sub_f32 %[w" #i "], %[w" #i "], %[t" #t "]\n\t"
-#define NM_BAND_IF(i) "s_bitcmp1_b32 %[stored], %[S]+" #i "\n\ts_cselect_b64 exec, %[sv], 0\n\t"
-#define NM_BAND_P64(i, t) NM_BAND_IF(i) NM_BAND_D64(i, t)
-#define NM_BAND_P32(i, t) NM_BAND_IF(i) NM_BAND_D32(i, t)
-#define NM_BAND_SEQ2(M, D) M(0, 0) M(1, 1) D(0, 0) D(1, 1)
-#define NM_BAND_SEQ3(M, D) M(0, 0) M(1, 1) M(2, 2) D(0, 0) D(1, 1) D(2, 2)
-#define NM_BAND_SEQ4(M, D) M(0, 0) M(1, 1) M(2, 2) M(3, 3) D(0, 0) D(1, 1) D(2, 2) D(3, 3)
-#define NM_BAND_ALL_LANES "s_mov_b64 exec, %[sv]\n\t"
-#define NM_BAND_TEXT(SEQ, M, D, P)                                                                                   \
-    "s_bfe_u32 %[bits], %[stored], %[field]\n\ts_cmp_eq_u32 %[bits], %[whole]\n\ts_cbranch_scc0 .Lpick_%=\n\t" SEQ(M, D)    \
-    "s_branch .Ldone_%=\n.Lpick_%=:\n\ts_mov_b64 %[sv], exec\n\t" SEQ(M, P) NM_BAND_ALL_LANES ".Ldone_%=:"
-#define NM_BAND_W(i) [w##i] "+v"(W[S + i][q])
-#define NM_BAND_U(i) [u##i] "s"(u[S + i])
-#define NM_BAND_LIST2(X) X(0), X(1)
-#define NM_BAND_LIST3(X) NM_BAND_LIST2(X), X(2)
-#define NM_BAND_LIST4(X) NM_BAND_LIST3(X), X(3)
-#define NM_BAND_CASE(N)                                                                                              \
-    if constexpr (CS - 2 == N) {                                                                                     \
-        if constexpr (sizeof(T) == 8)                                                                                \
-            NM_BAND_ASM_(NM_BAND_TEXT(NM_BAND_SEQ##N, NM_BAND_M64, NM_BAND_D64, NM_BAND_P64), N);                    \
-        else                                                                                                         \
-            NM_BAND_ASM_(NM_BAND_TEXT(NM_BAND_SEQ##N, NM_BAND_M32, NM_BAND_D32, NM_BAND_P32), N);                    \
-    }
-#define NM_BAND_ASM_(TEXT, N)                                                                                        \
-    asm volatile(TEXT : NM_BAND_LIST##N(NM_BAND_W), [t0] "=&v"(t0), [t1] "=&v"(t1), [t2] "=&v"(t2), [t3] "=&v"(t3),  \
-                 [sv] "=&s"(sv), [bits] "=&s"(bits) : [l] "v"(l), [stored] "s"(stored), [S] "n"(S),                  \
-                 [field] "n"(S | N << 16), [whole] "n"((1 << N) - 1), NM_BAND_LIST##N(NM_BAND_U) : "scc")
-// the places 1 .. CS - 2
-template <int CS, typename T, int RL>
-__device__ __forceinline__ void band_inner(T l, uint32_t stored, const T (&u)[CS], T (&W)[CS][RL], int q) {
-    constexpr int S = 1;
-    uint64_t sv;
-    uint32_t bits;
-    T t0, t1, t2, t3;
-    NM_BAND_CASE(2)
-    NM_BAND_CASE(3)
-    NM_BAND_CASE(4)
-}
-// the two outer places, bits 0 and 1 of `stored`
-template <typename T>
-__device__ __forceinline__ void band_outer(T l, uint32_t stored, T u0, T u1, T &w0, T &w1) {
-    uint64_t sv;
-    T t0, t1;
-    constexpr int S = 0;
-    if constexpr (sizeof(T) == 8)
-        asm volatile("s_mov_b64 %[sv], exec\n\t" NM_BAND_SEQ2(NM_BAND_M64, NM_BAND_P64) "s_mov_b64 exec, %[sv]"
-                     : [w0] "+v"(w0), [w1] "+v"(w1), [t0] "=&v"(t0), [t1] "=&v"(t1), [sv] "=&s"(sv)
-                     : [l] "v"(l), [stored] "s"(stored), [S] "n"(S), [u0] "s"(u0), [u1] "s"(u1) : "scc");
-    else
-        asm volatile("s_mov_b64 %[sv], exec\n\t" NM_BAND_SEQ2(NM_BAND_M32, NM_BAND_P32) "s_mov_b64 exec, %[sv]"
-                     : [w0] "+v"(w0), [w1] "+v"(w1), [t0] "=&v"(t0), [t1] "=&v"(t1), [sv] "=&s"(sv)
-                     : [l] "v"(l), [stored] "s"(stored), [S] "n"(S), [u0] "s"(u0), [u1] "s"(u1) : "scc");
-}
-
-// LDS accesses that stay in program order (no waits between them).
+template <typename T> struct Band {
+    int32_t n, panels, blb, bub;   // columns; blocks of eight rows below, columns right of a panel's own
+    int32_t rb, cb, pitch;         // blocks of the window (rings), entries from column to column (odd)
+    int32_t slack, kept;           // panels that the rings hold beyond the window; panels whose multipliers and rows are kept
+    T *win, *F, *U;                // F, U: the kept panels' multipliers [pivot][row - panel's first], rows [pivot][column - panel's end]
+    int32_t fr, fp, uc;            // rows of a panel, the same rounded up to whole registers, columns right of it
+    uint8_t *has;                  // [block of rows][column]: which of the eight are stored
+    int64_t *base;                 // by column of the window: where it starts in the arrays, its length, entries brought in, written
+    int32_t *len, *in, *out;
+    int32_t *count;
+    const int64_t *indices;
+    T *values;
+    const int64_t *indptr;
+    __device__ __forceinline__ T *column(int32_t slot) const { return win + slot * pitch; }
+    __device__ __forceinline__ T *multipliers(int32_t K) const { return F + (K & (kept - 1)) * (kPanel * fp); }
+    __device__ __forceinline__ T *rows(int32_t K) const { return U + (K & (kept - 1)) * (kPanel * uc); }
+};
+// LDS accesses that stay in program order: a wavefront's are carried out in that order.
 template <typename V> __device__ __forceinline__ V lds_get(V *p) {
     asm volatile("" ::: "memory");
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    const V v = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    asm volatile("" ::: "memory");
+    return v;
 }
 template <typename V> __device__ __forceinline__ void lds_put(V *p, V v) {
     asm volatile("" ::: "memory");
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    asm volatile("" ::: "memory");
 }
+// Waits until the count of every lane's number is at least the lane's `least`; false: the launch ends.
+template <bool SLEEP> __device__ __forceinline__ bool band_wait(int32_t *count, int32_t least) {
+    const int lane = threadIdx.x & 63;
+    while (true) {
+        const int32_t now = lds_get(count + min(lane, (int)kBandCounts - 1));
+        if (!__any(now < least)) return true;
+        if (__any(lane == kStop && now != 0)) return false;
+        if (SLEEP) __builtin_amdgcn_s_sleep(1);
+    }
+}
+// `least` with the counts [first, first + number) to be v at least
+__device__ __forceinline__ int32_t band_need(int32_t least, int first, int number, int32_t v) {
+    const int lane = threadIdx.x & 63;
+    return lane >= first && lane < first + number ? v : least;
+}
+constexpr int32_t kBandAny = -0x7fffffff;
+// (all lanes write the one word: less to issue than choosing one of them)
+__device__ __forceinline__ void band_tell(int32_t *count, int which, int32_t v) { lds_put(count + which, v); }
+__device__ __forceinline__ int32_t ring(int32_t at, int32_t size) { return at >= size ? at - size : at; }
 
-template <typename T, int RL, int CS>
-__device__ __forceinline__ void lu_band(int32_t n, int bl, const int64_t *__restrict__ indices,
-                                        const int64_t *__restrict__ indptr, T *values, BandShared &sh) {
-    constexpr int R = 64 * RL;
-    const int lane = threadIdx.x & 63, v = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    T W[CS][RL];              // the wavefront's columns
-    uint32_t pos[CS];         // entry number inside the column of each of this lane's rows, a byte each; 0xff: not stored
-    uint32_t has[RL];         // bit S: this lane's row of the register is stored in column S and not finished
-    T fetched[RL];            // the next column: entry e = lane + 64 q
-    int32_t fetched_row[RL];
-    int32_t fetched_len = 0;
-    int64_t base[CS], fetched_b = 0, staged_b = 0;   // where a column starts in the arrays: of the columns, of the
-                                                     // one requested, of the one in LDS
-    int64_t next_b, next_e;   // place of the column after that in the arrays
-    int32_t next_col = 0;
+// Eight values that are the same for all lanes.
+template <typename T> struct alignas(16) Eight { T v[kPanel]; };
 
-    // (vector loads: a scalar load would be waited for with the next access to LDS, microseconds later)
-    int32_t zero = 0;
-    asm volatile("" : "+v"(zero));
-    auto pointers = [&](int32_t col) NM_INLINE {
-        const int32_t at = min(col, n - 1) + zero;
-        next_b = indptr[at];
-        next_e = indptr[at + 1];
-        next_col = col;
+// Wavefronts 0 and 1: panels K = v, v + 2, ...  RL registers of 64 rows hold the panel's rows, the first RA of them
+// the rows that the panel before reaches.
+template <typename T, int RL, int RA> __device__ __forceinline__ void band_panels(const Band<T> &B, int v) {
+    const int lane = threadIdx.x & 63;
+    const int32_t cbs = B.cb * kPanel;
+    int32_t row_slot = lane / kPanel % B.rb, col_slot = 0;   // of panel 0
+    auto forward = [&](int32_t by) NM_INLINE {
+        row_slot = ring(row_slot + by, B.rb);
+        col_slot = ring(col_slot + by, B.cb);
     };
-    // Requests the column that `pointers` looked up last: unconditional loads (clamped to an entry
-    // that exists), so that nothing waits for them before `stage` does.
-    auto fetch = [&]() NM_INLINE {
-        fetched_len = next_col < n ? (int32_t)(next_e - next_b) : 0;
-        fetched_b = next_b;
+    if (v) forward(1);
+    __builtin_amdgcn_s_setprio(3);
+    for (int32_t K = v; K < B.panels; K += 2) {
+        int32_t least = band_need(kBandAny, kLoaded, kLoaders, K + 1);
+        least = band_need(least, kTrailing0 + K % kBandTrailing, 1, K - 2);   // (whose columns these are)
+        if (!band_wait<false>(B.count, least)) return;
+        T W[kPanel][RL];
+        uint32_t has_lo[RL], has_hi[RL];   // bit 8 (c & 3): stored in column c
 #pragma unroll
         for (int q = 0; q < RL; ++q) {
-            const int64_t t = max(min(next_b + q * 64 + lane, next_e - 1), (int64_t)0);
-            fetched_row[q] = reinterpret_cast<const int32_t *>(indices)[2 * t];   // (low half: rows fit 31 bits)
-            fetched[q] = values[t];
+            const bool mine = lane / kPanel + 8 * q <= B.blb;
+            const int32_t slot = mine ? (row_slot + 8 * q) % B.rb : row_slot;
+            const uint64_t m = *reinterpret_cast<const uint64_t *>(B.has + slot * cbs + col_slot * kPanel);
+            has_lo[q] = mine ? (uint32_t)m >> (lane & 7) : 0u;
+            has_hi[q] = mine ? (uint32_t)(m >> 32) >> (lane & 7) : 0u;
+#pragma unroll
+            for (int c = 0; c < kPanel; ++c) W[c][q] = B.column(col_slot * kPanel + c)[slot * kPanel + (lane & 7)];
         }
-    };
-    T *s_value = reinterpret_cast<T *>(sh.value[v]);
-    int32_t *s_entry = sh.entry[v];
-    auto stage = [&]() NM_INLINE {
-        staged_b = fetched_b;
+        // row t of the panel `back` before, whose rows are in W from the row 8 back - 8 of that panel's rest on
+        auto apply = [&](int back, int t) NM_INLINE {
+            const T *const F = B.multipliers(K - back) + t * B.fp;
+            const Eight<T> u = *reinterpret_cast<const Eight<T> *>(B.rows(K - back) + t * B.uc + (back - 1) * kPanel);
+            T l[RA];
 #pragma unroll
-        for (int q = 0; q < RL; ++q) s_entry[q * 64 + lane] = -1;
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-#pragma unroll
-        for (int q = 0; q < RL; ++q)
-            if (q * 64 + lane < fetched_len) {
-                const uint32_t at = (uint32_t)fetched_row[q] % (uint32_t)R;
-                s_value[at] = fetched[q];
-                s_entry[at] = q * 64 + lane;
+            for (int q = 0; q < RA; ++q) {
+                const int32_t at = back * kPanel + lane + 64 * q;
+                const T x = F[min(at, B.fp - 1)];
+                l[q] = at < B.fp ? x : T(0);
             }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    };
-    // the column in LDS takes the last place
-    auto unstage = [&]() NM_INLINE {
-        constexpr int S = CS - 1;
-        base[S] = staged_b;
-        pos[S] = 0;
 #pragma unroll
-        for (int q = 0; q < RL; ++q) {
-            const int32_t e = s_entry[q * 64 + lane];
-            W[S][q] = e >= 0 ? s_value[q * 64 + lane] : T(0);
-            pos[S] |= (uint32_t)(e >= 0 ? e : 0xff) << (8 * q);
-            has[q] |= e >= 0 ? 1u << S : 0u;
+            for (int c = 0; c < kPanel; ++c)
+#pragma unroll
+                for (int q = 0; q < RA; ++q) {
+                    const T p = l[q] * u.v[c];
+                    W[c][q] = W[c][q] - p;
+                }
+        };
+        if (K > 1 && B.bub > 1) {
+            if (!band_wait<false>(B.count, band_need(kBandAny, kRows0, 1, (K - 1) * kPanel))) return;
+#pragma unroll 1
+            for (int t = 0; t < kPanel; ++t) apply(2, t);
         }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    };
-    // the columns move up, so that the next one to finish is always in place 0
-    auto shift = [&]() NM_INLINE {
-#pragma unroll
-        for (int S = 0; S + 1 < CS; ++S) {
-            pos[S] = pos[S + 1];
-            base[S] = base[S + 1];
-#pragma unroll
-            for (int q = 0; q < RL; ++q) W[S][q] = W[S + 1][q];
+        if (K > 0) {
+#pragma unroll 1   // (registers: unrolled, 370 of them are spilled)
+            for (int t = 0; t < kPanel; ++t) {
+                if (!band_wait<false>(B.count, band_need(kBandAny, kPivots, 2, (K - 1) * kPanel + t + 1))) return;
+                apply(1, t);
+            }
         }
-#pragma unroll
-        for (int q = 0; q < RL; ++q) has[q] >>= 1;
-    };
-    // f(constant q) for the register that holds ring position p
-    auto by_ring = [&](int p, auto f) NM_INLINE {
-        if (RL == 1 || p < 64)
-            f(std::integral_constant<int, 0>{});
-        else if (RL == 2 || p < 128)
-            f(std::integral_constant<int, RL < 2 ? 0 : 1>{});
-        else
-            f(std::integral_constant<int, RL - 1>{});
-    };
-    // which of this lane's rows are stored below the diagonal (ring position p) of the column in place 0
-    bool below[RL];
-    uint64_t below_mask[RL];
-    bool has_diagonal = false;
-    auto look_below = [&](int p) NM_INLINE {
-#pragma unroll
-        for (int q = 0; q < RL; ++q) {
-            int delta = q * 64 + lane - p;
-            if (delta < 0) delta += R;
-            below[q] = delta >= 1 && delta <= bl && (has[q] & 1u) != 0;
-            below_mask[q] = __ballot(below[q]);
-        }
-        by_ring(p, [&](auto q) NM_INLINE { has_diagonal = (nm::read_lane((int)has[q], p & 63) & 1) != 0; });
-    };
-    // Divides column c, in place 0 (diagonal at ring position p), and leaves its multipliers for everybody.
-    // A wavefront's LDS accesses are carried out in order: who sees the column's number sees them.
-    auto finish = [&](int32_t c, int p) NM_INLINE {
-        const int buffer = c % kBandDepth;
-        T *s_l = reinterpret_cast<T *>(sh.l[buffer]);
-        if (has_diagonal) {
-            T d = T(0);
-            by_ring(p, [&](auto q) NM_INLINE { d = nm::read_lane(W[0][q], p & 63); });
+        // (the panel whose place this one takes is written, and applied to the rest and to the rows of the next)
+        least = band_need(kBandAny, kWritten, 1, K + 1 - B.kept);
+        least = band_need(least, kTrailing0, kBandTrailing, K + 1 - B.kept);
+        if (!band_wait<false>(B.count, band_need(least, kRows0, 2, (K + 2 - B.kept) * kPanel))) return;
+        T *const F = B.multipliers(K);
+        T finite = T(0);
+        nm::static_for<kPanel>([&](auto pivot) NM_INLINE {
+            constexpr int t = decltype(pivot)::value;
+            const uint32_t row_lo = (uint32_t)__builtin_amdgcn_readlane((int)has_lo[0], t);
+            const uint32_t row_hi = (uint32_t)__builtin_amdgcn_readlane((int)has_hi[0], t);
+            const T d = nm::read_lane(W[t][0], t);
+            const bool divide = ((t < 4 ? row_lo : row_hi) >> 8 * (t & 3) & 1) != 0;   // (the diagonal is stored)
+            T l[RL];
 #pragma unroll
             for (int q = 0; q < RL; ++q) {
-                const T quot = W[0][q] / d;
-                W[0][q] = below[q] ? quot : W[0][q];
+                const bool stored = ((t < 4 ? has_lo[q] : has_hi[q]) >> 8 * (t & 3) & 1) != 0;
+                const bool below = q > 0 || lane > t;
+                const T quotient = W[t][q] / d;
+                T x = divide && below ? quotient : W[t][q];
+                x = stored ? x : T(0);
+                finite = __builtin_fma(x, T(0), finite);
+                F[t * B.fp + lane + 64 * q] = x;   // (nothing is stored in the rows past the panel's)
+                l[q] = below ? x : T(0);
             }
-        }
+            band_tell(B.count, kPivots, K * kPanel + t + 1);
 #pragma unroll
-        for (int q = 0; q < RL; ++q) lds_put(s_l + q * 64 + lane, W[0][q]);
-        if (lane == 0) {
+            for (int c = t + 1; c < kPanel; ++c) {
+                const bool stored = ((c < 4 ? row_lo : row_hi) >> 8 * (c & 3) & 1) != 0;
+                const T there = nm::read_lane(W[c][0], t);
+                const T u = stored ? there : T(0);
 #pragma unroll
-            for (int q = 0; q < RL; ++q) lds_put(&sh.head[buffer][q], below_mask[q]);
-            lds_put(reinterpret_cast<int32_t *>(&sh.head[buffer][kBandMaxRl]), c);
-        }
-#pragma unroll
-        for (int q = 0; q < RL; ++q) has[q] &= ~1u;
-    };
-    auto write_out = [&]() NM_INLINE {
-#pragma unroll
-        for (int q = 0; q < RL; ++q) {
-            const uint32_t e = pos[0] >> (8 * q) & 0xffu;
-            if (e != 0xffu) values[base[0] + e] = W[0][q];
-        }
-    };
-
-#pragma unroll
-    for (int q = 0; q < RL; ++q) has[q] = 0;
-#pragma unroll
-    for (int S = 0; S < CS; ++S) {
-        pos[S] = ~0u;
-        base[S] = 0;
-#pragma unroll
-        for (int q = 0; q < RL; ++q) W[S][q] = T(0);
-    }
-    pointers(v);
-#pragma unroll 1
-    for (int S = 0; S < CS; ++S) {
-        fetch();
-        pointers(v + kBandWaves * (S + 1));
-        stage();
-        shift();
-        unstage();
-    }
-    int32_t ahead = v + kBandWaves * CS;        // column `next_b` belongs to
-    if (threadIdx.x < kBandDepth) sh.head[threadIdx.x][kBandMaxRl] = ~0ull;
-    __syncthreads();
-    int p = 0;                                  // ring position of row k
-    auto next = [&](int p) NM_INLINE { return p + 1 == R ? 0 : p + 1; };
-    // the multipliers of column k into l, their mask into m; HURRY: asks for everything every time
-    auto receive = [&](int32_t k, T (&l)[RL], uint64_t (&m)[RL], auto HURRY) NM_INLINE {
-        const int buffer = k & (kBandDepth - 1);
-        T *s_l = reinterpret_cast<T *>(sh.l[buffer]);
-        int32_t *s_column = reinterpret_cast<int32_t *>(&sh.head[buffer][kBandMaxRl]);
-        auto read = [&]() NM_INLINE {
-            const int32_t there = lds_get(s_column);
-            uint64_t w[RL];
-#pragma unroll
-            for (int q = 0; q < RL; ++q) w[q] = lds_get(&sh.head[buffer][q]);
-#pragma unroll
-            for (int q = 0; q < RL; ++q) l[q] = lds_get(s_l + q * 64 + lane);
-#pragma unroll
-            for (int q = 0; q < RL; ++q)
-                m[q] = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(w[q] >> 32)) << 32 |
-                       (uint32_t)__builtin_amdgcn_readfirstlane((int)w[q]);
-            return __builtin_amdgcn_readfirstlane(there) == k;
-        };
-        if constexpr (HURRY) {
-            while (!read()) {}
-        } else if (__builtin_expect(!read(), 0)) {
-            while (__builtin_amdgcn_readfirstlane(lds_get(s_column)) != k) __builtin_amdgcn_s_sleep(1);
-            read();
-        }
-    };
-    // the column whose multipliers are l applied to the columns of this wavefront; OWN: but not to place 0
-    auto apply = [&](const T (&l)[RL], const uint64_t (&m)[RL], const T (&u)[CS], uint32_t stored, auto OWN) NM_INLINE {
-        stored = (uint32_t)__builtin_amdgcn_readfirstlane((int)stored);
-        const uint32_t first = OWN ? 0u : stored & 1u;
-        const uint32_t outer = (uint32_t)__builtin_amdgcn_readfirstlane((int)(first | stored >> (CS - 1) << 1));
-#pragma unroll
-        for (int q = 0; q < RL; ++q)
-            if (__builtin_amdgcn_inverse_ballot_w64(m[q])) {
-                band_inner<CS>(l[q], stored, u, W, q);
-                band_outer(l[q], outer, u[0], u[CS - 1], W[0][q], W[CS - 1][q]);
+                for (int q = 0; q < RL; ++q) {
+                    const T p = l[q] * u;
+                    W[c][q] = W[c][q] - p;
+                }
             }
-    };
-    // the entries of the row at ring position p in this wavefront's columns, and which of them are stored
-    auto row = [&](int p, T (&u)[CS]) NM_INLINE {
-        uint32_t stored = 0;
-        by_ring(p, [&](auto q) NM_INLINE {
-            stored = (uint32_t)nm::read_lane((int)has[q], p & 63);
-            nm::static_for<CS>([&](auto S) NM_INLINE { u[S] = nm::read_lane(W[S][q], p & 63); });
         });
-        return stored;
-    };
-    constexpr std::true_type yes;
-    constexpr std::false_type no;
-    auto step = [&](int32_t k) NM_INLINE {
-        T l[RL], u[CS];
-        uint64_t m[RL];
-        const uint32_t stored = row(p, u);
-        receive(k, l, m, no);
-        apply(l, m, u, stored, no);
-        p = next(p);
-    };
-    auto update_first = [&](const T (&l)[RL], const uint64_t (&m)[RL], T u0, uint32_t stored) NM_INLINE {
-        if ((uint32_t)__builtin_amdgcn_readfirstlane((int)stored) & 1u) {
+        if (__any(finite != T(0)) || __builtin_amdgcn_readfirstlane(lds_get(B.count + kNegativeZero)) != 0) {
+            band_tell(B.count, kStop, 1);
+            return;
+        }
+        band_tell(B.count, kGoodPanel0 + v, K + 1);
+        forward(2);
+    }
+}
+
+// Wavefronts 2 and 3: the panel's rows, columns 64 w .. right of it, a lane each.  They apply the panel before to these rows
+// themselves, so that they wait for the update of the one before that only.
+template <typename T> __device__ __forceinline__ void band_rows(const Band<T> &B, int w) {
+    const int lane = threadIdx.x & 63, at = 64 * w + lane;
+    const int32_t width = B.bub * kPanel, cbs = B.cb * kPanel;
+    if (64 * w >= width) return;
+    const bool mine = at < width;
+    int32_t row_slot = 0, col_slot = (1 + at / kPanel) % B.cb;
+    __builtin_amdgcn_s_setprio(2);
+    for (int32_t K = 0; K < B.panels; ++K) {
+        int32_t least = band_need(kBandAny, kLoaded, kLoaders, K + 1);
+        least = band_need(least, kTrailing0, kBandTrailing, K - 1);
+        least = band_need(least, kPivots, 3, K * kPanel);
+        least = band_need(least, kWritten, 1, K + 1 - B.kept);
+        if (!band_wait<false>(B.count, least)) return;
+        const int32_t slot = mine ? col_slot * kPanel + (lane & 7) : 0;
+        const T *const column = B.column(slot) + row_slot * kPanel;
+        const uint32_t stored = mine && (K + 1) * kPanel + at < B.n ? B.has[row_slot * cbs + slot] : 0u;
+        T X[kPanel];
 #pragma unroll
-            for (int q = 0; q < RL; ++q)
-                if (__builtin_amdgcn_inverse_ballot_w64(m[q])) {
-                    const T prod = l[q] * u0;
-                    W[0][q] = W[0][q] - prod;
-                }
-        }
-    };
-    // Step c - 1: column c is finished and handed on before the wavefront turns to its other columns.
-    auto own = [&](int32_t c) NM_INLINE {
-        T l[RL], u[CS];
-        uint64_t m[RL];
-        uint32_t stored = 0;
-        const int p1 = c >= 1 ? next(p) : p;    // row c
-        look_below(p1);
-        if (c >= 1) {
-            stored = row(p, u);
-            receive(c - 1, l, m, yes);
-            __builtin_amdgcn_s_setprio(3);
-            update_first(l, m, u[0], stored);
-        }
-        finish(c, p1);
-        __builtin_amdgcn_s_setprio(0);
-        if (c >= 1) apply(l, m, u, stored, yes);
-        p = p1;
-    };
-    // Sixteen steps a round: the wavefront finishes its column c, writes it out at step c, puts the column
-    // that waits in LDS in its place at step c + 1 and requests the next one, which has the rest of the
-    // round to arrive.
-#pragma unroll 1
-    for (int32_t c = v - kBandWaves; c < n; c += kBandWaves) {
-        int32_t k = 0;
-        if (c >= 0) {
-            own(c);
-#pragma unroll 1
-            for (k = c; k < min(c + 2, n); ++k) {
-                step(k);
-                if (k == c) {
-                    write_out();
-                    shift();
-                } else {
-                    unstage();
+        for (int s = 0; s < kPanel; ++s) X[s] = column[s];
+        if (K > 0) {
+            const T *const F = B.multipliers(K - 1), *const U = B.rows(K - 1);
+            const bool reached = at + kPanel < width;
+            T u[kPanel];
+#pragma unroll
+            for (int t = 0; t < kPanel; ++t) u[t] = reached ? U[t * B.uc + at + kPanel] : T(0);
+#pragma unroll
+            for (int t = 0; t < kPanel; ++t) {
+                const Eight<T> l = *reinterpret_cast<const Eight<T> *>(F + t * B.fp + kPanel);
+#pragma unroll
+                for (int s = 0; s < kPanel; ++s) {
+                    const T p = l.v[s] * u[t];
+                    X[s] = X[s] - p;
                 }
             }
         }
-        fetch();
-        ahead += kBandWaves;
-        pointers(ahead);
-        // a wavefront goes before the others of its SIMD as the step at which everybody waits for it comes up
-#pragma unroll 1
-        for (; k < min(c + kBandWaves - 1, n); ++k) {
-            if (k == c + kBandWaves - 8) __builtin_amdgcn_s_setprio(1);
-            if (k == c + kBandWaves - 4) __builtin_amdgcn_s_setprio(2);
-            step(k);
+        const T *const F = B.multipliers(K);
+        T *const U = B.rows(K);
+        T finite = T(0);
+        bool going = true;
+        nm::static_for<kPanel>([&](auto pivot) NM_INLINE {
+            constexpr int t = decltype(pivot)::value;
+            X[t] = stored >> t & 1u ? X[t] : T(0);
+            finite = __builtin_fma(X[t], T(0), finite);
+            if constexpr (t == 0)   // (panel K has taken the rows that these replace)
+                going = B.kept > 2 || band_wait<false>(B.count, band_need(kBandAny, kPivots, 1, K * kPanel + 1));
+            if (mine) U[t * B.uc + at] = X[t];
+            band_tell(B.count, kRows0 + w, K * kPanel + t + 1);
+            if constexpr (t + 1 < kPanel) {
+                going = going && band_wait<false>(B.count, band_need(kBandAny, kPivots, 1, K * kPanel + t + 1));
+                const Eight<T> l = *reinterpret_cast<const Eight<T> *>(F + t * B.fp);
+#pragma unroll
+                for (int s = t + 1; s < kPanel; ++s) {
+                    const T p = l.v[s] * X[t];
+                    X[s] = X[s] - p;
+                }
+            }
+        });
+        if (!going) return;
+        if (__any(finite != T(0))) {
+            band_tell(B.count, kStop, 1);
+            return;
         }
-        stage();
+        band_tell(B.count, kGoodRows0 + w, K + 1);
+        row_slot = ring(row_slot + 1, B.rb);
+        col_slot = ring(col_slot + 1, B.cb);
+    }
+}
+
+// Six wavefronts: the panel applied to the columns from the third block right of it on and the rows from the second
+// block below it on, a block of columns at a time.
+template <typename T, int RL> __device__ __forceinline__ void band_trailing(const Band<T> &B, int w) {
+    const int lane = threadIdx.x & 63;
+    if (B.bub < 3 || B.blb < 2) return;
+    // (a block of columns stays with the wavefront of its number modulo six, so nobody waits for another's update)
+    int32_t row_slot = (2 + lane / kPanel) % B.rb, col_slot = 3 % B.cb, first = w < 3 ? w + kBandTrailing - 3 : w - 3;
+    for (int32_t K = 0; K < B.panels; ++K, first = first == 0 ? kBandTrailing - 1 : first - 1) {
+        int32_t least = band_need(kBandAny, kPivots, 3, (K + 1) * kPanel);
+        least = band_need(least, kLoaded, kLoaders, K + 1);
+        if (!band_wait<true>(B.count, least)) return;
+        const T *const F = B.multipliers(K) + 2 * kPanel, *const U = B.rows(K);
+        for (int32_t b = 3 + first; b <= B.bub && K + b < B.panels; b += kBandTrailing) {
+            T *const block = B.column(ring(col_slot + (b - 3), B.cb) * kPanel);
+            int32_t at[RL];
+            bool mine[RL];
+            T W[RL][kPanel];
+#pragma unroll
+            for (int q = 0; q < RL; ++q) {
+                mine[q] = lane / kPanel + 8 * q + 1 < B.blb;
+                at[q] = (mine[q] ? (row_slot + 8 * q) % B.rb : 0) * kPanel + (lane & 7);
+#pragma unroll
+                for (int c = 0; c < kPanel; ++c) W[q][c] = block[c * B.pitch + at[q]];
+            }
+#pragma unroll 2
+            for (int t = 0; t < kPanel; ++t) {
+                const Eight<T> u = *reinterpret_cast<const Eight<T> *>(U + t * B.uc + (b - 1) * kPanel);
+#pragma unroll
+                for (int q = 0; q < RL; ++q) {
+                    const T l = F[t * B.fp + (mine[q] ? lane + 64 * q : 0)];
+#pragma unroll
+                    for (int c = 0; c < kPanel; ++c) {
+                        const T p = l * u.v[c];
+                        W[q][c] = W[q][c] - p;
+                    }
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < RL; ++q)
+                if (mine[q]) {
+#pragma unroll
+                    for (int c = 0; c < kPanel; ++c) block[c * B.pitch + at[q]] = W[q][c];
+                }
+        }
+        asm volatile("" ::: "memory");
+        band_tell(B.count, kTrailing0 + w, K + 1);
+        row_slot = ring(row_slot + 1, B.rb);
+        col_slot = ring(col_slot + 1, B.cb);
+    }
+}
+
+template <typename T> __device__ __forceinline__ bool negative_zero(T v) { return v == T(0) && __builtin_signbit(v); }
+
+// Wavefronts 14 and 15: the blocks of columns in turn, block n + bub coming into the window with panel n (the first ones with
+// panel 0), down to the window's last row then.  A block is requested before the one before it is placed.
+template <typename T> struct BandColumns {
+    int64_t ptr;                  // lane c: where column c starts
+    int32_t row[kPanel][2];
+    T value[kPanel][2];
+    __device__ __forceinline__ int64_t start(int c) const {
+        return (int64_t)((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(ptr >> 32), c) << 32 |
+                         (uint32_t)__builtin_amdgcn_readlane((int)ptr, c));
+    }
+};
+template <typename T> __device__ __forceinline__ void band_load_columns(const Band<T> &B, int w) {
+    const int lane = threadIdx.x & 63;
+    const int32_t cbs = B.cb * kPanel;
+    auto pointers = [&](int32_t block) NM_INLINE { return B.indptr[min(block * kPanel + min(lane, kPanel), B.n)]; };
+    auto fetch = [&](BandColumns<T> &C, int64_t ptr) NM_INLINE {
+        C.ptr = ptr;
+#pragma unroll
+        for (int c = 0; c < kPanel; ++c) {
+            const int64_t b = C.start(c);
+            const int32_t length = (int32_t)(C.start(c + 1) - b);
+            // (an empty column: the entry before it, or the first of all)
+            const int64_t from = length > 0 ? b : max(b - 1, (int64_t)0);
+            const T *const values = B.values + from;
+            const int32_t *const rows = reinterpret_cast<const int32_t *>(B.indices + from);   // (low halves: rows fit 31 bits)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                if (q > 0 && length <= 64) continue;
+                const uint32_t at = min(lane + 64 * q, max(length - 1, 0));
+                C.row[c][q] = rows[2 * at];
+                C.value[c][q] = values[at];
+            }
+        }
+    };
+    auto place = [&](const BandColumns<T> &C, int32_t block) NM_INLINE {
+        const int32_t n = max(block - B.bub, 0), slot = block % B.cb * kPanel;
+        int32_t least = band_need(kBandAny, kPivots, 3, (n + 1 - B.slack) * kPanel);
+        least = band_need(least, kWritten, 1, n + 1 - B.slack);
+        if (!band_wait<true>(B.count, least)) return false;
+        const int32_t limit = (n + B.blb + 1) * kPanel, row_slot = n % B.rb;
+#pragma unroll
+        for (int c = 0; c < kPanel; ++c)
+            for (int32_t r = lane; r < B.rb * kPanel; r += 64) B.column(slot + c)[r] = T(0);
+        if (lane < B.rb) *reinterpret_cast<uint64_t *>(B.has + lane * cbs + slot) = 0ull;
+        asm volatile("" ::: "memory");
+        bool negative = false;
+#pragma unroll
+        for (int c = 0; c < kPanel; ++c) {
+            const int64_t begin = C.start(c);
+            const int32_t length = (int32_t)(C.start(c + 1) - begin);
+            int32_t in = 0;
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                if (q > 0 && length <= 64) continue;
+                const bool there = lane + 64 * q < length && C.row[c][q] < limit;
+                const uint64_t all = __ballot(there);
+                in += __popcll(all);
+                if (all != 0 && there) {
+                    const int32_t at = ring(row_slot + (C.row[c][q] / kPanel - n), B.rb), s = C.row[c][q] & 7;
+                    B.column(slot + c)[at * kPanel + s] = C.value[c][q];
+                    atomicOr(reinterpret_cast<uint32_t *>(B.has + at * cbs + slot) + c / 4, 1u << (8 * (c & 3) + s));
+                    negative = negative || negative_zero(C.value[c][q]);
+                }
+            }
+            if (lane == 0) {
+                B.base[slot + c] = begin;
+                B.len[slot + c] = length;
+                B.in[slot + c] = in;
+                B.out[slot + c] = 0;
+            }
+        }
+        if (__any(negative)) band_tell(B.count, kNegativeZero, 1);
+        asm volatile("" ::: "memory");
+        // (the next block is the other wavefront's)
+        band_tell(B.count, kColumns0 + w, max(block + 2 - B.bub, 0));
+        return true;
+    };
+    // (two sets by name: a copy would wait for the loads; a block past the last one is nobody's, its columns are empty)
+    BandColumns<T> C, D;
+    int64_t next = pointers(w + 2);
+    fetch(C, pointers(w));
+    for (int32_t block = w; block < B.panels; block += 4) {
+        fetch(D, next);
+        next = pointers(block + 4);
+        if (!place(C, block)) return;
+        if (block + 2 >= B.panels) break;
+        fetch(C, next);
+        next = pointers(block + 6);
+        if (!place(D, block + 2)) return;
+    }
+    band_tell(B.count, kColumns0 + w, kBandNever);
+}
+
+// Wavefronts 6 and 7: the rows that come into the window with panel n.  A lane keeps to one place for a column, whose
+// entries it takes in their order, requested before the rows' place is free.
+template <typename T> __device__ __forceinline__ void band_load_rows(const Band<T> &B, int w) {
+    const int lane = threadIdx.x & 63, slot = 64 * w + lane;
+    const int32_t cbs = B.cb * kPanel;
+    if (64 * w >= cbs) return;
+    band_tell(B.count, kIn0 + w, 1);   // (panel 0 has nothing but new columns)
+    int32_t row_slot = (1 + B.blb) % B.rb, ahead = slot / kPanel;   // blocks from panel n's own to the lane's
+    int32_t left = 0;
+    int64_t from = 0;
+    for (int32_t n = 1; n < B.panels; ++n) {
+        ahead = ahead == 0 ? B.cb - 1 : ahead - 1;
+        const bool active = slot < cbs && ahead < B.bub && (n + ahead) * kPanel + (lane & 7) < B.n;
+        if (!band_wait<true>(B.count, band_need(kBandAny, kColumns0, 2, n))) return;
+        if (active && (n == 1 || ahead == B.bub - 1)) {
+            left = B.len[slot] - B.in[slot];
+            from = B.base[slot] + B.in[slot];
+        }
+        int32_t row[kPanel];
+        T value[kPanel];
+#pragma unroll
+        for (int s = 0; s < kPanel; ++s) {
+            const int64_t e = active ? max(from + min(s, left - 1), (int64_t)0) : 0;
+            row[s] = reinterpret_cast<const int32_t *>(B.indices)[2 * e];
+            value[s] = B.values[e];
+        }
+        int32_t least = band_need(kBandAny, kPivots, 3, (n + 1 - B.slack) * kPanel);
+        least = band_need(least, kWritten, 1, n + 1 - B.slack);
+        if (!band_wait<true>(B.count, least)) return;
+        if (active) {
+            const int32_t limit = (n + B.blb + 1) * kPanel;
+            T *const column = B.column(slot) + row_slot * kPanel;
+#pragma unroll
+            for (int s = 0; s < kPanel; ++s) column[s] = T(0);
+            asm volatile("" ::: "memory");
+            uint32_t has = 0;
+            int32_t taken = 0;
+            bool negative = false;
+#pragma unroll
+            for (int s = 0; s < kPanel; ++s)
+                if (s < left && row[s] < limit) {
+                    column[row[s] & 7] = value[s];
+                    has |= 1u << (row[s] & 7);
+                    ++taken;
+                    negative = negative || negative_zero(value[s]);
+                }
+            B.has[row_slot * cbs + slot] = (uint8_t)has;
+            left -= taken;
+            from += taken;
+            if (negative) lds_put(B.count + kNegativeZero, 1);
+        }
+        asm volatile("" ::: "memory");
+        band_tell(B.count, kIn0 + w, n + 1);
+        row_slot = ring(row_slot + 1, B.rb);
+    }
+}
+
+// Wavefront 4: a panel's rows and columns into the arrays, once all of them are known to be finite.
+template <typename T> __device__ __forceinline__ void band_write(const Band<T> &B) {
+    const int lane = threadIdx.x & 63;
+    const int32_t width = B.bub * kPanel, cbs = B.cb * kPanel;
+    int32_t row_slot = 0, col_slot = 0;
+    for (int32_t K = 0; K < B.panels; ++K) {
+        int32_t least = band_need(kBandAny, kGoodPanel0 + (K & 1), 1, K + 1);
+        least = band_need(least, kGoodRows0, 2, K + 1);
+        if (!band_wait<true>(B.count, least)) return;
+        const T *const F = B.multipliers(K), *const U = B.rows(K);
+        const int32_t own = col_slot * kPanel + (lane & 7);
+        const int64_t start = B.base[own] + B.out[own];   // of column lane % 8
+        int64_t at[kPanel];
+#pragma unroll
+        for (int c = 0; c < kPanel; ++c)
+            at[c] = (int64_t)((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(start >> 32), c) << 32 | (uint32_t)__builtin_amdgcn_readlane((int)start, c));
+        for (int32_t r0 = 0; r0 < B.fr; r0 += 64) {
+            const int32_t r = r0 + lane;
+            const uint64_t m = r < B.fr ? *reinterpret_cast<const uint64_t *>(B.has + ring(row_slot + r / kPanel, B.rb) * cbs + col_slot * kPanel) >> (r & 7) : 0;
+            T x[kPanel];
+#pragma unroll
+            for (int c = 0; c < kPanel; ++c) x[c] = F[c * B.fp + r];
+#pragma unroll
+            for (int c = 0; c < kPanel; ++c) {
+                const bool stored = (m >> 8 * c & 1) != 0;
+                const uint64_t all = __ballot(stored);
+                if (stored) B.values[at[c] + __popcll(all & ((1ull << lane) - 1ull))] = x[c];
+                at[c] += __popcll(all);
+            }
+        }
+        for (int32_t at0 = 0; at0 < width; at0 += 64) {
+            const int32_t at = at0 + lane;
+            if (at < width && (K + 1) * kPanel + at < B.n) {
+                const int32_t slot = ring(col_slot + 1 + at / kPanel, B.cb) * kPanel + (lane & 7);
+                const uint32_t has = B.has[row_slot * cbs + slot];
+                const int32_t before = B.out[slot];
+                T *const out = B.values + B.base[slot] + before;
+                T x[kPanel];
+#pragma unroll
+                for (int s = 0; s < kPanel; ++s) x[s] = U[s * B.uc + at];
+#pragma unroll
+                for (int s = 0; s < kPanel; ++s)
+                    if (has >> s & 1u) out[__popc(has & ((1u << s) - 1u))] = x[s];
+                B.out[slot] = before + __popc(has);
+            }
+        }
+        asm volatile("" ::: "memory");
+        band_tell(B.count, kWritten, K + 1);
+        row_slot = ring(row_slot + 1, B.rb);
+        col_slot = ring(col_slot + 1, B.cb);
     }
 }
 
 template <typename T>
 __global__ __launch_bounds__(kBandWaves * 64) void lu_band_kernel(int32_t n, const int64_t *__restrict__ indices,
                                                                   const int64_t *__restrict__ indptr, T *values,
-                                                                  int32_t *ctl) {
-    __shared__ BandShared sh;
+                                                                  int32_t *ctl, int32_t *done) {
+    __shared__ __align__(16) unsigned char s_band[kBandLds];
     const int bu = ctl[4], bl = ctl[5];
     if (ctl[6] > kBandMaxBreaks || n >= 1 << 30 || indptr[n] == 0) return;   // lu_flow_kernel's
-    // The smallest set of registers that holds the band: the ring (above), and room for bu + 4 columns, as
-    // a column is in place two steps after its predecessor is done.  us a column, fp64, this kernel
-    // and lu_flow_kernel: reach 28 0.27 and 1.24, reach 60 0.50 and 1.30, reach 76 0.61 and 2.2, reach
-    // 92 0.70 and 2.2.
-    auto fits = [&](int rl, int cs) { return bu + 4 <= kBandWaves * cs && bl + kBandWaves * cs <= 64 * rl; };
-    if (fits(1, 2)) lu_band<T, 1, 2>(n, bl, indices, indptr, values, sh);
-    else if (fits(2, 4)) lu_band<T, 2, 4>(n, bl, indices, indptr, values, sh);
-    else if (fits(3, 5)) lu_band<T, 3, 5>(n, bl, indices, indptr, values, sh);
-    else if (fits(3, 6)) lu_band<T, 3, 6>(n, bl, indices, indptr, values, sh);
-    else return;
-    // lu_flow_kernel finds no column left to draw.  (A flag that it looks at first is 8 us less of 2.5 ms
-    // here, and 50 us of 1.32 ms there for an arrowhead of 1000 columns: the test costs its loop over a column.)
-    if (threadIdx.x == 0) ctl[0] = n;
+    Band<T> B;
+    B.n = n;
+    B.panels = (n + kPanel - 1) / kPanel;
+    B.blb = max(1, (bl + kPanel - 1) / kPanel);
+    B.bub = max(1, (bu + kPanel - 1) / kPanel);
+    if (B.blb > 15 || B.bub > 13) return;
+    B.fr = (B.blb + 1) * kPanel;
+    B.fp = (B.fr + 63) / 64 * 64;
+    B.uc = B.bub * kPanel;
+    // room for the loads and the writes to lag behind, as much as LDS has
+    size_t used = 0;
+    for (B.slack = 5, B.kept = 4; ; B.slack = 3, B.kept = 2) {
+        B.rb = B.blb + B.slack;
+        B.cb = B.bub + B.slack;
+        B.pitch = B.rb * kPanel + 1;
+        used = 0;
+        auto take = [&](size_t bytes) {
+            unsigned char *p = s_band + used;
+            used += (bytes + 15) & ~size_t(15);
+            return p;
+        };
+        const int32_t columns = B.cb * kPanel;
+        B.count = reinterpret_cast<int32_t *>(take(kBandCounts * 4));
+        B.base = reinterpret_cast<int64_t *>(take(columns * 8));
+        B.len = reinterpret_cast<int32_t *>(take(columns * 4));
+        B.in = reinterpret_cast<int32_t *>(take(columns * 4));
+        B.out = reinterpret_cast<int32_t *>(take(columns * 4));
+        B.has = take(B.rb * columns);
+        B.F = reinterpret_cast<T *>(take((size_t)B.kept * kPanel * B.fp * sizeof(T)));
+        B.U = reinterpret_cast<T *>(take((size_t)B.kept * kPanel * B.uc * sizeof(T)));
+        B.win = reinterpret_cast<T *>(take((size_t)columns * B.pitch * sizeof(T)));
+        if ((used <= kBandLds && B.cb <= 16) || B.slack == 3) break;   // (128 places for columns: band_load_rows)
+    }
+    if (used > kBandLds || B.cb > 16 || B.rb > 64) return;   // (the same in every thread, as are the other ways out above)
+    B.indices = indices;
+    B.indptr = indptr;
+    B.values = values;
+    const int v = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (threadIdx.x < kBandCounts) {
+        // wavefronts with nothing to do keep nobody waiting
+        const int i = threadIdx.x;
+        const bool idle = (B.bub <= 8 && (i == kRows1 || i == kGoodRows1)) || (B.cb <= 8 && i == kIn1) ||
+                          (i >= kTrailing0 && (B.bub < 3 || B.blb < 2));
+        B.count[i] = idle ? kBandNever : 0;
+    }
+    __syncthreads();
+    // (a SIMD takes every fourth wavefront: the panels' have the least company)
+    if (v < 2) {
+        if (B.fr <= 64) band_panels<T, 1, 1>(B, v);
+        else if (B.fr <= 72) band_panels<T, 2, 1>(B, v);
+        else band_panels<T, 2, 2>(B, v);
+    } else if (v < 4) {
+        band_rows<T>(B, v - 2);
+    } else if (v == 4) {
+        __builtin_amdgcn_s_setprio(1);
+        band_write<T>(B);
+    } else if (v == 8 || v == 9) {
+        __builtin_amdgcn_s_setprio(1);
+        band_load_rows<T>(B, v - 8);
+    } else if (v == 14 || v == 15) {
+        __builtin_amdgcn_s_setprio(1);
+        band_load_columns<T>(B, v - 14);
+    } else if (v != 12) {
+        const int w = v == 6 ? 0 : v == 7 ? 1 : v == 10 ? 2 : v == 11 ? 3 : v == 5 ? 4 : 5;
+        if (B.blb <= 9) band_trailing<T, 1>(B, w);
+        else band_trailing<T, 2>(B, w);
+    }
+    __syncthreads();
+    // lu_flow_kernel finds no column left to draw, or goes on behind the last panel that is written (ctl[7]).
+    const int32_t written = min(B.count[kWritten] * kPanel, n);
+    if (written < n) {
+        for (int32_t k = threadIdx.x; k < written; k += kBandWaves * 64) done[k] = 1;
+        if (written == 0) return;   // (from the start)
+    }
+    if (threadIdx.x == 0) {
+        ctl[0] = n;
+        ctl[7] = written < n ? written : 0;
+        ctl[8] = written < n ? written : n;
+    }
 }
 
 int check_rows(int64_t rows) {
@@ -994,11 +1215,10 @@ extern "C" int nm_splu_numeric(nm_dtype dt, int64_t cols, void *Mt_data, const i
         return nm::fail(NM_ERR_WORKSPACE, "workspace of %zu bytes, %zu needed", workspace_bytes, need);
     hipStream_t s = nm::as_stream(stream);
     if (int rc = nm::fill_async(F.ctl, 16, (int32_t)0, s)) return rc;
-    if (int rc = nm::fill_async(F.done, cols, (int32_t)0, s)) return rc;
     {
         int64_t g = nm::ceil_div(cols, kBlock);
         hipLaunchKernelGGL(lu_below_kernel, dim3((unsigned)(g > 65536 ? 65536 : g)), dim3(kBlock), 0, s, cols,
-                           Mt_indices, Mt_indptr, F.below, F.ctl);
+                           Mt_indices, Mt_indptr, F.below, F.done, F.ctl);
         NM_LAUNCH_CHECK("lu_below_kernel");
     }
     // Whether the factors are a band is known on the device only: the band kernel leaves at once
@@ -1007,28 +1227,27 @@ extern "C" int nm_splu_numeric(nm_dtype dt, int64_t cols, void *Mt_data, const i
     if (poll_limit <= 0) {
         if (dt == NM_F32)
             hipLaunchKernelGGL(lu_band_kernel<float>, dim3(1), dim3(kBandWaves * 64), 0, s, (int32_t)cols, Mt_indices,
-                               Mt_indptr, (float *)Mt_data, F.ctl);
+                               Mt_indptr, (float *)Mt_data, F.ctl, F.done);
         else
             hipLaunchKernelGGL(lu_band_kernel<double>, dim3(1), dim3(kBandWaves * 64), 0, s, (int32_t)cols, Mt_indices,
-                               Mt_indptr, (double *)Mt_data, F.ctl);
+                               Mt_indptr, (double *)Mt_data, F.ctl, F.done);
         NM_LAUNCH_CHECK("lu_band_kernel");
     }
     int64_t grid = nm::ceil_div(cols, kLuWavesPerBlock);
     if (grid > 1024) grid = 1024;
     const int64_t limit = poll_limit > 0 ? poll_limit : kLuSpinLimit;
     const size_t lds = (size_t)kLuWavesPerBlock * kLuCap * ((dt == NM_F32 ? 4 : 8) + 4);
-    if (lds > 64 * 1024) {
-        const void *fn = dt == NM_F32 ? reinterpret_cast<const void *>(lu_flow_kernel<float>)
-                                      : reinterpret_cast<const void *>(lu_flow_kernel<double>);
-        NM_HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    }
-    if (dt == NM_F32)
-        hipLaunchKernelGGL(lu_flow_kernel<float>, dim3((unsigned)grid), dim3(kLuFlowBlock), lds, s, cols, Mt_indices,
-                           Mt_indptr, F.below, (float *)Mt_data, F.done, F.ctl, limit);
-    else
-        hipLaunchKernelGGL(lu_flow_kernel<double>, dim3((unsigned)grid), dim3(kLuFlowBlock), lds, s, cols, Mt_indices,
-                           Mt_indptr, F.below, (double *)Mt_data, F.done, F.ctl, limit);
-    NM_LAUNCH_CHECK("lu_flow_kernel");
+    auto flow = [&](auto value) -> int {
+        using T = decltype(value);
+        if (lds > 64 * 1024)
+            NM_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(lu_flow_kernel<T>),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        hipLaunchKernelGGL(lu_flow_kernel<T>, dim3((unsigned)grid), dim3(kLuFlowBlock), lds, s, cols, Mt_indices,
+                           Mt_indptr, F.below, (T *)Mt_data, F.done, F.ctl, limit);
+        NM_LAUNCH_CHECK("lu_flow_kernel");
+        return NM_OK;
+    };
+    if (int rc = dt == NM_F32 ? flow(0.f) : flow(0.)) return rc;
     int32_t ctl_h[2] = {0, 0};
     if (hipMemcpyAsync(ctl_h, F.ctl, sizeof(ctl_h), hipMemcpyDeviceToHost, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess)
