@@ -259,6 +259,12 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_num_sgpr(72))) void sp
     // rt <= R: rows per block of this launch (block_rows)
     constexpr bool STAGE = LISTS && NM_STAGE_FWD && NM_FWD32_VEC && sizeof(IDX) == 4 && !UNIT && R == nm::kPackRows;
     constexpr bool HAS_LISTS = NM_STAGE_FWD && sizeof(IDX) == 4 && !UNIT && R == nm::kPackRows;
+    // 64-bit structure, fp64: a lane takes 2 consecutive entries per request (16 bytes of values and of columns, aligned
+    // to 8), three requests in flight, and the row pointers wait in registers as below.  Requests bound it, not
+    // bytes: 127 x 113 x 101 seven-point 41.4 -> 36.7 us (two and four in flight 37.7, 38.8), 27-point on 60^3 24.1 ->
+    // 21.5, 1024^2 five-point 21.4 -> 20.9, 20 random entries a row the same.  Not in fp32, whose 8-byte value
+    // requests gain nothing there (29.3 -> 29.2) and lose on 1024^2 (16.5 -> 18.7).
+    constexpr bool PAIRS = sizeof(IDX) == 8 && sizeof(T) == 8 && !UNIT;
     __shared__ int32_t s_off[R + 1];
     __shared__ __align__(16) T s_prod[CAP];
     __shared__ __align__(16) T s_x[STAGE ? nm::kStageFwd * nm::kStageSeg : 4];
@@ -316,7 +322,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_num_sgpr(72))) void sp
         int32_t po[Q];
         bool early = false;
         int n_early = 0;
-        if (NM_FWD_EARLY && NM_FWD32_VEC && sizeof(IDX) == 4 && !UNIT) {
+        if (NM_FWD_EARLY && NM_FWD32_VEC && !UNIT && (sizeof(IDX) == 4 || PAIRS)) {
             const int64_t span = (int64_t)indptr[r0 + nr] - base;
             early = span <= CAP;
             n_early = (int)span;
@@ -393,28 +399,64 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_num_sgpr(72))) void sp
         } else if (n <= CAP) {
             const T *__restrict__ d = data + base;
             const IDX *__restrict__ ci = indices + base;
-            // K entries in flight per lane: all their streams, then all their gathers of x.
-            // Loads are unconditional on a clamped position (a predicated load would sit in
-            // its own branch with its own wait).
-            constexpr int K = sizeof(IDX) == 4 ? NM_FWD32_K : 5;   // int64: 4, 5 and 10 measure the same on the 2048 x 2048 Poisson matrix
-            for (int k0 = threadIdx.x; k0 < n; k0 += K * BLOCK) {
-                T aa[K], xx[K];
-                IDX cc[K];
+            if constexpr (PAIRS) {
+                typedef T TV __attribute__((ext_vector_type(2), aligned(sizeof(T))));
+                typedef IDX IV __attribute__((ext_vector_type(2), aligned(sizeof(IDX))));
+                const int n2 = n & ~1;
+                constexpr int U = 3;
+                for (int k0 = threadIdx.x * 2; k0 < n2; k0 += U * 2 * BLOCK) {
+                    TV aa[U];
+                    IV cc[U];
+                    T xx[U][2];
 #pragma unroll
-                for (int u = 0; u < K; ++u) {
-                    const int kc = k0 + u * BLOCK < n ? k0 + u * BLOCK : n - 1;
-                    aa[u] = nm::stream_load(d + kc);
-                    if (!UNIT) cc[u] = nm::stream_load(ci + kc);
+                    for (int u = 0; u < U; ++u) {
+                        const int kc = k0 + u * 2 * BLOCK < n2 ? k0 + u * 2 * BLOCK : n2 - 2;
+                        aa[u] = __builtin_nontemporal_load(reinterpret_cast<const TV *>(d + kc));
+                        cc[u] = __builtin_nontemporal_load(reinterpret_cast<const IV *>(ci + kc));
+                    }
+#pragma unroll
+                    for (int u = 0; u < U; ++u)
+#pragma unroll
+                        for (int q = 0; q < 2; ++q) xx[u][q] = x[cc[u][q]];
+#pragma unroll
+                    for (int u = 0; u < U; ++u)
+                        if (k0 + u * 2 * BLOCK < n2) {
+#pragma unroll
+                            for (int q = 0; q < 2; ++q) s_prod[k0 + u * 2 * BLOCK + q] = aa[u][q] * xx[u][q];
+                        }
                 }
+                if (n2 < n && threadIdx.x == 0) s_prod[n2] = d[n2] * x[ci[n2]];
+            } else {
+                // K entries in flight per lane: all their streams, then all their gathers of x.
+                // Loads are unconditional on a clamped position (a predicated load would sit in
+                // its own branch with its own wait).
+                constexpr int K = sizeof(IDX) == 4 ? NM_FWD32_K : 5;   // int64: 4, 5 and 10 measure the same on the 2048 x 2048 Poisson matrix
+                for (int k0 = threadIdx.x; k0 < n; k0 += K * BLOCK) {
+                    T aa[K], xx[K];
+                    IDX cc[K];
 #pragma unroll
-                for (int u = 0; u < K; ++u) xx[u] = UNIT ? T(1) : x[cc[u]];
-                if (k0 + (K - 1) * BLOCK < n) {
+                    for (int u = 0; u < K; ++u) {
+                        const int kc = k0 + u * BLOCK < n ? k0 + u * BLOCK : n - 1;
+                        aa[u] = nm::stream_load(d + kc);
+                        if (!UNIT) cc[u] = nm::stream_load(ci + kc);
+                    }
 #pragma unroll
-                    for (int u = 0; u < K; ++u) s_prod[k0 + u * BLOCK] = aa[u] * xx[u];
-                } else {
+                    for (int u = 0; u < K; ++u) xx[u] = UNIT ? T(1) : x[cc[u]];
+                    if (k0 + (K - 1) * BLOCK < n) {
 #pragma unroll
-                    for (int u = 0; u < K; ++u)
-                        if (k0 + u * BLOCK < n) s_prod[k0 + u * BLOCK] = aa[u] * xx[u];
+                        for (int u = 0; u < K; ++u) s_prod[k0 + u * BLOCK] = aa[u] * xx[u];
+                    } else {
+#pragma unroll
+                        for (int u = 0; u < K; ++u)
+                            if (k0 + u * BLOCK < n) s_prod[k0 + u * BLOCK] = aa[u] * xx[u];
+                    }
+                }
+            }
+            if (early) {
+#pragma unroll
+                for (int q = 0; q < Q; ++q) {
+                    const int t = (int)threadIdx.x + q * BLOCK;
+                    if (t <= nr) s_off[t] = po[q];
                 }
             }
             __syncthreads();
