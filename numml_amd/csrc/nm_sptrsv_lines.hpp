@@ -21,9 +21,15 @@
 //
 // The division is the hardware's own sequence (reciprocal, two refinements, quotient, remainder,
 // quotient) with the first half, which knows the diagonal only, done in that pass.  The sequence is valid as it
-// stands where nothing has to be scaled: the pass leaves NaN for a diagonal outside 2^-128 .. 2^128, a quotient
-// outside 2^-256 .. 2^256 (a zero, an infinity, NaN among them) is looked for once a block of eight steps, and
-// the wavefront takes a block that has one again with divisions in full.
+// stands where nothing has to be scaled: the pass leaves NaN for a diagonal outside 2^-128 .. 2^128, and a quotient
+// outside 2^-800 .. 2^800 (a zero, an infinity, NaN among them) is looked for once a block of eight steps.  (The
+// remainder's last bit is then 2^-128-800-104 at least, so none of the sequence is rounded as a denormal.)
+// The wavefront goes on with divisions in full at a block that has such a quotient, 90 ns a step instead of 68, and
+// returns to the short ones after sixteen blocks that have none.  Zeros are what it meets in earnest: the
+// rows ahead of the first right-hand side that is not zero.  us with a dense right-hand side, with zeros
+// throughout, and that level by level (a wavefront that made such blocks again one by one and always
+// tried the short division first: the figure in brackets): 1024 x 1024 fp64 209, 281 (684), 700;
+// 97 x 89 x 101 120, 136 (284), 325; 300 x 70 38, 54 (119), 104; 64 x 64 18, 21 (44), 37.
 //
 // Sums run in double in the serial loop's order (cpp/sparse_csr_cpu.cpp:672-718: the farthest dependency
 // first), a dependency that is not there adding a zero product to a sum that is never -0: the same bits.
@@ -39,10 +45,11 @@ constexpr int kAhead = 16;         // steps that operands are requested ahead
 // Steps of a block, after which a wavefront looks at what the others have done (four: 64 x 4096 282 -> 330 us, and no
 // more than 2 % off what hands over most, 97 x 89 x 101).
 constexpr int kBlockSteps = 8;
+constexpr int kFullBlocks = 16;    // blocks without a quotient that needs it for which the division in full is kept up
 constexpr int kPatch = 8;          // lines of a patch in either direction of a volume
 constexpr int kSkewPlane = 2;      // steps from a line to the one of the next plane
 constexpr unsigned long long kUnsolved = ~0ull;   // a NaN; a result with these bits is handed on as the default NaN
-constexpr unsigned kSafeDiag = 128, kSafeQuotient = 256;   // exponents
+constexpr unsigned kSafeDiag = 128, kSafeQuotient = 800;   // exponents
 
 // A grid in the roles that its directions have here: lines run along one of them, a patch's lanes b (neighbours a step
 // apart) and a (kSkewPlane steps apart) lie along the others.
@@ -254,13 +261,10 @@ __device__ __forceinline__ void leave(unsigned long long *at, double v) {
 // LINE_LAST: the row before of the line is the nearest, whose product the serial sum adds last; else b's is.
 template <typename T, bool THREE, bool LINE_LAST> __device__ __forceinline__ void solve_patch(const Args<T> &k, const Patch &P, Shared &sh) {
     struct Operands { double2 near, rd; double y, far; };
-    typedef unsigned quad __attribute__((ext_vector_type(4)));
-    typedef unsigned pair __attribute__((ext_vector_type(2)));
     const int lane = threadIdx.x & 63;
     const int32_t length = k.g.length, w = P.na * P.nb, deepest = skew(P.na - 1, P.nb - 1), steps = length + deepest;
     const int a0 = THREE ? lane / kPatch : 0, b0 = THREE ? lane % kPatch : lane;
     const bool valid = a0 < P.na && b0 < P.nb;
-    const unsigned long long valid_lanes = __ballot(valid);
     const int32_t depth = valid ? skew(a0, b0) : 0x40000000;
     constexpr int kWidthY = THREE ? 16 : 8;
     const int32_t bytes = w * length * 16;
@@ -289,13 +293,7 @@ template <typename T, bool THREE, bool LINE_LAST> __device__ __forceinline__ voi
         place += w * 16;
         place = place == bytes ? 0 : place;
     };
-    // (in the order of the steps, here too: else the first step of every round waits for all that is under way)
     Operands o[kAhead];
-#pragma unroll
-    for (int s = 0; s < kAhead; ++s) {
-        request(o[s]);
-        asm volatile("" ::: "memory");
-    }
     double x = 0.;
     uint32_t worst = 0;   // of the block's quotients: how far from the smallest exponent that is safe
     auto step = [&](Operands &v, double import_n, double xg, int32_t t, double *keep, auto ramp, auto in_full) __attribute__((always_inline)) {
@@ -316,17 +314,12 @@ template <typename T, bool THREE, bool LINE_LAST> __device__ __forceinline__ voi
         const double n = v.rd.x - acc;
         bool live = true;
         if constexpr (ramp) live = (uint32_t)(t - depth) < (uint32_t)length;
-        double q;
-        if constexpr (in_full) {
-            q = n / v.rd.y;
-        } else {
-            q = n * v.y;
-            int high = __double2hiint(q);
-            asm volatile("" : "+v"(high));
-            const uint32_t off = ((uint32_t)high << 1) - ((1023u - kSafeQuotient) << 21);
-            worst = max(worst, live ? off : 0u);
-            q = __builtin_fma(__builtin_fma(-v.rd.y, q, n), v.y, q);
-        }
+        double q = in_full ? n / v.rd.y : n * v.y;
+        int high = __double2hiint(q);
+        asm volatile("" : "+v"(high));
+        const uint32_t off = ((uint32_t)high << 1) - ((1023u - kSafeQuotient) << 21);
+        worst = max(worst, live ? off : 0u);
+        if constexpr (!in_full) q = __builtin_fma(__builtin_fma(-v.rd.y, q, n), v.y, q);
         x = live ? q : 0.;
         *keep = x;
         // The lane of the next plane reads this from its own `lane`, an address that the compiler can prove is never the
@@ -350,9 +343,12 @@ template <typename T, bool THREE, bool LINE_LAST> __device__ __forceinline__ voi
     auto await = [&](int32_t t, double (&n)[kSteps]) __attribute__((always_inline)) {
         while (__any(missing(t))) ask(t, n);
     };
+    auto refused = [&]() __attribute__((always_inline)) { return valid && worst >= (2u * kSafeQuotient) << 21; };
+    // The first block that has a quotient which is not the short division's (-1: none).  It is made again with divisions in
+    // full; what comes after it in its round is nothing that anybody has been told of.
+    int32_t bad = -1;
     auto block = [&](Operands *ops, double (&n)[kSteps], double (&next_n)[kSteps], int32_t t, auto ramp) __attribute__((always_inline)) {
         double *const row = sh.x[t & (kKept - 1)];
-        const double before = x;
         worst = 0;
         // entry `lane` of the row two steps before, asked for a step ahead
         double xg = THREE ? sh.x[(t - 2) & (kKept - 1)][lane] : 0.;
@@ -365,39 +361,80 @@ template <typename T, bool THREE, bool LINE_LAST> __device__ __forceinline__ voi
             request(ops[s]);
             if constexpr (s == kSteps / 2) ask(t + kSteps, next_n);
         });
-        // (one test for all that hardly ever is)
-        const bool again = valid && worst >= (2u * kSafeQuotient) << 21;
-        if (__builtin_expect(__any(again || missing(t + kSteps)), 0)) {
-            if (__any(again)) {
-                x = before;
-#pragma unroll 1
-                for (int32_t s = t; s < t + kSteps; ++s) {
-                    Operands o;
-                    request_at(o, s % length * w * 16);
-                    step(o, sh.from_n[s & (kKept - 1)][THREE ? a0 : 0], THREE ? sh.x[(s - 2) & (kKept - 1)][lane] : 0., s,
-                         &sh.x[s & (kKept - 1)][kPatch + lane], std::true_type{}, std::true_type{});
-                }
-            }
-            lds_put(&sh.now.done, t + kSteps);
+        // (one test for all that hardly ever is.  In a volume most blocks have to wait: 97 x 89 x 101 120.6 us with that test,
+        // 119.5 without; 1024^2 446 and 462, both solves.)
+        const bool again = refused();
+        if (THREE || __builtin_expect(__any(again || missing(t + kSteps)) || bad >= 0, 0)) {
+            if (bad < 0 && __any(again)) bad = t;
+            if (bad < 0) lds_put(&sh.now.done, t + kSteps);
             await(t + kSteps, next_n);
         } else {
             lds_put(&sh.now.done, t + kSteps);
         }
     };
-    auto round = [&](int32_t t, auto ramp) __attribute__((always_inline)) {
+    int32_t t = 0;
+    auto round = [&](auto ramp) __attribute__((always_inline)) {
         nm::static_for<kAhead / kSteps>([&](auto part) __attribute__((always_inline)) {
             constexpr int i = decltype(part)::value;
             block(o + i * kSteps, import_n[i % 2], import_n[(i + 1) % 2], t + i * kSteps, ramp);
         });
+        t += kAhead;
     };
-    await(0, import_n[0]);
-    int32_t t = 0;
+    // From step t on with divisions in full, until kFullBlocks blocks in a row could have done without.
+    auto go_in_full = [&]() __attribute__((always_inline)) {
+        Operands v[kSteps];
+        double n[kSteps];
+        place = t % length * w * 16;
+#pragma unroll
+        for (int s = 0; s < kSteps; ++s) {
+            request(v[s]);
+            asm volatile("" ::: "memory");
+        }
+        ask(t, n);
 #pragma unroll 1
-    for (; t < deepest; t += kAhead) round(t, std::true_type{});
+        for (int left = kFullBlocks; left > 0 && t < steps; t += kSteps) {
+            double *const row = sh.x[t & (kKept - 1)];
+            worst = 0;
+            double xg = THREE ? sh.x[(t - 2) & (kKept - 1)][lane] : 0.;
+            nm::static_for<kSteps>([&](auto at) __attribute__((always_inline)) {
+                constexpr int s = decltype(at)::value;
+                const double xg_now = xg;
+                if constexpr (THREE && s == 0) xg = sh.x[(t - 1) & (kKept - 1)][lane];
+                else if constexpr (THREE && s + 1 < kSteps) xg = row[(s - 1) * kRow + lane];
+                step(v[s], n[s], xg_now, t + s, row + s * kRow + kPatch + lane, std::true_type{}, std::true_type{});
+                request(v[s]);
+            });
+            left = __any(refused()) ? kFullBlocks : left - 1;
+            lds_put(&sh.now.done, t + kSteps);
+            ask(t + kSteps, n);
+            await(t + kSteps, n);
+        }
+    };
+    while (true) {
+        // (in the order of the steps, here too: else the first step of every round waits for all that is under way)
+#pragma unroll
+        for (int s = 0; s < kAhead; ++s) {
+            request(o[s]);
+            asm volatile("" ::: "memory");
+        }
+        ask(t, import_n[0]);
+        await(t, import_n[0]);
+        bad = -1;
+        // (a patch that a right-hand side reaches late, or never, starts with zeros)
+        if (t == 0 && __any(lane == 0 && o[0].rd.x == 0. && import_n[0][0] == 0.)) bad = 0;
 #pragma unroll 1
-    for (; t + kAhead <= length; t += kAhead) round(t, std::false_type{});
+        while (t < deepest && bad < 0) round(std::true_type{});
 #pragma unroll 1
-    for (; t < steps; t += kAhead) round(t, std::true_type{});
+        while (t + kAhead <= length && bad < 0) round(std::false_type{});
+#pragma unroll 1
+        while (t < steps && bad < 0) round(std::true_type{});
+        if (bad < 0) break;
+        t = bad;
+        x = sh.x[(t - 1) & (kKept - 1)][kPatch + lane];
+        go_in_full();
+        place = t % length * w * 16;
+        if (t >= steps) break;
+    }
     // (nobody waits for more steps than there are, whatever multiple they count in)
     if (lane == 0) lds_put(&sh.now.done, kAll);
 }

@@ -96,6 +96,66 @@ def test_values_that_the_short_division_does_not_take(dev, dims):
     _compare(dev, d, i, p, n, np.float64, True, False, b)
 
 
+# lines along each direction, one patch and several, lines longer than sixteen blocks of eight steps
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("dims, lower", [((130, 400), True), ((400, 70), False), ((33, 9), True), ((9, 80, 300), False), ((300, 10, 11), True),
+                                         ((10, 300, 17), True)])
+def test_zeros_here_and_there(dev, dims, lower, dtype):
+    # Half of the couplings are zero, so that a zero of the right-hand side makes a zero quotient: the wavefront changes to
+    # divisions in full and back at any block, the first, the second of a round, the ramps at both ends.
+    d, i, p, n = _triangle(dims, lower, 11)
+    rng = np.random.default_rng(n)
+    row = np.repeat(np.arange(n), np.diff(p))
+    d[(row != i) & (rng.random(d.size) < 0.5)] = 0.
+    for share in (2 / n, 30 / n, 0.01, 0.5):
+        b = randn(12, n, np.float64)
+        b[rng.random(n) < share] = 0.
+        b[rng.random(n) < share / 4] = -0.
+        _compare(dev, d, i, p, n, dtype, lower, False, b)
+
+
+@pytest.mark.parametrize("dims, lower", [((70, 33), False), ((33, 70), True), ((10, 11, 12), False), ((9, 70, 10), True)])
+def test_quotients_at_the_ends_of_the_short_division(dev, dims, lower):
+    # diagonals around 2^+-128 and quotients around 2^+-800; decoupled rows, so that each has the quotient it is given
+    d, i, p, n = _triangle(dims, lower, 13)
+    rng = np.random.default_rng(13)
+    row = np.repeat(np.arange(n), np.diff(p))
+    d[row != i] = 0.
+    for far in (790, 799, 801, 1010):
+        e = rng.integers(-128, 128, n)
+        d[row == i] = np.ldexp(rng.uniform(1, 2, n) * rng.choice([-1, 1], n), e)
+        b = np.ldexp(rng.uniform(1, 2, n), np.clip(e + rng.choice([-far, far], n) + rng.integers(-2, 3, n), -1060, 1022))
+        _compare(dev, d, i, p, n, np.float64, lower, False, b)
+
+
+def _solve_time(solve):
+    for _ in range(3):
+        solve()
+    best = np.inf
+    for _ in range(5):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        for _ in range(10):
+            solve()
+        b.record()
+        torch.cuda.synchronize()
+        best = min(best, a.elapsed_time(b))
+    return best
+
+
+@pytest.mark.parametrize("dims", [(300, 70), (64, 64), (20, 21, 22)])
+def test_zeros_ahead_of_the_first_source_cost_little(dev, dims):
+    # Measured 1.4, 1.2 and 1.1 times a dense right-hand side's time; 3.1, 2.4 and 2.0 when every block that has a zero was
+    # made twice.
+    ext = numml_amd.load_compiled()
+    d, i, p, n = _triangle(dims, True, 14)
+    D, I, P, dense = to_dev(dev, d, i, p, randn(15, n, np.float64))
+    source = torch.zeros_like(dense)
+    source[n - 1] = 1.
+    t = [_solve_time(lambda: ext.sptrsv_forward(n, n, D, I, P, True, False, b)) for b in (dense, source)]
+    assert t[1] < 1.75 * t[0], t
+
+
 @pytest.mark.parametrize("what", ["missing", "extra", "far", "diagonal"])
 def test_patterns_that_are_almost_a_grids(dev, what):
     d, i, p, n = _triangle((300, 200), True, 5)
