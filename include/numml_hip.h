@@ -460,16 +460,18 @@ int nm_sptrsv_analyse(int64_t rows, int64_t nnz,
                       void *plan_mem, size_t plan_bytes, void *work, size_t work_bytes,
                       nm_sptrsv_plan **plan, nm_stream stream);
 
-/* Number of dependency levels / of level-kernel launches one solve with A issues. */
+/* Number of dependency levels / of level-kernel launches one solve with A issues (one where a grid's
+ * lines take it). */
 int64_t nm_sptrsv_plan_levels(const nm_sptrsv_plan *plan);
 int64_t nm_sptrsv_plan_launches(const nm_sptrsv_plan *plan);
 /* Levels of the solve with A (transposed = 0) or with A^T (1) that sit in runs of one-row levels
  * which a single wavefront walks with the newest solution in a register (banded factors,
- * bidiagonal and tridiagonal triangles); diagnostics. */
+ * bidiagonal and tridiagonal triangles); none where a grid's lines take the solve; diagnostics. */
 int64_t nm_sptrsv_plan_chain_levels(const nm_sptrsv_plan *plan, int transposed);
 /* Launches of the solve with A (transposed = 0) or with A^T (1) whose levels are each shared by
  * several workgroups (levels of more than 256 rows whose dependencies cross between the
- * workgroups' parts in a way that can be pipelined: triangles of grid stencils); diagnostics. */
+ * workgroups' parts in a way that can be pipelined: triangles of nine-point stencils, say); none where a
+ * grid's lines take the solve (nm_sptrsv_configure); diagnostics. */
 int64_t nm_sptrsv_plan_shared_launches(const nm_sptrsv_plan *plan, int transposed);
 
 void nm_sptrsv_plan_destroy(nm_sptrsv_plan *plan);

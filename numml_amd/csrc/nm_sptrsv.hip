@@ -2899,6 +2899,7 @@ extern "C" int64_t nm_sptrsv_plan_launches(const nm_sptrsv_plan *plan) {
 
 extern "C" int64_t nm_sptrsv_plan_chain_levels(const nm_sptrsv_plan *plan, int transposed) {
     if (!plan) return -1;
+    if (by_lines(plan)) return 0;
     int64_t n = 0;
     for (const auto &L : plan->launches)
         if (L.chain[transposed ? 1 : 0] != 0) n += L.l1 - L.l0;
@@ -2907,6 +2908,7 @@ extern "C" int64_t nm_sptrsv_plan_chain_levels(const nm_sptrsv_plan *plan, int t
 
 extern "C" int64_t nm_sptrsv_plan_shared_launches(const nm_sptrsv_plan *plan, int transposed) {
     if (!plan) return -1;
+    if (by_lines(plan)) return 0;
     int64_t n = 0;
     for (const auto &L : plan->launches)
         if (L.team[transposed ? 1 : 0].P > 1) ++n;

@@ -730,13 +730,11 @@ class _Plan:
             rows, nnz, _ptr(indices), _ptr(indptr), int(lower), _ptr(self.mem), pbytes.value,
             _ptr(work), wbytes.value, ctypes.byref(handle), _stream(dev)), "nm_sptrsv_analyse")
         self.handle = handle
-        self.levels = int(L.nm_sptrsv_plan_levels(handle))
-        self.launches = int(L.nm_sptrsv_plan_launches(handle))
-        self.chain_levels = (int(L.nm_sptrsv_plan_chain_levels(handle, 0)),
-                             int(L.nm_sptrsv_plan_chain_levels(handle, 1)))
-        self.shared_launches = (int(L.nm_sptrsv_plan_shared_launches(handle, 0)),
-                                int(L.nm_sptrsv_plan_shared_launches(handle, 1)))
         # nm_sptrsv_analyse synchronised its stream, so the plan is complete for every stream
+
+    def both(self, count):
+        # (of the solve with A and with A^T, under the switches as they are now)
+        return int(count(self.handle, 0)), int(count(self.handle, 1))
 
     def __del__(self):
         try:
@@ -860,7 +858,8 @@ def sptrsv_schedule(A_rows, A_indices, A_indptr, lower):
     A_indices, A_indptr = _idx(A_indices, "A_indices"), _idx(A_indptr, "A_indptr")
     with torch.cuda.device(dev):
         plan = _plan_for(A_indices, A_indptr, A_rows, lower, dev)
-    return plan.levels, plan.launches
+    L = _lib.lib()
+    return int(L.nm_sptrsv_plan_levels(plan.handle)), int(L.nm_sptrsv_plan_launches(plan.handle))
 
 
 def sptrsv_chain_levels(A_rows, A_indices, A_indptr, lower):
@@ -872,7 +871,7 @@ def sptrsv_chain_levels(A_rows, A_indices, A_indptr, lower):
     A_indices, A_indptr = _idx(A_indices, "A_indices"), _idx(A_indptr, "A_indptr")
     with torch.cuda.device(dev):
         plan = _plan_for(A_indices, A_indptr, A_rows, lower, dev)
-    return plan.chain_levels
+    return plan.both(_lib.lib().nm_sptrsv_plan_chain_levels)
 
 
 def sptrsv_shared_launches(A_rows, A_indices, A_indptr, lower):
@@ -884,7 +883,7 @@ def sptrsv_shared_launches(A_rows, A_indices, A_indptr, lower):
     A_indices, A_indptr = _idx(A_indices, "A_indices"), _idx(A_indptr, "A_indptr")
     with torch.cuda.device(dev):
         plan = _plan_for(A_indices, A_indptr, A_rows, lower, dev)
-    return plan.shared_launches
+    return plan.both(_lib.lib().nm_sptrsv_plan_shared_launches)
 
 
 def plan_cache_size():

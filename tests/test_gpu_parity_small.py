@@ -373,7 +373,7 @@ def test_sptrsv_signalling_equals_barriers_and_gives_up_instead_of_waiting_forev
     g = randn(4, n, np.float64)
     gA_ref, gb_ref = oracle.sptrsv_backward(g, x_ref, n, n, d, i, p, True, False)
     try:
-        for signalling in (1, 0):
+        for signalling in (1, 2, 0):   # signals, barriers, the grid's lines
             assert L.nm_sptrsv_configure(0, signalling) == 0
             x = ext.sptrsv_forward(n, n, D, I, P, True, False, Bv)
             assert_same(host(x), x_ref, f"x (signalling={signalling})")

@@ -42,6 +42,8 @@ def _compare(dev, d, i, p, n, dtype, lower, unit, b=None, by_lines=True):
     g = randn(6, n, dtype)
     D, I, P, Bv, Gv = to_dev(dev, d, i, p, b, g)
     assert (ext.sptrsv_schedule(n, I, P, lower)[1] == 1) == by_lines
+    if by_lines:   # and by nothing else
+        assert tuple(ext.sptrsv_shared_launches(n, I, P, lower)) == tuple(ext.sptrsv_chain_levels(n, I, P, lower)) == (0, 0)
     with np.errstate(all="ignore"):
         x_ref = oracle.sptrsv_forward(n, n, d, i, p, lower, unit, b)
         refs = oracle.sptrsv_backward(g, x_ref, n, n, d, i, p, lower, unit, b)
