@@ -505,7 +505,8 @@ int nm_sptrsv_solve(const nm_sptrsv_plan *plan, nm_dtype dt, int transposed,
  * solved line by line by one launch (unless bit 0 is set), goes by levels as well.  Results are
  * the same bits either way.
  * Bit 2 (for tests): the launch of a stretch of wide levels has more workgroups than the
- * device runs at once.
+ * device runs at once.  Bit 3 (for tests): a grid's lines are taken by two workgroups, a patch of them
+ * after the other.
  * All waiting is for rows of lower levels.  A shared launch needs as many free compute
  * units as it has workgroups, at most sixteen; a stretch of wide levels and a grid's lines are
  * solved by whatever part of their launch runs.  So the waits end; `poll_limit` bounds the polls of one wait all the same (0: the

@@ -167,6 +167,7 @@ std::atomic<bool> g_sig_enabled{[] {
     return e && e[0] == '1';
 }()};
 std::atomic<bool> g_flow_crowd{false};   // sptrsv_flow_kernel with kFlowCrowd workgroups
+std::atomic<bool> g_few_groups{false};   // a grid's lines with two workgroups
 
 struct Layout {
     nm::TPlan t;
@@ -2178,7 +2179,8 @@ int solve_typed(const nm_sptrsv_plan *p, int transposed, const void *data, int u
     if (by_lines(p)) {
         const T *dat = p->nnz > 0 ? (const T *)data : (const T *)b;
         return lines::solve<T>(p->grid, p->rows, transposed ? p->lower : !p->lower, P.lines, dat, unit, (const T *)b, (T *)x,
-                               a.w.ell_coef, a.w.rb, a.w.coef, a.w.status, g_sig_poll_limit.load(), s);
+                               a.w.ell_coef, a.w.rb, a.w.coef, a.w.status, g_sig_poll_limit.load(),
+                               g_few_groups.load() ? 2 : lines::kMaxGroups, s);
     }
     // the launches [flow_a, flow_b) that one sptrsv_flow_kernel takes
     int flow_a = 0, flow_b = 0;
@@ -3008,11 +3010,13 @@ extern "C" int nm_sptrsv_solve_static(const nm_sptrsv_plan *plan, nm_dtype dt, i
 //                a row more than one wavefront away, instead of meeting at a barrier after every
 //                level (default off); bit 1: launches that the plan would share among several
 //                workgroups are taken by one, wide levels by a launch each (default: shared); bit 2
-//                (tests): a stretch of wide levels is launched with more workgroups than can run at once.
+//                (tests): a stretch of wide levels is launched with more workgroups than can run at once;
+//                bit 3 (tests): a grid's lines are taken by two workgroups.
 extern "C" int nm_sptrsv_configure(int64_t poll_limit, int signalling) {
     g_sig_poll_limit.store(poll_limit == 0 ? int64_t(1) << 22 : poll_limit);
     g_sig_enabled.store((signalling & 1) != 0);
     g_team_enabled.store((signalling & 2) == 0);
     g_flow_crowd.store((signalling & 4) != 0);
+    g_few_groups.store((signalling & 8) != 0);
     return NM_OK;
 }

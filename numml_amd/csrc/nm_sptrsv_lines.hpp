@@ -577,12 +577,12 @@ template <typename T> __global__ __launch_bounds__(256) void failed_kernel(int32
     for (int32_t i = blockIdx.x * 256 + threadIdx.x; i < rows; i += gridDim.x * 256) x[i] = (T)__longlong_as_double(0x7ff8000000000000ll);
 }
 
-constexpr int kMaxWaves = 1024;
+constexpr int kMaxGroups = 1024;   // workgroups, which draw patches until there are none
 
 // Room in the per-call areas of doubles: `wide` takes four a row, `pairs` two, `edges` the edges.
 template <typename T>
 int solve(const Grid &g, int64_t rows, bool mirrored, const int32_t *src, const T *data, int unit, const T *b, T *x,
-          double *wide, double *pairs, double *edges, int32_t *status, int64_t poll_limit, hipStream_t s) {
+          double *wide, double *pairs, double *edges, int32_t *status, int64_t poll_limit, int most_groups, hipStream_t s) {
     Args<T> k;
     k.g = g;
     k.rows = (int32_t)rows;
@@ -602,14 +602,14 @@ int solve(const Grid &g, int64_t rows, bool mirrored, const int32_t *src, const 
     const int64_t entries = (int64_t)g.ah * g.bw * g.length;
     int64_t gx = nm::ceil_div(entries, (int64_t)256), gy = patches < 4096 ? patches : 4096;
     if (gx > 1024) gx = 1024;
-    const dim3 grid((unsigned)gx, (unsigned)gy), waves((unsigned)(patches < kMaxWaves ? patches : kMaxWaves));
+    const dim3 grid((unsigned)gx, (unsigned)gy), groups((unsigned)(patches < most_groups ? patches : most_groups));
     if (g.planes > 1) {
         hipLaunchKernelGGL((gather_kernel<T, true>), grid, dim3(256), 0, s, k);
-        if (g.along == 1) hipLaunchKernelGGL((solve_kernel<T, true, true>), waves, dim3(256), 0, s, k);
-        else hipLaunchKernelGGL((solve_kernel<T, true, false>), waves, dim3(256), 0, s, k);
+        if (g.along == 1) hipLaunchKernelGGL((solve_kernel<T, true, true>), groups, dim3(256), 0, s, k);
+        else hipLaunchKernelGGL((solve_kernel<T, true, false>), groups, dim3(256), 0, s, k);
     } else {
         hipLaunchKernelGGL((gather_kernel<T, false>), grid, dim3(256), 0, s, k);
-        hipLaunchKernelGGL((solve_kernel<T, false, true>), waves, dim3(256), 0, s, k);
+        hipLaunchKernelGGL((solve_kernel<T, false, true>), groups, dim3(256), 0, s, k);
     }
     NM_LAUNCH_CHECK("lines::solve_kernel");
     if (patches > 1) {

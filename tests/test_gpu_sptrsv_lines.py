@@ -181,6 +181,21 @@ def test_patterns_that_are_almost_a_grids(dev, what):
     _compare(dev, v[order], c[order], p, n, np.float64, True, False, by_lines=what == "diagonal")
 
 
+# what a workgroup does from its second patch on: a launch has a workgroup per patch up to 1024 of them, so without this only
+# grids of 257^3 and more come to it
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("dims, lower, unit", [((300, 301), True, False), ((301, 150), False, True), ((25, 31, 40), True, False),
+                                               ((33, 40, 18), False, False), ((20, 70, 21), True, True)])
+def test_two_workgroups_take_all_patches(dev, dims, lower, unit, dtype):
+    d, i, p, n = _triangle(dims, lower, 16)
+    try:
+        assert _lib.lib().nm_sptrsv_configure(0, 8) == 0
+        _compare(dev, d, i, p, n, dtype, lower, unit)
+        _compare(dev, d, i, p, n, dtype, lower, unit, np.where(np.arange(n) == n // 2, 1., 0.))
+    finally:
+        assert _lib.lib().nm_sptrsv_configure(0, 0) == 0
+
+
 def test_gives_up_instead_of_waiting_forever(dev):
     ext = numml_amd.load_compiled()
     for dims in ((300, 70), (20, 21, 22)):
