@@ -252,13 +252,24 @@ struct OwnColumn {
 
 // below[k] = position of the first entry of column k with a row index > k; no column is done.  Also what the choice of
 // the numeric kernel depends on: ctl[4] / ctl[5] = entries the widest column reaches above / below its
-// diagonal, ctl[6] = columns that do not name the column before them.
+// diagonal, ctl[6] = columns that do not name the column before them, ctl[9] = whether a value is -0.
+template <typename T>
 __global__ __launch_bounds__(kBlock) void lu_below_kernel(int64_t cols, const int64_t *__restrict__ indices,
-                                                          const int64_t *__restrict__ indptr,
+                                                          const int64_t *__restrict__ indptr, const T *__restrict__ values,
                                                           int64_t *__restrict__ below, int32_t *__restrict__ done, int32_t *ctl) {
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x, first = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t nnz = indptr[cols];
+    bool negative = false;
+    for (int64_t e = first; e < nnz; e += 8 * stride) {
+        T v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = values[e + u * stride < nnz ? e + u * stride : nnz - 1];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) negative = negative || (v[u] == T(0) && __builtin_signbit(v[u]));
+    }
+    if (__any(negative) && (threadIdx.x & 63) == 0) __hip_atomic_store(ctl + 9, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     int32_t up = 0, down = 0, breaks = 0;
-    for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < cols; k += stride) {
+    for (int64_t k = first; k < cols; k += stride) {
         const int64_t pb = indptr[k], pe = indptr[k + 1];
         int64_t lo = pb, hi = pe;
         while (lo < hi) {
@@ -506,12 +517,18 @@ __global__ __launch_bounds__(kLuFlowBlock) void lu_flow_kernel(int64_t cols, con
 // reach of 64 and more the update of the window takes over.  us for 4096 columns with everything around it (a kernel
 // that kept the window in registers and handed every column round by itself took the figure in brackets):
 //   reach      1            8            28           56           64           76           92
-//   fp64  1100 (1166)  1110 (1169)  1105 (1164)  1151 (2070)  1391 (2491)  2214 (2559)  2495 (2942)
-//   fp32  1064 (1162)  1064 (1160)  1055 (1178)  1091 (1780)  1205 (2187)  1481 (2231)  2013 (2375)
+//   fp64  1116 (1166)  1120 (1169)  1121 (1164)  1170 (2070)  1328 (2491)  2191 (2559)  2501 (2942)
+//   fp32  1052 (1162)  1055 (1160)  1052 (1178)  1090 (1780)  1182 (2187)  1490 (2231)  1918 (2375)
+// with a -0 among the inputs (SIGNED, below; ending the launch there and going on column by column took 3100 at a
+// reach of 1, 5600 at 64, 9300 at 92)
+//   fp64  1508         1508         1515         1663         1866         3589         4192
+//   fp32  1390         1382         1371         1401         1482         2198         2422
 // A 100 x 100 grid in fp32, which did not fit the registers, takes 4.9 ms instead of 25.
 // Entries that the pattern does not have are zeros when they are handed on, whatever a product has left in
 // their places, and a zero takes no part in a sum of finite numbers (no input is -0, a difference is
-// -0 only where one operand was).  A -0 among the inputs, an infinity or a NaN among the factors ends
+// -0 only where one operand was).  Where an input IS -0 (a masked or negated matrix with explicit zeros), it must keep its
+// sign until a product of two stored entries comes: there such entries are handed on as NaN, and a product that is NaN
+// counts as +0, which leaves every operand as it is (SIGNED).  An infinity or a NaN among the factors ends
 // the launch before they are written or used further: lu_flow_kernel goes on at that panel.
 #define NM_INLINE __attribute__((always_inline))   // (lambdas over register arrays)
 constexpr int kBandWaves = 16;
@@ -531,7 +548,6 @@ enum BandCount : int {
     kGoodPanel0, kGoodPanel1,    // panels found finite, by the wavefront that factors them
     kGoodRows0, kGoodRows1,
     kStop,                       // somebody found one that is not
-    kNegativeZero,
     kTrailing0 = 16,             // per wavefront: panels applied to the rest of the window
     kBandCounts = kTrailing0 + kBandTrailing
 };
@@ -590,9 +606,15 @@ __device__ __forceinline__ int32_t ring(int32_t at, int32_t size) { return at >=
 // Eight values that are the same for all lanes.
 template <typename T> struct alignas(16) Eight { T v[kPanel]; };
 
+template <bool SIGNED, typename T> __device__ __forceinline__ T absent() { return SIGNED ? (T)__builtin_nanf("") : T(0); }
+template <bool SIGNED, typename T> __device__ __forceinline__ T product(T l, T u) {
+    const T p = l * u;
+    return SIGNED && p != p ? T(0) : p;
+}
+
 // Wavefronts 0 and 1: panels K = v, v + 2, ...  RL registers of 64 rows hold the panel's rows, the first RA of them
 // the rows that the panel before reaches.
-template <typename T, int RL, int RA> __device__ __forceinline__ void band_panels(const Band<T> &B, int v) {
+template <bool SIGNED, typename T, int RL, int RA> __device__ __forceinline__ void band_panels(const Band<T> &B, int v) {
     const int lane = threadIdx.x & 63;
     const int32_t cbs = B.cb * kPanel;
     int32_t row_slot = lane / kPanel % B.rb, col_slot = 0;   // of panel 0
@@ -627,13 +649,13 @@ template <typename T, int RL, int RA> __device__ __forceinline__ void band_panel
             for (int q = 0; q < RA; ++q) {
                 const int32_t at = back * kPanel + lane + 64 * q;
                 const T x = F[min(at, B.fp - 1)];
-                l[q] = at < B.fp ? x : T(0);
+                l[q] = at < B.fp ? x : absent<SIGNED, T>();
             }
 #pragma unroll
             for (int c = 0; c < kPanel; ++c)
 #pragma unroll
                 for (int q = 0; q < RA; ++q) {
-                    const T p = l[q] * u.v[c];
+                    const T p = product<SIGNED>(l[q], u.v[c]);
                     W[c][q] = W[c][q] - p;
                 }
         };
@@ -670,23 +692,24 @@ template <typename T, int RL, int RA> __device__ __forceinline__ void band_panel
                 T x = divide && below ? quotient : W[t][q];
                 x = stored ? x : T(0);
                 finite = __builtin_fma(x, T(0), finite);
+                if (SIGNED) x = stored ? x : absent<SIGNED, T>();
                 F[t * B.fp + lane + 64 * q] = x;   // (nothing is stored in the rows past the panel's)
-                l[q] = below ? x : T(0);
+                l[q] = below ? x : absent<SIGNED, T>();
             }
             band_tell(B.count, kPivots, K * kPanel + t + 1);
 #pragma unroll
             for (int c = t + 1; c < kPanel; ++c) {
                 const bool stored = ((c < 4 ? row_lo : row_hi) >> 8 * (c & 3) & 1) != 0;
                 const T there = nm::read_lane(W[c][0], t);
-                const T u = stored ? there : T(0);
+                const T u = stored ? there : absent<SIGNED, T>();
 #pragma unroll
                 for (int q = 0; q < RL; ++q) {
-                    const T p = l[q] * u;
+                    const T p = product<SIGNED>(l[q], u);
                     W[c][q] = W[c][q] - p;
                 }
             }
         });
-        if (__any(finite != T(0)) || __builtin_amdgcn_readfirstlane(lds_get(B.count + kNegativeZero)) != 0) {
+        if (__any(finite != T(0))) {
             band_tell(B.count, kStop, 1);
             return;
         }
@@ -697,7 +720,7 @@ template <typename T, int RL, int RA> __device__ __forceinline__ void band_panel
 
 // Wavefronts 2 and 3: the panel's rows, columns 64 w .. right of it, a lane each.  They apply the panel before to these rows
 // themselves, so that they wait for the update of the one before that only.
-template <typename T> __device__ __forceinline__ void band_rows(const Band<T> &B, int w) {
+template <bool SIGNED, typename T> __device__ __forceinline__ void band_rows(const Band<T> &B, int w) {
     const int lane = threadIdx.x & 63, at = 64 * w + lane;
     const int32_t width = B.bub * kPanel, cbs = B.cb * kPanel;
     if (64 * w >= width) return;
@@ -721,13 +744,13 @@ template <typename T> __device__ __forceinline__ void band_rows(const Band<T> &B
             const bool reached = at + kPanel < width;
             T u[kPanel];
 #pragma unroll
-            for (int t = 0; t < kPanel; ++t) u[t] = reached ? U[t * B.uc + at + kPanel] : T(0);
+            for (int t = 0; t < kPanel; ++t) u[t] = reached ? U[t * B.uc + at + kPanel] : absent<SIGNED, T>();
 #pragma unroll
             for (int t = 0; t < kPanel; ++t) {
                 const Eight<T> l = *reinterpret_cast<const Eight<T> *>(F + t * B.fp + kPanel);
 #pragma unroll
                 for (int s = 0; s < kPanel; ++s) {
-                    const T p = l.v[s] * u[t];
+                    const T p = product<SIGNED>(l.v[s], u[t]);
                     X[s] = X[s] - p;
                 }
             }
@@ -740,6 +763,7 @@ template <typename T> __device__ __forceinline__ void band_rows(const Band<T> &B
             constexpr int t = decltype(pivot)::value;
             X[t] = stored >> t & 1u ? X[t] : T(0);
             finite = __builtin_fma(X[t], T(0), finite);
+            if (SIGNED) X[t] = stored >> t & 1u ? X[t] : absent<SIGNED, T>();
             if constexpr (t == 0)   // (panel K has taken the rows that these replace)
                 going = B.kept > 2 || band_wait<false>(B.count, band_need(kBandAny, kPivots, 1, K * kPanel + 1));
             if (mine) U[t * B.uc + at] = X[t];
@@ -749,7 +773,7 @@ template <typename T> __device__ __forceinline__ void band_rows(const Band<T> &B
                 const Eight<T> l = *reinterpret_cast<const Eight<T> *>(F + t * B.fp);
 #pragma unroll
                 for (int s = t + 1; s < kPanel; ++s) {
-                    const T p = l.v[s] * X[t];
+                    const T p = product<SIGNED>(l.v[s], X[t]);
                     X[s] = X[s] - p;
                 }
             }
@@ -767,7 +791,7 @@ template <typename T> __device__ __forceinline__ void band_rows(const Band<T> &B
 
 // Six wavefronts: the panel applied to the columns from the third block right of it on and the rows from the second
 // block below it on, a block of columns at a time.
-template <typename T, int RL> __device__ __forceinline__ void band_trailing(const Band<T> &B, int w) {
+template <bool SIGNED, typename T, int RL> __device__ __forceinline__ void band_trailing(const Band<T> &B, int w) {
     const int lane = threadIdx.x & 63;
     if (B.bub < 3 || B.blb < 2) return;
     // (a block of columns stays with the wavefront of its number modulo six, so nobody waits for another's update)
@@ -797,7 +821,7 @@ template <typename T, int RL> __device__ __forceinline__ void band_trailing(cons
                     const T l = F[t * B.fp + (mine[q] ? lane + 64 * q : 0)];
 #pragma unroll
                     for (int c = 0; c < kPanel; ++c) {
-                        const T p = l * u.v[c];
+                        const T p = product<SIGNED>(l, u.v[c]);
                         W[q][c] = W[q][c] - p;
                     }
                 }
@@ -815,8 +839,6 @@ template <typename T, int RL> __device__ __forceinline__ void band_trailing(cons
         col_slot = ring(col_slot + 1, B.cb);
     }
 }
-
-template <typename T> __device__ __forceinline__ bool negative_zero(T v) { return v == T(0) && __builtin_signbit(v); }
 
 // Wavefronts 14 and 15: the blocks of columns in turn, block n + bub coming into the window with panel n (the first ones with
 // panel 0), down to the window's last row then.  A block is requested before the one before it is placed.
@@ -863,7 +885,6 @@ template <typename T> __device__ __forceinline__ void band_load_columns(const Ba
             for (int32_t r = lane; r < B.rb * kPanel; r += 64) B.column(slot + c)[r] = T(0);
         if (lane < B.rb) *reinterpret_cast<uint64_t *>(B.has + lane * cbs + slot) = 0ull;
         asm volatile("" ::: "memory");
-        bool negative = false;
 #pragma unroll
         for (int c = 0; c < kPanel; ++c) {
             const int64_t begin = C.start(c);
@@ -879,7 +900,6 @@ template <typename T> __device__ __forceinline__ void band_load_columns(const Ba
                     const int32_t at = ring(row_slot + (C.row[c][q] / kPanel - n), B.rb), s = C.row[c][q] & 7;
                     B.column(slot + c)[at * kPanel + s] = C.value[c][q];
                     atomicOr(reinterpret_cast<uint32_t *>(B.has + at * cbs + slot) + c / 4, 1u << (8 * (c & 3) + s));
-                    negative = negative || negative_zero(C.value[c][q]);
                 }
             }
             if (lane == 0) {
@@ -889,7 +909,6 @@ template <typename T> __device__ __forceinline__ void band_load_columns(const Ba
                 B.out[slot + c] = 0;
             }
         }
-        if (__any(negative)) band_tell(B.count, kNegativeZero, 1);
         asm volatile("" ::: "memory");
         // (the next block is the other wavefront's)
         band_tell(B.count, kColumns0 + w, max(block + 2 - B.bub, 0));
@@ -911,7 +930,7 @@ template <typename T> __device__ __forceinline__ void band_load_columns(const Ba
     band_tell(B.count, kColumns0 + w, kBandNever);
 }
 
-// Wavefronts 6 and 7: the rows that come into the window with panel n.  A lane keeps to one place for a column, whose
+// Wavefronts 8 and 9: the rows that come into the window with panel n.  A lane keeps to one place for a column, whose
 // entries it takes in their order, requested before the rows' place is free.
 template <typename T> __device__ __forceinline__ void band_load_rows(const Band<T> &B, int w) {
     const int lane = threadIdx.x & 63, slot = 64 * w + lane;
@@ -948,19 +967,16 @@ template <typename T> __device__ __forceinline__ void band_load_rows(const Band<
             asm volatile("" ::: "memory");
             uint32_t has = 0;
             int32_t taken = 0;
-            bool negative = false;
 #pragma unroll
             for (int s = 0; s < kPanel; ++s)
                 if (s < left && row[s] < limit) {
                     column[row[s] & 7] = value[s];
                     has |= 1u << (row[s] & 7);
                     ++taken;
-                    negative = negative || negative_zero(value[s]);
                 }
             B.has[row_slot * cbs + slot] = (uint8_t)has;
             left -= taken;
             from += taken;
-            if (negative) lds_put(B.count + kNegativeZero, 1);
         }
         asm volatile("" ::: "memory");
         band_tell(B.count, kIn0 + w, n + 1);
@@ -1021,11 +1037,9 @@ template <typename T> __device__ __forceinline__ void band_write(const Band<T> &
     }
 }
 
-template <typename T>
-__global__ __launch_bounds__(kBandWaves * 64) void lu_band_kernel(int32_t n, const int64_t *__restrict__ indices,
-                                                                  const int64_t *__restrict__ indptr, T *values,
-                                                                  int32_t *ctl, int32_t *done) {
-    __shared__ __align__(16) unsigned char s_band[kBandLds];
+template <bool SIGNED, typename T>
+__device__ __forceinline__ void lu_band(int32_t n, const int64_t *__restrict__ indices, const int64_t *__restrict__ indptr, T *values, int32_t *ctl,
+                                        int32_t *done, unsigned char *s_band) {
     const int bu = ctl[4], bl = ctl[5];
     if (ctl[6] > kBandMaxBreaks || n >= 1 << 30 || indptr[n] == 0) return;   // lu_flow_kernel's
     Band<T> B;
@@ -1076,11 +1090,11 @@ __global__ __launch_bounds__(kBandWaves * 64) void lu_band_kernel(int32_t n, con
     __syncthreads();
     // (a SIMD takes every fourth wavefront: the panels' have the least company)
     if (v < 2) {
-        if (B.fr <= 64) band_panels<T, 1, 1>(B, v);
-        else if (B.fr <= 72) band_panels<T, 2, 1>(B, v);
-        else band_panels<T, 2, 2>(B, v);
+        if (B.fr <= 64) band_panels<SIGNED, T, 1, 1>(B, v);
+        else if (B.fr <= 72) band_panels<SIGNED, T, 2, 1>(B, v);
+        else band_panels<SIGNED, T, 2, 2>(B, v);
     } else if (v < 4) {
-        band_rows<T>(B, v - 2);
+        band_rows<SIGNED, T>(B, v - 2);
     } else if (v == 4) {
         __builtin_amdgcn_s_setprio(1);
         band_write<T>(B);
@@ -1092,8 +1106,8 @@ __global__ __launch_bounds__(kBandWaves * 64) void lu_band_kernel(int32_t n, con
         band_load_columns<T>(B, v - 14);
     } else if (v != 12) {
         const int w = v == 6 ? 0 : v == 7 ? 1 : v == 10 ? 2 : v == 11 ? 3 : v == 5 ? 4 : 5;
-        if (B.blb <= 9) band_trailing<T, 1>(B, w);
-        else band_trailing<T, 2>(B, w);
+        if (B.blb <= 9) band_trailing<SIGNED, T, 1>(B, w);
+        else band_trailing<SIGNED, T, 2>(B, w);
     }
     __syncthreads();
     // lu_flow_kernel finds no column left to draw, or goes on behind the last panel that is written (ctl[7]).
@@ -1107,6 +1121,15 @@ __global__ __launch_bounds__(kBandWaves * 64) void lu_band_kernel(int32_t n, con
         ctl[7] = written < n ? written : 0;
         ctl[8] = written < n ? written : n;
     }
+}
+
+template <typename T>
+__global__ __launch_bounds__(kBandWaves * 64) void lu_band_kernel(int32_t n, const int64_t *__restrict__ indices,
+                                                                  const int64_t *__restrict__ indptr, T *values,
+                                                                  int32_t *ctl, int32_t *done) {
+    __shared__ __align__(16) unsigned char s_band[kBandLds];
+    if (ctl[9] == 0) lu_band<false>(n, indices, indptr, values, ctl, done, s_band);
+    else lu_band<true>(n, indices, indptr, values, ctl, done, s_band);
 }
 
 int check_rows(int64_t rows) {
@@ -1216,9 +1239,15 @@ extern "C" int nm_splu_numeric(nm_dtype dt, int64_t cols, void *Mt_data, const i
     hipStream_t s = nm::as_stream(stream);
     if (int rc = nm::fill_async(F.ctl, 16, (int32_t)0, s)) return rc;
     {
-        int64_t g = nm::ceil_div(cols, kBlock);
-        hipLaunchKernelGGL(lu_below_kernel, dim3((unsigned)(g > 65536 ? 65536 : g)), dim3(kBlock), 0, s, cols,
-                           Mt_indices, Mt_indptr, F.below, F.done, F.ctl);
+        // (a workgroup for 32 columns, since it looks at their values as well)
+        const int64_t g = nm::ceil_div(cols, 32);
+        const dim3 grid((unsigned)(g > 65536 ? 65536 : g));
+        if (dt == NM_F32)
+            hipLaunchKernelGGL(lu_below_kernel<float>, grid, dim3(kBlock), 0, s, cols, Mt_indices, Mt_indptr,
+                               (const float *)Mt_data, F.below, F.done, F.ctl);
+        else
+            hipLaunchKernelGGL(lu_below_kernel<double>, grid, dim3(kBlock), 0, s, cols, Mt_indices, Mt_indptr,
+                               (const double *)Mt_data, F.below, F.done, F.ctl);
         NM_LAUNCH_CHECK("lu_below_kernel");
     }
     // Whether the factors are a band is known on the device only: the band kernel leaves at once
