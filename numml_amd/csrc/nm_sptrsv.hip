@@ -59,10 +59,10 @@ struct Packed {        // one solve direction, level-major (all int32, device)
     int32_t *dslot;    // [nnz]    slot of the row a dependency refers to
     int32_t *dsrc;     // [nnz]    position of its coefficient in A's data
     int32_t *diag;     // [rows]   position of the diagonal coefficient, -1 when not stored
-    int32_t *ell_ds;   // [ell_capacity] room for the fixed-width dependency entries: 16 bits each, `pre` per row
+    int32_t *ell_ds;   // [ell_capacity] room for the fixed-width dependency entries: 16 bits each, `pre` per row; at its end `lines`
     int32_t *lvl_sig;  // [levels] which neighbouring wavefronts the rows of a level wait for (kSigLower | kSigHigher)
     int32_t *team;     // [team_capacity] exchange tables of the launches that several workgroups share
-    int32_t *lines;    // [rows][4] where a grid's lines find their values (lines::plan_kernel)
+    int32_t *lines = nullptr;   // [rows][4] where a grid's lines find their values (lines::plan_kernel)
 };
 // Entries of the fixed-width (ELLPACK) arrays; the layout is used when (rows + kEllPad) * pre
 // fits.  kEllPad slots of padding follow the last row in every array the fixed-width kernel
@@ -70,6 +70,14 @@ struct Packed {        // one solve direction, level-major (all int32, device)
 // the level's width, so the slots behind a level's end must be readable.
 constexpr int64_t kEllPad = 1024;   // == kNarrow, the widest single-workgroup launch
 inline int64_t ell_capacity(int64_t rows, int64_t nnz) { return 2 * nnz + 2 * rows + 8 + 8 * kEllPad; }
+// Width of the fixed-width layout for rows of up to `most` dependencies (0: none).
+inline int ell_width(int32_t most) { return most <= 2 ? 2 : (most <= 4 ? 4 : (most <= 8 ? 8 : 0)); }
+// The 16-bit entries leave half of the area and more: where a grid's lines have their table, so that plans of other
+// patterns do not pay for it; null where it does not fit (no grid has so few entries).
+inline int32_t *lines_table(int32_t *ell_ds, int64_t rows, int64_t nnz, int pre) {
+    const int64_t at = (ell_capacity(rows, nnz) - 4 * rows) & ~int64_t(3);   // (read 16 bytes at a time)
+    return at * 4 >= (rows + kEllPad) * pre * 2 ? ell_ds + at : nullptr;
+}
 // Doubles of the per-call coefficient area: the fixed-width layout, or the coefficient rows of
 // the chain kernels (64 per chain row, whatever the band's width: room for chains of up to
 // 65536 rows in all; longer ones take what fits).
@@ -197,7 +205,6 @@ size_t plan_layout(int64_t rows, int64_t nnz, void *base, Layout *L) {
         l.dir[d].ell_ds = take(ell_capacity(rows, nnz));
         l.dir[d].lvl_sig = take(rows + 1);
         l.dir[d].team = take(team_capacity(rows));
-        l.dir[d].lines = take(4 * rows);
     }
     if (L) *L = l;
     return off;
@@ -2488,6 +2495,10 @@ extern "C" int nm_sptrsv_analyse(int64_t rows, int64_t nnz, const int64_t *indic
         !lines::make_grid(rows, meta_h[6], meta_h[7] > meta_h[6] ? meta_h[7] : 0, &grid) || grid.edges() > nnz)
         grid = lines::Grid();
     for (int d = 0; d < 2 && grid.length > 0; ++d) {
+        p->dir[d].lines = lines_table(p->dir[d].ell_ds, rows, nnz, ell_width(p->max_deps[d]));
+        if (!p->dir[d].lines) grid = lines::Grid();
+    }
+    for (int d = 0; d < 2 && grid.length > 0; ++d) {
         hipLaunchKernelGGL(lines::plan_kernel, dim3((unsigned)(rgrid > 4096 ? 4096 : rgrid)), dim3(kBlock), 0, s, grid,
                            (int32_t)rows, d == 0 ? !p->lower : p->lower, p->order, p->dir[d].dptr, p->dir[d].dslot,
                            p->dir[d].dsrc, p->dir[d].diag, reinterpret_cast<int4 *>(p->dir[d].lines), L.meta + 8);
@@ -2710,7 +2721,7 @@ extern "C" int nm_sptrsv_analyse(int64_t rows, int64_t nnz, const int64_t *indic
     }
     for (int d = 0; d < 2; ++d) {
         const int32_t md = p->max_deps[d];
-        const int pre = chains[d] ? 0 : (md <= 2 ? 2 : (md <= 4 ? 4 : (md <= 8 ? 8 : 0)));
+        const int pre = chains[d] ? 0 : ell_width(md);
         if (pre > 0 && rows < (1 << 30) && (rows + kEllPad) * pre <= ell_capacity(rows, nnz)) {
             p->ell_pre[d] = pre;
             int64_t grid = nm::ceil_div(rows * pre, kBlock);

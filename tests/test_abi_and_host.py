@@ -66,6 +66,21 @@ def test_argument_checks_report_through_nm_last_error():
                                   ctypes.byref(usable), None) == 0 and usable.value == 0    # rows on the hash path
 
 
+def test_a_triangular_plan_keeps_what_its_pattern_needs():
+    # Per row two directions of pointers, diagonals, marks and half the fixed-width layout, and the level order: 17 integers;
+    # per entry positions, dependencies and the layout's other half.  The table of a grid's lines (8 integers a row) lies in
+    # the layout's spare half: other patterns' plans, which count against the plan cache, must not grow by it.
+    def size(rows, nnz):
+        plan, work = ctypes.c_size_t(0), ctypes.c_size_t(0)
+        assert L.nm_sptrsv_plan_bytes(rows, nnz, ctypes.byref(plan), ctypes.byref(work)) == 0
+        return plan.value
+
+    L = _lib.lib()
+    rows, nnz = 10 ** 6, 3 * 10 ** 6
+    assert size(2 * rows, nnz) - size(rows, nnz) < 69 * rows
+    assert size(rows, 2 * nnz) - size(rows, nnz) < 51 * nnz
+
+
 def test_mirror_has_the_reference_signatures():
     # cpp/sparse_csr.hpp:32-105
     want = {
