@@ -233,13 +233,17 @@ def _banded(n, below, above, dtype, seed, holes=0.0):
     return a[r, c].astype(dtype), c.astype(np.int64), p
 
 
-# reaches at the edges of the band kernel's register sets (32, 64, 112, 96 below and 28, 60, 76, 92 above the
-# diagonal), sizes that are no multiples of a round of sixteen columns, one of them below sixteen
+# reaches at the edges of the band kernel's blocks of eight and of its wavefronts' 64 rows and columns; of what it takes (15
+# blocks below the diagonal and 13 right of it, and one more; in fp64 as much as fits 160 KB); sizes that are no
+# multiples of a panel of eight columns, one of them below eight
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("n, below, above", [(5, 1, 1), (16, 3, 1), (33, 1, 14), (130, 28, 28), (131, 29, 29), (150, 32, 28),
                                              (150, 33, 28), (190, 60, 60), (190, 61, 61), (210, 64, 60), (210, 65, 60),
                                              (230, 76, 76), (231, 77, 77), (290, 112, 76), (290, 113, 76),
-                                             (260, 92, 92), (261, 96, 92), (261, 97, 92), (262, 93, 93), (100, 5, 28), (300, 2, 92)])
+                                             (260, 92, 92), (261, 96, 92), (261, 97, 92), (262, 93, 93), (100, 5, 28), (300, 2, 92),
+                                             (300, 120, 104), (300, 121, 104), (300, 120, 105), (299, 104, 104), (260, 88, 88), (261, 97, 96),
+                                             (301, 120, 1), (301, 1, 104), (270, 96, 88), (300, 96, 104), (300, 120, 88),
+                                             (300, 120, 96), (290, 64, 80), (290, 64, 88)])
 def test_banded_factors_match_the_oracle_bit_for_bit(dev, dtype, n, below, above):
     ext = numml_amd.load_compiled()
     for holes in (0.0, 0.6):

@@ -61,7 +61,7 @@ DIMS = [(2, 3), (3, 2), (64, 2), (65, 2), (63, 7), (64, 8), (65, 9), (128, 15), 
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
-@pytest.mark.parametrize("lower, unit", [(True, False), (False, False), (True, True)])
+@pytest.mark.parametrize("lower, unit", [(True, False), (False, False), (True, True), (False, True)])
 @pytest.mark.parametrize("dims", DIMS)
 def test_grids(dev, dims, lower, unit, dtype):
     print("case", dims, lower, unit, dtype.__name__, flush=True)
@@ -76,9 +76,11 @@ def test_the_other_half_is_passed_over(dev, dims, lower):
     _compare(dev, d, i, p, n, np.float64, lower, False)
 
 
-@pytest.mark.parametrize("dims", [(70, 33), (10, 11, 12)])
-def test_values_that_the_short_division_does_not_take(dev, dims):
-    d, i, p, n = _triangle(dims, True, 4)
+# (lines along each of the directions)
+@pytest.mark.parametrize("lower", [True, False])
+@pytest.mark.parametrize("dims", [(70, 33), (33, 70), (10, 11, 12), (10, 70, 9), (70, 9, 10)])
+def test_values_that_the_short_division_does_not_take(dev, dims, lower):
+    d, i, p, n = _triangle(dims, lower, 4)
     row = np.repeat(np.arange(n), np.diff(p))
     diag = np.flatnonzero(row == i)
     rng = np.random.default_rng(4)
@@ -90,12 +92,42 @@ def test_values_that_the_short_division_does_not_take(dev, dims):
             b[rng.random(n) < 0.2] = -0.
         for v in special:
             b[rng.choice(n, 3, False)] = v
-        _compare(dev, d, i, p, n, np.float64, True, False, b)
+        _compare(dev, d, i, p, n, np.float64, lower, False, b)
     d[diag[n // 2]] = 0.
-    _compare(dev, d, i, p, n, np.float64, True, False)
+    _compare(dev, d, i, p, n, np.float64, lower, False)
     b = randn(8, n, np.float64)
     b.view(np.uint64)[[0, n // 3, n - 1]] = 0xffffffffffffffff   # the bits that mark a row as not solved
-    _compare(dev, d, i, p, n, np.float64, True, False, b)
+    _compare(dev, d, i, p, n, np.float64, lower, False, b)
+
+
+@pytest.mark.parametrize("dims", [(70, 33), (10, 11, 12)])
+@pytest.mark.parametrize("lower", [True, False])
+def test_fp32_values_out_of_the_ordinary(dev, dims, lower):
+    d, i, p, n = _triangle(dims, lower, 17)
+    rng = np.random.default_rng(17)
+    row = np.repeat(np.arange(n), np.diff(p))
+    diag = np.flatnonzero(row == i)
+    d[diag[rng.choice(n, 40, False)]] *= 10.0 ** rng.integers(-35, 35, 40)
+    for special in ((), (np.inf,), (np.nan, -np.inf), (-0., 1e-44)):
+        b = randn(18, n, np.float64) * 10.0 ** rng.integers(-30, 30, n)
+        b[rng.random(n) < 0.3] = 0.
+        for v in special:
+            b[rng.choice(n, 3, False)] = v
+        with np.errstate(all="ignore"):
+            _compare(dev, d, i, p, n, np.float32, lower, False, b)
+    d[diag[n // 2]] = 0.
+    _compare(dev, d, i, p, n, np.float32, lower, False)
+
+
+@pytest.mark.parametrize("dims", [(2, 40), (70, 33), (2, 2, 30), (10, 11, 12)])
+@pytest.mark.parametrize("lower", [True, False])
+def test_no_diagonal_stored(dev, dims, lower):
+    d, i, p, n = _triangle(dims, lower, 19)
+    row = np.repeat(np.arange(n), np.diff(p))
+    keep = row != i
+    p = np.concatenate(([0], np.cumsum(np.bincount(row[keep], minlength=n)))).astype(np.int64)
+    for dtype in (np.float32, np.float64):
+        _compare(dev, d[keep], i[keep], p, n, dtype, lower, True)
 
 
 # lines along each direction, one patch and several, lines longer than sixteen blocks of eight steps

@@ -64,19 +64,26 @@ def test_a_pattern_edited_in_place(dev, ext):
     for _ in range(5):
         (A + A.T).data
     T = A.T
-    # the transpose's own tensors, edited: their key is not the plan's any more
-    k = int(np.flatnonzero(np.diff(p) > 0)[0])
-    T.indices.copy_(r - 1 - T.indices.flip(0))
+    # the transpose's own tensors, edited: their key is not the plan's any more.  Every row's columns are mirrored in turn,
+    # so they stay sorted and distinct.
     td, ti, tp = host(T.data), host(T.indices), host(T.indptr)
-    order = np.concatenate([tp[q] + np.argsort(ti[tp[q]:tp[q + 1]], kind="stable") for q in range(r)])
-    T.indices.copy_(to_dev(dev, ti[order])[0])
-    ti = ti[order]
+    mirrored = np.concatenate([r - 1 - ti[tp[q]:tp[q + 1]][::-1] for q in range(r)])
+    assert (mirrored != ti).any()
+    T.indices.copy_(to_dev(dev, mirrored)[0])
     S = A + T
-    if all(np.unique(ti[tp[q]:tp[q + 1]]).size == tp[q + 1] - tp[q] for q in range(r)):
-        Cd, Ci, Cp = oracle.splincomb_forward(r, r, 1., d, i, p, 1., td, ti, tp)
-        assert_same(host(S.indices), Ci)
-        assert_same(host(S.data), Cd)
+    Cd, Ci, Cp = oracle.splincomb_forward(r, r, 1., d, i, p, 1., td, mirrored, tp)
+    for a, b in zip((S.data, S.indices, S.indptr), (Cd, Ci, Cp)):
+        assert_same(host(a), b)
+    # a product with it as well, and with the transpose as it was
+    Cd, Ci, Cp = oracle.spgemm_forward(r, r, td, mirrored, tp, r, r, d, i, p)
+    S = T @ A
+    assert_same(host(S.indices), Ci)
+    assert_same(host(S.data), Cd)
+    T.indices.copy_(to_dev(dev, ti)[0])
+    for a, b in zip((A + T).data, oracle.splincomb_forward(r, r, 1., d, i, p, 1., td, ti, tp)[0]):
+        assert a == b
     # the matrix's, edited: another pattern altogether
+    k = int(np.flatnonzero(np.diff(p) > 0)[0])
     row = np.repeat(np.arange(r), np.diff(p))
     i2 = i.copy()
     last = p[k + 1] - 1
