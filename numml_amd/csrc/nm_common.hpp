@@ -154,6 +154,19 @@ __device__ __forceinline__ double read_lane(double v, int l) {
 }
 __device__ __forceinline__ int read_lane(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
 
+// LDS accesses in program order: a wavefront's are carried out in that order, so who sees a count sees what it counts.
+template <typename V> __device__ __forceinline__ V lds_get(V *p) {
+    asm volatile("" ::: "memory");
+    const V v = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    asm volatile("" ::: "memory");
+    return v;
+}
+template <typename V> __device__ __forceinline__ void lds_put(V *p, V v) {
+    asm volatile("" ::: "memory");
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    asm volatile("" ::: "memory");
+}
+
 // Sum over the 64 lanes of a wavefront with DPP adds (no LDS traffic); every
 // lane gets the total.  Steps: swap within pairs, within quads, rotate the
 // 16-lane row by 4 and 8 (row totals everywhere), then carry lane 15 into rows

@@ -571,23 +571,11 @@ template <typename T> struct Band {
     __device__ __forceinline__ T *multipliers(int32_t K) const { return F + (K & (kept - 1)) * (kPanel * fp); }
     __device__ __forceinline__ T *rows(int32_t K) const { return U + (K & (kept - 1)) * (kPanel * uc); }
 };
-// LDS accesses that stay in program order: a wavefront's are carried out in that order.
-template <typename V> __device__ __forceinline__ V lds_get(V *p) {
-    asm volatile("" ::: "memory");
-    const V v = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    asm volatile("" ::: "memory");
-    return v;
-}
-template <typename V> __device__ __forceinline__ void lds_put(V *p, V v) {
-    asm volatile("" ::: "memory");
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    asm volatile("" ::: "memory");
-}
 // Waits until the count of every lane's number is at least the lane's `least`; false: the launch ends.
 template <bool SLEEP> __device__ __forceinline__ bool band_wait(int32_t *count, int32_t least) {
     const int lane = threadIdx.x & 63;
     while (true) {
-        const int32_t now = lds_get(count + min(lane, (int)kBandCounts - 1));
+        const int32_t now = nm::lds_get(count + min(lane, (int)kBandCounts - 1));
         if (!__any(now < least)) return true;
         if (__any(lane == kStop && now != 0)) return false;
         if (SLEEP) __builtin_amdgcn_s_sleep(1);
@@ -600,7 +588,7 @@ __device__ __forceinline__ int32_t band_need(int32_t least, int first, int numbe
 }
 constexpr int32_t kBandAny = -0x7fffffff;
 // (all lanes write the one word: less to issue than choosing one of them)
-__device__ __forceinline__ void band_tell(int32_t *count, int which, int32_t v) { lds_put(count + which, v); }
+__device__ __forceinline__ void band_tell(int32_t *count, int which, int32_t v) { nm::lds_put(count + which, v); }
 __device__ __forceinline__ int32_t ring(int32_t at, int32_t size) { return at >= size ? at - size : at; }
 
 // Eight values that are the same for all lanes.

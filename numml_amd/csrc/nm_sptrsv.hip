@@ -41,6 +41,7 @@
 //   nnz*(s+8) + (rows+1)*8 + 2*rows*s
 #include "nm_common.hpp"
 #include "nm_scan.hpp"
+#include "nm_sptrsv_lines.hpp"
 #include "nm_transpose.hpp"
 
 #include <algorithm>
@@ -52,8 +53,6 @@
 #include <vector>
 
 namespace {
-#include "nm_sptrsv_lines.hpp"
-
 struct Packed {        // one solve direction, level-major (all int32, device)
     int32_t *dptr;     // [rows+1] dependency range of slot q
     int32_t *dslot;    // [nnz]    slot of the row a dependency refers to

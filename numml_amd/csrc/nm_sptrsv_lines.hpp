@@ -39,6 +39,12 @@
 // 282 us, 68 ns a level where a workgroup with a barrier a level takes 270; fp64, ms before and now: 1024 x 1024
 // 0.70 and 0.21, 60 x 60 0.036 and 0.018, 97 x 89 x 101 0.325 and 0.12, 16 x 16 x 16 0.031 and 0.021, 300^3
 // 2.17 and 1.68.
+#pragma once
+#include "nm_common.hpp"
+
+#include <type_traits>
+
+namespace {
 namespace lines {
 
 constexpr int kAhead = 16;         // steps that operands are requested ahead
@@ -233,18 +239,6 @@ struct Shared {
     double x[kKept][kPatch + 64 + 1];
     double from_n[kKept][kPatch];   // by step and plane: what the planes' first lines need
 };
-// LDS accesses in program order: a wavefront's are carried out in that order, so who sees a count sees what it counts.
-template <typename V> __device__ __forceinline__ V lds_get(V *p) {
-    asm volatile("" ::: "memory");
-    const V v = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    asm volatile("" ::: "memory");
-    return v;
-}
-template <typename V> __device__ __forceinline__ void lds_put(V *p, V v) {
-    asm volatile("" ::: "memory");
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    asm volatile("" ::: "memory");
-}
 __device__ __forceinline__ unsigned long long look(const unsigned long long *at) {
     return __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -366,10 +360,10 @@ template <typename T, bool THREE, bool LINE_LAST> __device__ __forceinline__ voi
         const bool again = refused();
         if (THREE || __builtin_expect(__any(again || missing(t + kSteps)) || bad >= 0, 0)) {
             if (bad < 0 && __any(again)) bad = t;
-            if (bad < 0) lds_put(&sh.now.done, t + kSteps);
+            if (bad < 0) nm::lds_put(&sh.now.done, t + kSteps);
             await(t + kSteps, next_n);
         } else {
-            lds_put(&sh.now.done, t + kSteps);
+            nm::lds_put(&sh.now.done, t + kSteps);
         }
     };
     int32_t t = 0;
@@ -405,7 +399,7 @@ template <typename T, bool THREE, bool LINE_LAST> __device__ __forceinline__ voi
                 request(v[s]);
             });
             left = __any(refused()) ? kFullBlocks : left - 1;
-            lds_put(&sh.now.done, t + kSteps);
+            nm::lds_put(&sh.now.done, t + kSteps);
             ask(t + kSteps, n);
             await(t + kSteps, n);
         }
@@ -436,7 +430,7 @@ template <typename T, bool THREE, bool LINE_LAST> __device__ __forceinline__ voi
         if (t >= steps) break;
     }
     // (nobody waits for more steps than there are, whatever multiple they count in)
-    if (lane == 0) lds_put(&sh.now.done, kAll);
+    if (lane == 0) nm::lds_put(&sh.now.done, kAll);
 }
 
 // Wavefront 1: the rows of other patches that this one needs, from the edges into LDS.  False: it gave up.
@@ -454,18 +448,18 @@ template <typename T, bool THREE> __device__ __forceinline__ bool import_edges(c
     int64_t waited = 0;
     for (int32_t t = 0; t < steps;) {
         if (k.poll_limit < 0 || waited > k.poll_limit) return false;
-        const int32_t room = __builtin_amdgcn_readfirstlane(lds_get(&sh.now.done)) + kKept - 2;
+        const int32_t room = __builtin_amdgcn_readfirstlane(nm::lds_get(&sh.now.done)) + kKept - 2;
         const int32_t at = t + ahead, cn = at - skew(e, 0), cg = at - skew(0, e);
         const unsigned long long n = in_n && cn >= 0 && cn < length && e < P.na ? look(edge_n + (int64_t)cn * P.na + e) : 0ull;
         const unsigned long long g = in_g && cg >= 0 && cg < length && e < P.nb ? look(edge_g + (int64_t)cg * P.nb + e) : 0ull;
         const unsigned long long open = __ballot(n == kUnsolved || g == kUnsolved || at >= room);
         const int got = (open ? __builtin_ctzll(open) : 64) / (THREE ? kPatch : 1);
         if (ahead < got) {
-            lds_put(&sh.from_n[at & (kKept - 1)][e], __longlong_as_double((long long)n));
-            if (THREE) lds_put(&sh.x[(at - 2) & (kKept - 1)][e], __longlong_as_double((long long)g));
+            nm::lds_put(&sh.from_n[at & (kKept - 1)][e], __longlong_as_double((long long)n));
+            if (THREE) nm::lds_put(&sh.x[(at - 2) & (kKept - 1)][e], __longlong_as_double((long long)g));
         }
         t += got;
-        if (got > 0 && lane == 0) lds_put(&sh.now.imported, t);
+        if (got > 0 && lane == 0) nm::lds_put(&sh.now.imported, t);
         waited = got > 0 || t + 1 >= room ? 0 : waited + 1;
     }
     return true;
@@ -473,7 +467,7 @@ template <typename T, bool THREE> __device__ __forceinline__ bool import_edges(c
 
 // Waits until `upto` steps are solved.
 __device__ __forceinline__ void await_steps(Shared &sh, int32_t upto) {
-    while (__builtin_amdgcn_readfirstlane(lds_get(&sh.now.done)) < upto) __builtin_amdgcn_s_sleep(1);
+    while (__builtin_amdgcn_readfirstlane(nm::lds_get(&sh.now.done)) < upto) __builtin_amdgcn_s_sleep(1);
 }
 
 // Wavefront 2: the patch's last lines into the edges.
@@ -492,10 +486,10 @@ template <typename T, bool THREE> __device__ __forceinline__ void export_edges(c
         const int32_t at = t + s, cn = at - skew(e, P.nb - 1), cg = at - skew(P.na - 1, e);
         const double *row = sh.x[at & (kKept - 1)] + kPatch;
         if (to_n && s < kSteps && e < P.na && cn >= 0 && cn < length)
-            leave(edge_n + (int64_t)cn * P.na + e, lds_get(row + (THREE ? e * kPatch : 0) + P.nb - 1));
+            leave(edge_n + (int64_t)cn * P.na + e, nm::lds_get(row + (THREE ? e * kPatch : 0) + P.nb - 1));
         if (THREE && to_g && s < kSteps && e < P.nb && cg >= 0 && cg < length)
-            leave(edge_g + (int64_t)cg * P.nb + e, lds_get(row + (P.na - 1) * kPatch + e));
-        if (lane == 0) lds_put(&sh.now.exported, t + kSteps);
+            leave(edge_g + (int64_t)cg * P.nb + e, nm::lds_get(row + (P.na - 1) * kPatch + e));
+        if (lane == 0) nm::lds_put(&sh.now.exported, t + kSteps);
     }
 }
 
@@ -519,7 +513,7 @@ template <typename T, bool THREE> __device__ __forceinline__ void write_rows(con
                 v[g] = sh.x[(t & (kKept - 1)) + s][kPatch + l];
             });
             asm volatile("" ::: "memory");
-            if (lane == 0) lds_put(&sh.now.written, t + kRows);
+            if (lane == 0) nm::lds_put(&sh.now.written, t + kRows);
             nm::static_for<kRows>([&](auto at) __attribute__((always_inline)) {
                 constexpr int g = decltype(at)::value;
                 constexpr int first = kApart ? g / 2 * 8 : g * 4, a = THREE ? first / kPatch : 0, b0 = THREE ? first % kPatch : first;
@@ -560,7 +554,7 @@ template <typename T, bool THREE, bool LINE_LAST> __global__ __launch_bounds__(2
             const bool ok = import_edges<T, THREE>(k, P, sh);
             if (!ok && (threadIdx.x & 63) == 0)
                 __hip_atomic_store(k.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if ((threadIdx.x & 63) == 0) lds_put(&sh.now.imported, kAll);
+            if ((threadIdx.x & 63) == 0) nm::lds_put(&sh.now.imported, kAll);
         } else if (wave == 2) {
             export_edges<T, THREE>(k, P, sh);
         } else {
@@ -620,3 +614,4 @@ int solve(const Grid &g, int64_t rows, bool mirrored, const int32_t *src, const 
 }
 
 }  // namespace lines
+}  // namespace
