@@ -1227,8 +1227,8 @@ extern "C" int nm_splu_numeric(nm_dtype dt, int64_t cols, void *Mt_data, const i
     hipStream_t s = nm::as_stream(stream);
     if (int rc = nm::fill_async(F.ctl, 16, (int32_t)0, s)) return rc;
     {
-        // (a workgroup for 32 columns, since it looks at their values as well)
-        const int64_t g = nm::ceil_div(cols, 32);
+        // (a workgroup for 8 columns, since it looks at their values as well)
+        const int64_t g = nm::ceil_div(cols, 8);
         const dim3 grid((unsigned)(g > 65536 ? 65536 : g));
         if (dt == NM_F32)
             hipLaunchKernelGGL(lu_below_kernel<float>, grid, dim3(kBlock), 0, s, cols, Mt_indices, Mt_indptr,
