@@ -1,5 +1,9 @@
 // CSR x dense (SpMM) forward and backward for gfx950.
 //
+// Dense operands of up to 1 KB a row take the kernels of nm_spmm_groups.hpp (a group of lanes an
+// entry, several entries a request); the kernels below are for wider ones, for index and stride
+// ranges beyond 32 bits, and for both gradients without a plan.
+//
 // Forward: lane = output column (a 64-column fp32 row of B is one 256-byte
 // line, so every gather is a single coalesced request).  A wavefront owns a few
 // consecutive rows of A and walks their entries as one range, 64 (column,
@@ -20,6 +24,7 @@
 //   forward : nnz*(s+8) + (rows+1)*8 + cols*n*s + rows*n*s
 //   backward: nnz*(s+8) + (rows+1)*8 + rows*n*s + cols*n*s + nnz*s + cols*n*s
 #include "nm_common.hpp"
+#include "nm_spmm_groups.hpp"
 #include "nm_transpose.hpp"
 
 namespace {
@@ -289,8 +294,7 @@ template <typename T> __device__ __forceinline__ T fold8(const T (&p)[kBatch], i
 // wavefront owns 64 consecutive stored entries whatever rows they belong to
 // (every entry costs the same), finds its first row by bisection and walks on;
 // gathers go out eight at a time and the dot products are reduced with DPP adds.
-// FAST: grad_A only and n <= 64 (one column tile), which allows the pipelined loop below.
-template <typename T, bool FAST>
+template <typename T>
 __global__ __launch_bounds__(kBlock) void spdmm_bwd_kernel(
     int64_t rows, int64_t nnz, const T *__restrict__ data, const int64_t *__restrict__ indices,
     const int64_t *__restrict__ indptr, const T *__restrict__ B, int64_t ldb,
@@ -393,69 +397,37 @@ __global__ __launch_bounds__(kBlock) void spdmm_bwd_kernel(
                 if ((lane >> 3) == (j0 >> 3)) mydot += t;   // lane j0 + u takes vector u
             }
         };
-        if (FAST) {
-            // grad_A alone, at most 64 dense columns: one column tile per batch, so a batch is
-            // just its 16 operand vectors.  Two batches are kept in flight: the gathers of the
-            // next batch are issued before the current one is reduced.  The two stages
-            // alternate in place (copying a stage whose loads are still in flight would wait
-            // for them), and the scalar rows and columns of a batch die with its address
-            // arithmetic, which keeps them out of vector registers.
-            const bool live = lane < n;
-            auto issue = [&](int j0, T (&gv)[kBatch], T (&bv)[kBatch]) {
-                int64_t col[kBatch], rw[kBatch];
-                locate(j0, col, rw);
-                fetch(col, rw, lane, live, gv, bv);
-            };
-            auto finish = [&](int j0, const T (&gv)[kBatch], const T (&bv)[kBatch]) {
-                T p[kBatch];
+        for (int j0 = 0; j0 < cnt; j0 += kBatch) {
+            int64_t col[kBatch], rw[kBatch];
+            locate(j0, col, rw);
+            if (wide) {
+                // (with fewer columns: the tile-by-tile sums below, which are the one-walk kernel's,
+                // bit for bit)  A lane keeps its
+                // columns' share of the eight sums and the lanes are added up once, behind the
+                // last tile (a reduction per tile is 27 instructions for 16 loads; at 16 384 dense
+                // columns that was most of the kernel)
+                T part[kBatch];
 #pragma unroll
-                for (int u = 0; u < kBatch; ++u) p[u] = live ? gv[u] * bv[u] : T(0);
-                const T t = reduce8(p);
-                if ((lane >> 3) == (j0 >> 3)) mydot += t;
-            };
-            T gva[kBatch], bva[kBatch], gvb[kBatch], bvb[kBatch];
-            issue(0, gva, bva);
-            for (int j0 = 0;; j0 += 2 * kBatch) {
-                if (j0 + kBatch < cnt) issue(j0 + kBatch, gvb, bvb);
-                finish(j0, gva, bva);
-                if (j0 + kBatch >= cnt) break;
-                if (j0 + 2 * kBatch < cnt) issue(j0 + 2 * kBatch, gva, bva);
-                finish(j0 + kBatch, gvb, bvb);
-                if (j0 + 2 * kBatch >= cnt) break;
-            }
-        } else {
-            for (int j0 = 0; j0 < cnt; j0 += kBatch) {
-                int64_t col[kBatch], rw[kBatch];
-                locate(j0, col, rw);
-                if (wide) {
-                    // (with fewer columns: the tile-by-tile sums below, which are the one-walk kernel's,
-                    // bit for bit)  A lane keeps its
-                    // columns' share of the eight sums and the lanes are added up once, behind the
-                    // last tile (a reduction per tile is 27 instructions for 16 loads; at 16 384 dense
-                    // columns that was most of the kernel)
-                    T part[kBatch];
-#pragma unroll
-                    for (int u = 0; u < kBatch; ++u) part[u] = T(0);
+                for (int u = 0; u < kBatch; ++u) part[u] = T(0);
 #pragma unroll 2
-                    for (int64_t c0 = (int64_t)wave * kWave; c0 < n; c0 += kWavesPerBlock * kWave) {
-                        const int64_t c = c0 + lane;
-                        const bool live = c < n;
-                        T bv[kBatch], gv[kBatch];
-                        fetch(col, rw, c, live, gv, bv);
-#pragma unroll
-                        for (int u = 0; u < kBatch; ++u) part[u] += live ? gv[u] * bv[u] : T(0);
-                    }
-                    const T t = reduce8(part);
-                    if ((lane >> 3) == (j0 >> 3)) mydot += t;
-                    continue;
-                }
-                for (int64_t c0 = 0; c0 < n; c0 += kWave) {
+                for (int64_t c0 = (int64_t)wave * kWave; c0 < n; c0 += kWavesPerBlock * kWave) {
                     const int64_t c = c0 + lane;
                     const bool live = c < n;
                     T bv[kBatch], gv[kBatch];
                     fetch(col, rw, c, live, gv, bv);
-                    consume(j0, col, c, live, gv, bv);
+#pragma unroll
+                    for (int u = 0; u < kBatch; ++u) part[u] += live ? gv[u] * bv[u] : T(0);
                 }
+                const T t = reduce8(part);
+                if ((lane >> 3) == (j0 >> 3)) mydot += t;
+                continue;
+            }
+            for (int64_t c0 = 0; c0 < n; c0 += kWave) {
+                const int64_t c = c0 + lane;
+                const bool live = c < n;
+                T bv[kBatch], gv[kBatch];
+                fetch(col, rw, c, live, gv, bv);
+                consume(j0, col, c, live, gv, bv);
             }
         }
         if (wide) {
@@ -667,105 +639,6 @@ __global__ __launch_bounds__(kBlock) void spdmm_bwd_fused_kernel(
     }
 }
 
-// ---- narrow dense operands (n <= 32) -----------------------------------------------
-//
-// With lane = dense column, a 16-column operand leaves three quarters of every gather and
-// every multiply idle, and the kernels above take as long for n = 8 as for n = 64 (their time
-// is instruction issue and latency per ENTRY).  In the dot products of the backward a wavefront
-// therefore works on 64 / W entries per instruction, W = n rounded up to 8, 16 or 32: lane =
-// (entry slot, column); 1.03 -> 0.73 ms for the whole backward at n = 16 on the 1M x 1M
-// power-law matrix.  (The same mapping for the forward product, with the products of a chunk
-// staged in LDS and added per row in storage order, measured no faster than the wide kernel:
-// 0.41-0.77 ms against 0.51 ms, and was dropped.)
-
-// Sum over aligned groups of W lanes; every lane of the group gets it.
-template <int W, typename T> __device__ __forceinline__ T narrow_sum(T v) {
-    v += nm::dpp_move<0xB1>(v);                  // quad_perm [1,0,3,2]
-    v += nm::dpp_move<0x4E>(v);                  // quad_perm [2,3,0,1]
-    if (W == 8) v += nm::dpp_move<0x141>(v);     // row_half_mirror: the other quad of the 8
-    if (W >= 16) {
-        v += nm::dpp_move<0x124>(v);             // row_ror 4
-        v += nm::dpp_move<0x128>(v);             // row_ror 8
-    }
-    if (W == 32) v += __shfl_xor(v, 16, kWave);
-    return v;
-}
-
-// grad_A[k] = <gC[row(k), :], B[col(k), :]> for n <= W.  Entry-balanced like the wide kernel:
-// a wavefront owns 64 consecutive entries; every lane first finds the row of "its" entry by a
-// bisection over the ends of the next 64 rows (held one per lane), then the wavefront takes
-// 64 / W entries per step, four steps' gathers in flight.
-template <typename T, int W>
-__global__ __launch_bounds__(kBlock) void sddmm_narrow_kernel(
-    int64_t rows, int64_t nnz, const int64_t *__restrict__ indices, const int64_t *__restrict__ indptr,
-    const T *__restrict__ B, int64_t ldb, const T *__restrict__ gC, int64_t ldg, int n, T *__restrict__ grad_A,
-    const int32_t *__restrict__ chunk_row) {
-    constexpr int GPW = kWave / W;   // entries per step
-    constexpr int U = 4;             // steps per batch
-    const int lane = threadIdx.x & (kWave - 1);
-    const int64_t wave0 = (int64_t)blockIdx.x * kWavesPerBlock + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int64_t nwaves = (int64_t)gridDim.x * kWavesPerBlock;
-    const int64_t nchunks = (nnz + kWave - 1) / kWave;
-    const int slot = lane / W, c = lane % W;
-    const bool col_live = c < n;
-    const int cs = col_live ? c : 0;
-    for (int64_t ch = wave0; ch < nchunks; ch += nwaves) {
-        const int64_t kb = ch * kWave;
-        const int cnt = (int)(nnz - kb < kWave ? nnz - kb : kWave);
-        const int64_t k = kb + (lane < cnt ? lane : cnt - 1);
-        const int64_t mycol = indices[k];
-        int64_t row0;   // row of the chunk's first entry
-        if (chunk_row) {
-            row0 = chunk_row[ch];
-        } else {
-            int64_t lo = 0, hi = rows + 1;
-            while (lo < hi) {
-                const int64_t mid = (lo + hi) >> 1;
-                if (indptr[mid] <= kb) lo = mid + 1; else hi = mid;
-            }
-            row0 = lo - 1;
-        }
-        // my entry's row: row0 + number of row ends at or before it
-        const int64_t er = row0 + 1 + lane;
-        const int64_t my_end = indptr[er <= rows ? er : rows];
-        int lo = 0, hi = kWave;
-#pragma unroll
-        for (int step = 0; step < 7; ++step) {   // 65 possible answers: seven halvings
-            const int mid = (lo + hi) >> 1;      // == 64 only once lo == hi == 64: the read is ignored then
-            const int64_t e = __shfl(my_end, mid & (kWave - 1), kWave);
-            if (lo < hi) {
-                if (e <= k) lo = mid + 1; else hi = mid;
-            }
-        }
-        int64_t myrow = row0 + lo;
-        if (lo == kWave) {   // more than 64 rows end inside this chunk (empty rows): look the row up
-            int64_t l2 = myrow, h2 = rows + 1;
-            while (l2 < h2) {
-                const int64_t mid = (l2 + h2) >> 1;
-                if (indptr[mid] <= k) l2 = mid + 1; else h2 = mid;
-            }
-            myrow = l2 - 1;
-        }
-        for (int j0 = 0; j0 < cnt; j0 += U * GPW) {
-            T gv[U], bv[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int j = j0 + u * GPW + slot;
-                const int js = j < cnt ? j : cnt - 1;
-                const int64_t col = __shfl(mycol, js, kWave), rw = __shfl(myrow, js, kWave);
-                gv[u] = gC[rw * ldg + cs];
-                bv[u] = B[col * ldb + cs];
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int j = j0 + u * GPW + slot;
-                const T dot = narrow_sum<W>(col_live ? gv[u] * bv[u] : T(0));
-                if (c == 0 && j < cnt) grad_A[kb + j] = dot;
-            }
-        }
-    }
-}
-
 // Launches the forward product (A as delivered, or A^T through the plan).
 template <typename T, typename IDX, bool PERM>
 void launch_product(unsigned grid, hipStream_t s, int64_t rows, const T *data, const IDX *indices, const IDX *indptr,
@@ -789,6 +662,29 @@ inline unsigned flat_grid_for(int64_t rows) {
     return (unsigned)(g < 1 ? 1 : g);
 }
 
+// The kernels of nm_spmm_groups.hpp over the structure (ptr, idx, perm): out = sums of rows of `dense`,
+// dots = products of these with the rows of `own`.
+template <typename T, typename IDX>
+nm_groups::Args<T, IDX> group_args(int64_t rows, const void *data, const IDX *idx, const IDX *ptr, const int32_t *perm,
+                                   const void *dense, int64_t ld, int64_t n, void *out, int64_t ldo, const void *own,
+                                   int64_t ldw, void *dots) {
+    nm_groups::Args<T, IDX> a{};
+    a.rows = rows;
+    a.ptr = ptr;
+    a.idx = idx;
+    a.perm = perm;
+    a.data = (const T *)data;
+    a.dense = (const T *)dense;
+    a.ld = ld;
+    a.n = (int)n;
+    a.out = (T *)out;
+    a.ldo = ldo;
+    a.own = (const T *)own;
+    a.ldw = ldw;
+    a.dots = (T *)dots;
+    return a;
+}
+
 inline unsigned wave_grid(int64_t units, int per_block) {
     int64_t grid = nm::ceil_div(units, per_block);
     if (grid > nm::kMaxGrid) grid = nm::kMaxGrid;
@@ -806,6 +702,12 @@ extern "C" int nm_spdmm_forward(nm_dtype dt, int64_t rows, int64_t cols, int64_t
     NM_REQUIRE(ldb >= n && ldc >= n, "row stride smaller than the row (ldb=%lld ldc=%lld n=%lld)",
                (long long)ldb, (long long)ldc, (long long)n);
     hipStream_t s = nm::as_stream(stream);
+    if (dt == NM_F32 && nm_groups::takes<float>(cols, ldb, n))
+        return nm_groups::launch<float, int64_t, false, false>(
+            group_args<float>(rows, data, indices, indptr, nullptr, B, ldb, n, C, ldc, nullptr, 0, nullptr), s);
+    if (dt == NM_F64 && nm_groups::takes<double>(cols, ldb, n))
+        return nm_groups::launch<double, int64_t, false, false>(
+            group_args<double>(rows, data, indices, indptr, nullptr, B, ldb, n, C, ldc, nullptr, 0, nullptr), s);
     const unsigned flat_grid = flat_grid_for(rows);
     if (dt == NM_F32)
         launch_product<float, int64_t, false>(flat_grid, s, rows, (const float *)data, indices, indptr, nullptr,
@@ -844,28 +746,16 @@ int backward_impl(nm_dtype dt, int64_t rows, int64_t cols, int64_t nnz, const vo
     NM_REQUIRE(ldb >= n && ldg >= n, "row stride smaller than the row");
     // (dot products alone over thousands of dense columns: a workgroup per chunk of 64 entries)
     const dim3 grid(wave_grid(nm::ceil_div(nnz, kWave), grad_A && !grad_B && n > 4 * kColsPerSlice ? 1 : kWavesPerBlock));
-    if (grad_A && !grad_B && n <= 32) {
-#define NM_NARROW(T, W)                                                                                          \
-    hipLaunchKernelGGL((sddmm_narrow_kernel<T, W>), grid, dim3(kBlock), 0, s, rows, nnz, indices, indptr,          \
-                       (const T *)B, ldb, (const T *)gC, ldg, (int)n, (T *)grad_A, chunk_row)
-        if (dt == NM_F32) {
-            if (n <= 8) NM_NARROW(float, 8); else if (n <= 16) NM_NARROW(float, 16); else NM_NARROW(float, 32);
-        } else {
-            if (n <= 8) NM_NARROW(double, 8); else if (n <= 16) NM_NARROW(double, 16); else NM_NARROW(double, 32);
-        }
-#undef NM_NARROW
-        NM_LAUNCH_CHECK("sddmm_narrow_kernel");
-        return NM_OK;
-    }
-    const bool fast = grad_A && !grad_B && n <= kWave;
-#define NM_SDDMM(T, FAST)                                                                                         \
-    hipLaunchKernelGGL((spdmm_bwd_kernel<T, FAST>), grid, dim3(kBlock), 0, s, rows, nnz, (const T *)data, indices, \
+    if (grad_A && !grad_B && dt == NM_F32 && nm_groups::takes<float>(cols, ldb, n, rows, ldg))
+        return nm_groups::launch_dots(
+            group_args<float>(rows, data, indices, indptr, nullptr, B, ldb, n, nullptr, 0, gC, ldg, grad_A), nnz, chunk_row, s);
+    if (grad_A && !grad_B && dt == NM_F64 && nm_groups::takes<double>(cols, ldb, n, rows, ldg))
+        return nm_groups::launch_dots(
+            group_args<double>(rows, data, indices, indptr, nullptr, B, ldb, n, nullptr, 0, gC, ldg, grad_A), nnz, chunk_row, s);
+#define NM_SDDMM(T)                                                                                               \
+    hipLaunchKernelGGL((spdmm_bwd_kernel<T>), grid, dim3(kBlock), 0, s, rows, nnz, (const T *)data, indices,        \
                        indptr, (const T *)B, ldb, (const T *)gC, ldg, n, (T *)grad_A, (T *)grad_B, ldgb, chunk_row)
-    if (dt == NM_F32) {
-        if (fast) NM_SDDMM(float, true); else NM_SDDMM(float, false);
-    } else {
-        if (fast) NM_SDDMM(double, true); else NM_SDDMM(double, false);
-    }
+    if (dt == NM_F32) NM_SDDMM(float); else NM_SDDMM(double);
 #undef NM_SDDMM
     NM_LAUNCH_CHECK("spdmm_bwd_kernel");
     return NM_OK;
@@ -892,13 +782,22 @@ extern "C" int nm_spdmm_backward_planned(nm_dtype dt, int64_t rows, int64_t cols
     NM_REQUIRE(plan_mem != nullptr, "plan is null");
     nm::TPlan t;
     nm::tplan_layout(rows, cols, nnz, const_cast<void *>(plan_mem), &t);
+    if (grad_B && rows > 0 && cols > 0 && nnz > 0 &&
+        (dt == NM_F32 ? nm_groups::takes<float>(rows, ldg, n) : nm_groups::takes<double>(rows, ldg, n))) {
+        NM_REQUIRE((!grad_A || B != nullptr) && gC != nullptr, "B or gC is null");
+        NM_REQUIRE((!grad_A || ldb >= n) && ldg >= n && ldgb >= n, "row stride smaller than the row");
+        hipStream_t s = nm::as_stream(stream);
+        if (dt == NM_F32) {
+            const auto a = group_args<float>(cols, data, t.t_row, t.t_indptr, t.t_perm, gC, ldg, n, grad_B, ldgb, B, ldb, grad_A);
+            return grad_A ? nm_groups::launch<float, int32_t, true, true>(a, s) : nm_groups::launch<float, int32_t, true, false>(a, s);
+        }
+        const auto a = group_args<double>(cols, data, t.t_row, t.t_indptr, t.t_perm, gC, ldg, n, grad_B, ldgb, B, ldb, grad_A);
+        return grad_A ? nm_groups::launch<double, int32_t, true, true>(a, s) : nm_groups::launch<double, int32_t, true, false>(a, s);
+    }
     // (a dense operand of thousands of columns: the fused walk takes its column tiles one after the
     // other, the product below is cut into slices of kColsPerSlice over the grid)
     if (grad_A && grad_B && rows > 0 && cols > 0 && nnz > 0 && n > 32 && n <= 4 * kColsPerSlice) {
-        // both gradients from a single walk over A by column (measured on the 16 M-entry power-law
-        // matrix: 1.02 against 1.29 ms at 64 dense columns, 2.18 against 2.80 ms at 128, even at 32;
-        // with 16 or fewer the narrow dot-product kernel below and a separate product are faster,
-        // 0.70-0.74 against 0.81-0.82 ms)
+        // both gradients from a single walk over A by column
         NM_REQUIRE(B != nullptr && gC != nullptr, "B or gC is null");
         NM_REQUIRE(ldb >= n && ldg >= n && ldgb >= n, "row stride smaller than the row");
         hipStream_t s = nm::as_stream(stream);

@@ -1,0 +1,511 @@
+// CSR x dense with a dense operand of up to 1 KB a row: several entries of A per request.
+//
+// What bounds these products is the rows of the dense operand that the entries name.  With uniformly
+// random columns every entry fetches its row from beyond L2, and this part delivers about 57 cache
+// lines (128 bytes) a nanosecond from there, whether a line is wanted whole or by half: 15.6 M rows
+// of 256 bytes take 535 us, of 128 bytes 287, of 64 bytes 275.  A kernel reaches that only if it
+// asks for rows fast enough.  With lane = dense column (the kernels of nm_spmm.hip) an entry costs
+// the compute unit one request of ~16 cycles and a wavefront some eight instructions however narrow
+// the operand is: 520 us at 16 columns, where the lines would allow 275.
+//
+// Here a group of G lanes takes an entry, V = 16 bytes of its row a lane, so that a wavefront's
+// request covers 64 / G entries.  Every group walks its own rows of A and adds each row's terms in
+// storage order, like the serial loop (cpp/sparse_csr_cpu.cpp:586-598): same bits.  The groups of a
+// workgroup draw rows from a counter in LDS, so one that has a longer row holds nobody up.  Rows of
+// more than kShared entries are left to the workgroups at the head of the grid, which look for them and
+// share each one among all their groups: up to kSplit entries the products meet in LDS and are added in
+// storage order, beyond that chunks of 16 entries are summed and the sums added in order
+// (deterministic, the serial sum up to rounding).
+//
+// The walk gives out[r, :] = sum of value * dense[index, :] over the entries of row r and, with DOT,
+// dots[position] = <dense[index, :], own[r, :]>: the backward by column needs the same row of gC for
+// grad_B and for grad_A.  Dot products alone go by entry (dots_kernel).
+//
+// Measured on graphs with power-law rows and uniformly random columns, forward / with both gradients, against
+// lane = column: 1 M rows, 15.6 M entries, fp32: 64 columns 676 -> 650 / 1708 -> 1592 us (the rows' lines
+// alone take 535, index, values and result 60 more), 16 columns 520 -> 326 / 1276 -> 1040, 128 columns of 8.2 M
+// entries 804 -> 702 / 2172 -> 1618; 60 000 rows, 64 columns 190 -> 89 / 254 -> 145.  Seven-point matrix on 96^3,
+// 16 columns, fp32: 171 -> 60 / 462 -> 163.
+#pragma once
+
+#include "nm_common.hpp"
+
+namespace nm_groups {
+
+using nm::kWave;
+constexpr int kThreads = 256;
+// Rows of more than kShared entries are shared by the groups of a workgroup, up to kSplit entries with
+// their terms in storage order.  (Taken by one group each up to 512 entries, such rows kept the rest of
+// their workgroup waiting: 957 against 650 us.  From 65 entries on: 655 us; from 33: 745.)
+constexpr int kShared = 128, kSplit = 512;
+constexpr int kChunk = 16;         // entries of a row a group takes from memory at once
+constexpr int kPass = 4;           // entries of a shared row a group takes at once where their order counts
+// A matrix of few rows leaves compute units free while one workgroup after the other is at work on the
+// longest rows: there a workgroup looks through fewer rows, and a shared row's result is cut into slices of
+// 128 bytes (kSliceLanes lanes), a workgroup each, which has more of the row's entries in flight (60 000 rows,
+// up to 10 000 entries, 64 columns: 205 -> 89 us).  Where the chip is full anyway slices only cost
+// (1 M rows of 37 columns: 650 -> 785 us, the slices of a row share lines).
+constexpr int kSliceLanes = 8;
+constexpr int64_t kFewBlocks = 2048, kFewRows = 64;
+constexpr int kScan = kThreads;    // rows a workgroup at the head of the grid looks through
+constexpr int kDrawRows = 4;       // rows of a workgroup per group: enough to draw from, few enough that the
+                                   // rows of `own` (16 KB) leave room for eight workgroups a compute unit
+
+// V consecutive elements at an address that need only suit one of them
+template <typename T, int V> struct Vec { typedef T type __attribute__((ext_vector_type(V), aligned(sizeof(T)))); };
+template <typename T> struct Vec<T, 1> { typedef T type; };
+template <typename T, int V> struct Held { typedef T type __attribute__((ext_vector_type(V))); };   // the same in LDS
+template <typename T> struct Held<T, 1> { typedef T type; };
+template <typename T, int V> __device__ __forceinline__ T part(const typename Vec<T, V>::type &v, int i) {
+    if constexpr (V == 1) return v; else return v[i];
+}
+
+template <typename T, typename IDX> struct Args {
+    int64_t rows;             // rows that are walked (columns of A on the transposed structure)
+    const IDX *ptr, *idx;
+    const int32_t *perm;      // PERM: where an entry's value is and its dot product goes
+    const T *data;
+    const T *dense;           // gathered rows
+    int64_t ld;
+    int n;
+    T *out;
+    int64_t ldo;
+    const T *own;             // DOT: row r belongs to walked row r
+    int64_t ldw;
+    T *dots;
+    int scan_rows;            // rows each of the workgroups that look for long rows looks through
+    unsigned scan_blocks;     // workgroups that look for long rows, a multiple of nm::kXcds
+    unsigned tiles;           // workgroups that walk rows, the same
+};
+
+// Sum over the G lanes of a group, in every one of them and with the same bits in each (every step adds
+// two lanes' sums that are added the other way round in the other lane).
+template <int G, typename T> __device__ __forceinline__ T group_total(T v) {
+    v += nm::dpp_move<0xB1>(v);                          // quad_perm [1,0,3,2]
+    v += nm::dpp_move<0x4E>(v);                          // quad_perm [2,3,0,1]
+    if constexpr (G >= 8) v += nm::dpp_move<0x141>(v);   // row_half_mirror: the other quad of the 8
+    if constexpr (G >= 16) v += nm::dpp_move<0x140>(v);  // row_mirror: the other 8 of the 16
+    if constexpr (G >= 32) v += __shfl_xor(v, 16, kWave);
+    if constexpr (G == 64) v += __shfl_xor(v, 32, kWave);
+    return v;
+}
+
+template <typename T, int V, int G, typename IDX, bool PERM, bool DOT>
+struct Walker {
+    static constexpr int kGroups = kThreads / G, kRows = kGroups * kDrawRows;
+    // rows of the dense operand in flight at once: with 16 too few wavefronts fit (936 against 650 us)
+    static constexpr int kBatch = G >= 32 ? 4 : 8;
+    static constexpr int kHeld = G < kChunk ? kChunk / G : 1;   // entries of a chunk a lane holds
+    using vec = typename Vec<T, V>::type;
+    using held = typename Held<T, V>::type;
+
+    const Args<T, IDX> &a;
+    int l, first;          // lane of the group, the group's first lane
+    int c0;                // first column of the lane (the last lane's are moved back to end at n)
+    bool live;             // the lane has columns of its own
+    int fresh;             // the lane's first column that the lane before has not
+    const char *dense_c;
+    uint32_t row_bytes;
+    T dot[kHeld];          // dot products of the entries the lane holds
+
+    // (slice: the columns from slice * G * V on)
+    __device__ __forceinline__ Walker(const Args<T, IDX> &args, int slice = 0) : a(args) {
+        const int lane = threadIdx.x & (kWave - 1);
+        l = lane & (G - 1);
+        first = lane & ~(G - 1);
+        const int c = (slice * G + l) * V;
+        live = c < a.n;
+        c0 = c + V <= a.n ? c : a.n - V;
+        fresh = c - c0;
+        dense_c = reinterpret_cast<const char *>(a.dense + c0);
+        row_bytes = (uint32_t)(a.ld * (int64_t)sizeof(T));
+    }
+    // entries [kc, kc + cnt) of the chunk, cnt >= 1; places beyond them hold the last one
+    struct Chunk {
+        uint32_t col[kHeld];
+        T val[kHeld];
+        int32_t pos[kHeld];
+    };
+    __device__ __forceinline__ void load(Chunk &c, int64_t kc, int cnt) const {
+#pragma unroll
+        for (int h = 0; h < kHeld; ++h) {
+            const int e = h * G + l;
+            const int64_t k = kc + (e < cnt ? e : cnt - 1);
+            c.col[h] = (uint32_t)nm::stream_load(a.idx + k);
+            if constexpr (PERM) c.pos[h] = nm::stream_load(a.perm + k);
+            if constexpr (!PERM) c.val[h] = nm::stream_load(a.data + k);
+        }
+        if constexpr (PERM) {
+#pragma unroll
+            for (int h = 0; h < kHeld; ++h) c.val[h] = a.data[c.pos[h]];
+        }
+    }
+    __device__ __forceinline__ vec gather(const Chunk &c, int e) const {
+        const uint32_t col = (uint32_t)__shfl((int)c.col[e / G], first + e % G, kWave);
+        return *reinterpret_cast<const vec *>(dense_c + (uint64_t)col * row_bytes);
+    }
+    __device__ __forceinline__ void add(const Chunk &c, int e, const vec &b, T (&acc)[V]) const {
+        const T x = __shfl(c.val[e / G], first + e % G, kWave);
+#pragma unroll
+        for (int v = 0; v < V; ++v) acc[v] += x * part<T, V>(b, v);
+    }
+    __device__ __forceinline__ vec product(const Chunk &c, int e, const vec &b) const {
+        return __shfl(c.val[e / G], first + e % G, kWave) * b;
+    }
+    __device__ __forceinline__ T product_sum(const vec &b, const vec &mine) const {
+        T p[V];
+#pragma unroll
+        for (int v = 0; v < V; ++v) p[v] = live && v >= fresh ? part<T, V>(b, v) * part<T, V>(mine, v) : T(0);
+        T s = p[0];
+        if constexpr (V == 2) s = p[0] + p[1];
+        if constexpr (V == 4) s = (p[0] + p[1]) + (p[2] + p[3]);
+        return group_total<G>(s);
+    }
+    __device__ __forceinline__ void multiply(int e, const vec &b, const vec &mine) {
+        const T s = product_sum(b, mine);
+        if (l == e % G) dot[e / G] = s;
+    }
+    __device__ __forceinline__ void store_dots(const Chunk &c, int64_t kc, int cnt) const {
+#pragma unroll
+        for (int h = 0; h < kHeld; ++h) {
+            const int e = h * G + l;
+            if (e < cnt && e < kChunk) a.dots[PERM ? (int64_t)c.pos[h] : kc + e] = dot[h];
+        }
+    }
+    static __device__ __forceinline__ vec pack(const T (&acc)[V]) {
+        vec o;
+        if constexpr (V == 1) {
+            o = acc[0];
+        } else {
+#pragma unroll
+            for (int v = 0; v < V; ++v) o[v] = acc[v];
+        }
+        return o;
+    }
+    __device__ __forceinline__ void store_row(int64_t row, const T (&acc)[V]) const {
+        if (live) *reinterpret_cast<vec *>(a.out + row * a.ldo + c0) = pack(acc);
+    }
+    __device__ __forceinline__ vec own_row(int64_t row) const {
+        return *reinterpret_cast<const vec *>(a.own + row * a.ldw + c0);
+    }
+};
+
+template <typename T, int V, int G, typename IDX, bool PERM, bool DOT, bool SLICED>
+__global__ __launch_bounds__(kThreads, 5) void groups_kernel(const Args<T, IDX> a) {
+    using W = Walker<T, V, G, IDX, PERM, DOT>;
+    using vec = typename W::vec;
+    constexpr int kGroups = W::kGroups, kRows = W::kRows;
+    __shared__ int64_t s_ptr[kRows + 1];
+    // the walked rows' rows of `own`; in the workgroups that share rows: products, partial sums
+    __shared__ typename W::held s_mem[(DOT ? kRows * G : 1) > kThreads * kPass ? kRows * G : kThreads * kPass];
+    typename W::held *const s_own = s_mem, *const s_pass = s_mem;
+    __shared__ int s_list[kScan];
+    __shared__ int s_next;
+    const int t = threadIdx.x;
+
+    if (blockIdx.x < a.scan_blocks) {
+        // ---- rows of more than kShared entries, each shared by the groups of the workgroup ----
+        // (sums alone: a workgroup takes 128 bytes of the row's result, so that wide operands have
+        // more workgroups and more entries at once on a row; a dot product wants the whole row)
+        constexpr int GS = SLICED ? kSliceLanes : G, kGroups = kThreads / GS;
+        using WS = Walker<T, V, GS, IDX, PERM, DOT>;
+        using Chunk = typename WS::Chunk;
+        constexpr int kBatch = WS::kBatch;
+        const int slices = SLICED ? (a.n + GS * V - 1) / (GS * V) : 1;
+        WS w(a, SLICED ? blockIdx.x % slices : 0);
+        const int g = t / GS;
+        const int64_t r0 = (int64_t)(blockIdx.x / slices) * a.scan_rows;
+        if (t == 0) s_next = 0;
+        __syncthreads();
+        if (t < a.scan_rows && r0 + t < a.rows && (int64_t)(a.ptr[r0 + t + 1] - a.ptr[r0 + t]) > kShared)
+            s_list[atomicAdd(&s_next, 1)] = t;
+        __syncthreads();
+        const int found = s_next;
+        for (int i = 0; i < found; ++i) {   // (the order of the list does not matter)
+            const int64_t row = r0 + s_list[i], b = a.ptr[row], e = a.ptr[row + 1];
+            T acc[V] = {};
+            vec mine{};
+            if constexpr (DOT) mine = w.own_row(row);
+            Chunk c, later;
+            if (e - b <= kSplit) {
+                // every group takes four entries of a pass; their products meet in LDS, where one group
+                // adds them up in storage order
+                auto mine_of = [&](int64_t base) {   // entries of the pass at `base` that are this group's
+                    const int64_t left = e - base - g * kPass;
+                    return (int)(left < kPass ? left : kPass);
+                };
+                if (mine_of(b) > 0) w.load(c, b + g * kPass, mine_of(b));
+                for (int64_t base = b; base < e; base += kGroups * kPass) {
+                    const int cnt = mine_of(base), next = mine_of(base + kGroups * kPass);
+                    if (next > 0) w.load(later, base + kGroups * kPass + g * kPass, next);
+                    if (cnt > 0) {
+                        vec d[kPass];
+#pragma unroll
+                        for (int u = 0; u < kPass; ++u) d[u] = w.gather(c, u);
+#pragma unroll
+                        for (int u = 0; u < kPass; ++u) {
+                            if (u < cnt) {
+                                s_pass[(g * kPass + u) * GS + w.l] = w.product(c, u, d[u]);
+                                if constexpr (DOT) w.multiply(u, d[u], mine);
+                            }
+                        }
+                        if constexpr (DOT) w.store_dots(c, base + g * kPass, cnt);
+                    }
+                    __syncthreads();
+                    if (g == 0) {
+                        const int all = (int)(e - base < kGroups * kPass ? e - base : kGroups * kPass);
+#pragma unroll 4
+                        for (int j = 0; j < all; ++j) {
+                            const vec p = s_pass[j * GS + w.l];
+#pragma unroll
+                            for (int v = 0; v < V; ++v) acc[v] += part<T, V>(p, v);
+                        }
+                    }
+                    __syncthreads();
+                    c = later;
+                }
+                if (g == 0) w.store_row(row, acc);
+                continue;
+            }
+            // longer ones: a chunk of entries a group and pass, whose sums are added in the order of the
+            // chunks (so the bits do not depend on how many groups there are)
+            constexpr int64_t kStep = (int64_t)kGroups * kChunk;
+            auto count = [&](int64_t kc) { return (int)(e - kc < kChunk ? e - kc : kChunk); };
+            int64_t kc = b + (int64_t)g * kChunk;
+            if (kc < e) w.load(c, kc, count(kc));
+            for (int64_t base = b; base < e; base += kStep, kc += kStep) {
+                if (kc + kStep < e) w.load(later, kc + kStep, count(kc + kStep));
+                if (kc < e) {
+                    const int cnt = count(kc);
+                    T sum[V] = {};
+#pragma unroll
+                    for (int j0 = 0; j0 < kChunk; j0 += kBatch) {
+                        vec d[kBatch];
+#pragma unroll
+                        for (int u = 0; u < kBatch; ++u) d[u] = w.gather(c, j0 + u);
+#pragma unroll
+                        for (int u = 0; u < kBatch; ++u) {
+                            if (j0 + u < cnt) {
+                                w.add(c, j0 + u, d[u], sum);
+                                if constexpr (DOT) w.multiply(j0 + u, d[u], mine);
+                            }
+                        }
+                    }
+                    if constexpr (DOT) w.store_dots(c, kc, cnt);
+                    s_pass[t] = WS::pack(sum);
+                }
+                {
+                    __syncthreads();
+                    if (g == 0) {
+                        const int64_t left = (e - base + kChunk - 1) / kChunk;
+                        const int all = (int)(left < kGroups ? left : kGroups);
+#pragma unroll 4
+                        for (int j = 0; j < all; ++j) {
+                            const vec p = s_pass[j * GS + w.l];
+#pragma unroll
+                            for (int v = 0; v < V; ++v) acc[v] += part<T, V>(p, v);
+                        }
+                    }
+                    __syncthreads();
+                }
+                c = later;
+            }
+            if (g == 0) w.store_row(row, acc);
+        }
+        return;
+    }
+
+    // ---- all other rows, drawn by the groups one at a time ----
+    W w(a);
+    constexpr int kBatch = W::kBatch;
+    const int g = t / G;
+    typename W::Chunk c;
+    const int64_t r0 = nm::xcd_tile(blockIdx.x - a.scan_blocks, a.tiles) * kRows;
+    if (r0 >= a.rows) return;
+    const int nr = (int)(a.rows - r0 < kRows ? a.rows - r0 : kRows);
+    for (int i = t; i <= nr; i += kThreads) s_ptr[i] = (int64_t)a.ptr[r0 + i];
+    if constexpr (DOT) {
+        for (int i = g; i < nr; i += kGroups) s_own[i * G + w.l] = w.own_row(r0 + i);
+    }
+    if (t == 0) s_next = kGroups;
+    __syncthreads();
+    // A turn of the loop takes a chunk of every group's row, whatever the rows' lengths.  (The first row
+    // of a group is its own number: no draw.)
+    int r = g;
+    int64_t kc = 0, e = 0;
+    T acc[V] = {};
+    vec mine{};
+    auto draw = [&]() {
+        int next = 0;
+        if (w.l == 0) next = atomicAdd(&s_next, 1);
+        r = __shfl(next, w.first, kWave);
+    };
+    auto begin = [&]() {   // on to the next row that has entries and is not shared
+        for (; r < nr; draw()) {
+            kc = s_ptr[r];
+            e = s_ptr[r + 1];
+#pragma unroll
+            for (int v = 0; v < V; ++v) acc[v] = T(0);
+            if (e == kc) {
+                w.store_row(r0 + r, acc);
+            } else if (e - kc <= kShared) {
+                if constexpr (DOT) mine = s_own[r * G + w.l];
+                return;
+            }
+        }
+    };
+    begin();
+    while (r < nr) {
+        const int cnt = (int)(e - kc < kChunk ? e - kc : kChunk);
+        w.load(c, kc, cnt);
+#pragma unroll
+        for (int j0 = 0; j0 < kChunk; j0 += kBatch) {
+            if (j0 < cnt) {
+                vec d[kBatch];
+#pragma unroll
+                for (int u = 0; u < kBatch; ++u) d[u] = w.gather(c, j0 + u);
+#pragma unroll
+                for (int u = 0; u < kBatch; ++u) {
+                    if (j0 + u < cnt) {
+                        w.add(c, j0 + u, d[u], acc);
+                        if constexpr (DOT) w.multiply(j0 + u, d[u], mine);
+                    }
+                }
+            }
+        }
+        if constexpr (DOT) w.store_dots(c, kc, cnt);
+        kc += cnt;
+        if (kc == e) {
+            w.store_row(r0 + r, acc);
+            draw();
+            begin();
+        }
+    }
+}
+
+// Dot products alone: dots[k] = <dense[idx[k], :], own[row of k, :]>, by entry and not by row, since nothing is
+// added up over a row (one row may hold all entries).  A wavefront takes 64 consecutive entries, lane l entry
+// l: it finds that entry's row among the ends of the next 64 rows; a group then takes its lanes' entries one
+// after the other, a request a side, and every lane keeps its own entry's product (in the order of
+// groups_kernel: same bits).  `chunk_row`, when given, holds the row of every 64th entry.
+template <typename T, int V, int G>
+__global__ __launch_bounds__(kThreads) void dots_kernel(const Args<T, int64_t> a, int64_t nnz, const int32_t *__restrict__ chunk_row) {
+    using W = Walker<T, V, G, int64_t, false, true>;
+    using vec = typename W::vec;
+    constexpr int kFlight = G < 8 ? G : 8;
+    const W w(a);
+    const int lane = threadIdx.x & (kWave - 1);
+    const int64_t chunk = (int64_t)blockIdx.x * (kThreads / kWave) + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int64_t kb = chunk * kWave;
+    if (kb >= nnz) return;
+    const int64_t k = kb + lane < nnz ? kb + lane : nnz - 1;
+    const uint32_t mycol = (uint32_t)nm::stream_load(a.idx + k);
+    auto row_of = [&](int64_t entry, int64_t lo) {   // the last row r >= lo - 1 with ptr[r] <= entry
+        int64_t hi = a.rows + 1;
+        while (lo < hi) {
+            const int64_t mid = (lo + hi) >> 1;
+            if (a.ptr[mid] <= entry) lo = mid + 1; else hi = mid;
+        }
+        return lo - 1;
+    };
+    const int64_t row0 = chunk_row ? (int64_t)chunk_row[chunk] : row_of(kb, 0);
+    const int64_t end = row0 + 1 + lane;
+    const int64_t my_end = a.ptr[end <= a.rows ? end : a.rows];
+    int lo = 0, hi = kWave;
+#pragma unroll
+    for (int step = 0; step < 7; ++step) {   // 65 possible answers: seven halvings
+        const int mid = (lo + hi) >> 1;      // == 64 only once lo == hi == 64: the read is ignored then
+        const int64_t e = __shfl(my_end, mid & (kWave - 1), kWave);
+        if (lo < hi) {
+            if (e <= k) lo = mid + 1; else hi = mid;
+        }
+    }
+    // (more than 64 rows that end inside the chunk: empty ones)
+    const uint32_t myrow = (uint32_t)(lo == kWave ? row_of(k, row0 + lo) : row0 + lo);
+    const char *const own_c = reinterpret_cast<const char *>(a.own + w.c0);
+    const uint32_t own_bytes = (uint32_t)(a.ldw * (int64_t)sizeof(T));
+    T dot = T(0);
+#pragma unroll 1
+    for (int s0 = 0; s0 < G; s0 += kFlight) {
+        vec d[kFlight], o[kFlight];
+#pragma unroll
+        for (int u = 0; u < kFlight; ++u) {
+            const uint32_t c = (uint32_t)__shfl((int)mycol, w.first + s0 + u, kWave), r = (uint32_t)__shfl((int)myrow, w.first + s0 + u, kWave);
+            d[u] = *reinterpret_cast<const vec *>(w.dense_c + (uint64_t)c * w.row_bytes);
+            o[u] = *reinterpret_cast<const vec *>(own_c + (uint64_t)r * own_bytes);
+        }
+#pragma unroll
+        for (int u = 0; u < kFlight; ++u) {
+            const T s = w.product_sum(d[u], o[u]);
+            if (w.l == s0 + u) dot = s;
+        }
+    }
+    if (kb + lane < nnz) a.dots[kb + lane] = dot;
+}
+
+// The widest dense operand these kernels take: 64 lanes of 16 bytes.
+template <typename T> constexpr int64_t most_columns() { return kWave * (16 / (int64_t)sizeof(T)); }
+
+// Whether a product may go this way: indices that fit 32 bits and row strides that fit them in bytes.
+// (`own_rows`, `ldw`: of the operand the dot products are with)
+template <typename T> bool takes(int64_t indexed, int64_t ld, int64_t n, int64_t own_rows = 0, int64_t ldw = 0) {
+    return n >= 1 && n <= most_columns<T>() && indexed <= 0x7fffffff && own_rows <= 0x7fffffff &&
+           ld * (int64_t)sizeof(T) <= 0xffffffffll && ldw * (int64_t)sizeof(T) <= 0xffffffffll;
+}
+
+template <typename T, int V, int G, typename IDX, bool PERM, bool DOT>
+int launch_shape(Args<T, IDX> a, hipStream_t s) {
+    constexpr int64_t rows = (int64_t)(kThreads / G) * kDrawRows;
+    // rows a workgroup at the head of the grid looks through: few where the matrix has few, since it takes
+    // the long ones that it finds one after the other
+    a.scan_rows = kScan;
+    while (a.scan_rows > 16 && nm::ceil_div(a.rows, a.scan_rows) < kFewBlocks) a.scan_rows /= 2;
+    constexpr bool kMaySlice = !DOT && G > kSliceLanes;
+    const bool sliced = kMaySlice && nm::ceil_div(a.rows, kFewRows) < kFewBlocks;
+    const int64_t slices = sliced ? nm::ceil_div(a.n, kSliceLanes * V) : 1;
+    const int64_t scan = nm::xcd_padded(nm::ceil_div(a.rows, a.scan_rows) * slices), tiles = nm::xcd_padded(nm::ceil_div(a.rows, rows));
+    NM_REQUIRE(scan + tiles <= 0x7fffffff, "too many rows");
+    a.scan_blocks = (unsigned)scan;
+    a.tiles = (unsigned)tiles;
+    const dim3 grid((unsigned)(scan + tiles));
+    if constexpr (kMaySlice) {
+        if (sliced) {
+            hipLaunchKernelGGL((groups_kernel<T, V, G, IDX, PERM, DOT, true>), grid, dim3(kThreads), 0, s, a);
+            NM_LAUNCH_CHECK("groups_kernel");
+            return NM_OK;
+        }
+    }
+    hipLaunchKernelGGL((groups_kernel<T, V, G, IDX, PERM, DOT, false>), grid, dim3(kThreads), 0, s, a);
+    NM_LAUNCH_CHECK("groups_kernel");
+    return NM_OK;
+}
+
+// f(std::integral_constant<int, V>, std::integral_constant<int, G>) for a dense operand of n columns
+template <typename T, typename F> int by_width(int n, F f) {
+    constexpr int V = 16 / (int)sizeof(T);
+    using Wide = std::integral_constant<int, V>;
+    if (n < V) return f(std::integral_constant<int, 1>{}, std::integral_constant<int, 4>{});
+    if (n <= 4 * V) return f(Wide{}, std::integral_constant<int, 4>{});
+    if (n <= 8 * V) return f(Wide{}, std::integral_constant<int, 8>{});
+    if (n <= 16 * V) return f(Wide{}, std::integral_constant<int, 16>{});
+    if (n <= 32 * V) return f(Wide{}, std::integral_constant<int, 32>{});
+    return f(Wide{}, std::integral_constant<int, 64>{});
+}
+
+// out = sums of rows of `dense`, with DOT dots as well
+template <typename T, typename IDX, bool PERM, bool DOT> int launch(const Args<T, IDX> &a, hipStream_t s) {
+    if (a.rows == 0) return NM_OK;
+    return by_width<T>(a.n, [&](auto v, auto g) { return launch_shape<T, v(), g(), IDX, PERM, DOT>(a, s); });
+}
+
+template <typename T> int launch_dots(const Args<T, int64_t> &a, int64_t nnz, const int32_t *chunk_row, hipStream_t s) {
+    const int64_t grid = nm::ceil_div(nnz, (int64_t)kThreads);
+    NM_REQUIRE(grid <= 0x7fffffff, "too many entries");
+    return by_width<T>(a.n, [&](auto v, auto g) {
+        hipLaunchKernelGGL((dots_kernel<T, v(), g()>), dim3((unsigned)grid), dim3(kThreads), 0, s, a, nnz, chunk_row);
+        NM_LAUNCH_CHECK("dots_kernel");
+        return (int)NM_OK;
+    });
+}
+
+}  // namespace nm_groups
