@@ -114,7 +114,9 @@ int nm_csr_transpose_plan_build(int64_t rows, int64_t cols, int64_t nnz,
 
 /* What a built plan found out about the pattern, copied to the host: info[0]
  * pattern symmetric, info[1] / info[2] the packed words of the backward / the
- * 16-bit column offsets of the forward are valid, info[4] blocks of 512 rows
+ * 16-bit column offsets of the forward are valid, info[3] how many of every 64th
+ * entry in column-major order lie more than 2^18 entries from that place in
+ * row-major order, info[4] blocks of 512 rows
  * with a staging list (the SpMV forward loads the segments of x such a block
  * names into LDS), info[5] blocks of 256 columns with one (the same for the
  * backward), info[6] / info[7] entries of the longest column / row, info[8] the
@@ -226,6 +228,21 @@ int nm_spdmm_backward_planned(nm_dtype dt, int64_t rows, int64_t cols, int64_t n
                               const void *plan_mem,
                               const void *B, int64_t ldb, const void *gC, int64_t ldg, int64_t n,
                               void *grad_A, void *grad_B, int64_t ldgb, nm_stream stream);
+
+/* Values between row-major and column-major order, for patterns whose transpose scatters them over more memory than
+ * a cache holds.  The plan (8 bytes an entry, from the pattern's transposed-structure plan) makes that two
+ * passes with coalesced requests; nm_spdmm_backward_staged is nm_spdmm_backward_planned with the values
+ * brought into column-major order beforehand and grad_A brought back from it (work: nm_spdmm_staged_bytes), the same
+ * bits.  grad_B is required, a dense operand of more than 1 KB a row is refused.  Nothing waits.  No
+ * counterpart in the reference. */
+int nm_permute_plan_bytes(int64_t nnz, size_t *plan_bytes, size_t *work_bytes);
+int nm_permute_plan_build(int64_t rows, int64_t cols, int64_t nnz, const void *transpose_plan,
+                          void *plan, size_t plan_bytes, void *work, size_t work_bytes, nm_stream stream);
+int nm_spdmm_staged_bytes(nm_dtype dt, int64_t nnz, size_t *bytes);
+int nm_spdmm_backward_staged(nm_dtype dt, int64_t rows, int64_t cols, int64_t nnz, const void *data,
+                             const void *plan_mem, const void *permute_plan, void *work, size_t work_bytes,
+                             const void *B, int64_t ldb, const void *gC, int64_t ldg, int64_t n,
+                             void *grad_A, void *grad_B, int64_t ldgb, nm_stream stream);
 
 /* ---------------------------------------------------------------- SpGEMM
  * C = A B, both CSR.  Stands in for spgemm_forward (cpp/sparse_csr.hpp:45-48,

@@ -74,6 +74,11 @@ _SIGNATURES = {
                                   _c_ptr, _c_ptr, _c_ptr, _c_size, _c_int, _c_ptr, ctypes.POINTER(_c_int), _c_ptr],
     "nm_spgemm_backward_mapped_wide": [_c_int, _c_int, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_ptr,
                                        _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr],
+    "nm_permute_plan_bytes": [_c_i64, ctypes.POINTER(_c_size), ctypes.POINTER(_c_size)],
+    "nm_permute_plan_build": [_c_i64, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_size, _c_ptr, _c_size, _c_ptr],
+    "nm_spdmm_staged_bytes": [_c_int, _c_i64, ctypes.POINTER(_c_size)],
+    "nm_spdmm_backward_staged": [_c_int, _c_i64, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_size, _c_ptr, _c_i64,
+                                 _c_ptr, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_i64, _c_ptr],
     "nm_sptrsv_plan_bytes": [_c_i64, _c_i64, ctypes.POINTER(_c_size), ctypes.POINTER(_c_size)],
     "nm_sptrsv_analyse": [_c_i64, _c_i64, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_size, _c_ptr, _c_size,
                           ctypes.POINTER(_c_ptr), _c_ptr],

@@ -24,6 +24,7 @@
 //   forward : nnz*(s+8) + (rows+1)*8 + cols*n*s + rows*n*s
 //   backward: nnz*(s+8) + (rows+1)*8 + rows*n*s + cols*n*s + nnz*s + cols*n*s
 #include "nm_common.hpp"
+#include "nm_permute.hpp"
 #include "nm_spmm_groups.hpp"
 #include "nm_transpose.hpp"
 
@@ -831,4 +832,48 @@ extern "C" int nm_spdmm_backward_planned(nm_dtype dt, int64_t rows, int64_t cols
                                               t.t_perm, (const double *)gC, ldg, n, (double *)grad_B, ldgb);
     NM_LAUNCH_CHECK("spdmm_fwd_flat_kernel (transposed)");
     return NM_OK;
+}
+
+extern "C" int nm_spdmm_staged_bytes(nm_dtype dt, int64_t nnz, size_t *bytes) {
+    NM_REQUIRE(dt == NM_F32 || dt == NM_F64, "unknown dtype %d", (int)dt);
+    NM_REQUIRE(bytes && nnz >= 0, "null output or negative size");
+    *bytes = 2 * nm::align256((size_t)nnz * (dt == NM_F32 ? 4 : 8));
+    return NM_OK;
+}
+
+namespace {
+template <typename T>
+int staged_backward(int64_t nnz, const nm::PermutePlan &p, char *work, nm_groups::Args<T, int32_t> a, hipStream_t s) {
+    T *const one = reinterpret_cast<T *>(work), *const two = reinterpret_cast<T *>(work + nm::align256((size_t)nnz * sizeof(T)));
+    T *const grad_A = a.dots;
+    if (int rc = nm::to_columns<T>(p, nnz, a.data, one, two, s)) return rc;
+    a.data = two;
+    a.dots = one;
+    if (!grad_A) return nm_groups::launch<T, int32_t, false, false>(a, s);
+    if (int rc = nm_groups::launch<T, int32_t, false, true>(a, s)) return rc;
+    return nm::to_rows<T>(p, nnz, one, two, grad_A, s);
+}
+}  // namespace
+
+extern "C" int nm_spdmm_backward_staged(nm_dtype dt, int64_t rows, int64_t cols, int64_t nnz, const void *data,
+                                        const void *plan_mem, const void *permute_plan, void *work, size_t work_bytes,
+                                        const void *B, int64_t ldb, const void *gC, int64_t ldg, int64_t n,
+                                        void *grad_A, void *grad_B, int64_t ldgb, nm_stream stream) {
+    NM_REQUIRE(dt == NM_F32 || dt == NM_F64, "unknown dtype %d", (int)dt);
+    NM_REQUIRE(rows > 0 && cols > 0 && nnz > 0, "an empty product");
+    NM_REQUIRE(data && plan_mem && permute_plan && work && gC && grad_B && (!grad_A || B), "null memory");
+    NM_REQUIRE(ldg >= n && ldgb >= n && (!grad_A || ldb >= n), "row stride smaller than the row");
+    NM_REQUIRE(dt == NM_F32 ? nm_groups::takes<float>(rows, ldg, n) : nm_groups::takes<double>(rows, ldg, n),
+               "dense operand of more than 1 KB a row, or a stride beyond 32 bits");
+    size_t need = 0;
+    if (int rc = nm_spdmm_staged_bytes(dt, nnz, &need)) return rc;
+    NM_REQUIRE(work_bytes >= need, "work memory too small");
+    nm::TPlan t;
+    nm::tplan_layout(rows, cols, nnz, const_cast<void *>(plan_mem), &t);
+    nm::PermutePlan p;
+    nm::permute_layout(nnz, const_cast<void *>(permute_plan), &p);
+    hipStream_t s = nm::as_stream(stream);
+    if (dt == NM_F32)
+        return staged_backward<float>(nnz, p, (char *)work, group_args<float>(cols, data, t.t_row, t.t_indptr, nullptr, gC, ldg, n, grad_B, ldgb, B, ldb, grad_A), s);
+    return staged_backward<double>(nnz, p, (char *)work, group_args<double>(cols, data, t.t_row, t.t_indptr, nullptr, gC, ldg, n, grad_B, ldgb, B, ldb, grad_A), s);
 }

@@ -506,12 +506,18 @@ __global__ __launch_bounds__(kBlock) void tp_stats_kernel(int64_t rows, int64_t 
                                                           const int32_t *__restrict__ c_ptr32,
                                                           const int32_t *__restrict__ f_desc,
                                                           const int32_t *__restrict__ b_desc,
-                                                          const int32_t *__restrict__ stats, int32_t *flags) {
-    __shared__ int32_t s_red[6][kBlock / kWave];
+                                                          const int32_t *__restrict__ stats, int64_t nnz,
+                                                          const int32_t *__restrict__ t_perm, int32_t *flags) {
+    constexpr int kFigures = 7;
+    __shared__ int32_t s_red[kFigures][kBlock / kWave];
     const int64_t stride = (int64_t)gridDim.x * kBlock, tid = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     // staged row blocks, staged column blocks, longest column, longest row, heavy, staged row blocks of
-    // at most 3072 entries (what the forward's fp64 tile holds)
-    int v[6] = {0, 0, 0, 0, 0, 0};
+    // at most 3072 entries (what the forward's fp64 tile holds), sampled entries that lie far off
+    int v[kFigures] = {0, 0, 0, 0, 0, 0, 0};
+    for (int64_t i = tid; i < (nnz + nm::kSampled - 1) / nm::kSampled; i += stride) {
+        const int64_t off = t_perm[i * nm::kSampled] - i * nm::kSampled;
+        v[6] += off > nm::kFarOff || off < -nm::kFarOff;
+    }
     for (int64_t b = tid; b < rblocks; b += stride) {
         const bool staged = f_desc[b * nm::kStageDesc] >= 0;
         const int64_t r1 = (b + 1) * nm::kPackRows < rows ? (b + 1) * nm::kPackRows : rows;
@@ -527,19 +533,19 @@ __global__ __launch_bounds__(kBlock) void tp_stats_kernel(int64_t rows, int64_t 
 #pragma unroll
     for (int off = kWave / 2; off > 0; off >>= 1)
 #pragma unroll
-        for (int k = 0; k < 6; ++k) {
+        for (int k = 0; k < kFigures; ++k) {
             const int o = __shfl_xor(v[k], off, kWave);
-            v[k] = (k < 2 || k == 5) ? v[k] + o : max(v[k], o);
+            v[k] = (k < 2 || k >= 5) ? v[k] + o : max(v[k], o);
         }
     if ((threadIdx.x & (kWave - 1)) == 0)
-        for (int k = 0; k < 6; ++k) s_red[k][threadIdx.x / kWave] = v[k];
+        for (int k = 0; k < kFigures; ++k) s_red[k][threadIdx.x / kWave] = v[k];
     __syncthreads();
-    if (threadIdx.x < 6) {
+    if (threadIdx.x < kFigures) {
         const int k = threadIdx.x;
-        const bool sum = k < 2 || k == 5;
+        const bool sum = k < 2 || k >= 5;
         int r = 0;
         for (int w = 0; w < kBlock / kWave; ++w) r = sum ? r + s_red[k][w] : max(r, s_red[k][w]);
-        const int slot = k == 0 ? 4 : k == 1 ? 5 : k == 2 ? 6 : k == 3 ? 7 : k == 4 ? 8 : 9;
+        const int slot = k == 0 ? 4 : k == 1 ? 5 : k == 2 ? 6 : k == 3 ? 7 : k == 4 ? 8 : k == 5 ? 9 : 3;
         if (sum) { if (r) atomicAdd(&flags[slot], r); }
         else if (r) atomicMax(&flags[slot], r);
     }
@@ -634,7 +640,7 @@ int tplan_build(int64_t rows, int64_t cols, int64_t nnz, const int64_t *indices,
         NM_LAUNCH_CHECK("tp_pack_kernel");
         hipLaunchKernelGGL(tp_stats_kernel, dim3(32), dim3(kBlock), 0, s, rows, ceil_div(rows, (int64_t)kPackRows),
                            ceil_div(cols, (int64_t)kPackCols), plan.c_ptr32, plan.f_desc, plan.b_desc, plan.stats,
-                           plan.flags);
+                           nnz, plan.t_perm, plan.flags);
         NM_LAUNCH_CHECK("tp_stats_kernel");
     }
     return NM_OK;

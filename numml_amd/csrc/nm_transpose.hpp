@@ -75,6 +75,10 @@ constexpr int kStageFwdCap = 4096, kStageBwdCap = 2048, kStageBwdMin = 1024;
 constexpr int kStagePlaceBits = 11;
 static_assert(kStageBwd * kStageSeg <= (1 << kStagePlaceBits), "a place fits its field");
 
+// Every kSampled-th entry in column-major order is looked at for flags[3]: is its row-major position more than
+// kFarOff entries away?  (Values that far apart do not meet in the 4 MB L2 of a die.)
+constexpr int kSampled = 64, kFarOff = 1 << 18;
+
 inline size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
 
 // Carves the plan arrays out of `base` (nullptr: size query only); returns bytes.

@@ -189,7 +189,7 @@ struct Alias {
 };
 
 struct Plan {
-    // 'T' transposed structure, 'L' level schedule, 'U' filled pattern of the LU factors,
+    // 'T' transposed structure, 'G' staged order of a pattern's values, 'L' level schedule, 'U' filled pattern of the LU factors,
     // 'P' product plan of A B (key: A's pattern, key2: B's), 'S' maps of a linear combination
     // alpha A + beta B (key: A's pattern, key2: B's)
     char kind;
@@ -477,6 +477,33 @@ std::shared_ptr<Plan> backward_plan(const Tensor &indices, const Tensor &indptr,
     const int mode = backward_mode_now();
     if (mode == kAtomic || !fits_a_plan(rows, cols, indices.numel())) return nullptr;
     return transpose_plan(indices, indptr, rows, cols, dev, mode == kPlanned);
+}
+
+// The plan that brings A's values into column-major order and back (nm_permute_plan_build), where that pays, or
+// nullptr.  It pays where neighbouring entries of a column lie further apart among the values than a cache holds
+// (of every 64th entry the plan of the transposed structure counts those that do; an eighth of them suffices) and
+// the values are more than that.  Graphs with random columns, a step with gradients on either side of the line,
+// without -> with: 0.94 M fp32 entries 147 -> 146 us at 64 dense columns and 137 -> 113 at 16; 0.51 M fp64 112 -> 116;
+// 1.0 M fp32 129 -> 130 at 64; 1.5 M fp32 173 -> 135 at 16; 15.6 M fp32 1597 -> 1373 at 64, 1060 -> 770 at 16, fp64
+// 1602 -> 1425 at 32.  In the default mode the plan is noted at the pattern's first backward on the transposed
+// structure and built at the next (15.6 M entries: 1.4 ms, seven steps' gain).
+constexpr int64_t kScatteredBytes = (int64_t)4 << 20;
+std::shared_ptr<Plan> permute_plan(const std::shared_ptr<Plan> &transposed, const Tensor &indices, const Tensor &indptr,
+                                   int64_t rows, int64_t cols, size_t value_bytes, const c10::Device &dev) {
+    const int64_t nnz = indices.numel();
+    if (rows == 0 || nnz * (int64_t)value_bytes < kScatteredBytes) return nullptr;
+    const bool capturing = c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None;
+    if (capturing) return transposed->info_loaded.load(std::memory_order_acquire) ? peek_plan('G', indices, indptr, rows, cols, dev) : nullptr;
+    if ((int64_t)plan_info(*transposed, rows, cols, nnz, dev)[3] * 64 * 8 < nnz) return nullptr;
+    return cached('G', indices, indptr, rows, cols, backward_mode_now() == kPlanned, dev, [&](Plan &p) {
+        size_t pbytes = 0, wbytes = 0;
+        check(nm_permute_plan_bytes(nnz, &pbytes, &wbytes), "nm_permute_plan_bytes");
+        p.mem = scratch(pbytes, dev);
+        Tensor work = scratch(wbytes, dev);
+        check(nm_permute_plan_build(rows, cols, nnz, transposed->mem.data_ptr(), p.mem.data_ptr(), pbytes,
+                                    work.data_ptr(), wbytes, current_stream(dev)),
+              "nm_permute_plan_build");
+    });
 }
 
 std::shared_ptr<Plan> level_plan(const Tensor &indices, const Tensor &indptr, int64_t rows, bool lower,
@@ -1115,7 +1142,20 @@ std::vector<Tensor> spdmm_backward(int A_rows, int A_cols, Tensor A_data, Tensor
         if (heavy * (want.first ? 1000 : 100) > A_data.numel()) plan = nullptr;
     }
     g_last_spdmm_backward.store(plan ? kOnTransposedPlan : kStateless, std::memory_order_relaxed);
-    if (plan) {
+    const int64_t value_bytes = A_data.element_size();
+    auto staged = plan && n > 0 && n * value_bytes <= 1024 && ldg <= 0x3fffffff / value_bytes
+                      ? permute_plan(plan, A_indices, A_indptr, A_rows, B.size(0), value_bytes, dev)
+                      : nullptr;
+    if (staged) {
+        size_t bytes = 0;
+        check(nm_spdmm_staged_bytes(dtype_of(A_data), A_data.numel(), &bytes), "nm_spdmm_staged_bytes");
+        Tensor work = scratch(bytes, dev);
+        check(nm_spdmm_backward_staged(dtype_of(A_data), A_rows, B.size(0), A_data.numel(), A_data.data_ptr(),
+                                       plan->mem.data_ptr(), staged->mem.data_ptr(), work.data_ptr(), bytes, B.data_ptr(),
+                                       ldb, grad_C.data_ptr(), ldg, n, ptr_or_null(grad_A), ptr_or_null(grad_B),
+                                       std::max<int64_t>(n, 1), current_stream(dev)),
+              "nm_spdmm_backward_staged");
+    } else if (plan) {
         check(nm_spdmm_backward_planned(dtype_of(A_data), A_rows, B.size(0), A_data.numel(), A_data.data_ptr(),
                                         A_indices.data_ptr<int64_t>(), A_indptr.data_ptr<int64_t>(),
                                         plan->mem.data_ptr(), B.data_ptr(), ldb, grad_C.data_ptr(), ldg, n,
