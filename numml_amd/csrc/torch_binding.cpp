@@ -1647,6 +1647,155 @@ std::string backward_mode() {
     return m == kAtomic ? "atomic" : m == kEager ? "eager" : "planned";
 }
 
+// ---- autograd nodes ----------------------------------------------------------------
+//
+// The autograd Functions of numml_amd/sparse/{_csr,linalg}.py once more, as native nodes: the same calls in
+// the same order on the same saved tensors, without Python's Function on the way there and without the
+// interpreter on the way back (256 x 256 five-point SpMV with gradients, two kernels of 5 us: 72 -> 46 us, of which 35 are the engine's hand-over to its device thread).  The
+// Python layer takes them for plain tensors in plain eager mode only; tracing, functorch transforms,
+// forward-mode AD, tensor subclasses and dispatch modes stay with the Python Functions.
+
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+Tensor grad_or_zeros(const Tensor &grad, const Tensor &pattern, const Tensor &like) {
+    return grad.defined() ? grad : torch::zeros(pattern.sizes(), pattern.options().dtype(like.scalar_type()));
+}
+
+struct SpgemvNode : torch::autograd::Function<SpgemvNode> {
+    static Tensor forward(AutogradContext *ctx, int64_t rows, int64_t cols, const Tensor &A, const Tensor &ci, const Tensor &cp,
+                          const Tensor &x) {
+        Tensor y = spgemv_forward((int)rows, (int)cols, A, ci, cp, x);
+        ctx->save_for_backward({x, A, ci, cp});
+        ctx->saved_data["rows"] = rows;
+        ctx->saved_data["cols"] = cols;
+        return y;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grad) {
+        const auto s = ctx->get_saved_variables();
+        auto g = spgemv_backward(grad[0], (int)ctx->saved_data["rows"].toInt(), (int)ctx->saved_data["cols"].toInt(), s[1], s[2],
+                                 s[3], s[0]);
+        return {Tensor(), Tensor(), g[0], Tensor(), Tensor(), g[1]};
+    }
+};
+
+struct SpdmmNode : torch::autograd::Function<SpdmmNode> {
+    static Tensor forward(AutogradContext *ctx, int64_t rows, int64_t cols, const Tensor &A, const Tensor &ci, const Tensor &cp,
+                          const Tensor &B) {
+        ctx->save_for_backward({A, ci, cp, B});
+        ctx->saved_data["rows"] = rows;
+        ctx->saved_data["cols"] = cols;
+        return spdmm_forward((int)rows, (int)cols, A, ci, cp, B);
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grad) {
+        const auto s = ctx->get_saved_variables();
+        auto g = spdmm_backward((int)ctx->saved_data["rows"].toInt(), (int)ctx->saved_data["cols"].toInt(), s[0], s[1], s[2], s[3],
+                                grad[0]);
+        return {Tensor(), Tensor(), g[0], Tensor(), Tensor(), g[1]};
+    }
+};
+
+struct SpgemmNode : torch::autograd::Function<SpgemmNode> {
+    static variable_list forward(AutogradContext *ctx, int64_t rows, int64_t inner, int64_t cols, const Tensor &A, const Tensor &ai,
+                                 const Tensor &ap, const Tensor &B, const Tensor &bi, const Tensor &bp) {
+        variable_list C = spgemm_forward((int)rows, (int)inner, A, ai, ap, (int)inner, (int)cols, B, bi, bp);
+        ctx->save_for_backward({A, ai, ap, B, bi, bp, C[1], C[2]});
+        ctx->saved_data["rows"] = rows;
+        ctx->saved_data["inner"] = inner;
+        ctx->saved_data["cols"] = cols;
+        ctx->mark_non_differentiable({C[1], C[2]});
+        ctx->set_materialize_grads(false);
+        return C;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grad) {
+        const auto s = ctx->get_saved_variables();
+        const int rows = (int)ctx->saved_data["rows"].toInt(), inner = (int)ctx->saved_data["inner"].toInt(),
+                  cols = (int)ctx->saved_data["cols"].toInt();
+        auto g = spgemm_backward(grad_or_zeros(grad[0], s[6], s[0]), s[6], s[7], rows, inner, s[0], s[1], s[2], inner, cols, s[3],
+                                 s[4], s[5]);
+        return {Tensor(), Tensor(), Tensor(), g[0], Tensor(), Tensor(), g[1], Tensor(), Tensor()};
+    }
+};
+
+struct TransposeNode : torch::autograd::Function<TransposeNode> {
+    static variable_list forward(AutogradContext *ctx, int64_t rows, int64_t cols, const Tensor &A, const Tensor &ci, const Tensor &cp) {
+        variable_list t = csr_transpose_forward((int)rows, (int)cols, A, ci, cp);
+        ctx->save_for_backward({t[3]});
+        ctx->saved_data["dtype"] = (int64_t)A.scalar_type();
+        t.pop_back();
+        ctx->mark_non_differentiable({t[1], t[2]});
+        ctx->set_materialize_grads(false);
+        return t;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grad) {
+        const auto s = ctx->get_saved_variables();
+        Tensor g = grad[0];
+        if (!g.defined())
+            g = torch::zeros(s[0].sizes(), s[0].options().dtype((c10::ScalarType)ctx->saved_data["dtype"].toInt()));
+        return {Tensor(), Tensor(), csr_transpose_backward(g, s[0]), Tensor(), Tensor()};
+    }
+};
+
+struct LincombNode : torch::autograd::Function<LincombNode> {
+    static variable_list forward(AutogradContext *ctx, int64_t rows, int64_t cols, const Tensor &alpha, const Tensor &A,
+                                 const Tensor &ai, const Tensor &ap, const Tensor &beta, const Tensor &B, const Tensor &bi,
+                                 const Tensor &bp) {
+        variable_list C = splincomb_forward((int)rows, (int)cols, alpha, A, ai, ap, beta, B, bi, bp);
+        ctx->save_for_backward({alpha, A, ai, ap, beta, B, bi, bp, C[1], C[2]});
+        ctx->saved_data["rows"] = rows;
+        ctx->saved_data["cols"] = cols;
+        ctx->mark_non_differentiable({C[1], C[2]});
+        ctx->set_materialize_grads(false);
+        return C;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grad) {
+        const auto s = ctx->get_saved_variables();
+        auto g = splincomb_backward((int)ctx->saved_data["rows"].toInt(), (int)ctx->saved_data["cols"].toInt(), s[0], s[1], s[2],
+                                    s[3], s[4], s[5], s[6], s[7], grad_or_zeros(grad[0], s[8], s[1]), s[8], s[9]);
+        Tensor g_alpha, g_beta;
+        if (s[0].requires_grad()) g_alpha = s[1].sum().to(s[0].device());
+        if (s[4].requires_grad()) g_beta = s[5].sum().to(s[4].device());
+        return {Tensor(), Tensor(), g_alpha, g[0], Tensor(), Tensor(), g_beta, g[1], Tensor(), Tensor()};
+    }
+};
+
+struct SptrsvNode : torch::autograd::Function<SptrsvNode> {
+    static Tensor forward(AutogradContext *ctx, int64_t rows, const Tensor &A, const Tensor &ci, const Tensor &cp, bool lower,
+                          bool unit, const Tensor &b) {
+        Tensor x = sptrsv_forward((int)rows, (int)rows, A, ci, cp, lower, unit, b);
+        ctx->save_for_backward({A, ci, cp, b, x});
+        ctx->saved_data["rows"] = rows;
+        ctx->saved_data["lower"] = lower;
+        ctx->saved_data["unit"] = unit;
+        return x;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grad) {
+        const auto s = ctx->get_saved_variables();
+        const int rows = (int)ctx->saved_data["rows"].toInt();
+        auto g = sptrsv_backward(grad[0], s[4], rows, rows, s[0], s[1], s[2], ctx->saved_data["lower"].toBool(),
+                                 ctx->saved_data["unit"].toBool(), s[3]);
+        return {Tensor(), g[0], Tensor(), Tensor(), Tensor(), Tensor(), g[1]};
+    }
+};
+
+struct SpsolveNode : torch::autograd::Function<SpsolveNode> {
+    static Tensor forward(AutogradContext *ctx, int64_t rows, const Tensor &A, const Tensor &ci, const Tensor &cp, const Tensor &b) {
+        const int n = (int)rows;
+        const variable_list f = splu(n, n, A, ci, cp);
+        Tensor y = sptrsv_forward(n, n, f[0], f[1], f[2], true, true, b);
+        Tensor x = sptrsv_forward(n, n, f[0], f[1], f[2], false, false, y);
+        ctx->save_for_backward({A, ci, cp, f[3], f[4], f[5], x});
+        ctx->saved_data["rows"] = rows;
+        return x;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grad) {
+        const auto s = ctx->get_saved_variables();
+        const int n = (int)ctx->saved_data["rows"].toInt();
+        auto g = spsolve_backward(grad[0], s[6], n, n, s[3], s[4], s[5], s[0], s[1], s[2]);
+        return {Tensor(), g[0], Tensor(), Tensor(), g[1]};
+    }
+};
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -1675,6 +1824,30 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("csr_row_sum_backward", &csr_row_sum_backward, "CSR row sum backward");
     m.def("csr_extract_diagonal_forward", &csr_extract_diagonal_forward, "CSR extract diagonal forward");
     m.def("csr_extract_diagonal_backward", &csr_extract_diagonal_backward, "CSR extract diagonal backward");
+    // The autograd nodes (what the Python layer's Functions of these names give, for plain tensors).
+    m.def("spgemv_node", [](int rows, int cols, const Tensor &A, const Tensor &ci, const Tensor &cp, const Tensor &x) {
+        return SpgemvNode::apply((int64_t)rows, (int64_t)cols, A, ci, cp, x);
+    });
+    m.def("spdmm_node", [](int rows, int cols, const Tensor &A, const Tensor &ci, const Tensor &cp, const Tensor &B) {
+        return SpdmmNode::apply((int64_t)rows, (int64_t)cols, A, ci, cp, B);
+    });
+    m.def("spgemm_node", [](int rows, int inner, int cols, const Tensor &A, const Tensor &ai, const Tensor &ap, const Tensor &B,
+                            const Tensor &bi, const Tensor &bp) {
+        return SpgemmNode::apply((int64_t)rows, (int64_t)inner, (int64_t)cols, A, ai, ap, B, bi, bp);
+    });
+    m.def("sptranspose_node", [](int rows, int cols, const Tensor &A, const Tensor &ci, const Tensor &cp) {
+        return TransposeNode::apply((int64_t)rows, (int64_t)cols, A, ci, cp);
+    });
+    m.def("splincomb_node", [](int rows, int cols, const Tensor &alpha, const Tensor &A, const Tensor &ai, const Tensor &ap,
+                               const Tensor &beta, const Tensor &B, const Tensor &bi, const Tensor &bp) {
+        return LincombNode::apply((int64_t)rows, (int64_t)cols, alpha, A, ai, ap, beta, B, bi, bp);
+    });
+    m.def("sptrsv_node", [](int rows, const Tensor &A, const Tensor &ci, const Tensor &cp, bool lower, bool unit, const Tensor &b) {
+        return SptrsvNode::apply((int64_t)rows, A, ci, cp, lower, unit, b);
+    });
+    m.def("spsolve_node", [](int rows, const Tensor &A, const Tensor &ci, const Tensor &cp, const Tensor &b) {
+        return SpsolveNode::apply((int64_t)rows, A, ci, cp, b);
+    });
     m.def("sptrsv_schedule", &sptrsv_schedule, "(levels, launches per solve) of a triangular pattern");
     m.def("sptrsv_chain_levels", &sptrsv_chain_levels,
           "levels of the solves with A and with A^T that the single-wavefront chain kernels take");

@@ -23,6 +23,21 @@ __all__ = ["SparseCSRTensor", "coo_to_csr", "eye", "diag", "spgemv", "spgemm", "
            "splincomb", "sptodense", "sprowsum", "spdiag"]
 
 
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+_NODES = hasattr(_ext, "spgemv_node")     # the compiled binding's autograd nodes
+
+
+def _native(first, second):
+    """Whether an operation on these values may go through the compiled binding's autograd node in place of the
+    Function below: plain tensors of one type on one device, in plain eager mode.  Tracing, functorch transforms,
+    forward-mode AD, dispatch and function modes and tensor subclasses see the Function."""
+    return (_NODES and type(first) in _PLAIN and type(second) in _PLAIN and first.dtype is second.dtype
+            and first.is_cuda and first.device == second.device
+            and not torch._C._are_functorch_transforms_active() and torch._C._get_tracing_state() is None
+            and torch.autograd.forward_ad._current_level < 0 and torch._C._len_torch_dispatch_stack() == 0
+            and torch._C._len_torch_function_stack() == 0 and not torch.compiler.is_compiling())
+
+
 def _type_error(kind_a, a, kind_b, b):
     return RuntimeError(f"{kind_a} should be same data type, got {a.type()} and {b.type()}, respectively.")
 
@@ -278,24 +293,35 @@ class SparseCSRTensor(object):
         if self.shape[1] != torch.numel(x):
             raise RuntimeError("Number of columns of tensor must equal number of rows of vector.  "
                                f"Got shapes: {self.shape} and {x.shape}")
-        y = spgemv.apply(self.shape, self.data, self.indices, self.indptr, x.squeeze())
+        flat = x.squeeze()
+        if _native(self.data, flat):
+            y = _ext.spgemv_node(self.shape[0], self.shape[1], self.data, self.indices, self.indptr, flat)
+        else:
+            y = spgemv.apply(self.shape, self.data, self.indices, self.indptr, flat)
         return _unsqueeze_like(y, x)
 
     def spdmm(self, othr):
+        if _native(self.data, othr) and self.shape[1] == othr.shape[0]:
+            return _ext.spdmm_node(self.shape[0], self.shape[1], self.data, self.indices, self.indptr, othr)
         return spdmm.apply(self.shape, self.data, self.indices, self.indptr, othr)
 
     def spspmm(self, othr):
-        C_shape, C_data, C_indices, C_indptr = spgemm.apply(
-            self.shape, self.data, self.indices, self.indptr,
-            othr.shape, othr.data, othr.indices, othr.indptr)
+        if _native(self.data, othr.data) and self.shape[1] == othr.shape[0]:
+            C_shape = (self.shape[0], othr.shape[1])
+            C_data, C_indices, C_indptr = _ext.spgemm_node(
+                self.shape[0], self.shape[1], othr.shape[1], self.data, self.indices, self.indptr,
+                othr.data, othr.indices, othr.indptr)
+        else:
+            C_shape, C_data, C_indices, C_indptr = spgemm.apply(
+                self.shape, self.data, self.indices, self.indptr,
+                othr.shape, othr.data, othr.indices, othr.indptr)
         # The reference re-wraps with clone=True (numml/sparse/_csr.py:685); the three tensors are
         # fresh outputs of the product, so they are adopted as they are (no copy of C).
         return SparseCSRTensor((C_data, C_indices, C_indptr), C_shape, clone=False)
 
     def solve_triangular(self, upper, unit, b):
         from . import linalg
-        return linalg.sptrsv.apply(self.shape, self.data, self.indices, self.indptr,
-                                   not upper, unit, b)
+        return linalg.spsolve_triangular(self, b, not upper, unit)
 
     def __matmul__(self, x):
         if isinstance(x, SparseCSRTensor):
@@ -324,6 +350,10 @@ class SparseCSRTensor(object):
 
     def transpose(self):
         """A^T, computed eagerly as a new CSR matrix (numml/sparse/_csr.py:1074-1087)."""
+        if _native(self.data, self.data):
+            At_data, At_indices, At_indptr = _ext.sptranspose_node(self.shape[0], self.shape[1], self.data, self.indices,
+                                                                   self.indptr)
+            return SparseCSRTensor((At_data, At_indices, At_indptr), tuple(self.shape[::-1]), clone=False)
         At_shape, At_data, At_indices, At_indptr = sptranspose.apply(
             self.shape, self.data, self.indices, self.indptr)
         return SparseCSRTensor((At_data, At_indices, At_indptr), At_shape, clone=False)
@@ -350,8 +380,13 @@ class SparseCSRTensor(object):
         if self.shape != othr.shape:
             raise RuntimeError(f"Incompatible shapes for entrywise {what}, got {self.shape} and "
                                f"{othr.shape}, respectively.")
-        C = splincomb.apply(self.shape, torch.tensor(1.), self.data, self.indices, self.indptr,
-                            torch.tensor(beta), othr.data, othr.indices, othr.indptr)
+        if _native(self.data, othr.data):
+            C = tuple(_ext.splincomb_node(
+                self.shape[0], self.shape[1], torch.tensor(1.), self.data, self.indices, self.indptr,
+                torch.tensor(beta), othr.data, othr.indices, othr.indptr))
+        else:
+            C = splincomb.apply(self.shape, torch.tensor(1.), self.data, self.indices, self.indptr,
+                                torch.tensor(beta), othr.data, othr.indices, othr.indptr)
         return SparseCSRTensor(C, self.shape, clone=False)
 
     def __add__(self, othr):

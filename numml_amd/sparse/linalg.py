@@ -3,6 +3,7 @@ pivoting followed by two triangular solves (numml/sparse/linalg.py:8-137)."""
 import torch
 
 from .._binding import ops as _ext
+from ._csr import _native
 
 __all__ = ["sptrsv", "spsolve_triangular", "splu", "splu_solve", "spsolve_fn", "spsolve"]
 
@@ -37,6 +38,8 @@ class sptrsv(torch.autograd.Function):
 
 def spsolve_triangular(A, b, lower=True, unit_diagonal=False):
     """Solve A x = b for triangular A (numml/sparse/linalg.py:116-137)."""
+    if _native(A.data, b) and A.shape[0] == A.shape[1]:
+        return _ext.sptrsv_node(A.shape[0], A.data, A.indices, A.indptr, lower, unit_diagonal, b)
     return sptrsv.apply(A.shape, A.data, A.indices, A.indptr, lower, unit_diagonal, b)
 
 
@@ -80,4 +83,6 @@ class spsolve_fn(torch.autograd.Function):
 
 def spsolve(A, b):
     """Solve A x = b for a general sparse A (numml/sparse/linalg.py:113-114)."""
+    if _native(A.data, b) and A.shape[0] == A.shape[1]:
+        return _ext.spsolve_node(A.shape[0], A.data, A.indices, A.indptr, b)
     return spsolve_fn.apply(A.shape, A.data, A.indices, A.indptr, b)
