@@ -450,6 +450,29 @@ int nm_spgemm_backward_mapped_wide(nm_dtype dt, int plan_class, int64_t A_rows, 
                                    const int64_t *B_indptr, const void *plan_mem,
                                    void *grad_A, void *grad_B, nm_stream stream);
 
+/* Product plan by lists, for products beyond the records above: 24 bytes for every product of an entry of A with an
+ * entry of B, in the orders in which C, grad_A and grad_B add them up (the serial loops': the same bits).
+ * nm_spgemm_lists_products counts the products (work: (A_nnz + 1) * 8 bytes rounded up to 256, and
+ * A_nnz / 256 + 16 more); nm_spgemm_lists_build makes the plan from the three patterns and the
+ * transposed-structure plan of A, *usable = 0 where one workgroup would have more than 65 536
+ * products.  Both wait for `stream`; the passes do not.  No counterpart in the reference. */
+int nm_spgemm_lists_products(int64_t A_nnz, const int64_t *A_indices, const int64_t *B_indptr,
+                             void *work, size_t work_bytes, int64_t *products, nm_stream stream);
+int nm_spgemm_lists_bytes(int64_t B_rows, int64_t A_nnz, int64_t B_nnz, int64_t C_nnz, int64_t products,
+                          size_t *plan_bytes, size_t *work_bytes);
+int nm_spgemm_lists_build(int64_t A_rows, int64_t B_rows, int64_t A_nnz, int64_t B_nnz, int64_t C_nnz,
+                          int64_t products, const int64_t *A_indices, const int64_t *A_indptr,
+                          const int64_t *B_indices, const int64_t *B_indptr,
+                          const int64_t *C_indices, const int64_t *C_indptr, const void *A_plan_mem,
+                          void *plan_mem, size_t plan_bytes, void *work, size_t work_bytes,
+                          int *usable, nm_stream stream);
+int nm_spgemm_numeric_lists(nm_dtype dt, int64_t A_nnz, int64_t B_nnz, int64_t C_nnz, int64_t products,
+                            const void *A_data, const void *B_data, const void *plan_mem, void *C_data,
+                            nm_stream stream);
+int nm_spgemm_backward_lists(nm_dtype dt, int64_t A_nnz, int64_t B_nnz, int64_t C_nnz, int64_t products,
+                             const void *grad_C, const void *A_data, const void *B_data, const void *plan_mem,
+                             void *grad_A, void *grad_B, nm_stream stream);
+
 /* ---------------------------------------------------------------- SpTRSV
  * Level-scheduled triangular solve.  Stands in for sptrsv_forward /
  * sptrsv_backward (cpp/sparse_csr.hpp:94-105, cpp/sparse_csr_cpu.cpp:652-759).

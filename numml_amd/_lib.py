@@ -74,6 +74,13 @@ _SIGNATURES = {
                                   _c_ptr, _c_ptr, _c_ptr, _c_size, _c_int, _c_ptr, ctypes.POINTER(_c_int), _c_ptr],
     "nm_spgemm_backward_mapped_wide": [_c_int, _c_int, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_ptr,
                                        _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr],
+    "nm_spgemm_lists_products": [_c_i64, _c_ptr, _c_ptr, _c_ptr, _c_size, ctypes.POINTER(_c_i64), _c_ptr],
+    "nm_spgemm_lists_bytes": [_c_i64, _c_i64, _c_i64, _c_i64, _c_i64, ctypes.POINTER(_c_size), ctypes.POINTER(_c_size)],
+    "nm_spgemm_lists_build": [_c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr,
+                              _c_ptr, _c_ptr, _c_ptr, _c_size, _c_ptr, _c_size, ctypes.POINTER(_c_int), _c_ptr],
+    "nm_spgemm_numeric_lists": [_c_int, _c_i64, _c_i64, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr],
+    "nm_spgemm_backward_lists": [_c_int, _c_i64, _c_i64, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr,
+                                 _c_ptr],
     "nm_permute_plan_bytes": [_c_i64, ctypes.POINTER(_c_size), ctypes.POINTER(_c_size)],
     "nm_permute_plan_build": [_c_i64, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_size, _c_ptr, _c_size, _c_ptr],
     "nm_spdmm_staged_bytes": [_c_int, _c_i64, ctypes.POINTER(_c_size)],

@@ -201,6 +201,7 @@ struct Plan {
     std::vector<uint32_t> derived_versions;  //      and their version counters when built
     bool usable = true;                      // 'P': false when the product is beyond the plan's limits
     int plan_class = 1;                      // 'P': which forward kernel the product takes (nm_spgemm_plan_build)
+    int64_t products = 0;                    // 'P' by lists: products of an entry of A with one of B
     std::shared_ptr<Plan> parent;            // 'P': the transposed-structure plan of A it walks
     nm_sptrsv_plan *handle = nullptr;
     // 'T': what the build found out about the pattern (nm_csr_transpose_plan_info), read back
@@ -567,6 +568,34 @@ std::shared_ptr<Plan> peek_product_plan(const Tensor &A_indices, const Tensor &A
     return plan;
 }
 
+// A product beyond the records: the plan that lists its products (nm_spgemm_lists_build), where its 24 bytes a
+// product are at most a quarter of the cache.  Returns the plan's class, 0 where there is none.
+constexpr int kListClass = 100;
+int list_plan(Plan &plan, const Tensor &A_indices, const Tensor &A_indptr, const Tensor &B_indices, const Tensor &B_indptr,
+              const Tensor &C_indices, const Tensor &C_indptr, int64_t A_rows, int64_t A_cols, const c10::Device &dev) {
+    const int64_t A_nnz = A_indices.numel(), B_nnz = B_indices.numel(), C_nnz = C_indices.numel();
+    const nm_stream stream = current_stream(dev);
+    size_t pbytes = 0, wbytes = ((size_t)A_nnz + 33) * 8 + (size_t)A_nnz / 256 + 4096;
+    Tensor work = scratch(wbytes, dev);
+    int64_t products = 0;
+    check(nm_spgemm_lists_products(A_nnz, A_indices.data_ptr<int64_t>(), B_indptr.data_ptr<int64_t>(), work.data_ptr(),
+                                   wbytes, &products, stream),
+          "nm_spgemm_lists_products");
+    if (products <= 0 || products >= ((int64_t)1 << 31) - 2) return 0;
+    check(nm_spgemm_lists_bytes(A_cols, A_nnz, B_nnz, C_nnz, products, &pbytes, &wbytes), "nm_spgemm_lists_bytes");
+    if (pbytes > g_plan_bytes_limit.load(std::memory_order_relaxed) / 4) return 0;
+    plan.mem = scratch(pbytes, dev);
+    work = scratch(wbytes, dev);
+    int usable = 0;
+    check(nm_spgemm_lists_build(A_rows, A_cols, A_nnz, B_nnz, C_nnz, products, A_indices.data_ptr<int64_t>(),
+                                A_indptr.data_ptr<int64_t>(), B_indices.data_ptr<int64_t>(), B_indptr.data_ptr<int64_t>(),
+                                C_indices.data_ptr<int64_t>(), C_indptr.data_ptr<int64_t>(), plan.parent->mem.data_ptr(),
+                                plan.mem.data_ptr(), pbytes, work.data_ptr(), wbytes, &usable, stream),
+          "nm_spgemm_lists_build");
+    plan.products = products;
+    return usable ? kListClass : 0;
+}
+
 // After a stateless forward pass of a product without hash-path rows: notes the pair, or makes
 // its plan around the pattern of C that the pass has just produced.  `filled`: plan memory that
 // the pass filled as it went (nm_spgemm_symbolic_mapped / nm_spgemm_numeric_mapped), which only
@@ -641,6 +670,7 @@ void consider_product_plan(const Tensor &A_indices, const Tensor &A_indptr, cons
                   "nm_spgemm_plan_build_wide");
         }
     }
+    if (usable <= 0) usable = list_plan(*plan, A_indices, A_indptr, B_indices, B_indptr, C_indices, C_indptr, A_rows, A_cols, dev);
     plan->usable = usable > 0;
     plan->plan_class = usable > 0 ? usable : 0;
     if (plan->usable) {
@@ -1192,6 +1222,13 @@ std::vector<Tensor> spgemm_forward(int A_rows, int A_cols, Tensor A_data, Tensor
     auto on_plan = [&](const Plan &plan) -> std::vector<Tensor> {
         const Tensor &C_indices = plan.derived[0], &C_indptr = plan.derived[1];
         Tensor C_data = torch::empty({C_indices.numel()}, A_data.options());
+        if (plan.plan_class == kListClass) {
+            check(nm_spgemm_numeric_lists(dtype_of(A_data), A_data.numel(), B_data.numel(), C_indices.numel(), plan.products,
+                                          A_data.data_ptr(), B_data.data_ptr(), plan.mem.data_ptr(), C_data.data_ptr(),
+                                          current_stream(dev)),
+                  "nm_spgemm_numeric_lists");
+            return {C_data, C_indices, C_indptr};
+        }
         check(nm_spgemm_numeric_planned(dtype_of(A_data), plan.plan_class, A_rows, A_data.numel(), B_data.numel(),
                                         C_indices.numel(),
                                         A_data.data_ptr(), A_indptr.data_ptr<int64_t>(), B_data.data_ptr(),
@@ -1296,6 +1333,13 @@ std::vector<Tensor> spgemm_backward(Tensor grad_C, Tensor C_indices, Tensor C_in
         if (pp && pp->usable && pp->derived[0].data_ptr() == C_indices.data_ptr() &&
             pp->derived[1].data_ptr() == C_indptr.data_ptr() && pp->derived[0].numel() == C_indices.numel()) {
             g_last_spgemm_backward.store(kOnProductPlan, std::memory_order_relaxed);
+            if (pp->plan_class == kListClass) {
+                check(nm_spgemm_backward_lists(dtype_of(A_data), A_data.numel(), B_data.numel(), grad_C.numel(), pp->products,
+                                               grad_C.data_ptr(), A_data.data_ptr(), B_data.data_ptr(), pp->mem.data_ptr(),
+                                               ptr_or_null(grad_A), ptr_or_null(grad_B), current_stream(dev)),
+                      "nm_spgemm_backward_lists");
+                return {grad_A, grad_B};
+            }
             check(nm_spgemm_backward_mapped_wide(dtype_of(A_data), pp->plan_class, A_rows, A_cols, A_data.numel(),
                                                  B_data.numel(), grad_C.numel(), grad_C.data_ptr(),
                                                  A_data.data_ptr(), pp->parent->mem.data_ptr(), B_data.data_ptr(),
