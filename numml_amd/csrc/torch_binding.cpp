@@ -568,6 +568,18 @@ std::shared_ptr<Plan> peek_product_plan(const Tensor &A_indices, const Tensor &A
     return plan;
 }
 
+// Whether a usable product plan for patterns of these sizes is cached.
+bool product_plan_of_sizes(const Tensor &A_indices, const Tensor &A_indptr, const Tensor &B_indices, const Tensor &B_indptr,
+                           int64_t A_rows, int64_t B_cols) {
+    std::lock_guard<std::mutex> lock(g_plans_mutex);
+    for (const auto &p : g_plans)
+        if (p->kind == 'P' && p->usable && p->a == A_rows && p->b == B_cols && p->key.nnz == A_indices.numel() &&
+            p->key.nptr == A_indptr.numel() && p->key2.nnz == B_indices.numel() && p->key2.nptr == B_indptr.numel() &&
+            p->key.device == A_indices.device().index())
+            return true;
+    return false;
+}
+
 // A product beyond the records: the plan that lists its products (nm_spgemm_lists_build), where its 24 bytes a
 // product are at most a quarter of the cache.  Returns the plan's class, 0 where there is none.
 constexpr int kListClass = 100;
@@ -1238,7 +1250,10 @@ std::vector<Tensor> spgemm_forward(int A_rows, int A_cols, Tensor A_data, Tensor
         return {C_data, C_indices, C_indptr};
     };
     if (plans) {
-        auto plan = peek_product_plan(A_indices, A_indptr, B_indices, B_indptr, A_rows, B_cols, dev);
+        // A content key for patterns in tensors not seen before (a clone, a product computed again) where a plan
+        // of the same sizes exists: it may be theirs, and the symbolic phase is several times the key's pass
+        const bool likely = product_plan_of_sizes(A_indices, A_indptr, B_indices, B_indptr, A_rows, B_cols);
+        auto plan = peek_product_plan(A_indices, A_indptr, B_indices, B_indptr, A_rows, B_cols, dev, likely);
         if (plan && plan->usable) return on_plan(*plan);
     }
     size_t bytes = 0;
@@ -1275,12 +1290,6 @@ std::vector<Tensor> spgemm_forward(int A_rows, int A_cols, Tensor A_data, Tensor
     check(nm_spgemm_symbolic_result(A_rows, B_cols, work.data_ptr(), bytes, &nnz_c, &hash_rows, host_landing(),
                                     st),
           "nm_spgemm_symbolic_result");
-    if (plans && nnz_c > 0) {
-        // a product plan may exist: worth a content key per pattern that arrives in tensors not
-        // seen before (a clone, a product computed again), which may find the pair's plan
-        auto plan = peek_product_plan(A_indices, A_indptr, B_indices, B_indptr, A_rows, B_cols, dev, true);
-        if (plan && plan->usable) return on_plan(*plan);
-    }
     Tensor C_indices = torch::empty({nnz_c}, iopt);
     Tensor C_data = torch::empty({nnz_c}, A_data.options());
     const bool on_map = filled.defined() && hash_rows == 0 && nnz_c > 0 && nnz_c < lim31;
