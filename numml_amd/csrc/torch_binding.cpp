@@ -568,12 +568,12 @@ std::shared_ptr<Plan> peek_product_plan(const Tensor &A_indices, const Tensor &A
     return plan;
 }
 
-// Whether a usable product plan for patterns of these sizes is cached.
-bool product_plan_of_sizes(const Tensor &A_indices, const Tensor &A_indptr, const Tensor &B_indices, const Tensor &B_indptr,
-                           int64_t A_rows, int64_t B_cols) {
+// Whether a usable plan for a product ('P') or a sum ('S') of patterns of these sizes is cached.
+bool plan_of_sizes(char kind, const Tensor &A_indices, const Tensor &A_indptr, const Tensor &B_indices, const Tensor &B_indptr,
+                   int64_t A_rows, int64_t B_cols) {
     std::lock_guard<std::mutex> lock(g_plans_mutex);
     for (const auto &p : g_plans)
-        if (p->kind == 'P' && p->usable && p->a == A_rows && p->b == B_cols && p->key.nnz == A_indices.numel() &&
+        if (p->kind == kind && p->usable && p->a == A_rows && p->b == B_cols && p->key.nnz == A_indices.numel() &&
             p->key.nptr == A_indptr.numel() && p->key2.nnz == B_indices.numel() && p->key2.nptr == B_indptr.numel() &&
             p->key.device == A_indices.device().index())
             return true;
@@ -863,8 +863,9 @@ std::vector<Tensor> spgemv_backward(Tensor grad_z, int A_rows, int A_cols, Tenso
 
 // ----------------------------------------------------------------------- transpose
 
-std::vector<Tensor> csr_transpose_forward(int A_rows, int A_columns, Tensor A_data, Tensor A_indices,
-                                          Tensor A_indptr) {
+// {At_data, At_indices, At_indptr, At_to_A}, or with the plan's memory in place of At_to_A.
+std::vector<Tensor> transpose_values(int A_rows, int A_columns, Tensor A_data, Tensor A_indices, Tensor A_indptr,
+                                     bool want_map) {
     check_csr("csr_transpose_forward", A_rows, A_columns, A_data, A_indices, A_indptr);
     const auto dev = need_device({&A_data, &A_indices, &A_indptr});
     A_data = A_data.contiguous();
@@ -877,10 +878,10 @@ std::vector<Tensor> csr_transpose_forward(int A_rows, int A_columns, Tensor A_da
     Tensor At_data = torch::empty_like(A_data);
     Tensor At_indices = torch::empty({nnz}, iopt);
     Tensor At_indptr = torch::empty({(int64_t)A_columns + 1}, iopt);
-    Tensor At_to_A = torch::empty({nnz}, iopt);
+    Tensor At_to_A = want_map ? torch::empty({nnz}, iopt) : plan->mem;
     check(nm_csr_transpose_forward(dtype_of(A_data), A_rows, A_columns, nnz, A_data.data_ptr(),
                                    plan->mem.data_ptr(), At_data.data_ptr(), At_indices.data_ptr<int64_t>(),
-                                   At_indptr.data_ptr<int64_t>(), At_to_A.data_ptr<int64_t>(),
+                                   At_indptr.data_ptr<int64_t>(), want_map ? At_to_A.data_ptr<int64_t>() : nullptr,
                                    current_stream(dev)),
           "nm_csr_transpose_forward");
     // A sum or a product with the transpose has fresh structure tensors on every call, and would merge the
@@ -906,6 +907,11 @@ std::vector<Tensor> csr_transpose_forward(int A_rows, int A_columns, Tensor A_da
         }
     }
     return {At_data, At_indices, At_indptr, At_to_A};
+}
+
+std::vector<Tensor> csr_transpose_forward(int A_rows, int A_columns, Tensor A_data, Tensor A_indices,
+                                          Tensor A_indptr) {
+    return transpose_values(A_rows, A_columns, A_data, A_indices, A_indptr, true);
 }
 
 Tensor csr_transpose_backward(Tensor grad_At, Tensor At_to_A_idx) {
@@ -942,9 +948,10 @@ std::vector<Tensor> splincomb_forward(int rows, int cols, Tensor alpha, Tensor A
     const double a = alpha.item<double>(), b = beta.item<double>();
     c10::hip::HIPGuard guard(dev.index());
     if (backward_mode_now() != kAtomic) {
-        // patterns seen before (alias lookup only): one pass over the cached maps; the result shares
-        // the plan's pattern tensors, as a planned product does
-        if (auto plan = peek_product_plan(A_indices, A_indptr, B_indices, B_indptr, rows, cols, dev, false, 'S')) {
+        // patterns seen before (tensors not seen before get a content key where a plan of the same sizes
+        // exists): one pass over the cached maps; the result shares the plan's pattern tensors, as a planned product does
+        const bool likely = plan_of_sizes('S', A_indices, A_indptr, B_indices, B_indptr, rows, cols);
+        if (auto plan = peek_product_plan(A_indices, A_indptr, B_indices, B_indptr, rows, cols, dev, likely, 'S')) {
             Tensor C_data = torch::empty({plan->derived[0].numel()}, A_data.options());
             check(nm_splincomb_numeric_planned(dtype_of(A_data), A_indices.numel(), B_indices.numel(), C_data.numel(),
                                                a, A_data.data_ptr(), b, B_data.data_ptr(), plan->mem.data_ptr(),
@@ -1252,7 +1259,7 @@ std::vector<Tensor> spgemm_forward(int A_rows, int A_cols, Tensor A_data, Tensor
     if (plans) {
         // A content key for patterns in tensors not seen before (a clone, a product computed again) where a plan
         // of the same sizes exists: it may be theirs, and the symbolic phase is several times the key's pass
-        const bool likely = product_plan_of_sizes(A_indices, A_indptr, B_indices, B_indptr, A_rows, B_cols);
+        const bool likely = plan_of_sizes('P', A_indices, A_indptr, B_indices, B_indptr, A_rows, B_cols);
         auto plan = peek_product_plan(A_indices, A_indptr, B_indices, B_indptr, A_rows, B_cols, dev, likely);
         if (plan && plan->usable) return on_plan(*plan);
     }
@@ -1770,10 +1777,14 @@ struct SpgemmNode : torch::autograd::Function<SpgemmNode> {
     }
 };
 
+// (keeps the plan's memory, which the cache may drop meanwhile, instead of a permutation of 8 bytes an entry)
 struct TransposeNode : torch::autograd::Function<TransposeNode> {
     static variable_list forward(AutogradContext *ctx, int64_t rows, int64_t cols, const Tensor &A, const Tensor &ci, const Tensor &cp) {
-        variable_list t = csr_transpose_forward((int)rows, (int)cols, A, ci, cp);
+        variable_list t = transpose_values((int)rows, (int)cols, A, ci, cp, false);
         ctx->save_for_backward({t[3]});
+        ctx->saved_data["rows"] = rows;
+        ctx->saved_data["cols"] = cols;
+        ctx->saved_data["nnz"] = A.numel();
         ctx->saved_data["dtype"] = (int64_t)A.scalar_type();
         t.pop_back();
         ctx->mark_non_differentiable({t[1], t[2]});
@@ -1781,11 +1792,20 @@ struct TransposeNode : torch::autograd::Function<TransposeNode> {
         return t;
     }
     static variable_list backward(AutogradContext *ctx, variable_list grad) {
-        const auto s = ctx->get_saved_variables();
-        Tensor g = grad[0];
-        if (!g.defined())
-            g = torch::zeros(s[0].sizes(), s[0].options().dtype((c10::ScalarType)ctx->saved_data["dtype"].toInt()));
-        return {Tensor(), Tensor(), csr_transpose_backward(g, s[0]), Tensor(), Tensor()};
+        const Tensor plan = ctx->get_saved_variables()[0];
+        const int64_t nnz = ctx->saved_data["nnz"].toInt();
+        const auto dtype = (c10::ScalarType)ctx->saved_data["dtype"].toInt();
+        c10::hip::HIPGuard guard(plan.device().index());
+        Tensor grad_A = torch::empty({nnz}, plan.options().dtype(dtype));
+        if (!grad[0].defined()) return {Tensor(), Tensor(), grad_A.zero_(), Tensor(), Tensor()};
+        check_vector("csr_transpose_backward", "grad_At", grad[0], nnz);
+        same_dtype(grad_A, grad[0], "grad_At");
+        const Tensor g = grad[0].contiguous();
+        const auto dev = need_device({&g, &plan});
+        check(nm_csr_transpose_backward_planned(dtype_of(g), ctx->saved_data["rows"].toInt(), ctx->saved_data["cols"].toInt(), nnz,
+                                                g.data_ptr(), plan.data_ptr(), grad_A.data_ptr(), current_stream(dev)),
+              "nm_csr_transpose_backward_planned");
+        return {Tensor(), Tensor(), grad_A, Tensor(), Tensor()};
     }
 };
 
