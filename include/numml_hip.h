@@ -177,6 +177,18 @@ int nm_spgemv_forward_planned_lists(nm_dtype dt, int64_t rows, int64_t cols, int
                                     const void *data, const void *plan_mem,
                                     const void *x, void *y, nm_stream stream);
 
+/* The part of the transposed-structure plan that these two read, by itself (6 bytes an entry, two passes over the
+ * structure): for patterns that are multiplied again and again and never walked by column.  info as in
+ * nm_csr_transpose_plan_info ([2], [4], [7], [9]; the build waits for `stream` to hand it over);
+ * `lists` != 0: the instantiation for blocks with a staging list.  An empty matrix is refused.  No
+ * counterpart in the reference. */
+int nm_spgemv_rows_plan_bytes(int64_t rows, int64_t cols, int64_t nnz, size_t *plan_bytes);
+int nm_spgemv_rows_plan_build(int64_t rows, int64_t cols, int64_t nnz, const int64_t *indices,
+                              const int64_t *indptr, void *plan_mem, size_t plan_bytes, int32_t info[16],
+                              nm_stream stream);
+int nm_spgemv_forward_rows(nm_dtype dt, int lists, int64_t rows, int64_t cols, int64_t nnz, const void *data,
+                           const void *plan_mem, const void *x, void *y, nm_stream stream);
+
 /* nm_spgemv_backward on a transposed-structure plan: walks A by column, so
  * grad_x needs neither clearing nor atomics, is summed in ascending row order
  * (the order of cpp/sparse_csr_cpu.cpp:68-73) and is identical on every run.

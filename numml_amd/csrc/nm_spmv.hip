@@ -1279,33 +1279,73 @@ extern "C" int nm_spgemv_forward(nm_dtype dt, int64_t rows, int64_t cols, int64_
 }
 
 namespace {
-template <bool LISTS>
-int forward_planned(nm_dtype dt, int64_t rows, int64_t cols, int64_t nnz, const void *data, const void *plan_mem,
-                    const void *x, void *y, nm_stream stream) {
+int forward_planned(nm_dtype dt, bool lists, int64_t rows, int64_t cols, int64_t nnz, const void *data, const nm::TPlan &t,
+                    const void *x, void *y, hipStream_t s) {
     NM_REQUIRE(dt == NM_F32 || dt == NM_F64, "unknown dtype %d", (int)dt);
-    NM_REQUIRE(rows >= 0 && cols >= 0 && nnz >= 0 && plan_mem != nullptr, "bad sizes or null plan");
-    if (rows == 0) return NM_OK;
     NM_REQUIRE(y != nullptr && (nnz == 0 || data != nullptr), "null pointer argument");
     NM_REQUIRE(cols == 0 || x != nullptr, "x is null");
+    auto launch = [&](auto *one, auto with_lists) {
+        using T = std::remove_pointer_t<decltype(one)>;
+        return launch_fwd<T, int32_t, with_lists()>(rows, nnz, (const T *)data, t.c_idx32, t.c_ptr32, (const T *)x, (T *)y, s,
+                                                    t.c_off16, t.flags, nnz > 0 ? t.f_desc : nullptr);
+    };
+    if (dt == NM_F32) return lists ? launch((float *)nullptr, std::true_type{}) : launch((float *)nullptr, std::false_type{});
+    return lists ? launch((double *)nullptr, std::true_type{}) : launch((double *)nullptr, std::false_type{});
+}
+
+int forward_on_transpose_plan(nm_dtype dt, bool lists, int64_t rows, int64_t cols, int64_t nnz, const void *data,
+                              const void *plan_mem, const void *x, void *y, nm_stream stream) {
+    NM_REQUIRE(rows >= 0 && cols >= 0 && nnz >= 0 && plan_mem != nullptr, "bad sizes or null plan");
+    NM_REQUIRE(dt == NM_F32 || dt == NM_F64, "unknown dtype %d", (int)dt);
+    if (rows == 0) return NM_OK;
     nm::TPlan t;
     nm::tplan_layout(rows, cols, nnz, const_cast<void *>(plan_mem), &t);
-    hipStream_t s = nm::as_stream(stream);
-    if (dt == NM_F32)
-        return launch_fwd<float, int32_t, LISTS>(rows, nnz, (const float *)data, t.c_idx32, t.c_ptr32, (const float *)x,
-                                                 (float *)y, s, t.c_off16, t.flags, nnz > 0 ? t.f_desc : nullptr);
-    return launch_fwd<double, int32_t, LISTS>(rows, nnz, (const double *)data, t.c_idx32, t.c_ptr32, (const double *)x,
-                                              (double *)y, s, t.c_off16, t.flags, nnz > 0 ? t.f_desc : nullptr);
+    return forward_planned(dt, lists, rows, cols, nnz, data, t, x, y, nm::as_stream(stream));
+}
+
+bool fits_rows_plan(int64_t rows, int64_t cols, int64_t nnz) {
+    return rows >= 0 && cols >= 0 && nnz >= 0 && rows < 0x7ffffffe && cols < 0x7ffffffe && nnz < 0x7ffffffe;
 }
 }  // namespace
 
 extern "C" int nm_spgemv_forward_planned(nm_dtype dt, int64_t rows, int64_t cols, int64_t nnz, const void *data,
                                          const void *plan_mem, const void *x, void *y, nm_stream stream) {
-    return forward_planned<false>(dt, rows, cols, nnz, data, plan_mem, x, y, stream);
+    return forward_on_transpose_plan(dt, false, rows, cols, nnz, data, plan_mem, x, y, stream);
 }
 
 extern "C" int nm_spgemv_forward_planned_lists(nm_dtype dt, int64_t rows, int64_t cols, int64_t nnz, const void *data,
                                                const void *plan_mem, const void *x, void *y, nm_stream stream) {
-    return forward_planned<true>(dt, rows, cols, nnz, data, plan_mem, x, y, stream);
+    return forward_on_transpose_plan(dt, true, rows, cols, nnz, data, plan_mem, x, y, stream);
+}
+
+extern "C" int nm_spgemv_rows_plan_bytes(int64_t rows, int64_t cols, int64_t nnz, size_t *plan_bytes) {
+    NM_REQUIRE(plan_bytes != nullptr, "null output");
+    if (!fits_rows_plan(rows, cols, nnz)) return nm::fail(NM_ERR_UNSUPPORTED, "plans index with 32 bits");
+    *plan_bytes = nm::rows_plan_layout(rows, nnz, nullptr, nullptr);
+    return NM_OK;
+}
+
+extern "C" int nm_spgemv_rows_plan_build(int64_t rows, int64_t cols, int64_t nnz, const int64_t *indices, const int64_t *indptr,
+                                         void *plan_mem, size_t plan_bytes, int32_t info[16], nm_stream stream) {
+    size_t need = 0;
+    if (int rc = nm_spgemv_rows_plan_bytes(rows, cols, nnz, &need)) return rc;
+    NM_REQUIRE(rows > 0 && nnz > 0, "an empty matrix");
+    NM_REQUIRE(indices && indptr && plan_mem && info && plan_bytes >= need, "null pointer argument or plan memory too small");
+    hipStream_t s = nm::as_stream(stream);
+    nm::TPlan t;
+    nm::rows_plan_layout(rows, nnz, plan_mem, &t);
+    if (int rc = nm::rows_plan_build(rows, cols, nnz, indices, indptr, t, s)) return rc;
+    NM_HIP_TRY(hipMemcpyAsync(info, t.flags, 16 * sizeof(int32_t), hipMemcpyDeviceToHost, s));
+    NM_HIP_TRY(hipStreamSynchronize(s));
+    return NM_OK;
+}
+
+extern "C" int nm_spgemv_forward_rows(nm_dtype dt, int lists, int64_t rows, int64_t cols, int64_t nnz, const void *data,
+                                      const void *plan_mem, const void *x, void *y, nm_stream stream) {
+    NM_REQUIRE(fits_rows_plan(rows, cols, nnz) && rows > 0 && nnz > 0 && plan_mem != nullptr, "bad sizes or null plan");
+    nm::TPlan t;
+    nm::rows_plan_layout(rows, nnz, const_cast<void *>(plan_mem), &t);
+    return forward_planned(dt, lists != 0, rows, cols, nnz, data, t, x, y, nm::as_stream(stream));
 }
 
 extern "C" int nm_csr_row_sum_forward(nm_dtype dt, int64_t rows, int64_t nnz, const void *data,

@@ -414,15 +414,15 @@ __device__ __forceinline__ int32_t stage_place(const StageTable &t, int32_t k) {
 
 // t_pack, c_off16 and the staging lists of the plan; clears flags[1] / flags[2] when a difference
 // does not fit 16 bits and counts the blocks that got a list in flags[4] (rows) / flags[5] (columns).
-// A workgroup takes blocks of kPackCols columns, then blocks of kPackRows rows, lane = entry.
+// A workgroup takes blocks of kPackCols columns (cblocks: all of them, or 0 where there is no transposed
+// structure), then blocks of kPackRows rows, lane = entry.
 __global__ __launch_bounds__(kBlock) void tp_pack_kernel(
-    int64_t rows, int64_t cols, const int32_t *__restrict__ t_indptr, const int32_t *__restrict__ t_row,
+    int64_t rows, int64_t cols, int64_t cblocks, const int32_t *__restrict__ t_indptr, const int32_t *__restrict__ t_row,
     const int32_t *__restrict__ t_perm, const int32_t *__restrict__ c_ptr32, const int32_t *__restrict__ c_idx32,
     int32_t *__restrict__ t_pack, int16_t *__restrict__ c_off16, int32_t *__restrict__ f_desc,
     int32_t *__restrict__ b_desc, int32_t *__restrict__ stats, int32_t *flags) {
     __shared__ StageTable table;
     bool fits_t = true, fits_c = true;
-    const int64_t cblocks = (cols + nm::kPackCols - 1) / nm::kPackCols;
     for (int64_t b = blockIdx.x; b < cblocks; b += gridDim.x) {
         const int64_t c0 = b * nm::kPackCols;
         const int64_t c1 = c0 + nm::kPackCols < cols ? c0 + nm::kPackCols : cols;
@@ -634,8 +634,8 @@ int tplan_build(int64_t rows, int64_t cols, int64_t nnz, const int64_t *indices,
     if (nnz > 0) {
         int64_t grid = ceil_div(cols > rows ? cols : rows, (int64_t)kPackCols);
         if (grid > 65536) grid = 65536;
-        hipLaunchKernelGGL(tp_pack_kernel, dim3((unsigned)grid), dim3(kBlock), 0, s, rows, cols, plan.t_indptr,
-                           plan.t_row, plan.t_perm, plan.c_ptr32, plan.c_idx32, plan.t_pack, plan.c_off16, plan.f_desc,
+        hipLaunchKernelGGL(tp_pack_kernel, dim3((unsigned)grid), dim3(kBlock), 0, s, rows, cols,
+                           ceil_div(cols, (int64_t)kPackCols), plan.t_indptr, plan.t_row, plan.t_perm, plan.c_ptr32, plan.c_idx32, plan.t_pack, plan.c_off16, plan.f_desc,
                            plan.b_desc, plan.stats, plan.flags);
         NM_LAUNCH_CHECK("tp_pack_kernel");
         hipLaunchKernelGGL(tp_stats_kernel, dim3(32), dim3(kBlock), 0, s, rows, ceil_div(rows, (int64_t)kPackRows),
@@ -643,6 +643,36 @@ int tplan_build(int64_t rows, int64_t cols, int64_t nnz, const int64_t *indices,
                            nnz, plan.t_perm, plan.flags);
         NM_LAUNCH_CHECK("tp_stats_kernel");
     }
+    return NM_OK;
+}
+
+namespace {
+__global__ __launch_bounds__(kBlock) void narrow_kernel(int64_t nnz, int64_t rows, const int64_t *__restrict__ indices,
+                                                        const int64_t *__restrict__ indptr, int32_t *__restrict__ idx,
+                                                        int32_t *__restrict__ ptr) {
+    const int64_t stride = (int64_t)gridDim.x * kBlock, tid = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    for (int64_t k = tid; k < nnz; k += stride) idx[k] = (int32_t)stream_load(indices + k);
+    for (int64_t r = tid; r <= rows; r += stride) ptr[r] = (int32_t)indptr[r];
+}
+}  // namespace
+
+int rows_plan_build(int64_t rows, int64_t cols, int64_t nnz, const int64_t *indices, const int64_t *indptr, const TPlan &plan,
+                    hipStream_t s) {
+    int64_t grid = ceil_div(nnz > rows + 1 ? nnz : rows + 1, (int64_t)kBlock * 4);
+    if (grid > 65536) grid = 65536;
+    hipLaunchKernelGGL(narrow_kernel, dim3((unsigned)grid), dim3(kBlock), 0, s, nnz, rows, indices, indptr, plan.c_idx32, plan.c_ptr32);
+    hipLaunchKernelGGL(symmetry_init_kernel, dim3(1), dim3(64), 0, s, plan.flags, 0);
+    NM_LAUNCH_CHECK("narrow_kernel");
+    grid = ceil_div(rows, (int64_t)kPackRows);
+    if (grid > 65536) grid = 65536;
+    hipLaunchKernelGGL(tp_pack_kernel, dim3((unsigned)grid), dim3(kBlock), 0, s, rows, cols, (int64_t)0, (const int32_t *)nullptr,
+                       (const int32_t *)nullptr, (const int32_t *)nullptr, plan.c_ptr32, plan.c_idx32, (int32_t *)nullptr,
+                       plan.c_off16, plan.f_desc, (int32_t *)nullptr, plan.stats, plan.flags);
+    NM_LAUNCH_CHECK("tp_pack_kernel");
+    hipLaunchKernelGGL(tp_stats_kernel, dim3(32), dim3(kBlock), 0, s, rows, ceil_div(rows, (int64_t)kPackRows), (int64_t)0,
+                       plan.c_ptr32, plan.f_desc, (const int32_t *)nullptr, plan.stats, (int64_t)0, (const int32_t *)nullptr,
+                       plan.flags);
+    NM_LAUNCH_CHECK("tp_stats_kernel");
     return NM_OK;
 }
 

@@ -105,6 +105,29 @@ inline size_t tplan_layout(int64_t rows, int64_t cols, int64_t nnz, void *base, 
     return off;
 }
 
+// The part of the plan that a walk by row reads (c_ptr32, c_idx32, c_off16, f_desc, flags) by itself, for
+// patterns that are only multiplied from the left: 6 bytes an entry and two passes.
+inline size_t rows_plan_layout(int64_t rows, int64_t nnz, void *base, TPlan *p) {
+    size_t off = 0;
+    auto take = [&](size_t bytes) {
+        void *q = base ? static_cast<char *>(base) + off : nullptr;
+        off += align256(bytes);
+        return q;
+    };
+    const size_t blocks = (size_t)((rows + kPackRows - 1) / kPackRows);
+    TPlan t{};
+    t.flags = (int32_t *)take(16 * 4);
+    t.c_ptr32 = (int32_t *)take((size_t)(rows + 2) * 4);
+    t.c_idx32 = (int32_t *)take((size_t)(nnz + 1) * 4);
+    t.c_off16 = (int16_t *)take((size_t)(nnz + 8) * 2);
+    t.f_desc = (int32_t *)take((blocks + 1) * kStageDesc * 4);
+    t.stats = (int32_t *)take((blocks * 4 + 8) * 4);
+    if (p) *p = t;
+    return off;
+}
+int rows_plan_build(int64_t rows, int64_t cols, int64_t nnz, const int64_t *indices, const int64_t *indptr, const TPlan &plan,
+                    hipStream_t s);
+
 // Scratch bytes tplan_build needs.
 size_t tplan_work_bytes(int64_t rows, int64_t cols, int64_t nnz);
 
