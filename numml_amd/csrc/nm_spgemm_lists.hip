@@ -12,8 +12,8 @@
 // so that each pass is one kernel without a merge, a hash table, a search or an atomic, and the serial loops'
 // bits.  24 bytes a product; the pattern of C is the caller's.  What bounds them: the requests for the factors that lie
 // scattered, one line each from beyond L2 for gC in grad_B.  Power-law graph of 150 000 rows squared (10.1 M
-// products, fp32): forward 781 -> 56 us (the hash path and its symbolic phase before), with gradients 1326 -> 318;
-// 50 000 rows, 5 entries a row, fp64: 445 -> 17, 600 -> 81.  Making the plan takes 2 ms of the former, 0.4 of the latter.
+// products, fp32): forward 781 -> 56 us (the hash path and its symbolic phase before), with gradients 1326 -> 230;
+// 50 000 rows, 5 entries a row, fp64: 445 -> 17, 600 -> 62.  Making the plan takes 2 ms of the former, 0.4 of the latter.
 //
 // The plan is refused where a workgroup would have more than kBusiest products (hub columns that meet long rows): its
 // segments are added up by one lane each.
@@ -236,7 +236,17 @@ __global__ __launch_bounds__(kBlock) void segments_kernel(int64_t segments, List
 #pragma unroll
         for (int i = 0; i < L; ++i) {
             const int stop = (e[i] < base + n ? e[i] : base + n) - base;
-            for (int p = (b[i] > base ? b[i] : base) - base; p < stop; ++p) acc[i] += s_p[p];
+            int p = (b[i] > base ? b[i] : base) - base;
+            // (eight reads under way at a time: a wavefront's lanes wait for the longest segment among theirs; 145 ->
+            // 59 us for grad_A of the power-law graph)
+            for (; p + 8 <= stop; p += 8) {
+                T term[8];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) term[k] = s_p[p + k];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) acc[i] += term[k];
+            }
+            for (; p < stop; ++p) acc[i] += s_p[p];
         }
         __syncthreads();
     }
