@@ -120,6 +120,25 @@ __device__ __forceinline__ int run_end(const int32_t *s_off, int s0, int nr, int
     return lo;
 }
 
+// The products [b, e) of a row in LDS, added one after the other by one lane.  A workgroup waits for the longest
+// row of its tile, and a row read one product after the other is a trip to LDS each (~100 cycles): sixteen are
+// under way at a time.  Power-law graphs in fp32,
+// forward: 100 000 rows, 1.2 M entries 53 -> 22 us; 20 000 rows of up to 5000 entries 63 -> 15.5; 400 000 rows,
+// 7.6 M entries 121 -> 90.  Grids, whose rows are shorter than sixteen, as before.
+template <typename T> __device__ __forceinline__ T serial_sum(const T *s_prod, int b, int e) {
+    T acc = 0;
+    constexpr int U = 16;
+    for (; b + U <= e; b += U) {
+        T term[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) term[u] = s_prod[b + u];
+#pragma unroll
+        for (int u = 0; u < U; ++u) acc += term[u];
+    }
+    for (; b < e; ++b) acc += s_prod[b];
+    return acc;
+}
+
 // Element idx of an array.  O32: the array is smaller than 4 GiB, so the address is the base (in
 // scalar registers) plus a 32-bit byte offset (one vector register instead of two per access).
 template <bool O32, typename X>
@@ -391,10 +410,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_num_sgpr(72))) void sp
             }
             __syncthreads();
             for (int t = threadIdx.x; t < nr; t += BLOCK) {
-                const int e = s_off[t + 1];
-                T acc = 0;
-                for (int j = s_off[t]; j < e; ++j) acc += s_prod[j];
-                nm::stream_store(y + r0 + t, acc);
+                nm::stream_store(y + r0 + t, serial_sum(s_prod, s_off[t], s_off[t + 1]));
             }
         } else if (n <= CAP) {
             const T *__restrict__ d = data + base;
@@ -461,10 +477,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_num_sgpr(72))) void sp
             }
             __syncthreads();
             for (int t = threadIdx.x; t < nr; t += BLOCK) {
-                const int e = s_off[t + 1];
-                T acc = 0;
-                for (int j = s_off[t]; j < e; ++j) acc += s_prod[j];
-                nm::stream_store(y + r0 + t, acc);
+                nm::stream_store(y + r0 + t, serial_sum(s_prod, s_off[t], s_off[t + 1]));
             }
         } else if (n < kHuge) {
             // The block's entries do not fit the tile: runs of consecutive rows that do are taken
