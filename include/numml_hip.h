@@ -212,6 +212,13 @@ int nm_spgemv_backward_planned_lists(nm_dtype dt, int64_t rows, int64_t cols, in
                                      const void *data, const void *plan_mem,
                                      const void *x, const void *g,
                                      void *grad_A, void *grad_x, nm_stream stream);
+/* nm_spgemv_backward_planned for scattered columns: the products g[row] * data[k] are made by rows, brought into
+ * column-major order by a plan of nm_permute_plan_build (work: nm_spgemv_staged_bytes) and summed by columns.  grad_x is
+ * always computed, grad_A may be null.  Nothing waits.  No counterpart in the reference. */
+int nm_spgemv_staged_bytes(nm_dtype dt, int64_t nnz, size_t *bytes);
+int nm_spgemv_backward_staged(nm_dtype dt, int64_t rows, int64_t cols, int64_t nnz, const void *data,
+                              const void *transpose_plan, const void *permute_plan, void *work, size_t work_bytes,
+                              const void *x, const void *g, void *grad_A, void *grad_x, nm_stream stream);
 
 /* Test hook (no counterpart in the reference): `wide_offsets` = 1 makes
  * nm_spgemv_backward_planned(_lists) address its arrays with 64-bit offsets whatever

@@ -87,6 +87,9 @@ _SIGNATURES = {
     "nm_spgemv_forward_rows": [_c_int, _c_int, _c_i64, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr],
     "nm_permute_plan_bytes": [_c_i64, ctypes.POINTER(_c_size), ctypes.POINTER(_c_size)],
     "nm_permute_plan_build": [_c_i64, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_size, _c_ptr, _c_size, _c_ptr],
+    "nm_spgemv_staged_bytes": [_c_int, _c_i64, ctypes.POINTER(_c_size)],
+    "nm_spgemv_backward_staged": [_c_int, _c_i64, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_size, _c_ptr, _c_ptr,
+                                  _c_ptr, _c_ptr, _c_ptr],
     "nm_spdmm_staged_bytes": [_c_int, _c_i64, ctypes.POINTER(_c_size)],
     "nm_spdmm_backward_staged": [_c_int, _c_i64, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_size, _c_ptr, _c_i64,
                                  _c_ptr, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_i64, _c_ptr],

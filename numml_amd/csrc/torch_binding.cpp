@@ -555,16 +555,17 @@ std::shared_ptr<Plan> backward_plan(const Tensor &indices, const Tensor &indptr,
 // The plan that brings A's values into column-major order and back (nm_permute_plan_build), where that pays, or
 // nullptr.  It pays where neighbouring entries of a column lie further apart among the values than a cache holds
 // (of every 64th entry the plan of the transposed structure counts those that do; an eighth of them suffices) and
-// the values are more than that.  Graphs with random columns, a step with gradients on either side of the line,
+// the entries are `fewest` at least (products with vectors: kStagedBoth, kStagedOne; with dense matrices values of
+// kScatteredBytes).  Graphs with random columns, a step with gradients on either side of the latter line,
 // without -> with: 0.94 M fp32 entries 147 -> 146 us at 64 dense columns and 137 -> 113 at 16; 0.51 M fp64 112 -> 116;
 // 1.0 M fp32 129 -> 130 at 64; 1.5 M fp32 173 -> 135 at 16; 15.6 M fp32 1597 -> 1373 at 64, 1060 -> 770 at 16, fp64
 // 1602 -> 1425 at 32.  In the default mode the plan is noted at the pattern's first backward on the transposed
 // structure and built at the next (15.6 M entries: 1.4 ms, seven steps' gain).
 constexpr int64_t kScatteredBytes = (int64_t)4 << 20;
 std::shared_ptr<Plan> permute_plan(const std::shared_ptr<Plan> &transposed, const Tensor &indices, const Tensor &indptr,
-                                   int64_t rows, int64_t cols, size_t value_bytes, const c10::Device &dev) {
+                                   int64_t rows, int64_t cols, int64_t fewest, const c10::Device &dev) {
     const int64_t nnz = indices.numel();
-    if (rows == 0 || nnz * (int64_t)value_bytes < kScatteredBytes) return nullptr;
+    if (rows == 0 || nnz < fewest) return nullptr;
     const bool capturing = c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None;
     if (capturing) return transposed->info_loaded.load(std::memory_order_acquire) ? peek_plan('G', indices, indptr, rows, cols, dev) : nullptr;
     if ((int64_t)plan_info(*transposed, rows, cols, nnz, dev)[3] * 64 * 8 < nnz) return nullptr;
@@ -904,6 +905,14 @@ Tensor spgemv_forward(int A_rows, int A_cols, Tensor A_data, Tensor A_col_ind, T
     return y;
 }
 
+// Entries from which scattered values go through column-major order (permute_plan), both gradients or grad_x alone (the
+// gradient of A alone is made by rows).  Graphs with random columns, on the plan's kernel -> through the order, us:
+//   both        fp32  1.1 M 40.7 -> 29.8   1.2 M 40.3 -> 31.0   2.1 M 75 -> 43   3.8 M 150 -> 77    7.6 M 304 -> 121
+//               fp64  0.6 M 27.6 -> 28.9   0.8 M 33.2 -> 33.4   1.0 M 41.5 -> 36.3   2.1 M 84 -> 59   7.6 M 320 -> 200
+//   grad_x      fp32  1.1 M 22.3 -> 24.3   1.2 M 22.2 -> 26.0   2.1 M 34.8 -> 30.8   3.8 M 66 -> 51   7.6 M 137 -> 88
+//               fp64  1.0 M 20.9 -> 30.0   1.2 M 25.3 -> 32.6   2.1 M 44.5 -> 41.4   3.8 M 77 -> 72   7.6 M 173 -> 130
+constexpr int64_t kStagedBoth = 900 << 10, kStagedOne = 1536 << 10;
+
 std::vector<Tensor> spgemv_backward(Tensor grad_z, int A_rows, int A_cols, Tensor A_data, Tensor A_col_ind,
                                     Tensor A_rowptr, Tensor x) {
     check_csr("spgemv_backward", A_rows, A_cols, A_data, A_col_ind, A_rowptr);
@@ -926,6 +935,19 @@ std::vector<Tensor> spgemv_backward(Tensor grad_z, int A_rows, int A_cols, Tenso
         // most blocks of 256 columns have a staging list: the instantiation that stages g and x in LDS
         const int32_t *info = plan_info(*plan, A_rows, x.size(0), A_data.numel(), dev);
         const bool lists = 2 * (int64_t)info[5] >= ((int64_t)x.size(0) + 255) / 256;
+        auto staged = want.second && !lists ? permute_plan(plan, A_col_ind, A_rowptr, A_rows, x.size(0),
+                                                           want.first ? kStagedBoth : kStagedOne, dev)
+                                            : nullptr;
+        if (staged) {
+            size_t bytes = 0;
+            check(nm_spgemv_staged_bytes(dtype_of(A_data), A_data.numel(), &bytes), "nm_spgemv_staged_bytes");
+            Tensor work = scratch(bytes, dev);
+            check(nm_spgemv_backward_staged(dtype_of(A_data), A_rows, x.size(0), A_data.numel(), A_data.data_ptr(),
+                                            plan->mem.data_ptr(), staged->mem.data_ptr(), work.data_ptr(), bytes, x.data_ptr(),
+                                            grad_z.data_ptr(), ptr_or_null(grad_A), ptr_or_null(grad_x), current_stream(dev)),
+                  "nm_spgemv_backward_staged");
+            return {grad_A, grad_x};
+        }
         check((lists ? nm_spgemv_backward_planned_lists : nm_spgemv_backward_planned)(
                   dtype_of(A_data), A_rows, x.size(0), A_data.numel(), A_data.data_ptr(), plan->mem.data_ptr(),
                   x.data_ptr(), grad_z.data_ptr(), ptr_or_null(grad_A), ptr_or_null(grad_x), current_stream(dev)),
@@ -1271,7 +1293,7 @@ std::vector<Tensor> spdmm_backward(int A_rows, int A_cols, Tensor A_data, Tensor
     g_last_spdmm_backward.store(plan ? kOnTransposedPlan : kStateless, std::memory_order_relaxed);
     const int64_t value_bytes = A_data.element_size();
     auto staged = plan && n > 0 && n * value_bytes <= 1024 && ldg <= 0x3fffffff / value_bytes
-                      ? permute_plan(plan, A_indices, A_indptr, A_rows, B.size(0), value_bytes, dev)
+                      ? permute_plan(plan, A_indices, A_indptr, A_rows, B.size(0), kScatteredBytes / value_bytes, dev)
                       : nullptr;
     if (staged) {
         size_t bytes = 0;
