@@ -133,23 +133,49 @@ __device__ __forceinline__ int run_end(const int32_t *s_off, int s0, int nr, int
     return lo;
 }
 
-// The products [b, e) of a row in LDS, added one after the other by one lane.  A workgroup waits for the longest
-// row of its tile, and a row read one product after the other is a trip to LDS each (~100 cycles): sixteen are
-// under way at a time.  Power-law graphs in fp32,
-// forward: 100 000 rows, 1.2 M entries 53 -> 22 us; 20 000 rows of up to 5000 entries 63 -> 15.5; 400 000 rows,
-// 7.6 M entries 121 -> 90.  Grids, whose rows are shorter than sixteen, as before.
+// The products [b, e) of a row in LDS, added one after the other by one lane.  A row read one product after the
+// other is a trip to LDS each (~100 cycles): sixteen are under way at a time, then four.
 template <typename T> __device__ __forceinline__ T serial_sum(const T *s_prod, int b, int e) {
     T acc = 0;
-    constexpr int U = 16;
-    for (; b + U <= e; b += U) {
-        T term[U];
+    auto add = [&](auto count) {
+        constexpr int U = count();
+        for (; b + U <= e; b += U) {
+            T term[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) term[u] = s_prod[b + u];
+            for (int u = 0; u < U; ++u) term[u] = s_prod[b + u];
 #pragma unroll
-        for (int u = 0; u < U; ++u) acc += term[u];
-    }
-    for (; b < e; ++b) acc += s_prod[b];
+            for (int u = 0; u < U; ++u) acc += term[u];
+        }
+    };
+    add(std::integral_constant<int, 16>{});
+    add(std::integral_constant<int, 4>{});
+    add(std::integral_constant<int, 1>{});
     return acc;
+}
+
+// Rows [s0, e0) of a tile whose products lie in LDS from s_off[s0] - o0 on: one lane a row in storage order, and rows of
+// kLongRow products by a wavefront, lane l adding products l, l + 64, ... before the lanes are summed.  A workgroup
+// waits for the longest row of its tile.  Forward, graphs in fp32, a lane for every row and a trip to LDS for every
+// product -> sixteen at a time -> this, with small tiles (launch_fwd): 100 000 rows, 1.2 M entries 53 -> 22 -> 15.6 us;
+// 20 000 rows of up to 5000 entries 63 -> 15.5 -> 5.5; 400 000 rows, 7.6 M entries 122 -> 90 -> 68.  (A line at 64 or
+// 128: the same within 3 %.  The error of a long row's sum against 64 bits is smaller in this order: 6.13e-8 -> 5.98e-8 over
+// 30 000 rows of 26.)
+template <typename T, int BLOCK>
+__device__ __forceinline__ void row_sums(const T *s_prod, const int32_t *s_off, int s0, int e0, int o0, T *__restrict__ y) {
+    for (int tb = s0; tb < e0; tb += BLOCK) {
+        const int t = tb + (int)threadIdx.x, lane = threadIdx.x & (kWave - 1);
+        const int b = t < e0 ? s_off[t] - o0 : 0, e = t < e0 ? s_off[t + 1] - o0 : 0;
+        const bool wide = e - b >= kLongRow;
+        if (t < e0 && !wide) nm::stream_store(y + t, serial_sum(s_prod, b, e));
+        for (unsigned long long todo = __ballot(wide); todo; todo &= todo - 1) {
+            const int src = __builtin_ctzll(todo);
+            const int wb = __shfl(b, src, kWave), we = __shfl(e, src, kWave);
+            T acc = 0;
+            for (int j = wb + lane; j < we; j += kWave) acc += s_prod[j];
+            acc = nm::wave_sum(acc);
+            if (lane == 0) y[t + src] = acc;
+        }
+    }
 }
 
 // Element idx of an array.  O32: the array is smaller than 4 GiB, so the address is the base (in
@@ -422,9 +448,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_num_sgpr(72))) void sp
                 }
             }
             __syncthreads();
-            for (int t = threadIdx.x; t < nr; t += BLOCK) {
-                nm::stream_store(y + r0 + t, serial_sum(s_prod, s_off[t], s_off[t + 1]));
-            }
+            row_sums<T, BLOCK>(s_prod, s_off, 0, nr, 0, y + r0);
         } else if (n <= CAP) {
             const T *__restrict__ d = data + base;
             const IDX *__restrict__ ci = indices + base;
@@ -489,14 +513,10 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_num_sgpr(72))) void sp
                 }
             }
             __syncthreads();
-            for (int t = threadIdx.x; t < nr; t += BLOCK) {
-                nm::stream_store(y + r0 + t, serial_sum(s_prod, s_off[t], s_off[t + 1]));
-            }
+            row_sums<T, BLOCK>(s_prod, s_off, 0, nr, 0, y + r0);
         } else if (n < kHuge) {
             // The block's entries do not fit the tile: runs of consecutive rows that do are taken
-            // one after the other.  Rows shorter than kLongRow are added by one lane in storage
-            // order as above; longer ones by a wavefront, lane l adding entries l, l + 64, ...
-            // of the row before the lanes are summed.
+            // one after the other.
             auto products = [&](int64_t first, int cnt) {   // s_prod[j] = data * x of entry first + j
                 const T *__restrict__ d = data + first;
                 const IDX *__restrict__ ci = indices + first;
@@ -543,24 +563,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_num_sgpr(72))) void sp
                 const int o0 = s_off[s0];
                 products(base + o0, s_off[e0] - o0);
                 __syncthreads();
-                for (int tb = s0; tb < e0; tb += BLOCK) {
-                    const int t = tb + threadIdx.x;
-                    const int b = t < e0 ? s_off[t] - o0 : 0, e = t < e0 ? s_off[t + 1] - o0 : 0;
-                    const bool wide = e - b >= kLongRow;
-                    if (t < e0 && !wide) {
-                        T acc = 0;
-                        for (int j = b; j < e; ++j) acc += s_prod[j];
-                        nm::stream_store(y + r0 + t, acc);
-                    }
-                    for (unsigned long long todo = __ballot(wide); todo; todo &= todo - 1) {
-                        const int src = __builtin_ctzll(todo);
-                        const int wb = __shfl(b, src, kWave), we = __shfl(e, src, kWave);
-                        T acc = 0;
-                        for (int j = wb + lane; j < we; j += kWave) acc += s_prod[j];
-                        acc = nm::wave_sum(acc);
-                        if (lane == 0) y[r0 + tb + wave * kWave + src] = acc;
-                    }
-                }
+                row_sums<T, BLOCK>(s_prod, s_off, s0, e0, o0, y + r0);
                 __syncthreads();
                 s0 = e0;
             }
@@ -1259,7 +1262,14 @@ int launch_fwd(int64_t rows, int64_t nnz, const T *data, const IDX *indices, con
     // workgroups in fp64 whether the tile has 3072 or 4096 products: it takes the whole 4096, so
     // that blocks of 512 rows with seven entries a row stay blocks of 512 rows)
     constexpr int R = kFwdR, CAP = LISTS ? NM_FWD_CAP : kFwdCap<T>;
-    const int rt = block_rows(rows, nnz, R, CAP);
+    // Long rows: tiles of about 1024 products (of 2048 or 4096, fp32 graphs of 200 000 rows, 20 entries each on average
+    // 45 -> 56, 63 us; of 100 000 and 12, 15.6 -> 17.8, 22).  Short ones: a tile of 512 rows reads the plan's packed
+    // columns; without a plan at least 512 tiles (60 x 55 x 50 seven-point fp64 7.7 -> 5.9 us, with 1024 6.9; 30 x 35 x 30
+    // 6.2 -> 4.4, with 1024 5.6).
+    const bool long_rows = nnz > 8 * rows;
+    int rt = block_rows(rows, nnz, R, long_rows ? 1024 : CAP);
+    if (long_rows || sizeof(IDX) == 8)
+        while (rt > 16 && rows < (int64_t)rt * 512) rt /= 2;
     int64_t grid = nm::xcd_padded(nm::ceil_div(rows, rt));
     if (grid > nm::kMaxGrid) grid = nm::kMaxGrid;
     hipLaunchKernelGGL((spmv_fwd_kernel<T, kFwdBlock, R, CAP, false, IDX, LISTS>), dim3((unsigned)grid), dim3(kFwdBlock), 0, s,

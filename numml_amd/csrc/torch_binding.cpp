@@ -487,8 +487,9 @@ constexpr size_t kSeenTableSize = 64;
 constexpr int kProductsBeforePlan = 3;
 constexpr int64_t kRowsPlanEntries = 1 << 20;
 // Where blocks have no staging lists and columns do not fit 16 bits the plan only halves the indices of a product that
-// waits for its gathers: fp64 graph of 1.2 M entries 44.5 -> 47 us, of 7.6 M 107 -> 101 (fp32 53 -> 52 and 122 -> 111).
-constexpr int64_t kScatteredEntries = 4 << 20;
+// waits for its gathers: graphs of 1.2 M entries fp32 15.7 -> 13.3 us, fp64 16.8 -> 15.5 (not made), of 3.9 M 35.1 -> 29.5 and
+// 40.0 -> 34.6, of 7.6 M 68.6 -> 59.2 and 76.5 -> 68.3.
+constexpr int64_t kScatteredEntries = 2 << 20;
 std::list<Seen> g_seen;   // most recently seen first
 
 // How often products of this pair of structure tensors have been seen, this time included.
