@@ -134,7 +134,8 @@ __device__ __forceinline__ int run_end(const int32_t *s_off, int s0, int nr, int
 }
 
 // The products [b, e) of a row in LDS, added one after the other by one lane.  A row read one product after the
-// other is a trip to LDS each (~100 cycles): sixteen are under way at a time, then four.
+// other is a trip to LDS each (~100 cycles): four are under way at a time (sixteen or eight: the same within 2 %, rows
+// of kLongRow being shared).
 template <typename T> __device__ __forceinline__ T serial_sum(const T *s_prod, int b, int e) {
     T acc = 0;
     auto add = [&](auto count) {
@@ -147,34 +148,56 @@ template <typename T> __device__ __forceinline__ T serial_sum(const T *s_prod, i
             for (int u = 0; u < U; ++u) acc += term[u];
         }
     };
-    add(std::integral_constant<int, 16>{});
     add(std::integral_constant<int, 4>{});
     add(std::integral_constant<int, 1>{});
     return acc;
 }
 
-// Rows [s0, e0) of a tile whose products lie in LDS from s_off[s0] - o0 on: one lane a row in storage order, and rows of
-// kLongRow products by a wavefront, lane l adding products l, l + 64, ... before the lanes are summed.  A workgroup
-// waits for the longest row of its tile.  Forward, graphs in fp32, a lane for every row and a trip to LDS for every
-// product -> sixteen at a time -> this, with small tiles (launch_fwd): 100 000 rows, 1.2 M entries 53 -> 22 -> 15.6 us;
-// 20 000 rows of up to 5000 entries 63 -> 15.5 -> 5.5; 400 000 rows, 7.6 M entries 122 -> 90 -> 68.  (A line at 64 or
-// 128: the same within 3 %.  The error of a long row's sum against 64 bits is smaller in this order: 6.13e-8 -> 5.98e-8 over
-// 30 000 rows of 26.)
+// Sums of a wavefront's slices [b, e) of the products in LDS, one a lane, left at out[t] where `on` (t ascends with the
+// lanes; a slice is empty where it is not on): by the lane in storage order, and slices of kLongRow products by the
+// wavefront, lane l adding products l, l + 64, ... before the lanes are summed.  A workgroup waits for the longest row
+// of its tile.  Forward, graphs in fp32, a lane for every row and a trip to LDS for every product -> this, with small
+// tiles (launch_fwd): 100 000 rows, 1.2 M entries 53 -> 15.7 us; 20 000 rows of up to 5000 entries 63 -> 5.5; 400 000 rows,
+// 7.6 M entries 122 -> 68.  (A line at 64 or 128: the same within 3 %.  The error of a long row's sum against 64 bits is
+// smaller in this order: 6.13e-8 -> 5.98e-8 over 30 000 rows of 26.)
+template <bool STREAM, typename T>
+__device__ __forceinline__ void slice_sums(const T *s_prod, int b, int e, bool on, T *__restrict__ out, int t) {
+    const int lane = threadIdx.x & (kWave - 1);
+    const bool wide = e - b >= kLongRow;
+    if (on && !wide) {
+        if constexpr (STREAM) nm::stream_store(out + t, serial_sum(s_prod, b, e));
+        else out[t] = serial_sum(s_prod, b, e);
+    }
+    for (unsigned long long todo = __ballot(wide); todo; todo &= todo - 1) {
+        const int src = __builtin_ctzll(todo);
+        const int wb = __shfl(b, src, kWave), we = __shfl(e, src, kWave);
+        T acc = 0;
+        for (int j = wb + lane; j < we; j += kWave) acc += s_prod[j];
+        acc = nm::wave_sum(acc);
+        if (lane == 0) out[t + src] = acc;
+    }
+}
+
+// Rows [s0, e0) of a tile whose products lie in LDS from s_off[s0] - o0 on.
 template <typename T, int BLOCK>
 __device__ __forceinline__ void row_sums(const T *s_prod, const int32_t *s_off, int s0, int e0, int o0, T *__restrict__ y) {
     for (int tb = s0; tb < e0; tb += BLOCK) {
-        const int t = tb + (int)threadIdx.x, lane = threadIdx.x & (kWave - 1);
-        const int b = t < e0 ? s_off[t] - o0 : 0, e = t < e0 ? s_off[t + 1] - o0 : 0;
-        const bool wide = e - b >= kLongRow;
-        if (t < e0 && !wide) nm::stream_store(y + t, serial_sum(s_prod, b, e));
-        for (unsigned long long todo = __ballot(wide); todo; todo &= todo - 1) {
-            const int src = __builtin_ctzll(todo);
-            const int wb = __shfl(b, src, kWave), we = __shfl(e, src, kWave);
-            T acc = 0;
-            for (int j = wb + lane; j < we; j += kWave) acc += s_prod[j];
-            acc = nm::wave_sum(acc);
-            if (lane == 0) y[t + src] = acc;
-        }
+        const int t = tb + (int)threadIdx.x;
+        slice_sums<true>(s_prod, t < e0 ? s_off[t] - o0 : 0, t < e0 ? s_off[t + 1] - o0 : 0, t < e0, y, t);
+    }
+}
+
+// One value for the places [b, e) of a wavefront's slices of LDS, one slice a lane; long ones by the wavefront.
+template <typename T> __device__ __forceinline__ void slice_fill(T *s_v, int b, int e, T v) {
+    const int lane = threadIdx.x & (kWave - 1);
+    const bool wide = e - b >= kLongRow;
+    if (!wide)
+        for (int j = b; j < e; ++j) s_v[j] = v;
+    for (unsigned long long todo = __ballot(wide); todo; todo &= todo - 1) {
+        const int src = __builtin_ctzll(todo);
+        const int wb = __shfl(b, src, kWave), we = __shfl(e, src, kWave);
+        const T wv = __shfl(v, src, kWave);
+        for (int j = wb + lane; j < we; j += kWave) s_v[j] = wv;
     }
 }
 
@@ -637,15 +660,7 @@ __global__ __launch_bounds__(kBlock) void spmv_bwd_kernel(
                 const int t = tb + threadIdx.x;
                 const int jb = t < e0 ? s_off[t] - o0 : 0, je = t < e0 ? s_off[t + 1] - o0 : 0;
                 const T av = t < e0 ? a[r0 + t] : T(0);
-                const bool wide = je - jb >= kLongRow;
-                if (!wide)
-                    for (int j = jb; j < je; ++j) s_a[j] = av;
-                for (unsigned long long todo = __ballot(wide); todo; todo &= todo - 1) {
-                    const int src = __builtin_ctzll(todo);
-                    const int wb = __shfl(jb, src, kWave), we = __shfl(je, src, kWave);
-                    const T wv = __shfl(av, src, kWave);
-                    for (int j = wb + lane; j < we; j += kWave) s_a[j] = wv;
-                }
+                slice_fill(s_a, jb, je, av);
             }
         };
         // `cnt` entries from `first` on, whose factors are s_a[0, cnt): four consecutive entries a lane, unless their
@@ -836,11 +851,7 @@ __device__ __forceinline__ void bwd_tile_staged(const int64_t c0, const int nc, 
     }
     __syncthreads();
     // grad_x[column] = sum of the column's slice in ascending row order
-    if (tid < nc) {
-        T acc = 0;
-        for (int j = pa - base; j < pb - base; ++j) acc += s_v[j];
-        grad_x[c0 + tid] = acc;
-    }
+    slice_sums<false>(s_v, pa - base, pb - base, tid < nc, grad_x + c0, tid);
 }
 
 // Backward over the transposed-structure plan (columns of A as rows of A^T):
@@ -868,7 +879,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? (LISTS ? 6 : 8) : (LISTS ? 3
     int64_t cols, const T *__restrict__ data, const int32_t *__restrict__ t_indptr,
     const int32_t *__restrict__ t_row, const int32_t *__restrict__ t_perm, const int32_t *__restrict__ t_pack,
     const int32_t *__restrict__ flags, const T *__restrict__ x, const T *__restrict__ g,
-    T *__restrict__ grad_A, T *__restrict__ grad_x, const int32_t *__restrict__ b_desc) {
+    T *__restrict__ grad_A, T *__restrict__ grad_x, const int32_t *__restrict__ b_desc, int width) {
     static_assert(R == nm::kPackCols, "t_pack holds rows relative to the first column of a workgroup's block");
     static_assert(nm::kStageBwdCap <= CAP, "a block with a staging list fits the tile");
     constexpr bool STAGE = LISTS && NM_STAGE_BWD != 0;
@@ -884,7 +895,8 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? (LISTS ? 6 : 8) : (LISTS ? 3
     // one packed word per entry in place of (t_row, t_perm): patterns near the diagonal
     const bool packed_plan = flags[1] != 0;
     static_assert(R == kBlock, "lane t of a workgroup stages column t of its block");
-    const int64_t ntiles = (cols + R - 1) / R, npad = nm::xcd_padded(ntiles);
+    const int rt = LISTS ? R : width;   // divides R
+    const int64_t ntiles = (cols + rt - 1) / rt, npad = nm::xcd_padded(ntiles);
     const bool fused = mirror && grad_A;
     // the factor a column's entries share: g[column] (symmetric pattern: the lane writes the mirror
     // entry) or x[column]
@@ -893,11 +905,12 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? (LISTS ? 6 : 8) : (LISTS ? 3
     for (int64_t id = blockIdx.x; id < npad; id += gridDim.x) {
         const int64_t tile = nm::xcd_tile_reversed(id, npad);
         if (tile >= ntiles) continue;
-        const int64_t c0 = tile * R;
-        const int nc = (int)(cols - c0 < R ? cols - c0 : R);
+        const int64_t c0 = tile * rt;
+        const int nc = (int)(cols - c0 < rt ? cols - c0 : rt);
+        const int32_t block0 = (int32_t)c0 & ~(R - 1);     // what packed rows are relative to
         bool packed = packed_plan;
         // (the low half of a packed word of a block with a list is a place in the listed segments)
-        if constexpr (!STAGE) if (packed_plan && b_desc != nullptr) packed = b_desc[tile * nm::kStageDesc] < 0;
+        if constexpr (!STAGE) if (packed_plan && b_desc != nullptr) packed = b_desc[c0 / R * nm::kStageDesc] < 0;
         if constexpr (STAGE) if (fused && packed && b_desc != nullptr) {
             // a block of columns with a staging list, both gradients: the tile's ends, the head of
             // its list and the wavefront's four places of the list come together (scalar loads);
@@ -978,8 +991,6 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? (LISTS ? 6 : 8) : (LISTS ? 3
         const int n = s_off[nc] - base;
 
         // s_v[j] = own[column] for the entries j of columns [s0, e0); o0 = offset of column s0.
-        // WHOLE (the tile fits): one lane per column.  Otherwise columns of kLongRow entries
-        // or more are spread by a wavefront.
         auto spread = [&](auto whole, const T *__restrict__ own, const int s0, const int e0, const int32_t o0) {
             constexpr bool WHOLE = decltype(whole)::value;
             for (int tb = s0; tb < e0; tb += kBlock) {
@@ -995,41 +1006,17 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? (LISTS ? 6 : 8) : (LISTS ? 3
                     je = t < e0 ? s_off[t + 1] - o0 : 0;
                     v = t < e0 ? own[c0 + t] : T(0);
                 }
-                const bool wide = !WHOLE && je - jb >= kLongRow;
-                if (!wide)
-                    for (int j = jb; j < je; ++j) s_v[j] = v;
-                if (!WHOLE)
-                    for (unsigned long long todo = __ballot(wide); todo; todo &= todo - 1) {
-                        const int src = __builtin_ctzll(todo);
-                        const int wb = __shfl(jb, src, kWave), we = __shfl(je, src, kWave);
-                        const T wv = __shfl(v, src, kWave);
-                        for (int j = wb + lane; j < we; j += kWave) s_v[j] = wv;
-                    }
+                slice_fill(s_v, jb, je, v);
             }
         };
-        // grad_x[column] = sum of the column's slice of s_v: in storage order by one lane, or
-        // (not WHOLE, kLongRow entries or more) lane l of a wavefront adds entries l, l + 64, ...
+        // grad_x[column] = sum of the column's slice of s_v
         auto sums = [&](auto whole, const int s0, const int e0, const int32_t o0) {
             constexpr bool WHOLE = decltype(whole)::value;
             for (int tb = s0; tb < e0; tb += kBlock) {
                 const int t = tb + threadIdx.x;
                 const int jb = t < e0 ? (WHOLE ? my_a : s_off[t]) - o0 : 0;
                 const int je = t < e0 ? (WHOLE ? my_b : s_off[t + 1]) - o0 : 0;
-                const bool wide = !WHOLE && je - jb >= kLongRow;
-                if (t < e0 && !wide) {
-                    T acc = 0;
-                    for (int j = jb; j < je; ++j) acc += s_v[j];
-                    grad_x[c0 + t] = acc;
-                }
-                if (!WHOLE)
-                    for (unsigned long long todo = __ballot(wide); todo; todo &= todo - 1) {
-                        const int src = __builtin_ctzll(todo);
-                        const int wb = __shfl(jb, src, kWave), we = __shfl(je, src, kWave);
-                        T acc = 0;
-                        for (int j = wb + lane; j < we; j += kWave) acc += s_v[j];
-                        acc = nm::wave_sum(acc);
-                        if (lane == 0) grad_x[c0 + tb + wave * kWave + src] = acc;
-                    }
+                slice_sums<false>(s_v, jb, je, t < e0, grad_x + c0, t);
             }
         };
         // Entries first .. first + cnt of the plan, lane = entry, s_v holding the own factor of
@@ -1100,7 +1087,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? (LISTS ? 6 : 8) : (LISTS ? 3
                         const int pc = p0 + u * kBlock < cnt ? p0 + u * kBlock : cnt - 1;
                         const int32_t w = nm::stream_load(at<O32>(t_pack, first + pc));
                         kk[u] = first + pc + (w >> 16);
-                        rr[u] = (int32_t)c0 + (int16_t)w;
+                        rr[u] = block0 + (int16_t)w;
                     }
                 } else {
 #pragma unroll
@@ -1135,23 +1122,41 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? (LISTS ? 6 : 8) : (LISTS ? 3
                 }
             }
         };
-        // The same for one gradient only or a pattern that is not symmetric.
+        // The same for one gradient only or a pattern that is not symmetric; two entries a lane under way (one: 127 x
+        // 113 x 101 seven-point, gradient of x, fp32 42.5 us, fp64 67.8; two 37.7 and 57.2; four 38.2 and 56.6, eight 41.5 and
+        // 46.1; 2000 x 1980 five-point fp32 82, 78, 84 and 90).
         auto entries_any = [&](const int32_t first, const int cnt) {
             const int32_t *__restrict__ tr = t_row + first;
             const int32_t *__restrict__ tp = t_perm + first;
-            for (int p = threadIdx.x; p < cnt; p += kBlock) {
-                int32_t k, r;
-                if (packed) {
-                    const int32_t w = nm::stream_load(t_pack + first + p);
-                    k = first + p + ((STAGE && staged) ? w >> nm::kStagePlaceBits : w >> 16);
-                    r = (STAGE && staged) ? (w & ((1 << nm::kStagePlaceBits) - 1)) : (int32_t)c0 + (int16_t)w;
-                } else {
-                    k = nm::stream_load(tp + p);
-                    r = nm::stream_load(tr + p);
+            constexpr int K = 2;
+            for (int p0 = threadIdx.x; p0 < cnt; p0 += K * kBlock) {
+                int32_t k[K], r[K];
+                T gr[K], dd[K];
+#pragma unroll
+                for (int u = 0; u < K; ++u) {
+                    const int p = p0 + u * kBlock < cnt ? p0 + u * kBlock : cnt - 1;
+                    if (packed) {
+                        const int32_t w = nm::stream_load(t_pack + first + p);
+                        k[u] = first + p + ((STAGE && staged) ? w >> nm::kStagePlaceBits : w >> 16);
+                        r[u] = (STAGE && staged) ? (w & ((1 << nm::kStagePlaceBits) - 1)) : block0 + (int16_t)w;
+                    } else {
+                        k[u] = nm::stream_load(tp + p);
+                        r[u] = nm::stream_load(tr + p);
+                    }
                 }
-                const T gr = (STAGE && staged) ? s_g[r] : g[r];
-                if (grad_A) grad_A[k] = gr * s_v[p];
-                s_v[p] = gr * data[k];
+#pragma unroll
+                for (int u = 0; u < K; ++u) {
+                    gr[u] = (STAGE && staged) ? s_g[r[u]] : g[r[u]];
+                    dd[u] = data[k[u]];
+                }
+#pragma unroll
+                for (int u = 0; u < K; ++u) {
+                    const int p = p0 + u * kBlock;
+                    if (p < cnt) {
+                        if (grad_A) grad_A[k[u]] = gr[u] * s_v[p];
+                        s_v[p] = gr[u] * dd[u];
+                    }
+                }
             }
         };
         // columns [s0, e0) through LDS
@@ -1451,17 +1456,24 @@ template <typename T, bool LISTS>
 void launch_bwd_planned(int64_t cols, int64_t nnz, const nm::TPlan &t, bool o32, const void *data, const void *x,
                         const void *g, void *grad_A, void *grad_x, hipStream_t s) {
     constexpr int R = kPlannedR, CAP = kPlannedCap;
-    int64_t grid = nm::xcd_padded(nm::ceil_div(cols, R));
+    // Columns of a tile: where they hold more than eight entries each and 256 at a time are fewer than 1024 tiles,
+    // fewer (a power of two: a tile lies in one block of packed rows).  Graphs, both gradients, 256 -> this many:
+    // 10 000 columns of 26 fp32 33.5 -> 8.0 us, fp64 37 -> 8.3; 30 000 of 18 23.4 -> 12.1 and 30.5 -> 17.0; 80 000 of 8 26.7
+    // -> 18.2 (512 tiles: 20.7).  Columns of five: 30 x 35 x 30 the same.
+    int width = R;
+    if (!LISTS && nnz > 8 * cols)
+        while (width > 16 && cols < (int64_t)width * 1024) width /= 2;
+    int64_t grid = nm::xcd_padded(nm::ceil_div(cols, width));
     if (grid > nm::kMaxGrid) grid = nm::kMaxGrid;
     const int32_t *desc = nnz > 0 ? t.b_desc : nullptr;
     if (o32)
         hipLaunchKernelGGL((spmv_bwd_planned_kernel<T, R, CAP, true, LISTS>), dim3((unsigned)grid), dim3(kBlock), 0, s,
                            cols, (const T *)data, t.t_indptr, t.t_row, t.t_perm, t.t_pack, t.flags, (const T *)x,
-                           (const T *)g, (T *)grad_A, (T *)grad_x, desc);
+                           (const T *)g, (T *)grad_A, (T *)grad_x, desc, width);
     else
         hipLaunchKernelGGL((spmv_bwd_planned_kernel<T, R, CAP, false, LISTS>), dim3((unsigned)grid), dim3(kBlock), 0, s,
                            cols, (const T *)data, t.t_indptr, t.t_row, t.t_perm, t.t_pack, t.flags, (const T *)x,
-                           (const T *)g, (T *)grad_A, (T *)grad_x, desc);
+                           (const T *)g, (T *)grad_A, (T *)grad_x, desc, width);
 }
 
 template <typename T>

@@ -908,11 +908,11 @@ Tensor spgemv_forward(int A_rows, int A_cols, Tensor A_data, Tensor A_col_ind, T
 
 // Entries from which scattered values go through column-major order (permute_plan), both gradients or grad_x alone (the
 // gradient of A alone is made by rows).  Graphs with random columns, on the plan's kernel -> through the order, us:
-//   both        fp32  1.1 M 40.7 -> 29.8   1.2 M 40.3 -> 31.0   2.1 M 75 -> 43   3.8 M 150 -> 77    7.6 M 304 -> 121
-//               fp64  0.6 M 27.6 -> 28.9   0.8 M 33.2 -> 33.4   1.0 M 41.5 -> 36.3   2.1 M 84 -> 59   7.6 M 320 -> 200
-//   grad_x      fp32  1.1 M 22.3 -> 24.3   1.2 M 22.2 -> 26.0   2.1 M 34.8 -> 30.8   3.8 M 66 -> 51   7.6 M 137 -> 88
-//               fp64  1.0 M 20.9 -> 30.0   1.2 M 25.3 -> 32.6   2.1 M 44.5 -> 41.4   3.8 M 77 -> 72   7.6 M 173 -> 130
-constexpr int64_t kStagedBoth = 900 << 10, kStagedOne = 1536 << 10;
+//   both        fp32  0.82 M 25.4 -> 25.2   0.92 M 29.7 -> 25.5   1.2 M 40 -> 31   2.1 M 73 -> 42   3.8 M 136 -> 77   7.6 M 288 -> 121
+//               fp64  0.82 M 28.8 -> 32.9   0.92 M 34.3 -> 33.3   1.2 M 45 -> 40   2.1 M 83 -> 59   3.8 M 149 -> 96   7.6 M 307 -> 200
+//   grad_x      fp32  1.2 M 19.1 -> 25.9   2.1 M 34.1 -> 30.6   2.5 M 40.4 -> 37.9   3.8 M 59 -> 51.5   7.6 M 130 -> 88
+//               fp64  1.2 M 21.4 -> 32.1   2.1 M 43.6 -> 41.4   2.5 M 48.7 -> 52.7   3.8 M 66 -> 71     7.6 M 165 -> 130
+constexpr int64_t kStagedBoth = 950 << 10, kStagedOne = 3 << 20;
 
 std::vector<Tensor> spgemv_backward(Tensor grad_z, int A_rows, int A_cols, Tensor A_data, Tensor A_col_ind,
                                     Tensor A_rowptr, Tensor x) {

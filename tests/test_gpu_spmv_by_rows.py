@@ -1,6 +1,6 @@
 """Gradients of matrix-vector products that are made by rows: the gradient of A alone, both with the products brought into
-column-major order, and the sums that are added to memory; at the edges of quads, tiles and long rows, against the
-oracle; and the default mode's choice among them."""
+column-major order, and the sums that are added to memory; those made by columns in narrow tiles; at the edges of
+quads, tiles and long rows, against the oracle; and the default mode's choice among them."""
 import ctypes
 
 import numpy as np
@@ -37,13 +37,22 @@ def _case(case):
         return _lengths([1] * 5000, cols=1)
     if case == "wide":
         return _lengths([7] * 300, cols=200_000)
+    if "band" in case:
+        reach = [0, 1, 2, 3, 4, 5] if case == "band" else [0, 1, 2, 90, 700, 1500, 3000]
+        n = 3000 if case == "band" else 9001
+        offs = np.array(sorted({-o for o in reach} | set(reach)))
+        c = np.arange(n)[:, None] + offs
+        ok = (c >= 0) & (c < n)
+        if case == "uneven band":                                   # not a symmetric pattern
+            ok[::7, :4] = False
+        return c[ok].astype(np.int64), np.concatenate([[0], np.cumsum(ok.sum(1))]).astype(np.int64), (n, n)
     d, i, p, shape = {"scattered": lambda: G.random_csr(3000, 2000, 0.01, 5), "ragged": lambda: G.ragged_csr(4000, 1500, 31, 8),
                       "grid": lambda: G.poisson2d(70)}[case]()
     return i, p, shape
 
 
 CASES = ["one entry", "quads 1", "quads 2", "quads 3", "quads 4", "long rows", "long rows of few", "one column", "wide",
-         "scattered", "ragged", "grid"]
+         "scattered", "ragged", "grid", "band", "far band", "uneven band"]
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
@@ -89,6 +98,14 @@ def test_against_the_oracle(dev, dtype, case):
         gA, _ = fresh()
         assert planned(dt, rows, cols, nnz, D.data_ptr(), plan.mem.data_ptr(), *vectors, gA.data_ptr(), None, None) == 0
         assert_same(host(gA), want_A, "grad_A alone, on the plan")
+        for both in (True, False):
+            gA, gx = fresh()
+            assert planned(dt, rows, cols, nnz, D.data_ptr(), plan.mem.data_ptr(), *vectors, gA.data_ptr() if both else None,
+                           gx.data_ptr(), None) == 0
+            if both:
+                assert_same(host(gA), want_A, "grad_A, on the plan")
+            assert_same(host(gx)[short], want_x[short], "grad_x, on the plan")
+            assert_sums(host(gx), "grad_x, on the plan")
     for both in (True, False):
         gA, gx = fresh()
         assert L.nm_spgemv_backward(dt, rows, cols, nnz, D.data_ptr(), I.data_ptr(), P.data_ptr(), *vectors, gA.data_ptr(),
@@ -112,7 +129,7 @@ def test_default_mode(dev):
             if case == "grid":
                 d, i, p, (rows, cols) = G.poisson2d(440, np.float32, jitter_seed=1)
             else:
-                rows = cols = 190_000
+                rows = cols = 200_000
                 rng = np.random.default_rng(3)
                 i = np.sort(rng.integers(0, cols, (rows, 5)), 1).reshape(-1)
                 p, d = np.arange(rows + 1, dtype=np.int64) * 5, randn(1, 5 * rows, np.float32)
