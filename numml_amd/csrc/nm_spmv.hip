@@ -613,15 +613,15 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_num_sgpr(72))) void sp
     }
 }
 
-// Fused backward by rows: out_A[k] = alpha * (a[row] * b[col]); when grad_x is given, grad_x[col] +=
-// a[row] * data[k]; when prod is given, prod[k] = a[row] * data[k].  With neither this is the masked outer
+// Fused backward by rows: out_A[k] = alpha * (a[row] * b[col]); ADD: grad_x[col] += a[row] * data[k] (a build of its own:
+// with the rest in one, 2048^2 five-point fp32 191 -> 216 us); when prod is given, prod[k] = a[row] * data[k].  With neither this is the masked outer
 // product (cpp/sparse_csr_cpu.cpp:60-65 and :750-755).
 //
 // It reads b once an entry and everything else in order, so that a grid moves its bytes (127 x 113 x 101 fp32, 32-bit
 // structure: 81 MB in 20.5 us) and a graph waits for its gathers from L2.  The gradient of A alone is made here
 // also where a transposed-structure plan exists: a walk by column writes it entry by entry where columns are
 // scattered (7.6 M entries fp32 243 -> 50 us) and gathers positions where they are not (the grid 46 -> 20.5).
-template <typename T, int R, int CAP, typename IDX>
+template <typename T, int R, int CAP, typename IDX, bool ADD>
 __global__ __launch_bounds__(kBlock) void spmv_bwd_kernel(
     int64_t rows, int rt, const T *__restrict__ data, const IDX *__restrict__ indices,
     const IDX *__restrict__ indptr, const T *__restrict__ a, const T *__restrict__ b, T alpha,
@@ -646,12 +646,14 @@ __global__ __launch_bounds__(kBlock) void spmv_bwd_kernel(
         const int n = s_off[nr];
         // entry k, whose row's factor is av
         auto entry = [&](int64_t k, T av) {
-            if (out_A || grad_x) {
+            if constexpr (ADD) {
                 const int64_t c = indices[k];
                 if (out_A) out_A[k] = alpha * (av * b[c]);
-                if (grad_x) nm::atomic_add(grad_x + c, av * data[k]);
+                nm::atomic_add(grad_x + c, av * data[k]);
+            } else {
+                if (out_A) out_A[k] = alpha * (av * b[indices[k]]);
+                if (prod) prod[k] = av * data[k];
             }
-            if (prod) prod[k] = av * data[k];
         };
         // a[row] to the entries of rows [s0, e0) in s_a, which begins at entry o0 of the block: one lane per short
         // row, a wavefront per row of kLongRow entries or more
@@ -666,7 +668,7 @@ __global__ __launch_bounds__(kBlock) void spmv_bwd_kernel(
         // `cnt` entries from `first` on, whose factors are s_a[0, cnt): four consecutive entries a lane, unless their
         // sums are added to memory (neighbouring lanes' additions to neighbouring columns go together)
         auto entries = [&](int64_t first, int cnt) {
-            if (grad_x) {
+            if constexpr (ADD) {
                 for (int k = threadIdx.x; k < cnt; k += kBlock) entry(first + k, s_a[k]);
                 return;
             }
@@ -1303,7 +1305,14 @@ int launch_bwd(int64_t rows, int64_t nnz, const T *data, const IDX *indices, con
     const int rt = small_block_rows(rows, nnz, R, CAP);
     int64_t grid = nm::xcd_padded(nm::ceil_div(rows, rt));
     if (grid > nm::kMaxGrid) grid = nm::kMaxGrid;
-    hipLaunchKernelGGL((spmv_bwd_kernel<T, R, CAP, IDX>), dim3((unsigned)grid), dim3(kBlock), 0, s, rows, rt, data,
+    if constexpr (sizeof(IDX) == 8)
+        if (grad_x) {
+            hipLaunchKernelGGL((spmv_bwd_kernel<T, R, CAP, IDX, true>), dim3((unsigned)grid), dim3(kBlock), 0, s, rows, rt,
+                               data, indices, indptr, a, b, alpha, out_A, grad_x, prod);
+            NM_LAUNCH_CHECK("spmv_bwd_kernel");
+            return NM_OK;
+        }
+    hipLaunchKernelGGL((spmv_bwd_kernel<T, R, CAP, IDX, false>), dim3((unsigned)grid), dim3(kBlock), 0, s, rows, rt, data,
                        indices, indptr, a, b, alpha, out_A, grad_x, prod);
     NM_LAUNCH_CHECK("spmv_bwd_kernel");
     return NM_OK;
