@@ -420,7 +420,8 @@ class SpMM(Workload):
                           + cols * n * s)
         self.bytes_per_step = self.fwd_bytes + self.bwd_bytes
         self.dominant_bytes = self.bwd_bytes
-        self.dominant_name = ("spdmm_bwd_fused_kernel: both gradients from one walk over A by column (transposed plan)"
+        self.dominant_name = ("groups_kernel<DOT>: both gradients from one walk over A by column (transposed plan)"
+                              + ("" if self.banded else ", values through column-major order by move_kernel")
                               if _binding.backward_mode() != "atomic"
                               else "spdmm_bwd_kernel (+ fill_kernel clearing grad_B)")
         # the plan of the default backward is built during one of these
@@ -440,11 +441,12 @@ class SpMM(Workload):
     def ops(self):
         from numml_amd import _binding
         planned = _binding.backward_mode() != "atomic"
-        return [("spdmm_fwd_flat_kernel",
+        return [("groups_kernel",
                  lambda: self.ext.spdmm_forward(self.rows, self.cols, self.D, self.I, self.P, self.B),
-                 self.fwd_bytes, "spdmm_fwd_flat_kernel"),
+                 self.fwd_bytes, "groups_kernel<float, 4, 16, long, false, false, false>"),
                 (self.dominant_name, self.dominant, self.bwd_bytes,
-                 "spdmm_bwd_fused_kernel" if planned else "spdmm_bwd_kernel")]
+                 "spdmm_bwd_kernel" if not planned else "groups_kernel<float, 4, 16, int, true, true, false>" if self.banded
+                 else ("groups_kernel<float, 4, 16, int, false, true, false>", "Move)0>", "Move)1>", "Move)2>", "Move)3>"))]
 
     def after(self, rec, steps):
         """The same step priced on the bytes that are gathered, not on the operands' sizes: what the
@@ -866,11 +868,11 @@ class Lincomb(Workload):
         bwd = 3 * (nnz * 8 + ptr) + nnz * s + 2 * nnz * s       # three patterns and grad_C in, two gradients out
         self.stateless_bytes = sym + num + bwd
         # on the cached maps of the pair of patterns (compiled binding, from the second sighting on):
-        # two int32 maps per entry of C and both value arrays in, C's values out; per gradient one
-        # int32 map, the gathered grad_C and the store
+        # both value arrays in, C's values out; grad_C in and both gradients out (operands of one
+        # pattern: the maps are the identity and nobody reads them)
         self.planned = _binding.name == "compiled" and _binding.backward_mode() != "atomic"
-        fwd_p = nnz * (2 * 4 + s) + 2 * nnz * s
-        bwd_p = 2 * (nnz * 4 + nnz * s + nnz * s)
+        fwd_p = 2 * nnz * s + nnz * s
+        bwd_p = nnz * s + 2 * nnz * s
         self.bytes_per_step = fwd_p + bwd_p if self.planned else self.stateless_bytes
         self.dominant_bytes = fwd_p if self.planned else sym + num
         self.dominant_name = ("lincomb_planned_kernel (one pass over the cached maps)" if self.planned
