@@ -337,7 +337,9 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_num_sgpr(72))) void sp
     const IDX *__restrict__ indptr, const T *__restrict__ x, T *__restrict__ y,
     const int16_t *__restrict__ off16 = nullptr, const int32_t *__restrict__ flags = nullptr,
     const int32_t *__restrict__ f_desc = nullptr) {
-    // rt <= R: rows per block of this launch (block_rows)
+    // rt <= R: rows per block of this launch (block_rows); the build for plans without lists finds in its high half those
+    // that a plan without packed columns is walked in
+    if constexpr (sizeof(IDX) == 4 && !UNIT && !LISTS) rt = flags[2] != 0 ? rt & 0xffff : rt >> 16;
     constexpr bool STAGE = LISTS && NM_STAGE_FWD && NM_FWD32_VEC && sizeof(IDX) == 4 && !UNIT && R == nm::kPackRows;
     constexpr bool HAS_LISTS = NM_STAGE_FWD && sizeof(IDX) == 4 && !UNIT && R == nm::kPackRows;
     // 64-bit structure, fp64: a lane takes 2 consecutive entries per request (16 bytes of values and of columns, aligned
@@ -1272,13 +1274,20 @@ int launch_fwd(int64_t rows, int64_t nnz, const T *data, const IDX *indices, con
     // Long rows: tiles of about 1024 products (of 2048 or 4096, fp32 graphs of 200 000 rows, 20 entries each on average
     // 45 -> 56, 63 us; of 100 000 and 12, 15.6 -> 17.8, 22).  Short ones: a tile of 512 rows reads the plan's packed
     // columns; without a plan at least 512 tiles (60 x 55 x 50 seven-point fp64 7.7 -> 5.9 us, with 1024 6.9; 30 x 35 x 30
-    // 6.2 -> 4.4, with 1024 5.6).
+    // 6.2 -> 4.4, with 1024 5.6).  On a plan whose columns are not packed, which only the device knows, at least 1024 (graphs, fp32,
+    // of 512 rows a tile -> 512 -> 1024 tiles: 200 000 rows of 7 entries on average 26.2 -> 23.9 -> 19.4 us, 130 000 of 5 14.6 ->
+    // 8.4 -> 8.1), and below 65 536 rows, where every column fits 16 bits, on any without lists (20 000 rows of 3 12.7 ->
+    // 5.6, 10 000 of 7 10.8 -> 5.0; grids the same).
     const bool long_rows = nnz > 8 * rows;
     int rt = block_rows(rows, nnz, R, long_rows ? 1024 : CAP);
     if (long_rows || sizeof(IDX) == 8)
         while (rt > 16 && rows < (int64_t)rt * 512) rt /= 2;
-    int64_t grid = nm::xcd_padded(nm::ceil_div(rows, rt));
+    int narrow = rt;
+    if (sizeof(IDX) == 4 && !LISTS && !long_rows)
+        while (narrow > 16 && rows < (int64_t)narrow * 1024) narrow /= 2;
+    int64_t grid = nm::xcd_padded(nm::ceil_div(rows, narrow));
     if (grid > nm::kMaxGrid) grid = nm::kMaxGrid;
+    if (sizeof(IDX) == 4 && !LISTS) rt = (rows < (1 << 16) ? narrow : rt) | narrow << 16;
     hipLaunchKernelGGL((spmv_fwd_kernel<T, kFwdBlock, R, CAP, false, IDX, LISTS>), dim3((unsigned)grid), dim3(kFwdBlock), 0, s,
                        rows, rt, data, indices, indptr, x, y, off16, flags, f_desc);
     NM_LAUNCH_CHECK("spmv_fwd_kernel");

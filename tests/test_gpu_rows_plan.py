@@ -23,8 +23,19 @@ def default_mode():
     _binding.set_backward_mode(old)
 
 
+def _some_long(rows, dtype):
+    """Three random columns a row, up to 6000 in seven of them."""
+    rng = np.random.default_rng(rows)
+    lens = np.full(rows, 3)
+    lens[[0, 15, 16, 5000, rows // 2, rows - 600, rows - 1]] = [31, 32, 2000, 4096, 4097, 6000, 5]
+    p = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    i = rng.integers(0, rows, p[-1])
+    return randn(5, p[-1], dtype), i, p, (rows, rows)
+
+
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
-@pytest.mark.parametrize("case", ["grid", "wide band", "scattered", "ragged", "one row", "511 rows", "513 rows"])
+@pytest.mark.parametrize("case", ["grid", "wide band", "scattered", "ragged", "one row", "511 rows", "513 rows", "65536 rows",
+                                  "65535 rows, some long", "70000 rows, some long"])
 def test_the_bits_of_the_plain_kernel(dev, dtype, case):
     d, i, p, (rows, cols) = {
         "grid": lambda: G.poisson2d(40, dtype, jitter_seed=1),
@@ -34,6 +45,9 @@ def test_the_bits_of_the_plain_kernel(dev, dtype, case):
         "one row": lambda: G.random_csr(1, 50, 0.5, 3, dtype, empty_rows=False),
         "511 rows": lambda: G.tridiag(511, dtype),
         "513 rows": lambda: G.tridiag(513, dtype),
+        "65536 rows": lambda: G.poisson2d(256, dtype, jitter_seed=1),
+        "65535 rows, some long": lambda: _some_long(65535, dtype),
+        "70000 rows, some long": lambda: _some_long(70000, dtype),
     }[case]()
     nnz = d.size
     x = randn(4, cols, dtype)
