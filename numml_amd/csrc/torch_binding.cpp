@@ -374,6 +374,29 @@ std::shared_ptr<Plan> peek_plan(char kind, const Tensor &indices, const Tensor &
     return plan;
 }
 
+// Takes a finished plan into the cache, which drops the least recently used ones beyond its bound.  These go when the
+// lock has been released: a plan's tensors may have been handed to Python, and dropping such a tensor
+// waits for the interpreter's lock, whose holder may be waiting for this one (a backward pass runs without
+// the interpreter's lock, a forward pass with it).
+void keep_plan(const std::shared_ptr<Plan> &plan, const c10::Device &dev) {
+    auto stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index());
+    plan->build_stream = stream.id();
+    plan->ready = std::make_unique<at::cuda::CUDAEvent>();
+    plan->ready->record(stream);
+    plan->bytes = plan->mem.defined() ? (size_t)plan->mem.nbytes() : 0;
+    for (const Tensor &t : plan->derived) plan->bytes += (size_t)t.nbytes();
+    g_plans_built.fetch_add(1, std::memory_order_relaxed);
+    std::list<std::shared_ptr<Plan>> dropped;
+    std::lock_guard<std::mutex> lock(g_plans_mutex);
+    g_plans.push_front(plan);
+    g_plan_bytes += plan->bytes;
+    const size_t limit = g_plan_bytes_limit.load(std::memory_order_relaxed);
+    while (g_plans.size() > 1 && g_plan_bytes > limit) {
+        g_plan_bytes -= g_plans.back()->bytes;
+        dropped.splice(dropped.end(), g_plans, std::prev(g_plans.end()));
+    }
+}
+
 // The plan of this kind for the pattern.  `second_sighting`: a pattern seen for the first time
 // is only noted and nullptr is returned (the caller then runs its stateless kernels); the plan
 // is built when the pattern shows up again.
@@ -409,21 +432,7 @@ std::shared_ptr<Plan> cached(char kind, const Tensor &indices, const Tensor &ind
     plan->a = a;
     plan->b = b;
     make(*plan);
-    auto stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index());
-    plan->build_stream = stream.id();
-    plan->ready = std::make_unique<at::cuda::CUDAEvent>();
-    plan->ready->record(stream);
-    plan->bytes = plan->mem.defined() ? (size_t)plan->mem.nbytes() : 0;
-    for (const Tensor &t : plan->derived) plan->bytes += (size_t)t.nbytes();
-    g_plans_built.fetch_add(1, std::memory_order_relaxed);
-    std::lock_guard<std::mutex> lock(g_plans_mutex);
-    g_plans.push_front(plan);
-    g_plan_bytes += plan->bytes;
-    const size_t limit = g_plan_bytes_limit.load(std::memory_order_relaxed);
-    while (g_plans.size() > 1 && g_plan_bytes > limit) {
-        g_plan_bytes -= g_plans.back()->bytes;
-        g_plans.pop_back();
-    }
+    keep_plan(plan, dev);
     return plan;
 }
 
@@ -766,21 +775,7 @@ void consider_product_plan(const Tensor &A_indices, const Tensor &A_indptr, cons
         plan->mem = Tensor();   // remembered as unusable, so that the pair is not analysed again
         plan->parent.reset();
     }
-    auto stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index());
-    plan->build_stream = stream.id();
-    plan->ready = std::make_unique<at::cuda::CUDAEvent>();
-    plan->ready->record(stream);
-    plan->bytes = plan->mem.defined() ? (size_t)plan->mem.nbytes() : 0;
-    for (const Tensor &t : plan->derived) plan->bytes += (size_t)t.nbytes();
-    g_plans_built.fetch_add(1, std::memory_order_relaxed);
-    std::lock_guard<std::mutex> lock(g_plans_mutex);
-    g_plans.push_front(plan);
-    g_plan_bytes += plan->bytes;
-    const size_t limit = g_plan_bytes_limit.load(std::memory_order_relaxed);
-    while (g_plans.size() > 1 && g_plan_bytes > limit) {
-        g_plan_bytes -= g_plans.back()->bytes;
-        g_plans.pop_back();
-    }
+    keep_plan(plan, dev);
 }
 
 // After a stateless linear combination: notes the pair of patterns, or (second sighting; first in
@@ -832,21 +827,7 @@ void consider_sum_plan(const Tensor &A_indices, const Tensor &A_indptr, const Te
           "nm_splincomb_plan_build");
     plan->derived = {C_indices, C_indptr};
     for (const Tensor &t : plan->derived) plan->derived_versions.push_back(version_of(t));
-    auto stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index());
-    plan->build_stream = stream.id();
-    plan->ready = std::make_unique<at::cuda::CUDAEvent>();
-    plan->ready->record(stream);
-    plan->bytes = (size_t)plan->mem.nbytes();
-    for (const Tensor &t : plan->derived) plan->bytes += (size_t)t.nbytes();
-    g_plans_built.fetch_add(1, std::memory_order_relaxed);
-    std::lock_guard<std::mutex> lock(g_plans_mutex);
-    g_plans.push_front(plan);
-    g_plan_bytes += plan->bytes;
-    const size_t limit = g_plan_bytes_limit.load(std::memory_order_relaxed);
-    while (g_plans.size() > 1 && g_plan_bytes > limit) {
-        g_plan_bytes -= g_plans.back()->bytes;
-        g_plans.pop_back();
-    }
+    keep_plan(plan, dev);
 }
 
 Tensor solve(const Plan &plan, bool transposed, const Tensor &A_data, bool unit, const Tensor &b, int64_t rows,
@@ -1770,8 +1751,9 @@ std::tuple<std::string, std::string> last_backward_paths() {
 }
 
 void clear_plan_cache() {
+    std::list<std::shared_ptr<Plan>> dropped;   // (goes after the lock: keep_plan)
     std::lock_guard<std::mutex> lock(g_plans_mutex);
-    g_plans.clear();
+    dropped.swap(g_plans);
     g_aliases.clear();
     g_sightings.clear();
     g_seen.clear();

@@ -166,3 +166,43 @@ def test_threads_at_once(dev):
     for t in threads:
         t.join()
     assert not failures, failures
+
+
+def test_threads_while_plans_leave_the_cache(dev):
+    """The same with room for one plan: every call drops plans, with pattern tensors that Python holds, has held
+    or still looks at, in backward passes too (no interpreter's lock) while other threads call forward passes (with
+    it)."""
+    want = {n: torch.autograd.grad(run().sum(), leaves) for n, (run, leaves) in _operations(dev).items()}
+    failures, held = [], []
+
+    def work():
+        try:
+            stream = torch.cuda.Stream()
+            with torch.cuda.stream(stream):
+                for k in range(5):
+                    for n, (run, leaves) in _operations(dev).items():
+                        A = _grid(dev)
+                        for C in (A @ A, A + A):
+                            C.indices, C.indptr     # wrapped here ...
+                            if k % 2:
+                                held.append(C)      # ... and kept by every second turn
+                        got = torch.autograd.grad(run().sum(), leaves)
+                        stream.synchronize()
+                        assert all(torch.allclose(a, b, rtol=1e-12) for a, b in zip(got, want[n])), n
+        except Exception as e:   # reported by the main thread
+            failures.append(repr(e))
+    ops = _binding.ops
+    ops.clear_plan_cache()
+    ops.set_plan_cache_limit(1)
+    try:
+        threads = [threading.Thread(target=work, daemon=True) for _ in range(4)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join(60)
+        assert not any(t.is_alive() for t in threads), "threads wait for each other"
+        assert not failures, failures
+        assert ops.plan_cache_size() == 1
+    finally:
+        ops.set_plan_cache_limit(4096 << 20)
+        ops.clear_plan_cache()
