@@ -87,9 +87,16 @@ Tensor row_major(const Tensor &M, int64_t *ld) {
     return R;
 }
 
+// Memory of plans and of the pattern tensors that they hand out: an ordinary tensor under torch.inference_mode()
+// too.  A plan made in an evaluation pass serves training passes later, whose autograd nodes save such tensors,
+// and autograd saves no inference tensors.
+Tensor lasting(int64_t numel, const torch::TensorOptions &options) {
+    c10::InferenceMode off(false);
+    return torch::empty({numel}, options);
+}
+
 Tensor scratch(size_t bytes, const c10::Device &dev) {
-    return torch::empty({(int64_t)std::max<size_t>(bytes, 8)},
-                        torch::TensorOptions().dtype(torch::kUInt8).device(dev));
+    return lasting((int64_t)std::max<size_t>(bytes, 8), torch::TensorOptions().dtype(torch::kUInt8).device(dev));
 }
 
 // ---- argument shapes ------------------------------------------------------------
@@ -252,10 +259,8 @@ void *host_landing() {
 // Tensors made under torch.inference_mode() carry no version counter (asking for it throws).
 // A pair of such structure tensors gets no entry in the alias table -- an edit in place could
 // not be noticed -- so a call that needs a plan computes their content key every time and one
-// that only peeks runs its stateless kernels; pattern tensors of this kind that a plan hands
-// out count as version 0.
+// that only peeks runs its stateless kernels.  (Tensors that a plan hands out are never of this kind.)
 bool tracked(const Tensor &t) { return !t.is_inference(); }
-uint32_t version_of(const Tensor &t) { return tracked(t) ? t._version() : 0; }
 
 bool alias_matches(const Alias &al, const Tensor &indices, const Tensor &indptr) {
     return al.idx_impl == indices.unsafeGetTensorImpl() && al.ptr_impl == indptr.unsafeGetTensorImpl() &&
@@ -642,7 +647,7 @@ std::shared_ptr<Plan> peek_product_plan(const Tensor &A_indices, const Tensor &A
     }
     if (!plan) return nullptr;
     for (size_t i = 0; i < plan->derived.size(); ++i)
-        if (version_of(plan->derived[i]) != plan->derived_versions[i]) {
+        if (plan->derived[i]._version() != plan->derived_versions[i]) {
             drop_plan(plan);
             return nullptr;
         }
@@ -770,7 +775,7 @@ void consider_product_plan(const Tensor &A_indices, const Tensor &A_indptr, cons
     plan->plan_class = usable > 0 ? usable : 0;
     if (plan->usable) {
         plan->derived = {C_indices, C_indptr};
-        for (const Tensor &t : plan->derived) plan->derived_versions.push_back(version_of(t));
+        for (const Tensor &t : plan->derived) plan->derived_versions.push_back(t._version());
     } else {
         plan->mem = Tensor();   // remembered as unusable, so that the pair is not analysed again
         plan->parent.reset();
@@ -826,7 +831,7 @@ void consider_sum_plan(const Tensor &A_indices, const Tensor &A_indptr, const Te
                                   pbytes, current_stream(dev)),
           "nm_splincomb_plan_build");
     plan->derived = {C_indices, C_indptr};
-    for (const Tensor &t : plan->derived) plan->derived_versions.push_back(version_of(t));
+    for (const Tensor &t : plan->derived) plan->derived_versions.push_back(t._version());
     keep_plan(plan, dev);
 }
 
@@ -1046,14 +1051,14 @@ std::vector<Tensor> splincomb_forward(int rows, int cols, Tensor alpha, Tensor A
     check(nm_splincomb_workspace_bytes(rows, &bytes), "nm_splincomb_workspace_bytes");
     Tensor work = scratch(bytes, dev);
     const auto iopt = torch::TensorOptions().dtype(torch::kInt64).device(dev);
-    Tensor C_indptr = torch::empty({(int64_t)rows + 1}, iopt);
+    Tensor C_indptr = lasting((int64_t)rows + 1, iopt);
     nm_stream st = current_stream(dev);
     check(nm_splincomb_symbolic(rows, A_indices.data_ptr<int64_t>(), A_indptr.data_ptr<int64_t>(),
                                 B_indices.data_ptr<int64_t>(), B_indptr.data_ptr<int64_t>(),
                                 C_indptr.data_ptr<int64_t>(), work.data_ptr(), bytes, st),
           "nm_splincomb_symbolic");
     const int64_t nnz_c = C_indptr[rows].item<int64_t>();   // C is returned exactly sized
-    Tensor C_indices = torch::empty({nnz_c}, iopt);
+    Tensor C_indices = lasting(nnz_c, iopt);
     Tensor C_data = torch::empty({nnz_c}, A_data.options());
     check(nm_splincomb_numeric(dtype_of(A_data), rows, a, A_data.data_ptr(), A_indices.data_ptr<int64_t>(),
                                A_indptr.data_ptr<int64_t>(), b, B_data.data_ptr(), B_indices.data_ptr<int64_t>(),
@@ -1349,7 +1354,7 @@ std::vector<Tensor> spgemm_forward(int A_rows, int A_cols, Tensor A_data, Tensor
     check(nm_spgemm_workspace_bytes(A_rows, B_cols, &bytes), "nm_spgemm_workspace_bytes");
     Tensor work = scratch(bytes, dev);
     const auto iopt = torch::TensorOptions().dtype(torch::kInt64).device(dev);
-    Tensor C_indptr = torch::empty({(int64_t)A_rows + 1}, iopt);
+    Tensor C_indptr = lasting((int64_t)A_rows + 1, iopt);
     nm_stream st = current_stream(dev);
     // The symbolic merge records where every product goes (16 bytes per entry of A, scratch of this
     // call): with no row on the hash path the numeric phase then adds the products up on those
@@ -1379,7 +1384,7 @@ std::vector<Tensor> spgemm_forward(int A_rows, int A_cols, Tensor A_data, Tensor
     check(nm_spgemm_symbolic_result(A_rows, B_cols, work.data_ptr(), bytes, &nnz_c, &hash_rows, host_landing(),
                                     st),
           "nm_spgemm_symbolic_result");
-    Tensor C_indices = torch::empty({nnz_c}, iopt);
+    Tensor C_indices = lasting(nnz_c, iopt);
     Tensor C_data = torch::empty({nnz_c}, A_data.options());
     const bool on_map = filled.defined() && hash_rows == 0 && nnz_c > 0 && nnz_c < lim31;
     check(nm_spgemm_numeric_mapped(dtype_of(A_data), A_rows, A_cols, B_cols, A_nnz, nnz_c, A_data.data_ptr(),
@@ -1554,12 +1559,12 @@ std::shared_ptr<Plan> lu_pattern(const Tensor &A_indices, const Tensor &A_indptr
             size_t bytes = 0;
             check(nm_splu_symbolic_bytes(rows, &bytes), "nm_splu_symbolic_bytes");
             Tensor work = scratch(bytes, dev);
-            Tensor M_indptr = torch::empty({rows + 1}, iopt);
+            Tensor M_indptr = lasting(rows + 1, iopt);
             check(nm_splu_symbolic(rows, A_indices.data_ptr<int64_t>(), A_indptr.data_ptr<int64_t>(),
                                    M_indptr.data_ptr<int64_t>(), work.data_ptr(), bytes, stream),
                   "nm_splu_symbolic");
             const int64_t nnz = M_indptr[rows].item<int64_t>();
-            Tensor M_indices = torch::empty({nnz}, iopt);
+            Tensor M_indices = lasting(nnz, iopt);
             Tensor zeros = torch::zeros({std::max<int64_t>(A_indices.numel(), 1)},
                                         torch::TensorOptions().dtype(torch::kFloat32).device(dev));
             Tensor As_data = torch::empty({nnz}, zeros.options());
@@ -1569,19 +1574,19 @@ std::shared_ptr<Plan> lu_pattern(const Tensor &A_indices, const Tensor &A_indptr
                   "nm_splu_fill");
             auto tplan = transpose_plan(M_indices, M_indptr, rows, rows, dev);
             Tensor Mt_data = torch::empty_like(As_data);
-            Tensor Mt_indices = torch::empty({nnz}, iopt);
-            Tensor Mt_indptr = torch::empty({rows + 1}, iopt);
-            Tensor Mt_to_M = torch::empty({nnz}, iopt);
+            Tensor Mt_indices = lasting(nnz, iopt);
+            Tensor Mt_indptr = lasting(rows + 1, iopt);
+            Tensor Mt_to_M = lasting(nnz, iopt);
             check(nm_csr_transpose_forward(NM_F32, rows, rows, nnz, As_data.data_ptr(), tplan->mem.data_ptr(),
                                            Mt_data.data_ptr(), Mt_indices.data_ptr<int64_t>(),
                                            Mt_indptr.data_ptr<int64_t>(), Mt_to_M.data_ptr<int64_t>(), stream),
                   "nm_csr_transpose_forward");
             p.derived = {M_indices, M_indptr, Mt_indices, Mt_indptr, Mt_to_M};
-            for (const Tensor &t : p.derived) p.derived_versions.push_back(version_of(t));
+            for (const Tensor &t : p.derived) p.derived_versions.push_back(t._version());
         });
         bool intact = true;   // a caller may have edited the tensors it was handed
         for (size_t i = 0; i < plan->derived.size(); ++i)
-            intact = intact && version_of(plan->derived[i]) == plan->derived_versions[i];
+            intact = intact && plan->derived[i]._version() == plan->derived_versions[i];
         if (intact || attempt > 0) {
             TORCH_CHECK(intact, "the cached factor pattern was modified in place");
             return plan;

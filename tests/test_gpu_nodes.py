@@ -108,6 +108,34 @@ def test_saved_tensor_hooks_are_seen(dev, name):
         assert np.allclose(host(a), host(b), rtol=1e-12)
 
 
+@pytest.mark.parametrize("mode", ["planned", "eager"])
+def test_an_evaluation_pass_first(dev, mode):
+    """Plans and pattern tensors made under torch.inference_mode() serve a training pass on the same patterns."""
+    _binding.set_backward_mode(mode)
+
+    def operations():
+        run = _operations(dev)
+        A, B = _grid(dev), _grid(dev)
+        run["symmetric part"] = (lambda: (A + A.T).data, (A.data,))
+        run["coarse"] = (lambda: (B.T @ (A @ B)).data, (A.data, B.data))
+        return run
+    want = {}
+    for name in operations():
+        _binding.ops.clear_plan_cache()
+        run, leaves = operations()[name]
+        want[name] = torch.autograd.grad(run().sum(), leaves)
+    for name in want:
+        _binding.ops.clear_plan_cache()
+        run, leaves = operations()[name]
+        with torch.inference_mode():
+            for _ in range(3):
+                run()
+        for _ in range(2):
+            got = torch.autograd.grad(run().sum(), leaves)
+            for a, b in zip(got, want[name]):
+                assert torch.allclose(a, b, rtol=1e-12, atol=1e-12), name
+
+
 @pytest.mark.parametrize("name", ["spmv", "sptrsv"])
 def test_functions_stay_where_an_operation_is_not_plain(dev, monkeypatch, name):
     run, leaves = _operations(dev)[name]
