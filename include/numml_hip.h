@@ -478,8 +478,9 @@ int nm_spgemm_backward_mapped_wide(nm_dtype dt, int plan_class, int64_t A_rows, 
  * entry of B, in the orders in which C, grad_A and grad_B add them up (the serial loops': the same bits).
  * nm_spgemm_lists_products counts the products (work: (A_nnz + 1) * 8 bytes rounded up to 256, and
  * A_nnz / 256 + 16 more); nm_spgemm_lists_build makes the plan from the three patterns and the
- * transposed-structure plan of A, *usable = 0 where one workgroup would have more than 65 536
- * products.  Both wait for `stream`; the passes do not.  No counterpart in the reference. */
+ * transposed-structure plan of A: *usable = 0 where one workgroup would have more than 65 536
+ * products, 2 (only nm_spgemm_numeric_lists may be called) where one of a gradient's would have more
+ * than 16 384, else 1.  Both wait for `stream`; the passes do not.  No counterpart in the reference. */
 int nm_spgemm_lists_products(int64_t A_nnz, const int64_t *A_indices, const int64_t *B_indptr,
                              void *work, size_t work_bytes, int64_t *products, nm_stream stream);
 int nm_spgemm_lists_bytes(int64_t B_rows, int64_t A_nnz, int64_t B_nnz, int64_t C_nnz, int64_t products,

@@ -15,8 +15,15 @@
 // products, fp32): forward 781 -> 56 us (the hash path and its symbolic phase before), with gradients 1326 -> 230;
 // 50 000 rows, 5 entries a row, fp64: 445 -> 17, 600 -> 62.  Making the plan takes 2 ms of the former, 0.4 of the latter.
 //
-// The plan is refused where a workgroup would have more than kBusiest products (hub columns that meet long rows): its
-// segments are added up by one lane each.
+// A workgroup takes its products a tile at a time and a lane adds up a segment alone, so a workgroup with very many
+// products makes everybody wait.  Counted before any list is made: the plan is refused where a workgroup would have more
+// than kBusiest products; where one of a gradient's would have more than kBusiestBack the gradients are
+// left to the kernels without a plan.  Measured in microseconds, this plan against none (fp32, forward + gradients):
+//   a workgroup of C:    48 x 48 from 48 x 256 (65 536)       137 + 33 -> 278 + 563
+//                        one entry of 32 768 products         301 + 12 -> 9923 + 19564
+//   of both gradients:   256 x 1 times 1 x 64 (16 384)          7 + 49 ->  89 + 40
+//                        256 x 1 times 1 x 128 (32 768)         8 + 98 -> 108 + 25
+//                        256 x 1 times 1 x 256 (65 536)        7 + 242 -> 105 + 28
 #include "nm_common.hpp"
 #include "nm_scan.hpp"
 #include "nm_transpose.hpp"
@@ -29,14 +36,14 @@ using nm::kWave;
 constexpr int kBlock = 256;
 constexpr int kTile = 2048;                // products in LDS at a time
 constexpr int kPerLane = kTile / kBlock;
-constexpr int kBusiest = 65536;            // most products of a workgroup
+constexpr int kBusiest = 65536, kBusiestBack = 16384;   // most products of a workgroup, and of one of a gradient's
 
 struct Lists {          // out[s] = sum over p in [ptr[s], ptr[s + 1]) of U[u[p]] * V[v[p]]
     int32_t *ptr, *u, *v;
 };
 struct Plan {
     Lists c, a, b;
-    int32_t *flags;     // [0] products of the busiest workgroup
+    int32_t *flags;     // products of the busiest workgroup [0] of C, [1] of a gradient, where they are many
 };
 
 size_t plan_layout(int64_t nnzA, int64_t nnzB, int64_t nnzC, int64_t products, void *base, Plan *plan) {
@@ -95,40 +102,53 @@ __global__ void narrow_kernel(int64_t n, const int64_t *__restrict__ wide, int32
     if (i < n) out[i] = (int32_t)wide[i];
 }
 
-// Rows of A, a wavefront each in turn: place in C, entry of A and entry of B of every product; counts the
-// products of C's entries.
+// The last index in [lo, hi) whose pointer is at or before p (ptr[lo] <= p): past empty ones, the one that p lies in.
+template <typename P> __device__ __forceinline__ int64_t last_at(const P *__restrict__ ptr, int64_t lo, int64_t hi, int64_t p) {
+    while (hi - lo > 1) {
+        const int64_t mid = (lo + hi) >> 1;
+        if (ptr[mid] <= p) lo = mid; else hi = mid;
+    }
+    return lo;
+}
+
+// Where a product lies: the entry in whose list it is and that entry's row.  Product by product, so that neither a row
+// nor an entry with millions of products keeps one wavefront busy; a workgroup's products are consecutive, and
+// its two ends bound what its lanes look through.
+struct Place {
+    int64_t entry, row;
+};
+__device__ __forceinline__ Place place_of(int64_t p, int64_t products, const int32_t *__restrict__ ptr, int64_t entries,
+                                          const int64_t *__restrict__ indptr, int64_t rows) {
+    __shared__ Place s_end[2];
+    if (threadIdx.x < 2) {
+        const int64_t end = (int64_t)(blockIdx.x + threadIdx.x) * kBlock - threadIdx.x;
+        const int64_t e = last_at(ptr, 0, entries, end < products ? end : products - 1);
+        s_end[threadIdx.x] = Place{e, last_at(indptr, 0, rows, e)};
+    }
+    __syncthreads();
+    const int64_t e = last_at(ptr, s_end[0].entry, s_end[1].entry + 1, p);
+    return Place{e, last_at(indptr, s_end[0].row, s_end[1].row + 1, e)};
+}
+
+// Place in C, entry of A and entry of B of every product; counts the products of C's entries.
 __global__ __launch_bounds__(kBlock) void products_kernel(
-    int64_t rows, const int64_t *__restrict__ A_indices, const int64_t *__restrict__ A_indptr,
+    int64_t products, int64_t rows, int64_t nnzA, const int64_t *__restrict__ A_indices, const int64_t *__restrict__ A_indptr,
     const int64_t *__restrict__ B_indices, const int64_t *__restrict__ B_indptr, const int64_t *__restrict__ C_indices,
     const int64_t *__restrict__ C_indptr, Lists a, int32_t *__restrict__ entry, unsigned long long *__restrict__ count) {
-    const int lane = threadIdx.x & (kWave - 1);
-    const int64_t waves = (int64_t)gridDim.x * (kBlock / kWave);
-    for (int64_t row = (int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave; row < rows; row += waves) {
-        const int64_t eb = A_indptr[row], ee = A_indptr[row + 1], cb = C_indptr[row], ce = C_indptr[row + 1];
-        // the row's products are consecutive: lane by lane, whatever the entries' lengths
-        int64_t e = eb;
-        for (int64_t p0 = a.ptr[eb]; p0 < a.ptr[ee]; p0 += kWave) {
-            const int64_t p = p0 + lane;
-            if (p >= a.ptr[ee]) continue;
-            int64_t lo = e, hi = ee;            // the last entry that starts at or before p (empty ones before it)
-            while (hi - lo > 1) {
-                const int64_t mid = (lo + hi) >> 1;
-                if (a.ptr[mid] <= p) lo = mid; else hi = mid;
-            }
-            e = lo;
-            const int64_t f = B_indptr[A_indices[lo]] + (p - a.ptr[lo]);
-            const int64_t column = B_indices[f];
-            int64_t l = cb, h = ce;
-            while (l < h) {
-                const int64_t mid = (l + h) >> 1;
-                if (C_indices[mid] < column) l = mid + 1; else h = mid;
-            }
-            a.u[p] = (int32_t)l;
-            a.v[p] = (int32_t)f;
-            entry[p] = (int32_t)lo;
-            atomicAdd(&count[l], 1ull);
-        }
+    const int64_t p = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    const Place at = place_of(p < products ? p : products - 1, products, a.ptr, nnzA, A_indptr, rows);
+    if (p >= products) return;
+    const int64_t f = B_indptr[A_indices[at.entry]] + (p - a.ptr[at.entry]);
+    const int64_t column = B_indices[f];
+    int64_t l = C_indptr[at.row], h = C_indptr[at.row + 1];
+    while (l < h) {
+        const int64_t mid = (l + h) >> 1;
+        if (C_indices[mid] < column) l = mid + 1; else h = mid;
     }
+    a.u[p] = (int32_t)l;
+    a.v[p] = (int32_t)f;
+    entry[p] = (int32_t)at.entry;
+    atomicAdd(&count[l], 1ull);
 }
 
 __global__ __launch_bounds__(kBlock) void place_kernel(int64_t products, const int32_t *__restrict__ dest, int32_t *__restrict__ cursor,
@@ -137,26 +157,14 @@ __global__ __launch_bounds__(kBlock) void place_kernel(int64_t products, const i
     if (p < products) raw[atomicAdd(&cursor[dest[p]], 1)] = (int32_t)p;
 }
 
-// The products of an entry of C into ascending order (each finds its rank among the others; entries of more than a few
-// are shared by the wavefront).
-__global__ __launch_bounds__(kBlock) void order_kernel(int64_t nnzC, const int32_t *__restrict__ raw, const int32_t *__restrict__ entry,
-                                                       const int32_t *__restrict__ f, Lists c) {
-    const int64_t s = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    const int lane = threadIdx.x & (kWave - 1);
-    const int b = s < nnzC ? c.ptr[s] : 0, n = s < nnzC ? c.ptr[s + 1] - b : 0;
-    auto put = [&](int first, int len, int i) {
-        const int32_t p = raw[first + i];
-        int rank = 0;
-        for (int k = 0; k < len; ++k) rank += raw[first + k] < p;
-        c.u[first + rank] = entry[p];
-        c.v[first + rank] = f[p];
-    };
-    if (n <= 8)
-        for (int i = 0; i < n; ++i) put(b, n, i);
-    for (unsigned long long left = __ballot(n > 8); left; left &= left - 1) {
-        const int l = __ffsll(left) - 1, first = __shfl(b, l, kWave), len = __shfl(n, l, kWave);
-        for (int i = lane; i < len; i += kWave) put(first, len, i);
-    }
+// The factors of C's products, whose numbers lie in `raw` entry by entry, ascending
+__global__ __launch_bounds__(kBlock) void c_lists_kernel(int64_t products, const int32_t *__restrict__ raw, const int32_t *__restrict__ entry,
+                                                         const int32_t *__restrict__ f, Lists c) {
+    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i >= products) return;
+    const int32_t p = raw[i];
+    c.u[i] = entry[p];
+    c.v[i] = f[p];
 }
 
 // count[j] = products of row j of B: its entries times the entries of A's column j
@@ -166,33 +174,38 @@ __global__ void row_products_kernel(int64_t rowsB, const int64_t *__restrict__ B
     if (j <= rowsB) count[j] = j < rowsB ? (B_indptr[j + 1] - B_indptr[j]) * (t_indptr[j + 1] - t_indptr[j]) : 0;
 }
 
-// Lists of B's entries: a wavefront a row of B in turn, the products with A's column beside it as a table of
-// (entry of B) x (entry of the column).
-__global__ __launch_bounds__(kBlock) void b_lists_kernel(int64_t rowsB, const int64_t *__restrict__ B_indptr,
-                                                         const int32_t *__restrict__ t_indptr, const int32_t *__restrict__ t_perm,
-                                                         const int64_t *__restrict__ start, Lists a, Lists b) {
+// Where the lists of B's entries begin: an entry of row j has a product with every entry of A's column j (a wavefront a
+// row of B in turn).
+__global__ __launch_bounds__(kBlock) void b_ptr_kernel(int64_t rowsB, int64_t products, const int64_t *__restrict__ B_indptr,
+                                                       const int32_t *__restrict__ t_indptr, const int64_t *__restrict__ start, Lists b) {
     const int lane = threadIdx.x & (kWave - 1);
     const int64_t waves = (int64_t)gridDim.x * (kBlock / kWave);
     for (int64_t j = (int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave; j < rowsB; j += waves) {
-        const int64_t fb = B_indptr[j], len = B_indptr[j + 1] - fb, tb = t_indptr[j], col = t_indptr[j + 1] - tb, p0 = start[j];
+        const int64_t fb = B_indptr[j], len = B_indptr[j + 1] - fb, col = t_indptr[j + 1] - t_indptr[j], p0 = start[j];
         for (int64_t k = lane; k < len; k += kWave) b.ptr[fb + k] = (int32_t)(p0 + k * col);
-        for (int64_t i = lane; i < len * col; i += kWave) {
-            const int64_t k = i / col, e = t_perm[tb + (i - k * col)];
-            b.u[p0 + i] = (int32_t)e;
-            b.v[p0 + i] = a.u[a.ptr[e] + k];
-        }
     }
+    if (blockIdx.x == 0 && threadIdx.x == 0) b.ptr[B_indptr[rowsB]] = (int32_t)products;
 }
-__global__ void last_ptr_kernel(int32_t *ptr, int32_t v) { *ptr = v; }
 
-// Products of the busiest workgroup of segments_kernel
-__global__ __launch_bounds__(kBlock) void busiest_kernel(int64_t segments, int per_block, const int32_t *__restrict__ ptr, int32_t *flags) {
+__global__ __launch_bounds__(kBlock) void b_lists_kernel(int64_t products, int64_t rowsB, int64_t nnzB, const int64_t *__restrict__ B_indptr,
+                                                         const int32_t *__restrict__ t_indptr, const int32_t *__restrict__ t_perm,
+                                                         Lists a, Lists b) {
+    const int64_t p = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    const Place at = place_of(p < products ? p : products - 1, products, b.ptr, nnzB, B_indptr, rowsB);
+    if (p >= products) return;
+    const int32_t e = t_perm[t_indptr[at.row] + (p - b.ptr[at.entry])];
+    b.u[p] = e;
+    b.v[p] = a.u[a.ptr[e] + (at.entry - B_indptr[at.row])];
+}
+
+// Products of the busiest workgroup of segments_kernel, where they are more than kBusiestBack
+__global__ __launch_bounds__(kBlock) void busiest_kernel(int64_t segments, int per_block, const int32_t *__restrict__ ptr, int32_t *flag) {
     const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x, s = i * per_block;
     int n = 0;
     if (s < segments) n = ptr[s + per_block < segments ? s + per_block : segments] - ptr[s];
 #pragma unroll
     for (int off = kWave / 2; off > 0; off >>= 1) n = max(n, __shfl_xor(n, off, kWave));
-    if ((threadIdx.x & (kWave - 1)) == 0 && n > kBusiest) atomicMax(flags, n);
+    if ((threadIdx.x & (kWave - 1)) == 0 && n > kBusiestBack) atomicMax(flag, n);
 }
 
 // out[s] = sum over p of U[u[p]] * V[v[p]], terms in the order of p from +0.0: a workgroup has kBlock * L
@@ -326,45 +339,55 @@ extern "C" int nm_spgemm_lists_build(int64_t A_rows, int64_t B_rows, int64_t A_n
     work_layout(B_rows, A_nnz, B_nnz, C_nnz, products, work, &w);
     nm::TPlan t;
     nm::tplan_layout(A_rows, B_rows, A_nnz, const_cast<void *>(A_plan_mem), &t);
-    // A's entries
+    // (a workgroup has these many at least: no need to look)
+    for (int64_t n : {C_nnz, A_nnz, B_nnz})
+        if (products > kBusiest * nm::ceil_div(n, (int64_t)kBlock * per_lane(n, products))) return NM_OK;
+    if (int rc = nm::fill_async(p.flags, (int64_t)2, (int32_t)0, s)) return rc;
+    auto look_at = [&](int64_t n, const Lists &list, int32_t *flag) {
+        const int per_block = kBlock * per_lane(n, products);
+        hipLaunchKernelGGL(busiest_kernel, dim3(grid_of(nm::ceil_div(n, per_block), kBlock)), dim3(kBlock), 0, s, n, per_block, list.ptr, flag);
+    };
+    // where the lists begin: A's entries
     hipLaunchKernelGGL(lengths_kernel, dim3(grid_of(A_nnz + 1, kBlock)), dim3(kBlock), 0, s, A_nnz, A_indices, B_indptr, w.count);
     NM_LAUNCH_CHECK("lengths_kernel");
     if (int rc = nm::scan_exclusive_i64(w.count, A_nnz + 1, w.scan, s)) return rc;
     hipLaunchKernelGGL(narrow_kernel, dim3(grid_of(A_nnz + 1, kBlock)), dim3(kBlock), 0, s, A_nnz + 1, w.count, p.a.ptr);
     NM_LAUNCH_CHECK("narrow_kernel");
+    look_at(A_nnz, p.a, p.flags + 1);
+    // B's entries
+    hipLaunchKernelGGL(row_products_kernel, dim3(grid_of(B_rows + 1, kBlock)), dim3(kBlock), 0, s, B_rows, B_indptr, t.t_indptr, w.count);
+    NM_LAUNCH_CHECK("row_products_kernel");
+    if (int rc = nm::scan_exclusive_i64(w.count, B_rows + 1, w.scan, s)) return rc;
+    const int64_t b_blocks = std::min<int64_t>(nm::ceil_div(B_rows, kBlock / kWave), 65536);
+    hipLaunchKernelGGL(b_ptr_kernel, dim3((unsigned)b_blocks), dim3(kBlock), 0, s, B_rows, products, B_indptr, t.t_indptr, w.count, p.b);
+    NM_LAUNCH_CHECK("b_ptr_kernel");
+    look_at(B_nnz, p.b, p.flags + 1);
     // C's entries
     if (int rc = nm::fill_async(w.count, C_nnz + 1, (int64_t)0, s)) return rc;
-    const int64_t row_blocks = std::min<int64_t>(nm::ceil_div(A_rows, kBlock / kWave), 65536);
-    hipLaunchKernelGGL(products_kernel, dim3((unsigned)row_blocks), dim3(kBlock), 0, s, A_rows, A_indices, A_indptr, B_indices,
+    const dim3 each(grid_of(products, kBlock));
+    hipLaunchKernelGGL(products_kernel, each, dim3(kBlock), 0, s, products, A_rows, A_nnz, A_indices, A_indptr, B_indices,
                        B_indptr, C_indices, C_indptr, p.a, w.entry, (unsigned long long *)w.count);
     NM_LAUNCH_CHECK("products_kernel");
     if (int rc = nm::scan_exclusive_i64(w.count, C_nnz + 1, w.scan, s)) return rc;
     hipLaunchKernelGGL(narrow_kernel, dim3(grid_of(C_nnz + 1, kBlock)), dim3(kBlock), 0, s, C_nnz + 1, w.count, p.c.ptr);
     hipLaunchKernelGGL(narrow_kernel, dim3(grid_of(C_nnz, kBlock)), dim3(kBlock), 0, s, C_nnz, w.count, w.cursor);
     NM_LAUNCH_CHECK("narrow_kernel");
-    hipLaunchKernelGGL(place_kernel, dim3(grid_of(products, kBlock)), dim3(kBlock), 0, s, products, p.a.u, w.cursor, w.raw);
-    NM_LAUNCH_CHECK("place_kernel");
-    hipLaunchKernelGGL(order_kernel, dim3(grid_of(C_nnz, kBlock)), dim3(kBlock), 0, s, C_nnz, w.raw, w.entry, p.a.v, p.c);
-    NM_LAUNCH_CHECK("order_kernel");
-    // B's entries
-    hipLaunchKernelGGL(row_products_kernel, dim3(grid_of(B_rows + 1, kBlock)), dim3(kBlock), 0, s, B_rows, B_indptr, t.t_indptr, w.count);
-    NM_LAUNCH_CHECK("row_products_kernel");
-    if (int rc = nm::scan_exclusive_i64(w.count, B_rows + 1, w.scan, s)) return rc;
-    const int64_t b_blocks = std::min<int64_t>(nm::ceil_div(B_rows, kBlock / kWave), 65536);
-    hipLaunchKernelGGL(b_lists_kernel, dim3((unsigned)b_blocks), dim3(kBlock), 0, s, B_rows, B_indptr, t.t_indptr, t.t_perm, w.count, p.a, p.b);
-    hipLaunchKernelGGL(last_ptr_kernel, dim3(1), dim3(1), 0, s, p.b.ptr + B_nnz, (int32_t)products);
-    NM_LAUNCH_CHECK("b_lists_kernel");
-    // within the limit?
-    if (int rc = nm::fill_async(p.flags, (int64_t)1, (int32_t)0, s)) return rc;
-    for (auto [n, list] : {std::pair<int64_t, const Lists *>{C_nnz, &p.c}, {A_nnz, &p.a}, {B_nnz, &p.b}}) {
-        const int per_block = kBlock * per_lane(n, products);
-        hipLaunchKernelGGL(busiest_kernel, dim3(grid_of(nm::ceil_div(n, per_block), kBlock)), dim3(kBlock), 0, s, n, per_block, list->ptr, p.flags);
-    }
+    look_at(C_nnz, p.c, p.flags);
     NM_LAUNCH_CHECK("busiest_kernel");
-    int32_t over = 0;
-    NM_HIP_TRY(hipMemcpyAsync(&over, p.flags, 4, hipMemcpyDeviceToHost, s));
+    int32_t most[2] = {0, 0};
+    NM_HIP_TRY(hipMemcpyAsync(most, p.flags, sizeof(most), hipMemcpyDeviceToHost, s));
     NM_HIP_TRY(hipStreamSynchronize(s));
-    *usable = over == 0;
+    if (most[0] > kBusiest || most[1] > kBusiest) return NM_OK;
+    // the lists; C's products are put into ascending order entry by entry (in the meantime c.u is scratch)
+    hipLaunchKernelGGL(place_kernel, each, dim3(kBlock), 0, s, products, p.a.u, w.cursor, w.raw);
+    NM_LAUNCH_CHECK("place_kernel");
+    if (int rc = nm::segments_sort_i32(nullptr, C_nnz, products, p.c.ptr, w.raw, p.c.u, s)) return rc;
+    hipLaunchKernelGGL(c_lists_kernel, each, dim3(kBlock), 0, s, products, w.raw, w.entry, p.a.v, p.c);
+    NM_LAUNCH_CHECK("c_lists_kernel");
+    *usable = most[1] > kBusiestBack ? 2 : 1;
+    if (*usable == 2) return NM_OK;
+    hipLaunchKernelGGL(b_lists_kernel, each, dim3(kBlock), 0, s, products, B_rows, B_nnz, B_indptr, t.t_indptr, t.t_perm, p.a, p.b);
+    NM_LAUNCH_CHECK("b_lists_kernel");
     return NM_OK;
 }
 

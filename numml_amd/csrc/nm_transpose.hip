@@ -679,10 +679,10 @@ int rows_plan_build(int64_t rows, int64_t cols, int64_t nnz, const int64_t *indi
 int segments_sort_i32(const int32_t *nseg_dev, int64_t nseg_max, int64_t nkeys, const int32_t *seg_ptr,
                       int32_t *keys, int32_t *tmp, hipStream_t s) {
     if (nkeys <= 0 || nseg_max <= 0) return NM_OK;
-    // few segments per workgroup: their number is not known here, and they may be long
-    const int ct = 8;
+    // few segments per workgroup where their number is not known here, and they may be long
+    const int ct = nseg_dev ? 8 : tile_rows(nseg_max, nkeys, 1);
     int64_t grid = xcd_padded(ceil_div(nseg_max, ct));
-    if (grid > 8192) grid = 8192;
+    if (grid > (nseg_dev ? 8192 : 65536)) grid = nseg_dev ? 8192 : 65536;
     hipLaunchKernelGGL(tp_order_kernel<false>, dim3((unsigned)grid), dim3(kBlock), 0, s, nseg_max, nseg_dev, ct, seg_ptr,
                        keys, (const int32_t *)nullptr, (int32_t *)nullptr, tmp);
     NM_LAUNCH_CHECK("tp_order_kernel (segments)");

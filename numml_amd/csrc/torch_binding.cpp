@@ -670,7 +670,7 @@ bool plan_of_sizes(char kind, const Tensor &A_indices, const Tensor &A_indptr, c
 
 // A product beyond the records: the plan that lists its products (nm_spgemm_lists_build), where its 24 bytes a
 // product are at most a quarter of the cache.  Returns the plan's class, 0 where there is none.
-constexpr int kListClass = 100;
+constexpr int kListClass = 100, kListForwardClass = 101;   // the latter: for forward passes only
 int list_plan(Plan &plan, const Tensor &A_indices, const Tensor &A_indptr, const Tensor &B_indices, const Tensor &B_indptr,
               const Tensor &C_indices, const Tensor &C_indptr, int64_t A_rows, int64_t A_cols, const c10::Device &dev) {
     const int64_t A_nnz = A_indices.numel(), B_nnz = B_indices.numel(), C_nnz = C_indices.numel();
@@ -693,7 +693,7 @@ int list_plan(Plan &plan, const Tensor &A_indices, const Tensor &A_indptr, const
                                 plan.mem.data_ptr(), pbytes, work.data_ptr(), wbytes, &usable, stream),
           "nm_spgemm_lists_build");
     plan.products = products;
-    return usable ? kListClass : 0;
+    return usable == 1 ? kListClass : usable == 2 ? kListForwardClass : 0;
 }
 
 // After a stateless forward pass of a product without hash-path rows: notes the pair, or makes
@@ -1328,7 +1328,7 @@ std::vector<Tensor> spgemm_forward(int A_rows, int A_cols, Tensor A_data, Tensor
     auto on_plan = [&](const Plan &plan) -> std::vector<Tensor> {
         const Tensor &C_indices = plan.derived[0], &C_indptr = plan.derived[1];
         Tensor C_data = torch::empty({C_indices.numel()}, A_data.options());
-        if (plan.plan_class == kListClass) {
+        if (plan.plan_class >= kListClass) {
             check(nm_spgemm_numeric_lists(dtype_of(A_data), A_data.numel(), B_data.numel(), C_indices.numel(), plan.products,
                                           A_data.data_ptr(), B_data.data_ptr(), plan.mem.data_ptr(), C_data.data_ptr(),
                                           current_stream(dev)),
@@ -1433,7 +1433,7 @@ std::vector<Tensor> spgemm_backward(Tensor grad_C, Tensor C_indices, Tensor C_in
     if (backward_mode_now() != kAtomic) {
         // the product plan applies when grad_C lies on the very pattern tensors the plan handed out
         auto pp = peek_product_plan(A_indices, A_indptr, B_indices, B_indptr, A_rows, B_cols, dev);
-        if (pp && pp->usable && pp->derived[0].data_ptr() == C_indices.data_ptr() &&
+        if (pp && pp->usable && pp->plan_class != kListForwardClass && pp->derived[0].data_ptr() == C_indices.data_ptr() &&
             pp->derived[1].data_ptr() == C_indptr.data_ptr() && pp->derived[0].numel() == C_indices.numel()) {
             g_last_spgemm_backward.store(kOnProductPlan, std::memory_order_relaxed);
             if (pp->plan_class == kListClass) {

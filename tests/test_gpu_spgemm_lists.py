@@ -91,6 +91,93 @@ def test_a_busy_workgroup_is_refused(dev, dtype):
             assert_close(host(g), w, "gradient")
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n", [127, 128, 129, 4096, 4097, 9000, 40_000])
+def test_an_entry_of_many_products(dev, dtype, n):
+    """One entry of C with n products, in the serial loop's order (put there by rank below 128 of them, sorted in LDS
+    up to 4096 and in pieces beyond).  The row of 40 entries keeps the product off the records."""
+    ops = _binding.ops
+    ops.clear_plan_cache()
+    ai, ap = np.arange(n), np.array([0, n], np.int64)
+    lengths = np.ones(n, np.int64)
+    lengths[n // 3] = 40
+    bp = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int64)
+    bi = np.concatenate([np.arange(m) for m in lengths]).astype(np.int64)
+    ad, bd = randn(n, n, dtype), randn(n + 1, bi.size, dtype)
+    ref = oracle.spgemm_forward(1, n, ad, ai, ap, n, 40, bd, bi, bp)
+    gC = randn(n + 2, ref[0].shape, dtype)
+    want = oracle.spgemm_backward(gC, ref[1], ref[2], 1, n, ad, ai, ap, n, 40, bd, bi, bp)
+    A, B, Gd = to_dev(dev, ad, ai, ap), to_dev(dev, bd, bi, bp), to_dev(dev, gC)[0]
+    for k in range(3):
+        C = ops.spgemm_forward(1, n, *A, n, 40, *B)
+        (assert_same if k == 2 else assert_close)(host(C[0]), ref[0], "values")
+    got = ops.spgemm_backward(Gd, C[1], C[2], 1, n, *A, n, 40, *B)
+    assert ops.last_backward_paths()[1] == "product plan"
+    for g, w in zip(got, want):
+        assert_same(host(g), w, "gradient")
+
+
+def _build(dev, A, B, C, products):
+    """`usable` of nm_spgemm_lists_build for patterns (indices, indptr, shape)."""
+    L, plan, work, usable = _lib.lib(), ctypes.c_size_t(), ctypes.c_size_t(), ctypes.c_int(-1)
+    (ai, ap, (m, k)), (bi, bp, _), (ci, cp, _) = A, B, C
+    t = [to_dev(dev, *x[:2]) for x in (A, B, C)]
+    assert L.nm_csr_transpose_plan_bytes(m, k, ai.size, plan, work) == 0
+    tp, tw = (torch.empty(s.value, dtype=torch.uint8, device=dev) for s in (plan, work))
+    assert L.nm_csr_transpose_plan_build(m, k, ai.size, t[0][0].data_ptr(), t[0][1].data_ptr(), tp.data_ptr(), plan, tw.data_ptr(), work, None) == 0
+    assert L.nm_spgemm_lists_bytes(k, ai.size, bi.size, ci.size, products, plan, work) == 0
+    lp, lw = (torch.empty(s.value, dtype=torch.uint8, device=dev) for s in (plan, work))
+    ptrs = [x.data_ptr() for pair in t for x in pair]
+    assert L.nm_spgemm_lists_build(m, k, ai.size, bi.size, ci.size, products, *ptrs, tp.data_ptr(), lp.data_ptr(), plan,
+                                   lw.data_ptr(), work, usable, None) == 0
+    torch.cuda.synchronize()
+    return usable.value
+
+
+def test_what_is_refused_depends_on_the_counts(dev):
+    """On either side of 65 536 products in a workgroup of C (one entry, and many entries that share one) and of 16 384 and
+    65 536 in one of a gradient."""
+    rows = lambda lengths, cols, pick: (np.concatenate([pick(r, n) for r, n in enumerate(lengths)]).astype(np.int64),
+                                        np.concatenate([[0], np.cumsum(lengths)]).astype(np.int64), (len(lengths), cols))
+    first = lambda r, n: np.arange(n)
+    full = lambda m, n: rows([n] * m, n, first)
+    # one entry of C with all products, alone (known from the sizes) and among 2048 more entries (counted)
+    for n, usable in ((65_536, 1), (65_537, 0)):
+        assert _build(dev, full(1, n), rows([1] * n, 1, first), full(1, 1), n) == usable
+    more = 2048
+    for n, usable in ((65_536 - 255, 1), (65_536 - 254, 0)):
+        A = rows([n] + [1] * more, n + more, lambda r, m: np.arange(m) if r == 0 else np.array([n + r - 1]))
+        B = rows([1] * (n + more), 1, first)
+        assert _build(dev, A, B, full(1 + more, 1), n + more) == usable
+    # 256 entries of A with n products each, as many entries of B (one row) with 256
+    for n, usable in ((64, 1), (65, 2), (256, 2), (257, 0)):
+        assert _build(dev, full(256, 1), full(1, n), full(256, n), 256 * n) == usable
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n, planned", [(64, True), (65, False)])
+def test_gradients_of_busy_workgroups_go_without_the_plan(dev, dtype, n, planned):
+    ops = _binding.ops
+    ops.clear_plan_cache()
+    ad, bd = randn(1, 256, dtype), randn(2, n, dtype)
+    ai, ap = np.zeros(256, np.int64), np.arange(257)
+    bi, bp = np.arange(n), np.array([0, n], np.int64)
+    A, B = to_dev(dev, ad, ai, ap), to_dev(dev, bd, bi, bp)
+    ref = oracle.spgemm_forward(256, 1, ad, ai, ap, 1, n, bd, bi, bp)
+    gC = randn(3, ref[0].shape, dtype)
+    want = oracle.spgemm_backward(gC, ref[1], ref[2], 256, 1, ad, ai, ap, 1, n, bd, bi, bp)
+    for k in range(3):
+        C = ops.spgemm_forward(256, 1, *A, 1, n, *B)
+        assert_same(host(C[0]), ref[0], "values")
+        got = ops.spgemm_backward(to_dev(dev, gC)[0], C[1], C[2], 256, 1, *A, 1, n, *B)
+        for g, w in zip(got, want):
+            assert_close(host(g), w, "gradient")
+    assert (ops.last_backward_paths()[1] == "product plan") == planned
+    built = ops.plan_cache_stats()[0]
+    C2 = ops.spgemm_forward(256, 1, *A, 1, n, *B)
+    assert C2[1].data_ptr() == C[1].data_ptr() and ops.plan_cache_stats()[0] == built, "the forward is on the plan"
+
+
 def test_sizes_and_memory_are_checked(dev):
     L = _lib.lib()
     n = ctypes.c_int64()
