@@ -3,12 +3,12 @@
 // Work mapping ("row-block streaming"): one 256-lane workgroup owns R
 // consecutive rows.  It stages the rows' offsets in LDS and, when the block's
 // stored entries fit the LDS tile, walks them with fully coalesced loads of
-// `data` and `indices` (lane k takes entry k), leaving the per-entry results in
-// LDS; one lane per row then adds its row's slice in storage order, which is
-// the summation order of the serial CPU loop (cpp/sparse_csr_cpu.cpp:29-35),
-// so short rows reproduce it bit for bit.  Blocks whose entries do not fit
-// (long rows) switch to one wavefront per long row with a cross-lane
-// reduction, and one lane per short row.
+// `data` and `indices`, leaving the per-entry results in LDS; blocks whose
+// entries do not fit take runs of rows that do, one after the other.  One lane
+// per row then adds its row's slice in storage order, which is the summation
+// order of the serial CPU loop (cpp/sparse_csr_cpu.cpp:29-35), so rows of fewer
+// than kLongRow entries reproduce it bit for bit.  Longer rows are added by a
+// wavefront each, entry k by lane k % 64, in every tile and kernel of this file.
 //
 // Algorithmic HBM bytes, s = sizeof(value):
 //   forward : nnz*(s+8) + (rows+1)*8 + cols*s + rows*s
@@ -28,7 +28,7 @@ using nm::kWave;
 
 constexpr int kBlock = 256;
 constexpr int kWavesPerBlock = kBlock / kWave;
-// Rows of at least this many entries get a whole wavefront on the long-row path.
+// Rows of at least this many entries get a whole wavefront.
 constexpr int kLongRow = 32;
 
 template <typename T> struct Tile;
@@ -153,29 +153,37 @@ template <typename T> __device__ __forceinline__ T serial_sum(const T *s_prod, i
     return acc;
 }
 
-// Sums of a wavefront's slices [b, e) of the products in LDS, one a lane, left at out[t] where `on` (t ascends with the
-// lanes; a slice is empty where it is not on): by the lane in storage order, and slices of kLongRow products by the
+// Sum of a lane's slice [b, e) of the products in LDS (all lanes of a wavefront call it; empty where b == e): by the lane in
+// storage order, and slices of kLongRow products by the
 // wavefront, lane l adding products l, l + 64, ... before the lanes are summed.  A workgroup waits for the longest row
 // of its tile.  Forward, graphs in fp32, a lane for every row and a trip to LDS for every product -> this, with small
 // tiles (launch_fwd): 100 000 rows, 1.2 M entries 53 -> 15.7 us; 20 000 rows of up to 5000 entries 63 -> 5.5; 400 000 rows,
 // 7.6 M entries 122 -> 68.  (A line at 64 or 128: the same within 3 %.  The error of a long row's sum against 64 bits is
-// smaller in this order: 6.13e-8 -> 5.98e-8 over 30 000 rows of 26.)
-template <bool STREAM, typename T>
-__device__ __forceinline__ void slice_sums(const T *s_prod, int b, int e, bool on, T *__restrict__ out, int t) {
+// smaller in this order: 6.13e-8 -> 5.98e-8 over 30 000 rows of 26.)  Every tile of a kernel sums by it, so a row's bits do
+// not depend on the tile it is in.
+template <typename T> __device__ __forceinline__ T slice_sum(const T *s_prod, int b, int e) {
     const int lane = threadIdx.x & (kWave - 1);
     const bool wide = e - b >= kLongRow;
-    if (on && !wide) {
-        if constexpr (STREAM) nm::stream_store(out + t, serial_sum(s_prod, b, e));
-        else out[t] = serial_sum(s_prod, b, e);
-    }
+    T total = 0;
+    if (!wide) total = serial_sum(s_prod, b, e);
     for (unsigned long long todo = __ballot(wide); todo; todo &= todo - 1) {
         const int src = __builtin_ctzll(todo);
         const int wb = __shfl(b, src, kWave), we = __shfl(e, src, kWave);
         T acc = 0;
         for (int j = wb + lane; j < we; j += kWave) acc += s_prod[j];
         acc = nm::wave_sum(acc);
-        if (lane == 0) out[t + src] = acc;
+        if (lane == src) total = acc;
     }
+    return total;
+}
+
+// The same, left at out[t] where `on` (a slice is empty where it is not on).
+template <bool STREAM, typename T>
+__device__ __forceinline__ void slice_sums(const T *s_prod, int b, int e, bool on, T *__restrict__ out, int t) {
+    const T total = slice_sum(s_prod, b, e);
+    if (!on) return;
+    if constexpr (STREAM) nm::stream_store(out + t, total);
+    else out[t] = total;
 }
 
 // Rows [s0, e0) of a tile whose products lie in LDS from s_off[s0] - o0 on.
@@ -306,10 +314,7 @@ __device__ __forceinline__ void fwd_tile_staged(const int64_t r0, const int nr, 
         }
     }
     __syncthreads();
-    // storage-order sums of the lane's two rows
-    T acc0 = 0, acc1 = 0;
-    for (int j = p0 - base; j < p1 - base; ++j) acc0 += s_prod[j];
-    for (int j = p1 - base; j < p2 - base; ++j) acc1 += s_prod[j];
+    const T acc0 = slice_sum(s_prod, p0 - base, p1 - base), acc1 = slice_sum(s_prod, p1 - base, p2 - base);
     if (2 * tid + 1 < nr) {
         T2 out;
         out[0] = acc0, out[1] = acc1;
