@@ -148,9 +148,11 @@ int nm_csr_transpose_backward(nm_dtype dt, int64_t nnz, const void *grad_At,
                               const int64_t *At_to_A_idx, void *grad_A, nm_stream stream);
 
 /* The same gradient by the transposed-structure plan that the transpose was made with, in place of its
- * At_to_A_idx (which nm_csr_transpose_forward does not write where it is NULL). */
-int nm_csr_transpose_backward_planned(nm_dtype dt, int64_t rows, int64_t cols, int64_t nnz, const void *grad_At,
-                                      const void *plan_mem, void *grad_A, nm_stream stream);
+ * At_to_A_idx (which nm_csr_transpose_forward does not write where it is NULL): of the plan it reads `bytes`
+ * bytes from `offset` on, about 4 an entry, which may be kept by themselves.  No counterpart in the reference. */
+int nm_csr_transpose_part(int64_t rows, int64_t cols, int64_t nnz, size_t *offset, size_t *bytes);
+int nm_csr_transpose_backward_planned(nm_dtype dt, int64_t nnz, const void *grad_At, const void *part, void *grad_A,
+                                      nm_stream stream);
 
 /* nm_spgemv_forward for a pattern whose transposed-structure plan has been
  * built: the kernel reads the plan's 32-bit copies of A's column indices and

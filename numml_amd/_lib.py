@@ -105,7 +105,8 @@ _SIGNATURES = {
     "nm_csr_transpose_forward": [_c_int, _c_i64, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr,
                                  _c_ptr],
     "nm_csr_transpose_backward": [_c_int, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr],
-    "nm_csr_transpose_backward_planned": [_c_int, _c_i64, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr],
+    "nm_csr_transpose_part": [_c_i64, _c_i64, _c_i64, ctypes.POINTER(_c_size), ctypes.POINTER(_c_size)],
+    "nm_csr_transpose_backward_planned": [_c_int, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr],
     "nm_splincomb_workspace_bytes": [_c_i64, ctypes.POINTER(_c_size)],
     "nm_splincomb_symbolic": [_c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_size, _c_ptr],
     "nm_splincomb_numeric": [_c_int, _c_i64, _c_dbl, _c_ptr, _c_ptr, _c_ptr, _c_dbl, _c_ptr, _c_ptr, _c_ptr,

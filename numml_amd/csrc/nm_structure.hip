@@ -647,21 +647,29 @@ extern "C" int nm_csr_transpose_backward(nm_dtype dt, int64_t nnz, const void *g
     return NM_OK;
 }
 
-extern "C" int nm_csr_transpose_backward_planned(nm_dtype dt, int64_t rows, int64_t cols, int64_t nnz, const void *grad_At,
-                                                 const void *plan_mem, void *grad_A, nm_stream stream) {
+extern "C" int nm_csr_transpose_part(int64_t rows, int64_t cols, int64_t nnz, size_t *offset, size_t *bytes) {
     NM_REQUIRE(rows >= 0 && cols >= 0 && nnz >= 0, "negative size");
+    NM_REQUIRE(offset && bytes, "null output");
+    *offset = nm::perm_part_offset(cols, nnz);
+    *bytes = nm::perm_part_layout(nnz, nullptr, nullptr, nullptr);
+    return NM_OK;
+}
+
+extern "C" int nm_csr_transpose_backward_planned(nm_dtype dt, int64_t nnz, const void *grad_At, const void *part, void *grad_A,
+                                                 nm_stream stream) {
+    NM_REQUIRE(nnz >= 0, "negative size");
     NM_REQUIRE(dt == NM_F32 || dt == NM_F64, "bad dtype %d", (int)dt);
     if (nnz == 0) return NM_OK;
-    NM_REQUIRE(grad_At && plan_mem && grad_A, "null pointer argument");
-    nm::TPlan plan;
-    nm::tplan_layout(rows, cols, nnz, const_cast<void *>(plan_mem), &plan);
+    NM_REQUIRE(grad_At && part && grad_A, "null pointer argument");
+    const int32_t *t_perm = nullptr, *flags = nullptr;
+    nm::perm_part_layout(nnz, part, &t_perm, &flags);
     hipStream_t s = nm::as_stream(stream);
     if (dt == NM_F32)
         hipLaunchKernelGGL(transpose_back_kernel<float>, dim3(grid_for(nnz)), dim3(kBlock), 0, s, nnz, (const float *)grad_At,
-                           plan.t_perm, plan.flags, (float *)grad_A);
+                           t_perm, flags, (float *)grad_A);
     else
         hipLaunchKernelGGL(transpose_back_kernel<double>, dim3(grid_for(nnz)), dim3(kBlock), 0, s, nnz, (const double *)grad_At,
-                           plan.t_perm, plan.flags, (double *)grad_A);
+                           t_perm, flags, (double *)grad_A);
     NM_LAUNCH_CHECK("transpose_back_kernel");
     return NM_OK;
 }

@@ -105,6 +105,16 @@ inline size_t tplan_layout(int64_t rows, int64_t cols, int64_t nnz, void *base, 
     return off;
 }
 
+// The part of the plan that takes a gradient of the transpose back to A (t_perm, chunk_row and flags as they lie in
+// tplan_layout, about 4 bytes an entry): where it begins, and its arrays.
+inline size_t perm_part_offset(int64_t cols, int64_t nnz) { return align256((size_t)(cols + 1) * 4) + align256((size_t)(nnz + 1) * 4); }
+inline size_t perm_part_layout(int64_t nnz, const void *base, const int32_t **t_perm, const int32_t **flags) {
+    const size_t at = align256((size_t)(nnz + 1) * 4) + align256((size_t)((nnz + 63) / 64 + 1) * 4);
+    if (t_perm) *t_perm = (const int32_t *)base;
+    if (flags) *flags = (const int32_t *)((const char *)base + at);
+    return at + align256(16 * 4);
+}
+
 // The part of the plan that a walk by row reads (c_ptr32, c_idx32, c_off16, f_desc, flags) by itself, for
 // patterns that are only multiplied from the left: 6 bytes an entry and two passes.
 inline size_t rows_plan_layout(int64_t rows, int64_t nnz, void *base, TPlan *p) {

@@ -950,7 +950,7 @@ std::vector<Tensor> spgemv_backward(Tensor grad_z, int A_rows, int A_cols, Tenso
 
 // ----------------------------------------------------------------------- transpose
 
-// {At_data, At_indices, At_indptr, At_to_A}, or with the plan's memory in place of At_to_A.
+// {At_data, At_indices, At_indptr, At_to_A}, or with the part of the plan that stands for At_to_A in its place.
 std::vector<Tensor> transpose_values(int A_rows, int A_columns, Tensor A_data, Tensor A_indices, Tensor A_indptr,
                                      bool want_map) {
     check_csr("csr_transpose_forward", A_rows, A_columns, A_data, A_indices, A_indptr);
@@ -965,7 +965,14 @@ std::vector<Tensor> transpose_values(int A_rows, int A_columns, Tensor A_data, T
     Tensor At_data = torch::empty_like(A_data);
     Tensor At_indices = torch::empty({nnz}, iopt);
     Tensor At_indptr = torch::empty({(int64_t)A_columns + 1}, iopt);
-    Tensor At_to_A = want_map ? torch::empty({nnz}, iopt) : plan->mem;
+    Tensor At_to_A;
+    if (want_map) {
+        At_to_A = torch::empty({nnz}, iopt);
+    } else {
+        size_t offset = 0, bytes = 0;
+        check(nm_csr_transpose_part(A_rows, A_columns, nnz, &offset, &bytes), "nm_csr_transpose_part");
+        At_to_A = plan->mem.narrow(0, (int64_t)offset, (int64_t)bytes);
+    }
     check(nm_csr_transpose_forward(dtype_of(A_data), A_rows, A_columns, nnz, A_data.data_ptr(),
                                    plan->mem.data_ptr(), At_data.data_ptr(), At_indices.data_ptr<int64_t>(),
                                    At_indptr.data_ptr<int64_t>(), want_map ? At_to_A.data_ptr<int64_t>() : nullptr,
@@ -1866,13 +1873,12 @@ struct SpgemmNode : torch::autograd::Function<SpgemmNode> {
     }
 };
 
-// (keeps the plan's memory, which the cache may drop meanwhile, instead of a permutation of 8 bytes an entry)
+// (keeps a view of the part of the plan that the backward reads, about 4 bytes an entry, instead of a permutation of 8.
+// Hooks that pack saved tensors see that part alone; a plan that the cache drops meanwhile lives as long as the node.)
 struct TransposeNode : torch::autograd::Function<TransposeNode> {
     static variable_list forward(AutogradContext *ctx, int64_t rows, int64_t cols, const Tensor &A, const Tensor &ci, const Tensor &cp) {
         variable_list t = transpose_values((int)rows, (int)cols, A, ci, cp, false);
         ctx->save_for_backward({t[3]});
-        ctx->saved_data["rows"] = rows;
-        ctx->saved_data["cols"] = cols;
         ctx->saved_data["nnz"] = A.numel();
         ctx->saved_data["dtype"] = (int64_t)A.scalar_type();
         t.pop_back();
@@ -1881,18 +1887,18 @@ struct TransposeNode : torch::autograd::Function<TransposeNode> {
         return t;
     }
     static variable_list backward(AutogradContext *ctx, variable_list grad) {
-        const Tensor plan = ctx->get_saved_variables()[0];
+        const Tensor part = ctx->get_saved_variables()[0];
         const int64_t nnz = ctx->saved_data["nnz"].toInt();
         const auto dtype = (c10::ScalarType)ctx->saved_data["dtype"].toInt();
-        c10::hip::HIPGuard guard(plan.device().index());
-        Tensor grad_A = torch::empty({nnz}, plan.options().dtype(dtype));
+        c10::hip::HIPGuard guard(part.device().index());
+        Tensor grad_A = torch::empty({nnz}, part.options().dtype(dtype));
         if (!grad[0].defined()) return {Tensor(), Tensor(), grad_A.zero_(), Tensor(), Tensor()};
         check_vector("csr_transpose_backward", "grad_At", grad[0], nnz);
         same_dtype(grad_A, grad[0], "grad_At");
         const Tensor g = grad[0].contiguous();
-        const auto dev = need_device({&g, &plan});
-        check(nm_csr_transpose_backward_planned(dtype_of(g), ctx->saved_data["rows"].toInt(), ctx->saved_data["cols"].toInt(), nnz,
-                                                g.data_ptr(), plan.data_ptr(), grad_A.data_ptr(), current_stream(dev)),
+        const auto dev = need_device({&g, &part});
+        check(nm_csr_transpose_backward_planned(dtype_of(g), nnz, g.data_ptr(), part.data_ptr(), grad_A.data_ptr(),
+                                                current_stream(dev)),
               "nm_csr_transpose_backward_planned");
         return {Tensor(), Tensor(), grad_A, Tensor(), Tensor()};
     }

@@ -108,6 +108,15 @@ def test_saved_tensor_hooks_are_seen(dev, name):
         assert np.allclose(host(a), host(b), rtol=1e-12)
 
 
+def test_a_transpose_saves_no_more_than_its_permutation(dev):
+    """Hooks that pack saved tensors (offloading) get at most the 8 bytes an entry that At_to_A has."""
+    A = _grid(dev)
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(t.numel() * t.element_size()) or t, lambda t: t):
+        A.T
+    assert 0 < sum(packed) <= 8 * A.nnz
+
+
 @pytest.mark.parametrize("mode", ["planned", "eager"])
 def test_an_evaluation_pass_first(dev, mode):
     """Plans and pattern tensors made under torch.inference_mode() serve a training pass on the same patterns."""
