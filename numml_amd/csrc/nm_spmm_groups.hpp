@@ -47,7 +47,12 @@ constexpr int kPass = 4;           // entries of a shared row a group takes at o
 // (1 M rows of 37 columns: 650 -> 785 us, the slices of a row share lines).
 constexpr int kSliceLanes = 8;
 constexpr int64_t kFewBlocks = 2048, kFewRows = 64;
-constexpr int kScan = kThreads;    // rows a workgroup at the head of the grid looks through
+constexpr int kScan = kThreads;    // rows a workgroup at the head of the grid looks through,
+// in kPlaces places far apart, so that neighbouring long rows (a sorted graph, a block of dense rows) get workgroups
+// of their own: with 256 neighbours a workgroup one had them all.  fp32, 64 columns, rows of 4 entries and among them 256
+// neighbours of 500: 1 M rows 4920 -> 192 us, 200 000 rows 1330 -> 59; power-law rows in descending order, 200 000: 4850 -> 336.
+// (A row by itself each: a line of row pointers a row, 1 M rows of 12 entries 242 -> 248 us at 16 columns.)
+constexpr int kPlaces = 32;
 constexpr int kDrawRows = 4;       // rows of a workgroup per group: enough to draw from, few enough that the
                                    // rows of `own` (16 KB) leave room for eight workgroups a compute unit
 
@@ -74,6 +79,8 @@ template <typename T, typename IDX> struct Args {
     int64_t ldw;
     T *dots;
     int scan_rows;            // rows each of the workgroups that look for long rows looks through
+    int stripe;               // neighbours among these, as a power of two
+    int64_t scan_sets;        // parts the rows are dealt into for that
     unsigned scan_blocks;     // workgroups that look for long rows, a multiple of nm::kXcds
     unsigned tiles;           // workgroups that walk rows, the same
 };
@@ -214,15 +221,18 @@ __global__ __launch_bounds__(kThreads, 5) void groups_kernel(const Args<T, IDX> 
         const int slices = SLICED ? (a.n + GS * V - 1) / (GS * V) : 1;
         WS w(a, SLICED ? blockIdx.x % slices : 0);
         const int g = t / GS;
-        const int64_t r0 = (int64_t)(blockIdx.x / slices) * a.scan_rows;
+        const int64_t set = blockIdx.x / slices;
+        auto row_of = [&](int place) { return (((place >> a.stripe) * a.scan_sets + set) << a.stripe) + (place & ((1 << a.stripe) - 1)); };
         if (t == 0) s_next = 0;
         __syncthreads();
-        if (t < a.scan_rows && r0 + t < a.rows && (int64_t)(a.ptr[r0 + t + 1] - a.ptr[r0 + t]) > kShared)
-            s_list[atomicAdd(&s_next, 1)] = t;
+        if (t < a.scan_rows && set < a.scan_sets) {
+            const int64_t row = row_of(t);
+            if (row < a.rows && (int64_t)(a.ptr[row + 1] - a.ptr[row]) > kShared) s_list[atomicAdd(&s_next, 1)] = t;
+        }
         __syncthreads();
         const int found = s_next;
         for (int i = 0; i < found; ++i) {   // (the order of the list does not matter)
-            const int64_t row = r0 + s_list[i], b = a.ptr[row], e = a.ptr[row + 1];
+            const int64_t row = row_of(s_list[i]), b = a.ptr[row], e = a.ptr[row + 1];
             T acc[V] = {};
             vec mine{};
             if constexpr (DOT) mine = w.own_row(row);
@@ -463,7 +473,10 @@ int launch_shape(Args<T, IDX> a, hipStream_t s) {
     constexpr bool kMaySlice = !DOT && G > kSliceLanes;
     const bool sliced = kMaySlice && nm::ceil_div(a.rows, kFewRows) < kFewBlocks;
     const int64_t slices = sliced ? nm::ceil_div(a.n, kSliceLanes * V) : 1;
-    const int64_t scan = nm::xcd_padded(nm::ceil_div(a.rows, a.scan_rows) * slices), tiles = nm::xcd_padded(nm::ceil_div(a.rows, rows));
+    a.scan_sets = nm::ceil_div(a.rows, a.scan_rows);
+    a.stripe = 0;
+    while ((kPlaces << a.stripe) < a.scan_rows) ++a.stripe;
+    const int64_t scan = nm::xcd_padded(a.scan_sets * slices), tiles = nm::xcd_padded(nm::ceil_div(a.rows, rows));
     NM_REQUIRE(scan + tiles <= 0x7fffffff, "too many rows");
     a.scan_blocks = (unsigned)scan;
     a.tiles = (unsigned)tiles;

@@ -75,3 +75,35 @@ def test_long_columns_and_rows_off_alignment(dev, dtype):
             assert_same(gB[kept], gB_ref[kept], f"n={n} grad_B, columns in storage order")
     finally:
         ext.BACKWARD_MODE = old
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("rows", [1, 15, 16, 17, 33, 2500, 40_000, 140_000, 300_001])
+def test_long_rows_side_by_side(dev, dtype, rows, mode):
+    """Blocks of long rows among short ones, where the rows are dealt to few and to many workgroups, singly and two and four
+    neighbours at a time."""
+    rng = np.random.default_rng(rows)
+    lengths = rng.integers(0, 3, rows)
+    for at in (0, rows // 2, rows - 20):
+        block = slice(max(at, 0), min(at + 20, rows))
+        lengths[block] = rng.choice([129, 130, 200, 512, 513, 600], block.stop - block.start)
+    cols = 700
+    p = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int64)
+    i = np.concatenate([np.sort(rng.choice(cols, n, replace=False)) if n > 2 else (7 * r + np.arange(n)) % (cols - 1)
+                        for r, n in enumerate(lengths)] + [[]]).astype(np.int64)
+    d = rng.standard_normal(i.size).astype(dtype)
+    t = oracle.csr_transpose(rows, cols, d, i, p)
+    for n in (4, 20):
+        B, gC = randn(3, (cols, n), dtype), randn(4, (rows, n), dtype)
+        C = host(ext.spdmm_forward(rows, cols, *to_dev(dev, d, i, p, B)))
+        C_ref = oracle.spdmm_forward(rows, cols, d, i, p, B)
+        kept = np.diff(p) <= 512
+        assert_same(C[kept], C_ref[kept], f"n={n} C, rows in storage order")
+        assert_close(C, C_ref, f"n={n} C")
+        # the same rows as columns: both gradients
+        ref = oracle.spdmm_backward(cols, rows, *t[:3], gC, B)
+        got = ext.spdmm_backward(cols, rows, *to_dev(dev, *t[:3], gC, B))
+        for g, w, what in zip(got, ref, ("grad_A", "grad_B")):
+            assert_close(host(g), w, f"n={n} {what}")
+        if mode == "eager":
+            assert_same(host(got[1])[kept], ref[1][kept], f"n={n} grad_B, columns in storage order")
