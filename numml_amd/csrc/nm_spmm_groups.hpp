@@ -13,9 +13,9 @@
 // storage order, like the serial loop (cpp/sparse_csr_cpu.cpp:586-598): same bits.  The groups of a
 // workgroup draw rows from a counter in LDS, so one that has a longer row holds nobody up.  Rows of
 // more than kShared entries are left to the workgroups at the head of the grid, which look for them and
-// share each one among all their groups: up to kSplit entries the products meet in LDS and are added in
-// storage order, beyond that chunks of 16 entries are summed and the sums added in order
-// (deterministic, the serial sum up to rounding).
+// share each one among all their groups (or, where they find many, deal them to their groups): up to kSplit entries the
+// products meet in LDS and are added in storage order, beyond that chunks of 16 entries are summed and the sums added in
+// order (deterministic, the serial sum up to rounding).
 //
 // The walk gives out[r, :] = sum of value * dense[index, :] over the entries of row r and, with DOT,
 // dots[position] = <dense[index, :], own[r, :]>: the backward by column needs the same row of gC for
@@ -38,6 +38,14 @@ constexpr int kThreads = 256;
 // their terms in storage order.  (Taken by one group each up to 512 entries, such rows kept the rest of
 // their workgroup waiting: 957 against 650 us.  From 65 entries on: 655 us; from 33: 745.)
 constexpr int kShared = 128, kSplit = 512;
+// Where kAlone eighths of the rows that a workgroup looks through have kShared to kSplit entries, its groups take one each:
+// there long rows are the rule and none keeps the others waiting, while sharing costs two barriers a turn and one group's addition.
+// Rows of 140 to 500 entries throughout, fp32, us, lane = column / all shared / this: 100 000 rows of 140, 16 columns 334 / 446 /
+// 182, 64 columns 449 / 956 / 366; 30 000 of 500, 64 columns 474 / 745 / 319; 3000 of 200, 64 columns 120 / 104 / 28.  (30 000
+// rows, of 16: from 3 or 4 on power-law rows up to 1000 entries take 50 instead of 26 us at 16 columns; from 12 on rows of 0 to 280
+// 236 instead of 157 at 64.  kShared at 192: power-law rows up to 1000 entries 15 % slower.)  Rows around kShared are
+// the least gain: 30 000 of 90 +- 30, fp64, 64 columns 172 / 209 / 207.
+constexpr int kAlone = 3;
 constexpr int kChunk = 16;         // entries of a row a group takes from memory at once
 constexpr int kPass = 4;           // entries of a shared row a group takes at once where their order counts
 // A matrix of few rows leaves compute units free while one workgroup after the other is at work on the
@@ -50,7 +58,7 @@ constexpr int64_t kFewBlocks = 2048, kFewRows = 64;
 constexpr int kScan = kThreads;    // rows a workgroup at the head of the grid looks through,
 // in kPlaces places far apart, so that neighbouring long rows (a sorted graph, a block of dense rows) get workgroups
 // of their own: with 256 neighbours a workgroup one had them all.  fp32, 64 columns, rows of 4 entries and among them 256
-// neighbours of 500: 1 M rows 4920 -> 192 us, 200 000 rows 1330 -> 59; power-law rows in descending order, 200 000: 4850 -> 336.
+// neighbours of 500: 1 M rows 4930 -> 255 us, 200 000 rows 1330 -> 58; power-law rows in descending order, 200 000: 4840 -> 340.
 // (A row by itself each: a line of row pointers a row, 1 M rows of 12 entries 242 -> 248 us at 16 columns.)
 constexpr int kPlaces = 32;
 constexpr int kDrawRows = 4;       // rows of a workgroup per group: enough to draw from, few enough that the
@@ -103,6 +111,9 @@ struct Walker {
     // rows of the dense operand in flight at once: with 16 too few wavefronts fit (936 against 650 us)
     static constexpr int kBatch = G >= 32 ? 4 : 8;
     static constexpr int kHeld = G < kChunk ? kChunk / G : 1;   // entries of a chunk a lane holds
+    static constexpr int kWidth = V;
+    static constexpr bool kDot = DOT;
+    using value = T;
     using vec = typename Vec<T, V>::type;
     using held = typename Held<T, V>::type;
 
@@ -197,6 +208,61 @@ struct Walker {
     }
 };
 
+// Places 0 .. nr - 1 of a workgroup's rows, each walked by one group in storage order.  The groups draw places from the
+// counter `next`; the first one of each is its own number r.  open(r, row, kc, e, mine) tells whether the row at r is to be
+// walked, and fills in the row, its entries and (DOT) its row of `own`.  A turn of the loop takes a chunk of every
+// group's row, whatever the rows' lengths.
+template <typename W, typename OPEN> __device__ __forceinline__ void walk_rows(W &w, int r, int nr, int *next, OPEN open) {
+    using T = typename W::value;
+    using vec = typename W::vec;
+    constexpr int V = W::kWidth, kBatch = W::kBatch;
+    constexpr bool DOT = W::kDot;
+    typename W::Chunk c;
+    int64_t row = 0, kc = 0, e = 0;
+    T acc[V] = {};
+    vec mine{};
+    auto draw = [&]() {
+        int drawn = 0;
+        if (w.l == 0) drawn = atomicAdd(next, 1);
+        r = __shfl(drawn, w.first, kWave);
+    };
+    auto begin = [&]() {
+        for (; r < nr; draw()) {
+            if (!open(r, row, kc, e, mine)) continue;
+#pragma unroll
+            for (int v = 0; v < V; ++v) acc[v] = T(0);
+            return;
+        }
+    };
+    begin();
+    while (r < nr) {
+        const int cnt = (int)(e - kc < kChunk ? e - kc : kChunk);
+        w.load(c, kc, cnt);
+#pragma unroll
+        for (int j0 = 0; j0 < kChunk; j0 += kBatch) {
+            if (j0 < cnt) {
+                vec d[kBatch];
+#pragma unroll
+                for (int u = 0; u < kBatch; ++u) d[u] = w.gather(c, j0 + u);
+#pragma unroll
+                for (int u = 0; u < kBatch; ++u) {
+                    if (j0 + u < cnt) {
+                        w.add(c, j0 + u, d[u], acc);
+                        if constexpr (DOT) w.multiply(j0 + u, d[u], mine);
+                    }
+                }
+            }
+        }
+        if constexpr (DOT) w.store_dots(c, kc, cnt);
+        kc += cnt;
+        if (kc == e) {
+            w.store_row(row, acc);
+            draw();
+            begin();
+        }
+    }
+}
+
 template <typename T, int V, int G, typename IDX, bool PERM, bool DOT, bool SLICED>
 __global__ __launch_bounds__(kThreads, 5) void groups_kernel(const Args<T, IDX> a) {
     using W = Walker<T, V, G, IDX, PERM, DOT>;
@@ -206,7 +272,7 @@ __global__ __launch_bounds__(kThreads, 5) void groups_kernel(const Args<T, IDX> 
     // the walked rows' rows of `own`; in the workgroups that share rows: products, partial sums
     __shared__ typename W::held s_mem[(DOT ? kRows * G : 1) > kThreads * kPass ? kRows * G : kThreads * kPass];
     typename W::held *const s_own = s_mem, *const s_pass = s_mem;
-    __shared__ int s_list[kScan];
+    __shared__ int s_list[kScan], s_found[2];
     __shared__ int s_next;
     const int t = threadIdx.x;
 
@@ -223,16 +289,33 @@ __global__ __launch_bounds__(kThreads, 5) void groups_kernel(const Args<T, IDX> 
         const int g = t / GS;
         const int64_t set = blockIdx.x / slices;
         auto row_of = [&](int place) { return (((place >> a.stripe) * a.scan_sets + set) << a.stripe) + (place & ((1 << a.stripe) - 1)); };
-        if (t == 0) s_next = 0;
+        // (listed from the front: up to kSplit entries; from the back: more)
+        if (t == 0) {
+            s_next = kGroups;
+            s_found[0] = s_found[1] = 0;
+        }
         __syncthreads();
         if (t < a.scan_rows && set < a.scan_sets) {
             const int64_t row = row_of(t);
-            if (row < a.rows && (int64_t)(a.ptr[row + 1] - a.ptr[row]) > kShared) s_list[atomicAdd(&s_next, 1)] = t;
+            const int64_t n = row < a.rows ? (int64_t)(a.ptr[row + 1] - a.ptr[row]) : 0;
+            if (n > kSplit) s_list[kScan - 1 - atomicAdd(&s_found[1], 1)] = t;
+            else if (n > kShared) s_list[atomicAdd(&s_found[0], 1)] = t;
         }
         __syncthreads();
-        const int found = s_next;
-        for (int i = 0; i < found; ++i) {   // (the order of the list does not matter)
-            const int64_t row = row_of(s_list[i]), b = a.ptr[row], e = a.ptr[row + 1];
+        int split = s_found[0];
+        const int longer = s_found[1];
+        if (split * 8 >= a.scan_rows * kAlone) {
+            walk_rows(w, g, split, &s_next, [&](int r, int64_t &row, int64_t &kc, int64_t &e, vec &mine) {
+                row = row_of(s_list[r]);
+                kc = a.ptr[row];
+                e = a.ptr[row + 1];
+                if constexpr (DOT) mine = w.own_row(row);
+                return true;
+            });
+            split = 0;
+        }
+        for (int i = 0; i < split + longer; ++i) {   // (the order of the list does not matter)
+            const int64_t row = row_of(s_list[i < split ? i : kScan - 1 - (i - split)]), b = a.ptr[row], e = a.ptr[row + 1];
             T acc[V] = {};
             vec mine{};
             if constexpr (DOT) mine = w.own_row(row);
@@ -327,9 +410,7 @@ __global__ __launch_bounds__(kThreads, 5) void groups_kernel(const Args<T, IDX> 
 
     // ---- all other rows, drawn by the groups one at a time ----
     W w(a);
-    constexpr int kBatch = W::kBatch;
     const int g = t / G;
-    typename W::Chunk c;
     const int64_t r0 = nm::xcd_tile(blockIdx.x - a.scan_blocks, a.tiles) * kRows;
     if (r0 >= a.rows) return;
     const int nr = (int)(a.rows - r0 < kRows ? a.rows - r0 : kRows);
@@ -339,58 +420,19 @@ __global__ __launch_bounds__(kThreads, 5) void groups_kernel(const Args<T, IDX> 
     }
     if (t == 0) s_next = kGroups;
     __syncthreads();
-    // A turn of the loop takes a chunk of every group's row, whatever the rows' lengths.  (The first row
-    // of a group is its own number: no draw.)
-    int r = g;
-    int64_t kc = 0, e = 0;
-    T acc[V] = {};
-    vec mine{};
-    auto draw = [&]() {
-        int next = 0;
-        if (w.l == 0) next = atomicAdd(&s_next, 1);
-        r = __shfl(next, w.first, kWave);
-    };
-    auto begin = [&]() {   // on to the next row that has entries and is not shared
-        for (; r < nr; draw()) {
-            kc = s_ptr[r];
-            e = s_ptr[r + 1];
-#pragma unroll
-            for (int v = 0; v < V; ++v) acc[v] = T(0);
-            if (e == kc) {
-                w.store_row(r0 + r, acc);
-            } else if (e - kc <= kShared) {
-                if constexpr (DOT) mine = s_own[r * G + w.l];
-                return;
-            }
+    walk_rows(w, g, nr, &s_next, [&](int r, int64_t &row, int64_t &kc, int64_t &e, vec &mine) {
+        row = r0 + r;
+        kc = s_ptr[r];
+        e = s_ptr[r + 1];
+        if (e == kc) {
+            const T zero[V] = {};
+            w.store_row(row, zero);
+            return false;
         }
-    };
-    begin();
-    while (r < nr) {
-        const int cnt = (int)(e - kc < kChunk ? e - kc : kChunk);
-        w.load(c, kc, cnt);
-#pragma unroll
-        for (int j0 = 0; j0 < kChunk; j0 += kBatch) {
-            if (j0 < cnt) {
-                vec d[kBatch];
-#pragma unroll
-                for (int u = 0; u < kBatch; ++u) d[u] = w.gather(c, j0 + u);
-#pragma unroll
-                for (int u = 0; u < kBatch; ++u) {
-                    if (j0 + u < cnt) {
-                        w.add(c, j0 + u, d[u], acc);
-                        if constexpr (DOT) w.multiply(j0 + u, d[u], mine);
-                    }
-                }
-            }
-        }
-        if constexpr (DOT) w.store_dots(c, kc, cnt);
-        kc += cnt;
-        if (kc == e) {
-            w.store_row(r0 + r, acc);
-            draw();
-            begin();
-        }
-    }
+        if (e - kc > kShared) return false;
+        if constexpr (DOT) mine = s_own[r * G + w.l];
+        return true;
+    });
 }
 
 // Dot products alone: dots[k] = <dense[idx[k], :], own[row of k, :]>, by entry and not by row, since nothing is

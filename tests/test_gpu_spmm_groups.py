@@ -81,7 +81,7 @@ def test_long_columns_and_rows_off_alignment(dev, dtype):
 @pytest.mark.parametrize("rows", [1, 15, 16, 17, 33, 2500, 40_000, 140_000, 300_001])
 def test_long_rows_side_by_side(dev, dtype, rows, mode):
     """Blocks of long rows among short ones, where the rows are dealt to few and to many workgroups, singly and two and four
-    neighbours at a time."""
+    neighbours at a time; in the small ones a workgroup has so many of them that its groups take one each."""
     rng = np.random.default_rng(rows)
     lengths = rng.integers(0, 3, rows)
     for at in (0, rows // 2, rows - 20):
@@ -93,7 +93,7 @@ def test_long_rows_side_by_side(dev, dtype, rows, mode):
                         for r, n in enumerate(lengths)] + [[]]).astype(np.int64)
     d = rng.standard_normal(i.size).astype(dtype)
     t = oracle.csr_transpose(rows, cols, d, i, p)
-    for n in (4, 20):
+    for n in (4, 20, 70, 200) if rows < 100 else (4, 20):
         B, gC = randn(3, (cols, n), dtype), randn(4, (rows, n), dtype)
         C = host(ext.spdmm_forward(rows, cols, *to_dev(dev, d, i, p, B)))
         C_ref = oracle.spdmm_forward(rows, cols, d, i, p, B)
