@@ -28,8 +28,10 @@ using nm::kWave;
 
 constexpr int kBlock = 256;
 constexpr int kWavesPerBlock = kBlock / kWave;
-// Rows of at least this many entries get a whole wavefront.
+// Rows of at least this many entries are added in the order of a wavefront (slice_sum).
 constexpr int kLongRow = 32;
+// A wavefront that has at least so many rows of kLongRow to 2 * kWave entries gives each to its lane.
+constexpr int kManyRows = 6;
 
 template <typename T> struct Tile;
 template <> struct Tile<float>  { static constexpr int R = 512; static constexpr int CAP = 4096; };
@@ -107,14 +109,17 @@ inline int block_rows(int64_t rows, int64_t nnz, int most, int cap) {
     return (int)(r > most ? most : (r < 8 ? 8 : r));
 }
 
-// The same for the kernels whose work is done when a tile's entries have come: tiles of fewer entries than LDS holds
-// where rows are long, and at least 1024 of them where there are rows enough.  (The tail of a power-law graph is the
+// The same for the kernels whose work is done when a tile's entries have come: tiles of long_cap entries where rows are long,
+// and at least 1024 of them where there are rows enough.  (The tail of a power-law graph is the
 // tile with the most entries; a wave that is nearly empty costs as much as a full one.)  Gradient of A,
-// fp32, tiles of up to 4096 entries -> these: 100 000 rows of 12 on average 15.7 -> 10.5 us, 50 000 12.7 -> 7.4, 200 000 of
-// 20 48 -> 36, 400 000 of 20 58 -> 53 (fp64 78 -> 79); row sums of these 13.0 -> 10.9, 13.3 -> 10.2, 41 -> 28, 35 -> 38;
-// 31 500 rows of seven points 5.5 -> 5.1; 512 or 2048 tiles at least: 60 x 55 x 50 fp32 5.3 -> 6.3 and 6.9.
-inline int small_block_rows(int64_t rows, int64_t nnz, int most, int cap) {
-    int r = block_rows(rows, nnz, most, nnz > 8 * rows ? 1024 : cap);
+// fp32, tiles of up to 4096 entries -> 1024: 100 000 rows of 12 on average 15.7 -> 10.5 us, 50 000 12.7 -> 7.4, 200 000 of
+// 20 48 -> 36; rows of 7 in 31 500 5.5 -> 5.1; 512 or 2048 tiles at least: 60 x 55 x 50 fp32 5.3 -> 6.3 and 6.9.
+// Matrices whose rows are all of one length, and large graphs, want more: row sums of 1 M rows of 20, fp64, with 1024 / 2048 / 4096
+// entries 44.6 / 33.9 / 31.4 us, of a graph of 400 000 rows of 20 42.3 / 40.5 / 41.2; gradients of A, rows of 35, 400 000,
+// 89 / 52 / 44, the graph 81.8 / 75.8 / 77.4.  With sums that are added to memory 1024 up to 48 entries a row (1 M rows of 20
+// 316 / 351 / 393), beyond that all that LDS holds (100 000 rows of 150 227 / 194 / 158).
+inline int small_block_rows(int64_t rows, int64_t nnz, int most, int cap, int long_cap) {
+    int r = block_rows(rows, nnz, most, nnz > 8 * rows ? std::min(long_cap, cap) : cap);
     while (r > 16 && rows < (int64_t)r * 1024) r /= 2;
     return r;
 }
@@ -153,22 +158,61 @@ template <typename T> __device__ __forceinline__ T serial_sum(const T *s_prod, i
     return acc;
 }
 
-// Sum of a lane's slice [b, e) of the products in LDS (all lanes of a wavefront call it; empty where b == e): by the lane in
-// storage order, and slices of kLongRow products by the
-// wavefront, lane l adding products l, l + 64, ... before the lanes are summed.  A workgroup waits for the longest row
-// of its tile.  Forward, graphs in fp32, a lane for every row and a trip to LDS for every product -> this, with small
-// tiles (launch_fwd): 100 000 rows, 1.2 M entries 53 -> 15.7 us; 20 000 rows of up to 5000 entries 63 -> 5.5; 400 000 rows,
-// 7.6 M entries 122 -> 68.  (A line at 64 or 128: the same within 3 %.  The error of a long row's sum against 64 bits is
-// smaller in this order: 6.13e-8 -> 5.98e-8 over 30 000 rows of 26.)  Every tile of a kernel sums by it, so a row's bits do
-// not depend on the tile it is in.
-template <typename T> __device__ __forceinline__ T slice_sum(const T *s_prod, int b, int e) {
+// The order of long rows: term l, l + 64, ... to part l, and the 64 parts pairwise (nm::wave_sum).  Here one lane does that for
+// its slice [b, e) of kLongRow to 2 * kWave products, eight terms at a time; the others of the wavefront do the same for
+// theirs.
+template <typename T> __device__ __forceinline__ T lane_sum_long(const T *s_prod, int b, int e, bool on) {
+    constexpr int C = 8;
+    const int n = on ? e - b : 0;
+    const bool twice = __any(n > kWave);
+    auto eight = [&](int c0) {      // parts c0 .. c0 + 7, pairwise
+        T v[C];
+        if (!__any(n > c0)) return T(0);
+#pragma unroll
+        for (int u = 0; u < C; ++u) v[u] = s_prod[c0 + u < n ? b + c0 + u : 0];
+#pragma unroll
+        for (int u = 0; u < C; ++u) v[u] = T(0) + (c0 + u < n ? v[u] : T(0));
+        if (twice) {
+#pragma unroll
+            for (int u = 0; u < C; ++u) {
+                const T w = s_prod[c0 + u + kWave < n ? b + c0 + u + kWave : 0];
+                v[u] += c0 + u + kWave < n ? w : T(0);
+            }
+        }
+        return ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+    };
+    auto quarter = [&](int c0) { const T lo = eight(c0); return lo + eight(c0 + C); };
+    auto half = [&](int c0) { const T lo = quarter(c0); return lo + quarter(c0 + 2 * C); };
+    const T lo = half(0);
+    return lo + half(4 * C);
+}
+
+// Sum of a lane's slice [b, e) of the products in LDS (all lanes of a wavefront call it; empty where b == e): in storage
+// order, and slices of kLongRow products in the order above, by the wavefront one after the other or (ALONE), where it has
+// many of up to 2 * kWave products, each by its lane: the same bits.  So a row's bits do not depend on the tile it is in.
+// What bounds it: a workgroup waits for the longest row of its tile, and the wavefront's sum of one row takes as many
+// instructions as 64 lanes' sums of their own.  Forward, graphs in fp32, a lane for every row and a trip to LDS for every
+// product -> the wavefront, with small tiles (launch_fwd): 100 000 rows, 1.2 M entries 53 -> 15.7 us; 20 000 rows of up to 5000
+// entries 63 -> 5.5; 400 000 rows, 7.6 M entries 122 -> 68.  Rows of 35 throughout, a band of 100 000, fp32 / fp64: the wavefront 20
+// / 31 us, a lane each 12 / 16.  (The error of a long row's sum against 64 bits is smaller in this order: 6.13e-8 -> 5.98e-8 over
+// 30 000 rows of 26.)
+template <bool ALONE = true, typename T> __device__ __forceinline__ T slice_sum(const T *s_prod, int b, int e) {
     const int lane = threadIdx.x & (kWave - 1);
-    const bool wide = e - b >= kLongRow;
+    const bool wide = e - b >= kLongRow, alone = wide && e - b <= 2 * kWave;
     T total = 0;
     if (!wide) total = serial_sum(s_prod, b, e);
-    for (unsigned long long todo = __ballot(wide); todo; todo &= todo - 1) {
+    unsigned long long todo = __ballot(wide);
+    if constexpr (ALONE) {
+        const unsigned long long many = __ballot(alone);
+        if (__popcll(many) >= kManyRows) {
+            const T sum = lane_sum_long(s_prod, b, e, alone);
+            if (alone) total = sum;
+            todo &= ~many;
+        }
+    }
+    for (; todo; todo &= todo - 1) {
         const int src = __builtin_ctzll(todo);
-        const int wb = __shfl(b, src, kWave), we = __shfl(e, src, kWave);
+        const int wb = ALONE ? nm::read_lane(b, src) : __shfl(b, src, kWave), we = ALONE ? nm::read_lane(e, src) : __shfl(e, src, kWave);
         T acc = 0;
         for (int j = wb + lane; j < we; j += kWave) acc += s_prod[j];
         acc = nm::wave_sum(acc);
@@ -178,33 +222,43 @@ template <typename T> __device__ __forceinline__ T slice_sum(const T *s_prod, in
 }
 
 // The same, left at out[t] where `on` (a slice is empty where it is not on).
-template <bool STREAM, typename T>
+template <bool STREAM, bool ALONE = true, typename T>
 __device__ __forceinline__ void slice_sums(const T *s_prod, int b, int e, bool on, T *__restrict__ out, int t) {
-    const T total = slice_sum(s_prod, b, e);
+    const T total = slice_sum<ALONE>(s_prod, b, e);
     if (!on) return;
     if constexpr (STREAM) nm::stream_store(out + t, total);
     else out[t] = total;
 }
 
+// Which of n rows of a tile thread t takes first: its own number, or where there are only a few, and so long ones, a share of
+// them for every wavefront (rows of 150, fp64: 55 -> 49 us, of 96 48 -> 33; with 64 or 128 rows shared rows of 20 take
+// 65 instead of 61).
+template <int BLOCK> __device__ __forceinline__ int row_of_thread(int n) {
+    const int t = threadIdx.x;
+    return n > 16 ? t : (t & (kWave - 1)) * (BLOCK / kWave) + t / kWave;
+}
+
 // Rows [s0, e0) of a tile whose products lie in LDS from s_off[s0] - o0 on.
-template <typename T, int BLOCK>
+template <typename T, int BLOCK, bool ALONE>
 __device__ __forceinline__ void row_sums(const T *s_prod, const int32_t *s_off, int s0, int e0, int o0, T *__restrict__ y) {
     for (int tb = s0; tb < e0; tb += BLOCK) {
-        const int t = tb + (int)threadIdx.x;
-        slice_sums<true>(s_prod, t < e0 ? s_off[t] - o0 : 0, t < e0 ? s_off[t + 1] - o0 : 0, t < e0, y, t);
+        const int t = tb + (ALONE ? row_of_thread<BLOCK>(e0 - s0) : (int)threadIdx.x);
+        slice_sums<true, ALONE>(s_prod, t < e0 ? s_off[t] - o0 : 0, t < e0 ? s_off[t + 1] - o0 : 0, t < e0, y, t);
     }
 }
 
-// One value for the places [b, e) of a wavefront's slices of LDS, one slice a lane; long ones by the wavefront.
+// One value for the places [b, e) of a wavefront's slices of LDS, one slice a lane; long ones by the wavefront, unless it has
+// many of up to 2 * kWave places.
 template <typename T> __device__ __forceinline__ void slice_fill(T *s_v, int b, int e, T v) {
     const int lane = threadIdx.x & (kWave - 1);
-    const bool wide = e - b >= kLongRow;
+    const bool alone = e - b <= 2 * kWave && __popcll(__ballot(e - b >= kLongRow && e - b <= 2 * kWave)) >= kManyRows;
+    const bool wide = e - b >= kLongRow && !alone;
     if (!wide)
         for (int j = b; j < e; ++j) s_v[j] = v;
     for (unsigned long long todo = __ballot(wide); todo; todo &= todo - 1) {
         const int src = __builtin_ctzll(todo);
-        const int wb = __shfl(b, src, kWave), we = __shfl(e, src, kWave);
-        const T wv = __shfl(v, src, kWave);
+        const int wb = nm::read_lane(b, src), we = nm::read_lane(e, src);
+        const T wv = nm::read_lane(v, src);
         for (int j = wb + lane; j < we; j += kWave) s_v[j] = wv;
     }
 }
@@ -314,7 +368,8 @@ __device__ __forceinline__ void fwd_tile_staged(const int64_t r0, const int nr, 
         }
     }
     __syncthreads();
-    const T acc0 = slice_sum(s_prod, p0 - base, p1 - base), acc1 = slice_sum(s_prod, p1 - base, p2 - base);
+    // (a tile with a list has eight entries a row at most: few long ones)
+    const T acc0 = slice_sum<false>(s_prod, p0 - base, p1 - base), acc1 = slice_sum<false>(s_prod, p1 - base, p2 - base);
     if (2 * tid + 1 < nr) {
         T2 out;
         out[0] = acc0, out[1] = acc1;
@@ -478,7 +533,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_num_sgpr(72))) void sp
                 }
             }
             __syncthreads();
-            row_sums<T, BLOCK>(s_prod, s_off, 0, nr, 0, y + r0);
+            row_sums<T, BLOCK, !LISTS>(s_prod, s_off, 0, nr, 0, y + r0);
         } else if (n <= CAP) {
             const T *__restrict__ d = data + base;
             const IDX *__restrict__ ci = indices + base;
@@ -543,7 +598,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_num_sgpr(72))) void sp
                 }
             }
             __syncthreads();
-            row_sums<T, BLOCK>(s_prod, s_off, 0, nr, 0, y + r0);
+            row_sums<T, BLOCK, !LISTS>(s_prod, s_off, 0, nr, 0, y + r0);
         } else if (n < kHuge) {
             // The block's entries do not fit the tile: runs of consecutive rows that do are taken
             // one after the other.
@@ -593,7 +648,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_num_sgpr(72))) void sp
                 const int o0 = s_off[s0];
                 products(base + o0, s_off[e0] - o0);
                 __syncthreads();
-                row_sums<T, BLOCK>(s_prod, s_off, s0, e0, o0, y + r0);
+                row_sums<T, BLOCK, !LISTS>(s_prod, s_off, s0, e0, o0, y + r0);
                 __syncthreads();
                 s0 = e0;
             }
@@ -666,7 +721,7 @@ __global__ __launch_bounds__(kBlock) void spmv_bwd_kernel(
         // row, a wavefront per row of kLongRow entries or more
         auto spread = [&](int s0, int e0, int o0) {
             for (int tb = s0; tb < e0; tb += kBlock) {
-                const int t = tb + threadIdx.x;
+                const int t = tb + row_of_thread<kBlock>(e0 - s0);
                 const int jb = t < e0 ? s_off[t] - o0 : 0, je = t < e0 ? s_off[t + 1] - o0 : 0;
                 const T av = t < e0 ? a[r0 + t] : T(0);
                 slice_fill(s_a, jb, je, av);
@@ -860,7 +915,7 @@ __device__ __forceinline__ void bwd_tile_staged(const int64_t c0, const int nc, 
     }
     __syncthreads();
     // grad_x[column] = sum of the column's slice in ascending row order
-    slice_sums<false>(s_v, pa - base, pb - base, tid < nc, grad_x + c0, tid);
+    slice_sums<false, false>(s_v, pa - base, pb - base, tid < nc, grad_x + c0, tid);
 }
 
 // Backward over the transposed-structure plan (columns of A as rows of A^T):
@@ -1025,7 +1080,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? (LISTS ? 6 : 8) : (LISTS ? 3
                 const int t = tb + threadIdx.x;
                 const int jb = t < e0 ? (WHOLE ? my_a : s_off[t]) - o0 : 0;
                 const int je = t < e0 ? (WHOLE ? my_b : s_off[t + 1]) - o0 : 0;
-                slice_sums<false>(s_v, jb, je, t < e0, grad_x + c0, t);
+                slice_sums<false, !LISTS>(s_v, jb, je, t < e0, grad_x + c0, t);
             }
         };
         // Entries first .. first + cnt of the plan, lane = entry, s_v holding the own factor of
@@ -1277,14 +1332,15 @@ int launch_fwd(int64_t rows, int64_t nnz, const T *data, const IDX *indices, con
     // that blocks of 512 rows with seven entries a row stay blocks of 512 rows)
     constexpr int R = kFwdR, CAP = LISTS ? NM_FWD_CAP : kFwdCap<T>;
     // Long rows: tiles of about 1024 products (of 2048 or 4096, fp32 graphs of 200 000 rows, 20 entries each on average
-    // 45 -> 56, 63 us; of 100 000 and 12, 15.6 -> 17.8, 22).  Short ones: a tile of 512 rows reads the plan's packed
+    // 45 -> 56, 63 us; of 100 000 and 12, 15.6 -> 17.8, 22), without a plan and in fp64 1280 (1 M rows of 9, band 35.6 -> 32.1 us,
+    // random the same; 1536: 29.7, but a graph of 400 000 rows of 10 38.0 -> 42.7).  Short ones: a tile of 512 rows reads the plan's packed
     // columns; without a plan at least 512 tiles (60 x 55 x 50 seven-point fp64 7.7 -> 5.9 us, with 1024 6.9; 30 x 35 x 30
     // 6.2 -> 4.4, with 1024 5.6).  On a plan whose columns are not packed, which only the device knows, at least 1024 (graphs, fp32,
     // of 512 rows a tile -> 512 -> 1024 tiles: 200 000 rows of 7 entries on average 26.2 -> 23.9 -> 19.4 us, 130 000 of 5 14.6 ->
     // 8.4 -> 8.1), and below 65 536 rows, where every column fits 16 bits, on any without lists (20 000 rows of 3 12.7 ->
     // 5.6, 10 000 of 7 10.8 -> 5.0; grids the same).
     const bool long_rows = nnz > 8 * rows;
-    int rt = block_rows(rows, nnz, R, long_rows ? 1024 : CAP);
+    int rt = block_rows(rows, nnz, R, long_rows ? (sizeof(T) == 8 && sizeof(IDX) == 8 ? 1280 : 1024) : CAP);
     if (long_rows || sizeof(IDX) == 8)
         while (rt > 16 && rows < (int64_t)rt * 512) rt /= 2;
     int narrow = rt;
@@ -1302,7 +1358,7 @@ int launch_fwd(int64_t rows, int64_t nnz, const T *data, const IDX *indices, con
 template <typename T, typename IDX>
 int launch_row_sum(int64_t rows, int64_t nnz, const T *data, const IDX *indptr, T *y, hipStream_t s) {
     constexpr int R = kFwdR, CAP = kFwdCap<T>;
-    const int rt = small_block_rows(rows, nnz, R, CAP);
+    const int rt = small_block_rows(rows, nnz, R, CAP, 2048);
     int64_t grid = nm::xcd_padded(nm::ceil_div(rows, rt));
     if (grid > nm::kMaxGrid) grid = nm::kMaxGrid;
     hipLaunchKernelGGL((spmv_fwd_kernel<T, kFwdBlock, R, CAP, true, IDX>), dim3((unsigned)grid), dim3(kFwdBlock), 0, s, rows,
@@ -1316,7 +1372,7 @@ template <typename T, typename IDX>
 int launch_bwd(int64_t rows, int64_t nnz, const T *data, const IDX *indices, const IDX *indptr, const T *a,
                const T *b, T alpha, T *out_A, T *grad_x, T *prod, hipStream_t s) {
     constexpr int R = Tile<T>::R, CAP = Tile<T>::CAP;
-    const int rt = small_block_rows(rows, nnz, R, CAP);
+    const int rt = small_block_rows(rows, nnz, R, CAP, !grad_x ? 2048 : nnz > 48 * rows ? CAP : 1024);
     int64_t grid = nm::xcd_padded(nm::ceil_div(rows, rt));
     if (grid > nm::kMaxGrid) grid = nm::kMaxGrid;
     if constexpr (sizeof(IDX) == 8)
