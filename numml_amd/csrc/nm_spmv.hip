@@ -675,21 +675,16 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_num_sgpr(72))) void sp
     }
 }
 
-// Fused backward by rows: out_A[k] = alpha * (a[row] * b[col]); ADD: grad_x[col] += a[row] * data[k] (a build of its own:
-// with the rest in one, 2048^2 five-point fp32 191 -> 216 us); when prod is given, prod[k] = a[row] * data[k].  With neither this is the masked outer
+// Fused backward by rows, without a plan: out_A[k] = alpha * (a[row] * b[col]); ADD: grad_x[col] += a[row] * data[k] (a build of
+// its own: with the rest in one, 2048^2 five-point fp32 191 -> 216 us).  Without ADD this is the masked outer
 // product (cpp/sparse_csr_cpu.cpp:60-65 and :750-755).
-//
-// It reads b once an entry and everything else in order, so that a grid moves its bytes (127 x 113 x 101 fp32, 32-bit
-// structure: 81 MB in 20.5 us) and a graph waits for its gathers from L2.  The gradient of A alone is made here
-// also where a transposed-structure plan exists: a walk by column writes it entry by entry where columns are
-// scattered (7.6 M entries fp32 243 -> 50 us) and gathers positions where they are not (the grid 46 -> 20.5).
-template <typename T, int R, int CAP, typename IDX, bool ADD>
+template <typename T, int R, int CAP, bool ADD>
 __global__ __launch_bounds__(kBlock) void spmv_bwd_kernel(
-    int64_t rows, int rt, const T *__restrict__ data, const IDX *__restrict__ indices,
-    const IDX *__restrict__ indptr, const T *__restrict__ a, const T *__restrict__ b, T alpha,
-    T *__restrict__ out_A, T *__restrict__ grad_x, T *__restrict__ prod) {
+    int64_t rows, int rt, const T *__restrict__ data, const int64_t *__restrict__ indices,
+    const int64_t *__restrict__ indptr, const T *__restrict__ a, const T *__restrict__ b, T alpha,
+    T *__restrict__ out_A, T *__restrict__ grad_x) {
     typedef T TV __attribute__((ext_vector_type(4), aligned(sizeof(T))));
-    typedef IDX IV __attribute__((ext_vector_type(4), aligned(sizeof(IDX))));
+    typedef int64_t IV __attribute__((ext_vector_type(4), aligned(8)));
     __shared__ int32_t s_off[R + 1];
     __shared__ T s_a[CAP];
     const int lane = threadIdx.x & (kWave - 1);
@@ -703,7 +698,7 @@ __global__ __launch_bounds__(kBlock) void spmv_bwd_kernel(
         int nr = (int)(rows - r0 < rt ? rows - r0 : rt);
         nr = nr < R ? nr : R;   // rt <= R
         const int64_t base = indptr[r0];
-        stage_offsets<R, CAP, kBlock, IDX>(indptr, r0, nr, base, s_off);
+        stage_offsets<R, CAP, kBlock>(indptr, r0, nr, base, s_off);
         __syncthreads();
         const int n = s_off[nr];
         // entry k, whose row's factor is av
@@ -713,8 +708,7 @@ __global__ __launch_bounds__(kBlock) void spmv_bwd_kernel(
                 if (out_A) out_A[k] = alpha * (av * b[c]);
                 nm::atomic_add(grad_x + c, av * data[k]);
             } else {
-                if (out_A) out_A[k] = alpha * (av * b[indices[k]]);
-                if (prod) prod[k] = av * data[k];
+                out_A[k] = alpha * (av * b[indices[k]]);
             }
         };
         // a[row] to the entries of rows [s0, e0) in s_a, which begins at entry o0 of the block: one lane per short
@@ -736,22 +730,13 @@ __global__ __launch_bounds__(kBlock) void spmv_bwd_kernel(
             }
             const int n4 = cnt & ~3;
             for (int k = 4 * threadIdx.x; k < n4; k += 4 * kBlock) {
-                IV c;
-                TV d, o;
-                if (out_A) c = *(const IV *)(indices + first + k);
-                if (prod) d = *(const TV *)(data + first + k);
-                if (out_A) {
+                const IV c = *(const IV *)(indices + first + k);
+                TV o;
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) o[v] = b[c[v]];
+                for (int v = 0; v < 4; ++v) o[v] = b[c[v]];
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) o[v] = alpha * (s_a[k + v] * o[v]);
-                    *(TV *)(out_A + first + k) = o;
-                }
-                if (prod) {
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) o[v] = s_a[k + v] * d[v];
-                    *(TV *)(prod + first + k) = o;
-                }
+                for (int v = 0; v < 4; ++v) o[v] = alpha * (s_a[k + v] * o[v]);
+                *(TV *)(out_A + first + k) = o;
             }
             if (threadIdx.x < (cnt & 3)) entry(first + n4 + threadIdx.x, s_a[n4 + threadIdx.x]);
         };
@@ -792,6 +777,86 @@ __global__ __launch_bounds__(kBlock) void spmv_bwd_kernel(
                 const T av = a[r0 + t];
                 for (int64_t k = rb + lane; k < re; k += kWave) entry(k, av);
             }
+        }
+        __syncthreads();
+    }
+}
+
+// The same on a transposed-structure plan: out_A[k] = a[row] * b[col] and / or prod[k] = a[row] * data[k].  A workgroup has
+// `tile` consecutive entries (a multiple of 64, at most CAP), whatever rows they are of: chunk_row tells the first one's.  (With
+// tiles of rows one workgroup has all of a long row and of long rows side by side: 20 rows of 100 000 1210 -> 9 us, power-law
+// rows in descending order, 100 000 rows, 2 M entries 403 -> 12.5.)
+//
+// It reads b once an entry and everything else in order, so that a grid moves its bytes (127 x 113 x 101 fp32: 81 MB in
+// 20 us) and a graph waits for its gathers from L2.  The gradient of A alone is made here too: a walk by column writes it
+// entry by entry where columns are scattered (7.6 M entries fp32 243 -> 50 us) and gathers positions where they are not
+// (the grid 46 -> 20).
+template <typename T, int R, int CAP>
+__global__ __launch_bounds__(kBlock) void spmv_bwd_entries_kernel(
+    int64_t rows, int64_t nnz, int tile, const T *__restrict__ data, const int32_t *__restrict__ idx32,
+    const int32_t *__restrict__ ptr32, const int32_t *__restrict__ chunk_row, const T *__restrict__ a, const T *__restrict__ b,
+    T *__restrict__ out_A, T *__restrict__ prod) {
+    typedef T TV __attribute__((ext_vector_type(4), aligned(sizeof(T))));
+    typedef int32_t IV __attribute__((ext_vector_type(4), aligned(4)));
+    __shared__ int32_t s_off[R + 1];
+    __shared__ T s_a[CAP];
+    const int64_t ntiles = (nnz + tile - 1) / tile, npad = nm::xcd_padded(ntiles);
+    for (int64_t id = blockIdx.x; id < npad; id += gridDim.x) {
+        const int64_t at = nm::xcd_tile(id, npad);
+        if (at >= ntiles) continue;
+        const int64_t base = at * tile, next = base + tile;
+        const int n = (int)(nnz - base < tile ? nnz - base : tile);
+        const int32_t r0 = chunk_row[base / kWave], r1 = next < nnz ? chunk_row[next / kWave] : (int32_t)(rows - 1);
+        // a[row] to the rows' entries: rows r0 .. r1 with their entries among these n
+        if (r1 - r0 < 4 * R) {
+            for (int32_t s0 = r0; s0 <= r1; s0 += R) {
+                const int nr = r1 - s0 + 1 < R ? r1 - s0 + 1 : R;
+                if (s0 > r0) __syncthreads();
+                for (int t = threadIdx.x; t <= nr; t += kBlock) {
+                    const int64_t d = (int64_t)ptr32[s0 + t] - base;
+                    s_off[t] = (int)(d < 0 ? 0 : d < n ? d : n);
+                }
+                __syncthreads();
+                for (int tb = 0; tb < nr; tb += kBlock) {
+                    const int t = tb + row_of_thread<kBlock>(nr);
+                    const int jb = t < nr ? s_off[t] : 0, je = t < nr ? s_off[t + 1] : 0;
+                    slice_fill(s_a, jb, je, je > jb ? a[s0 + t] : T(0));
+                }
+            }
+        } else {
+            // (nearly all of these rows are empty: every entry looks for its own)
+            for (int k = threadIdx.x; k < n; k += kBlock) {
+                int32_t lo = r0, hi = r1 + 1;
+                while (hi - lo > 1) {
+                    const int32_t mid = lo + (hi - lo) / 2;
+                    if (ptr32[mid] <= base + k) lo = mid; else hi = mid;
+                }
+                s_a[k] = a[lo];
+            }
+        }
+        __syncthreads();
+        const int n4 = n & ~3;
+        for (int k = 4 * threadIdx.x; k < n4; k += 4 * kBlock) {
+            IV c;
+            TV d, o;
+            if (out_A) c = *(const IV *)(idx32 + base + k);
+            if (prod) d = *(const TV *)(data + base + k);
+            if (out_A) {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) o[v] = b[c[v]];
+#pragma unroll
+                for (int v = 0; v < 4; ++v) o[v] = s_a[k + v] * o[v];
+                *(TV *)(out_A + base + k) = o;
+            }
+            if (prod) {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) o[v] = s_a[k + v] * d[v];
+                *(TV *)(prod + base + k) = o;
+            }
+        }
+        if (const int k = n4 + threadIdx.x; k < n) {
+            if (out_A) out_A[base + k] = s_a[k] * b[idx32[base + k]];
+            if (prod) prod[base + k] = s_a[k] * data[base + k];
         }
         __syncthreads();
     }
@@ -1368,22 +1433,19 @@ int launch_row_sum(int64_t rows, int64_t nnz, const T *data, const IDX *indptr, 
     return NM_OK;
 }
 
-template <typename T, typename IDX>
-int launch_bwd(int64_t rows, int64_t nnz, const T *data, const IDX *indices, const IDX *indptr, const T *a,
-               const T *b, T alpha, T *out_A, T *grad_x, T *prod, hipStream_t s) {
+template <typename T>
+int launch_bwd(int64_t rows, int64_t nnz, const T *data, const int64_t *indices, const int64_t *indptr, const T *a,
+               const T *b, T alpha, T *out_A, T *grad_x, hipStream_t s) {
     constexpr int R = Tile<T>::R, CAP = Tile<T>::CAP;
     const int rt = small_block_rows(rows, nnz, R, CAP, !grad_x ? 2048 : nnz > 48 * rows ? CAP : 1024);
     int64_t grid = nm::xcd_padded(nm::ceil_div(rows, rt));
     if (grid > nm::kMaxGrid) grid = nm::kMaxGrid;
-    if constexpr (sizeof(IDX) == 8)
-        if (grad_x) {
-            hipLaunchKernelGGL((spmv_bwd_kernel<T, R, CAP, IDX, true>), dim3((unsigned)grid), dim3(kBlock), 0, s, rows, rt,
-                               data, indices, indptr, a, b, alpha, out_A, grad_x, prod);
-            NM_LAUNCH_CHECK("spmv_bwd_kernel");
-            return NM_OK;
-        }
-    hipLaunchKernelGGL((spmv_bwd_kernel<T, R, CAP, IDX, false>), dim3((unsigned)grid), dim3(kBlock), 0, s, rows, rt, data,
-                       indices, indptr, a, b, alpha, out_A, grad_x, prod);
+    if (grad_x)
+        hipLaunchKernelGGL((spmv_bwd_kernel<T, R, CAP, true>), dim3((unsigned)grid), dim3(kBlock), 0, s, rows, rt,
+                           data, indices, indptr, a, b, alpha, out_A, grad_x);
+    else
+        hipLaunchKernelGGL((spmv_bwd_kernel<T, R, CAP, false>), dim3((unsigned)grid), dim3(kBlock), 0, s, rows, rt, data,
+                           indices, indptr, a, b, alpha, out_A, grad_x);
     NM_LAUNCH_CHECK("spmv_bwd_kernel");
     return NM_OK;
 }
@@ -1504,10 +1566,10 @@ extern "C" int nm_spgemv_backward(nm_dtype dt, int64_t rows, int64_t cols, int64
     if (rows == 0 || nnz == 0 || (!grad_A && !grad_x)) return NM_OK;
     NM_REQUIRE(g != nullptr && x != nullptr, "g or x is null");
     if (dt == NM_F32)
-        return launch_bwd<float, int64_t>(rows, nnz, (const float *)data, indices, indptr, (const float *)g,
-                                 (const float *)x, 1.0f, (float *)grad_A, (float *)grad_x, (float *)nullptr, s);
-    return launch_bwd<double, int64_t>(rows, nnz, (const double *)data, indices, indptr, (const double *)g,
-                              (const double *)x, 1.0, (double *)grad_A, (double *)grad_x, (double *)nullptr, s);
+        return launch_bwd<float>(rows, nnz, (const float *)data, indices, indptr, (const float *)g,
+                                 (const float *)x, 1.0f, (float *)grad_A, (float *)grad_x, s);
+    return launch_bwd<double>(rows, nnz, (const double *)data, indices, indptr, (const double *)g,
+                              (const double *)x, 1.0, (double *)grad_A, (double *)grad_x, s);
 }
 
 extern "C" int nm_masked_outer(nm_dtype dt, int64_t rows, int64_t nnz, const int64_t *indices,
@@ -1519,10 +1581,10 @@ extern "C" int nm_masked_outer(nm_dtype dt, int64_t rows, int64_t nnz, const int
     NM_REQUIRE(indices && a && b && out, "null pointer argument");
     hipStream_t s = nm::as_stream(stream);
     if (dt == NM_F32)
-        return launch_bwd<float, int64_t>(rows, nnz, nullptr, indices, indptr, (const float *)a, (const float *)b,
-                                 (float)alpha, (float *)out, (float *)nullptr, (float *)nullptr, s);
-    return launch_bwd<double, int64_t>(rows, nnz, nullptr, indices, indptr, (const double *)a, (const double *)b, alpha,
-                              (double *)out, (double *)nullptr, (double *)nullptr, s);
+        return launch_bwd<float>(rows, nnz, nullptr, indices, indptr, (const float *)a, (const float *)b,
+                                 (float)alpha, (float *)out, (float *)nullptr, s);
+    return launch_bwd<double>(rows, nnz, nullptr, indices, indptr, (const double *)a, (const double *)b, alpha,
+                              (double *)out, (double *)nullptr, s);
 }
 
 extern "C" int nm_spgemv_configure(int wide_offsets) {
@@ -1555,11 +1617,18 @@ void launch_bwd_planned(int64_t cols, int64_t nnz, const nm::TPlan &t, bool o32,
                            (const T *)g, (T *)grad_A, (T *)grad_x, desc, width);
 }
 
+// Tiles of 2048 entries (1 M rows of 12, band, fp32 / fp64, 1024 / 2048 / 4096 entries: 22.9, 19.7, 20.5 / 27.7, 27.0, 31.0
+// us), of fewer where these were not 1024 tiles.
 template <typename T>
 int by_rows(int64_t rows, int64_t nnz, const nm::TPlan &t, const void *data, const void *x, const void *g, void *grad_A,
             void *prod, hipStream_t s) {
-    return launch_bwd<T, int32_t>(rows, nnz, (const T *)data, t.c_idx32, t.c_ptr32, (const T *)g, (const T *)x, T(1),
-                                  (T *)grad_A, (T *)nullptr, (T *)prod, s);
+    constexpr int64_t kMost = 2048;
+    const int64_t tile = std::min(kMost, std::max<int64_t>(256, (nnz / 1024 + 255) / 256 * 256));
+    const int64_t grid = std::min<int64_t>(nm::xcd_padded(nm::ceil_div(nnz, tile)), nm::kMaxGrid);
+    hipLaunchKernelGGL((spmv_bwd_entries_kernel<T, 1024, kMost>), dim3((unsigned)grid), dim3(kBlock), 0, s, rows, nnz, (int)tile, (const T *)data,
+                       t.c_idx32, t.c_ptr32, t.chunk_row, (const T *)g, (const T *)x, (T *)grad_A, (T *)prod);
+    NM_LAUNCH_CHECK("spmv_bwd_entries_kernel");
+    return NM_OK;
 }
 
 // Scattered columns: the kernel on the plan alone gathers a value and writes a gradient per entry, each a cache line

@@ -158,3 +158,58 @@ def test_default_mode(dev):
     finally:
         ops.set_backward_mode(old)
         ops.clear_plan_cache()
+
+
+def _spread_rows(rows, at, lens):
+    n = np.zeros(rows, np.int64)
+    n[at] = lens
+    return n
+
+
+TILES = {   # lengths of the rows; a workgroup of the kernel by entries stages 1024 rows at a time, up to 4096 of them
+    "one row": np.array([70_000]),
+    "ends of tiles": np.array([255, 1, 256, 257, 511, 64, 63, 1, 1, 128, 2]),
+    "all empty but one": _spread_rows(100_000, [99_000], [3]),
+    "empty ones first and last": _spread_rows(20_000, [9_000, 9_001], [300, 5]),
+    "1023 to 1025 rows a tile": np.concatenate([_spread_rows(1022, [0, 500], [100, 156]), _spread_rows(1024, [1023], [256]),
+                                                _spread_rows(1025, [3, 1024], [1, 255]), [300]]),
+    "4095 to 4097 rows a tile": np.concatenate([_spread_rows(4094, [0, 500], [100, 156]), _spread_rows(4096, [4095], [256]),
+                                                _spread_rows(4098, [3, 4097], [1, 255]), [300]]),
+    "many entries": np.concatenate([np.full(500_000, 3), [600_000], np.zeros(9000, np.int64), [1, 2047, 2048, 2049], np.full(3000, 40), [17]]),
+}
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("case", list(TILES))
+def test_gradient_of_the_matrix_alone_on_the_plan(dev, dtype, case):
+    lens, cols = TILES[case], 1000
+    p = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    rows, nnz = lens.size, int(p[-1])
+    i = np.random.default_rng(nnz).integers(0, cols, nnz)
+    d, x, g = randn(1, nnz, dtype), randn(2, cols, dtype), randn(3, rows, dtype)
+    X, Gz = to_dev(dev, x, g)
+    L, dt = _lib.lib(), ext._dt(X)
+    for n in (nnz, nnz - 1, nnz - 63) if lens[-1] > 63 else (nnz,):      # other ends of the last tile
+        p[-1] = n
+        D, I, P = to_dev(dev, d[:n], i[:n], p)
+        plan = ext._transpose_plan(I, P, rows, cols, dev)
+        out = torch.full((n + 8,), 7, dtype=D.dtype, device=dev)
+        assert L.nm_spgemv_backward_planned(dt, rows, cols, n, D.data_ptr(), plan.mem.data_ptr(), X.data_ptr(), Gz.data_ptr(),
+                                            out.data_ptr(), None, None) == 0
+        want = g[np.repeat(np.arange(rows), np.diff(p))] * x[i[:n]]
+        assert_same(host(out)[:n], want, f"{case}, {n} entries")
+        assert (host(out)[n:] == 7).all()
+        # the products of the way through column-major order are made by the same kernel
+        pb, wb, sb = ctypes.c_size_t(), ctypes.c_size_t(), ctypes.c_size_t()
+        assert L.nm_permute_plan_bytes(n, pb, wb) == 0 and L.nm_spgemv_staged_bytes(dt, n, sb) == 0
+        perm, work, room = (torch.empty(b.value, dtype=torch.uint8, device=dev) for b in (pb, wb, sb))
+        assert L.nm_permute_plan_build(rows, cols, n, plan.mem.data_ptr(), perm.data_ptr(), pb, work.data_ptr(), wb, None) == 0
+        gA, gx = torch.empty_like(D), torch.empty_like(X)
+        assert L.nm_spgemv_backward_staged(dt, rows, cols, n, D.data_ptr(), plan.mem.data_ptr(), perm.data_ptr(), room.data_ptr(), sb,
+                                           X.data_ptr(), Gz.data_ptr(), gA.data_ptr(), gx.data_ptr(), None) == 0
+        assert_same(host(gA), want, f"{case}, {n} entries, with the gradient of x")
+        terms = np.abs(g[np.repeat(np.arange(rows), np.diff(p))] * d[:n]).astype(np.float64)
+        ref = np.bincount(i[:n], weights=(g[np.repeat(np.arange(rows), np.diff(p))] * d[:n]).astype(np.float64), minlength=cols)
+        # sums of n terms in any order: 2 n eps times the sum of their sizes
+        bound = 2 * np.finfo(dtype).eps * np.bincount(i[:n], minlength=cols) * np.bincount(i[:n], weights=terms, minlength=cols)
+        assert (np.abs(host(gx) - ref) <= bound + 1e-300).all(), f"{case}: gradient of x"
