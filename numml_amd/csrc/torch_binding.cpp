@@ -487,18 +487,27 @@ bool fits_a_plan(int64_t rows, int64_t cols, int64_t nnz) {
 // plan that the forward reads, 6 bytes an entry in place of 8 for the interface's structure, at the third product with the
 // same tensors: nothing is known of these until then but how often they were seen (weak references, as in the
 // alias table).  A pattern whose gradients are asked for has its transposed-structure plan by then, which
-// holds the same.  Only where a product takes long enough (kRowsPlanEntries: 1.2 M entries of a grid 9.2 -> 8.2 us, the
-// plan 30 to 70).  127 x 113 x 101 seven-point fp64 36.4 -> 25.5 us, fp32 29.2 -> 15.0; 2000 x 1900 five-point fp32 55.8 ->
-// 29.6, fp64 69 -> 49; 150^3 fp64 81.7 -> 74.4.
+// holds the same.  The product that makes the plan takes 60 us longer at a million entries, 185 at 21 million (content
+// key, build, a wait for the stream).  Products without -> with it, five- and seven-point grids, us, and after how many
+// products it has paid:
+//   1.3 M fp32 7.4 -> 6.1 (45)    fp64 7.8 -> 6.2 (36)       5.2 M fp32 15.9 -> 9.1 (13)    fp64 20.1 -> 15.5 (19)
+//   2.5 M fp32 9.7 -> 7.2 (27)    fp64 10.1 -> 9.5 (110)     10.0 M fp32 29.7 -> 14.8 (8)   fp64 36.7 -> 25.5 (10)
+//   3.5 M fp32 12.0 -> 7.0 (15)   fp64 14.4 -> 10.8 (20)     21.0 M fp32 56.6 -> 28.9 (7)   fp64 73.8 -> 51.2 (9)
+// and random rows of 40, 4.0 M, fp32 26.0 -> 22.7 (26).  At 1.06 M the two are equal: from there on (kRowsPlanEntries) it is
+// for solvers, whose products are hundreds; a call whose matrix is new each time never makes one.
+//
+// A plan that left the cache is made again after kProductsBeforeAgain further products only: matrices whose plans
+// don't fit beside each other would make one on every product otherwise.  None is made that exceeds the cache's limit
+// alone or that the device has no memory for.
 struct Seen {
     const c10::TensorImpl *idx_impl, *ptr_impl;
     WeakImpl idx_weak, ptr_weak;
     const void *idx_ptr, *ptr_ptr;
     uint32_t idx_version, ptr_version;
-    int times;
+    int left;       // products until the plan is made
 };
 constexpr size_t kSeenTableSize = 64;
-constexpr int kProductsBeforePlan = 3;
+constexpr int kProductsBeforePlan = 3, kProductsBeforeAgain = 64;
 constexpr int64_t kRowsPlanEntries = 1 << 20;
 // Where blocks have no staging lists and columns do not fit 16 bits the plan only halves the indices of a product that
 // waits for its gathers: graphs of 1.2 M entries fp32 15.7 -> 13.3 us, fp64 16.8 -> 15.5 (not made), of 3.9 M 35.1 -> 29.5 and
@@ -506,23 +515,24 @@ constexpr int64_t kRowsPlanEntries = 1 << 20;
 constexpr int64_t kScatteredEntries = 2 << 20;
 std::list<Seen> g_seen;   // most recently seen first
 
-// How often products of this pair of structure tensors have been seen, this time included.
-int times_seen(const Tensor &indices, const Tensor &indptr) {
+// Whether the product of this pair of structure tensors is the one that makes the plan.
+bool makes_rows_plan(const Tensor &indices, const Tensor &indptr) {
     std::lock_guard<std::mutex> lock(g_plans_mutex);
     for (auto it = g_seen.begin(); it != g_seen.end(); ++it)
         if (it->idx_impl == indices.unsafeGetTensorImpl() && it->ptr_impl == indptr.unsafeGetTensorImpl() &&
             it->idx_ptr == indices.data_ptr() && it->ptr_ptr == indptr.data_ptr() && it->idx_version == indices._version() &&
             it->ptr_version == indptr._version() && !it->idx_weak.expired() && !it->ptr_weak.expired()) {
-            const int times = ++it->times;
+            const bool now = --it->left == 0;
+            if (now) it->left = kProductsBeforeAgain;
             if (it != g_seen.begin()) g_seen.splice(g_seen.begin(), g_seen, it);
-            return times;
+            return now;
         }
     g_seen.remove_if([](const Seen &o) { return o.idx_weak.expired() || o.ptr_weak.expired(); });
     g_seen.push_front(Seen{indices.unsafeGetTensorImpl(), indptr.unsafeGetTensorImpl(), WeakImpl(indices.getIntrusivePtr()),
                            WeakImpl(indptr.getIntrusivePtr()), indices.data_ptr(), indptr.data_ptr(), indices._version(),
-                           indptr._version(), 1});
+                           indptr._version(), kProductsBeforePlan - 1});
     while (g_seen.size() > kSeenTableSize) g_seen.pop_back();
-    return 1;
+    return false;
 }
 
 // Most blocks of 512 rows have a staging list: the instantiation that stages x in LDS (it gives up resident
@@ -535,13 +545,19 @@ std::shared_ptr<Plan> rows_plan(const Tensor &indices, const Tensor &indptr, int
         !tracked(indices) || !tracked(indptr))
         return nullptr;
     if (auto plan = peek_plan('R', indices, indptr, rows, cols, dev)) return plan->usable ? plan : nullptr;
-    if (times_seen(indices, indptr) < kProductsBeforePlan ||
-        c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None)
+    if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None || !makes_rows_plan(indices, indptr))
         return nullptr;
+    size_t bytes = 0;
+    check(nm_spgemv_rows_plan_bytes(rows, cols, nnz, &bytes), "nm_spgemv_rows_plan_bytes");
+    if (bytes > g_plan_bytes_limit.load(std::memory_order_relaxed)) return nullptr;
+    Tensor mem;
+    try {
+        mem = scratch(bytes, dev);
+    } catch (const c10::OutOfMemoryError &) {
+        return nullptr;
+    }
     auto plan = cached('R', indices, indptr, rows, cols, false, dev, [&](Plan &p) {
-        size_t bytes = 0;
-        check(nm_spgemv_rows_plan_bytes(rows, cols, nnz, &bytes), "nm_spgemv_rows_plan_bytes");
-        p.mem = scratch(bytes, dev);
+        p.mem = mem;
         check(nm_spgemv_rows_plan_build(rows, cols, nnz, indices.data_ptr<int64_t>(), indptr.data_ptr<int64_t>(),
                                         p.mem.data_ptr(), bytes, p.info, current_stream(dev)),
               "nm_spgemv_rows_plan_build");

@@ -146,3 +146,55 @@ def test_under_capture_nothing_is_made(dev):
             graph.replay()
             torch.cuda.synchronize()
             assert torch.equal(z, ops.spgemv_forward(rows, cols, D, I, P, X))
+
+
+@needs_policy
+def test_a_plan_that_does_not_stay_is_not_made_on_every_product(dev):
+    ops = _binding.ops
+    d, i, p, (rows, cols) = G.poisson2d(480, np.float32, jitter_seed=1)
+    D, I, P, X = to_dev(dev, d, i, p, randn(1, cols, np.float32))
+    other = I.clone()
+    other[0], other[1] = int(I[1]), int(I[0])       # another content: a plan of its own
+    size = ctypes.c_size_t()
+    assert _lib.lib().nm_spgemv_rows_plan_bytes(rows, cols, d.size, size) == 0
+
+    def built(products, *index):
+        before = ops.plan_cache_stats()[0]
+        for _ in range(products):
+            for j in index:
+                ops.spgemv_forward(rows, cols, D, j, P, X)
+        return ops.plan_cache_stats()[0] - before
+    try:
+        ops.clear_plan_cache()
+        ops.set_plan_cache_limit(size.value * 3 // 2)           # room for one of the two
+        assert built(20, I, other) == 2
+        assert 1 <= built(200, I, other) <= 6                   # (every second of 400 without a bound)
+        ops.clear_plan_cache()
+        ops.set_plan_cache_limit(size.value - 1)
+        assert built(20, I) == 0
+        ops.set_plan_cache_limit(size.value + 64)               # (the plan's tensor may be a little larger than asked for)
+        assert built(64, I) == 1 and built(64, I) == 0
+    finally:
+        ops.set_plan_cache_limit(4 << 30)
+        ops.clear_plan_cache()
+
+
+@needs_policy
+def test_no_memory_for_the_plan(dev):
+    """The product is made without it."""
+    ops = _binding.ops
+    d, i, p, (rows, cols) = G.poisson2d(1000, np.float32, jitter_seed=1)        # 5 M entries, a plan of 30 MB
+    D, I, P, X = to_dev(dev, d, i, p, randn(1, cols, np.float32))
+    ops.clear_plan_cache()
+    want = [ops.spgemv_forward(rows, cols, D, I, P, X) for _ in range(2)][0]
+    out = torch.empty_like(want)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (8 << 20)) / torch.cuda.get_device_properties(0).total_memory)
+        for _ in range(3):
+            out.copy_(ops.spgemv_forward(rows, cols, D, I, P, X))
+        assert ops.plan_cache_size() == 0
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(out, want)
