@@ -909,11 +909,14 @@ Tensor spgemv_forward(int A_rows, int A_cols, Tensor A_data, Tensor A_col_ind, T
 }
 
 // Entries from which scattered values go through column-major order (permute_plan), both gradients or grad_x alone (the
-// gradient of A alone is made by rows).  Graphs with random columns, on the plan's kernel -> through the order, us:
-//   both        fp32  0.82 M 25.4 -> 25.2   0.92 M 29.7 -> 25.5   1.2 M 40 -> 31   2.1 M 73 -> 42   3.8 M 136 -> 77   7.6 M 288 -> 121
-//               fp64  0.82 M 28.8 -> 32.9   0.92 M 34.3 -> 33.3   1.2 M 45 -> 40   2.1 M 83 -> 59   3.8 M 149 -> 96   7.6 M 307 -> 200
-//   grad_x      fp32  1.2 M 19.1 -> 25.9   2.1 M 34.1 -> 30.6   2.5 M 40.4 -> 37.9   3.8 M 59 -> 51.5   7.6 M 130 -> 88
-//               fp64  1.2 M 21.4 -> 32.1   2.1 M 43.6 -> 41.4   2.5 M 48.7 -> 52.7   3.8 M 66 -> 71     7.6 M 165 -> 130
+// gradient of A alone is made by rows).  Graphs with random columns, 10 to 38 a row, on the plan's kernel -> through the
+// order, us:
+//   both     fp32  0.60 M 21 -> 20   0.90 M 32 -> 24   1.2 M 46 -> 29   2.1 M 81 -> 37   3.8 M 151 -> 55   8.0 M 324 -> 106
+//            fp64  0.60 M 24 -> 26   0.90 M 38 -> 31   1.2 M 50 -> 35   2.1 M 87 -> 51   3.8 M 160 -> 76   8.0 M 351 -> 178
+//   grad_x   fp32  1.2 M 20 -> 24    2.1 M 35 -> 28    2.5 M 43 -> 30   3.0 M 52 -> 33   3.8 M 70 -> 39    8.0 M 174 -> 78
+//            fp64  1.2 M 24 -> 29    2.1 M 42 -> 40    2.5 M 59 -> 43   3.0 M 63 -> 48   3.8 M 74 -> 61    8.0 M 218 -> 114
+// Both widths gain from 0.9 M and 2.1 M entries on.  The lines lie where the plan, which takes 0.1 to 0.3 ms to make, has
+// paid within some twenty steps.
 constexpr int64_t kStagedBoth = 950 << 10, kStagedOne = 3 << 20;
 
 std::vector<Tensor> spgemv_backward(Tensor grad_z, int A_rows, int A_cols, Tensor A_data, Tensor A_col_ind,
