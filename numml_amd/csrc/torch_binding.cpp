@@ -1293,19 +1293,31 @@ std::vector<Tensor> spdmm_backward(int A_rows, int A_cols, Tensor A_data, Tensor
     if (want.second) grad_B = torch::empty({B.size(0), n}, B.options());
     // (the dot products alone walk A by row and need no plan)
     auto plan = want.second ? backward_plan(A_indices, A_indptr, A_rows, B.size(0), dev) : nullptr;
+    // the kernels for groups of lanes (nm_spmm_groups.hpp) take the product
+    const int64_t value_bytes = A_data.element_size();
+    const bool grouped = n > 0 && n * value_bytes <= 1024 && ldg <= 0x3fffffff / value_bytes;
     if (plan && backward_mode_now() == kPlanned) {
-        // The kernels on the plan give every aligned group of 64 columns to one workgroup, which
-        // takes the group's columns of more than 512 entries one after the other (~0.12 us an entry
-        // with both gradients, ~0.02 us for the transposed product alone), while the stateless
-        // kernels spread every entry over the chip at ~0.2 ns: where one group holds more than a
-        // thousandth (a hundredth) of the matrix in such columns, the stateless kernels are the
-        // faster ones.  ("eager" asks for the deterministic sums whatever they cost.)
+        // On the plan a long column is summed by one workgroup; the stateless kernels
+        // spread every entry over the chip, with an atomic add for each of its values.  info[8] is the most entries
+        // that columns of more than 512 entries hold in one aligned group of 64: where these are more than a hundredth of
+        // the matrix the stateless kernels are taken.  Ten entries a column, 64 values a row, us on the plan / without
+        // it, both gradients and grad_B alone:
+        //   rows   in such columns   both, fp32     fp64           grad_B, fp32   fp64
+        //   1 M    none              716 / 2090     1521 / 3849    585 / 2038     982 / 3686
+        //   1 M    0.3 %, one        912 / 2757     2206 / 4460    795 / 2701     1601 / 4231
+        //   1 M    1 %, one          2059 / 4410    5389 / 5776    1812 / 4373    3923 / 5651
+        //   1 M    1.6 %, 64         1097 / 2179    2719 / 3926    964 / 2151     1990 / 3776
+        //   1 M    3 %, one          5274 / 9135    14395 / 9887   4645 / 9129    10480 / 9833
+        //   0.1 M  1 %, one          183 / 456      425 / 582      105 / 450      126 / 572
+        //   0.1 M  3 %, one          458 / 927      1173 / 994     245 / 926      264 / 989
+        // Rows over 1 KB go to kernels that give a workgroup the columns of such a group: both gradients of an entry of a
+        // long one cost about 0.12 us there, and a thousandth is the line.  ("eager" asks for the deterministic sums whatever
+        // they cost.)
         const int64_t heavy = plan_info(*plan, A_rows, B.size(0), A_data.numel(), dev)[8];
-        if (heavy * (want.first ? 1000 : 100) > A_data.numel()) plan = nullptr;
+        if (heavy * (want.first && !grouped ? 1000 : 100) > A_data.numel()) plan = nullptr;
     }
     g_last_spdmm_backward.store(plan ? kOnTransposedPlan : kStateless, std::memory_order_relaxed);
-    const int64_t value_bytes = A_data.element_size();
-    auto staged = plan && n > 0 && n * value_bytes <= 1024 && ldg <= 0x3fffffff / value_bytes
+    auto staged = plan && grouped
                       ? permute_plan(plan, A_indices, A_indptr, A_rows, B.size(0), kScatteredBytes / value_bytes, dev)
                       : nullptr;
     if (staged) {

@@ -434,6 +434,30 @@ def test_default_mode_judges_by_the_heaviest_rows_and_columns_not_by_means(dev, 
         cpp.clear_plan_cache()
 
 
+@pytest.mark.parametrize("n,share,want", [(40, 0.008, "transposed plan"), (40, 0.012, "stateless"), (128, 0.008, "transposed plan"),
+                                          (129, 0.008, "stateless"), (129, 0.0008, "transposed plan")])
+def test_default_mode_takes_the_plan_where_few_entries_lie_in_long_columns(dev, cpp, n, share, want):
+    """One long column: both gradients on the plan up to a hundredth of the entries (fp64 rows of up to 1 KB), a thousandth
+    beyond that."""
+    rows, deg = 25_000, 60
+    rng = np.random.default_rng(7)
+    cols = np.sort((rng.integers(1, rows // deg, (rows, deg)) + np.arange(deg) * (rows // deg)), axis=1)     # column 0 stays empty
+    long = np.sort(rng.choice(rows, int(share * rows * deg), replace=False))
+    i = np.insert(cols.reshape(-1), long * deg, 0).astype(np.int64)
+    p = (np.arange(rows + 1) * deg + np.searchsorted(long, np.arange(rows + 1))).astype(np.int64)
+    d, B, g = randn(1, i.size, np.float64), randn(2, (rows, n), np.float64), randn(3, (rows, n), np.float64)
+    ref = oracle.spdmm_backward(rows, rows, d, i, p, B, g)
+    D, I, P, Bd, Gd = to_dev(dev, d, i, p, B, g)
+    cpp.clear_plan_cache()
+    cpp.set_backward_mode("planned")
+    for _ in range(3):
+        gA, gB = cpp.spdmm_backward(rows, rows, D, I, P, Bd, Gd)
+        assert_close(host(gA), ref[0], "grad_A")
+        assert_close(host(gB), ref[1], "grad_B")
+    assert cpp.last_backward_paths()[0] == want
+    cpp.clear_plan_cache()
+
+
 def test_product_plan_for_rows_of_the_right_operand_of_up_to_32_entries(dev, cpp):
     """A (A A) on a 3D grid -- the right operand has 25-entry rows, so the product takes the hash path --
     in a loop with new values: the first call is stateless, the second leaves a product plan with four
