@@ -795,7 +795,8 @@ extern "C" int nm_spdmm_backward_planned(nm_dtype dt, int64_t rows, int64_t cols
         const auto a = group_args<double>(cols, data, t.t_row, t.t_indptr, t.t_perm, gC, ldg, n, grad_B, ldgb, B, ldb, grad_A);
         return grad_A ? nm_groups::launch<double, int32_t, true, true>(a, s) : nm_groups::launch<double, int32_t, true, false>(a, s);
     }
-    // (a dense operand of thousands of columns: the fused walk takes its column tiles one after the
+    // (Up to 32 columns come here only where rows of gC lie gigabytes apart; a wavefront of the fused walk would be half
+    // idle.  A dense operand of thousands of columns: the fused walk takes its column tiles one after the
     // other, the product below is cut into slices of kColsPerSlice over the grid)
     if (grad_A && grad_B && rows > 0 && cols > 0 && nnz > 0 && n > 32 && n <= 4 * kColsPerSlice) {
         // both gradients from a single walk over A by column

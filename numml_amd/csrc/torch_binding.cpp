@@ -1951,10 +1951,7 @@ struct LincombNode : torch::autograd::Function<LincombNode> {
         const auto s = ctx->get_saved_variables();
         auto g = splincomb_backward((int)ctx->saved_data["rows"].toInt(), (int)ctx->saved_data["cols"].toInt(), s[0], s[1], s[2],
                                     s[3], s[4], s[5], s[6], s[7], grad_or_zeros(grad[0], s[8], s[1]), s[8], s[9]);
-        Tensor g_alpha, g_beta;
-        if (s[0].requires_grad()) g_alpha = s[1].sum().to(s[0].device());
-        if (s[4].requires_grad()) g_beta = s[5].sum().to(s[4].device());
-        return {Tensor(), Tensor(), g_alpha, g[0], Tensor(), Tensor(), g_beta, g[1], Tensor(), Tensor()};
+        return {Tensor(), Tensor(), Tensor(), g[0], Tensor(), Tensor(), Tensor(), g[1], Tensor(), Tensor()};
     }
 };
 
