@@ -21,11 +21,12 @@
 // dots[position] = <dense[index, :], own[r, :]>: the backward by column needs the same row of gC for
 // grad_B and for grad_A.  Dot products alone go by entry (dots_kernel).
 //
-// Measured on graphs with power-law rows and uniformly random columns, forward / with both gradients, against
-// lane = column: 1 M rows, 15.6 M entries, fp32: 64 columns 676 -> 650 / 1708 -> 1592 us (the rows' lines
-// alone take 535, index, values and result 60 more), 16 columns 520 -> 326 / 1276 -> 1040, 128 columns of 8.2 M
-// entries 804 -> 702 / 2172 -> 1618; 60 000 rows, 64 columns 190 -> 89 / 254 -> 145.  Seven-point matrix on 96^3,
-// 16 columns, fp32: 171 -> 60 / 462 -> 163.
+// Measured on graphs with power-law rows and uniformly random columns, forward / backward with both gradients, against
+// lane = column: 1 M rows, 15.6 M entries, fp32: 64 columns 637 -> 608 / 1007 -> 696 us (the rows' lines
+// alone take 535, index, values and result 60 more), 16 columns 524 -> 321 / 747 -> 416; fp64, 16 columns 690 -> 355 / 975 -> 583.
+// 100 000 rows of mean 15, 64 columns fp32 97 -> 73.  Lane = column is the better one for rows of one to three entries of
+// 33 to 64 values (100 000 rows of one, fp64, 48 columns: 16 -> 22) and for fp64 rows of 48 to 64 values where a few
+// rows have thousands of entries (0.5 M rows, 20 M entries, 48 columns: 1067 -> 1300, the backward 1450 -> 1310).
 #pragma once
 
 #include "nm_common.hpp"
@@ -41,10 +42,10 @@ constexpr int kShared = 128, kSplit = 512;
 // Where kAlone eighths of the rows that a workgroup looks through have kShared to kSplit entries, its groups take one each:
 // there long rows are the rule and none keeps the others waiting, while sharing costs two barriers a turn and one group's addition.
 // Rows of 140 to 500 entries throughout, fp32, us, lane = column / all shared / this: 100 000 rows of 140, 16 columns 334 / 446 /
-// 182, 64 columns 449 / 956 / 366; 30 000 of 500, 64 columns 474 / 745 / 319; 3000 of 200, 64 columns 120 / 104 / 28.  (30 000
+// 126, 64 columns 449 / 956 / 262; 30 000 of 500, 64 columns 474 / 745 / 200; 3000 of 200, 64 columns 120 / 104 / 24.  (30 000
 // rows, of 16: from 3 or 4 on power-law rows up to 1000 entries take 50 instead of 26 us at 16 columns; from 12 on rows of 0 to 280
 // 236 instead of 157 at 64.  kShared at 192: power-law rows up to 1000 entries 15 % slower.)  Rows around kShared are
-// the least gain: 30 000 of 90 +- 30, fp64, 64 columns 172 / 209 / 207.
+// the least gain: 30 000 of 90 +- 30, 64 columns, lane = column / this: fp32 111 / 103, fp64 169 / 195.
 constexpr int kAlone = 3;
 constexpr int kChunk = 16;         // entries of a row a group takes from memory at once
 constexpr int kPass = 4;           // entries of a shared row a group takes at once where their order counts
@@ -53,12 +54,18 @@ constexpr int kPass = 4;           // entries of a shared row a group takes at o
 // 128 bytes (kSliceLanes lanes), a workgroup each, which has more of the row's entries in flight (60 000 rows,
 // up to 10 000 entries, 64 columns: 205 -> 89 us).  Where the chip is full anyway slices only cost
 // (1 M rows of 37 columns: 650 -> 785 us, the slices of a row share lines).
-constexpr int kSliceLanes = 8;
+// (In the slices a group takes kSliceBatch rows of the operand at once.  With eight the walk of the other rows, which
+// shares the kernel's registers, had five wavefronts a SIMD instead of seven: 100 000 rows of 5, 64 columns fp32 31 -> 27 us,
+// of 35 120 -> 95.)
+constexpr int kSliceLanes = 8, kSliceBatch = 4;
+// Workgroups at the head of the grid, slices included, that look for long rows: a matrix without any has them for nothing,
+// while few of them have one long row after the other.  2048 fill the chip once.  (2048 before slices, up to 12 500 with
+// them: 100 000 rows of one, fp64, 48 columns 26 -> 22 us; 1024: 200 000 rows of 4 and 256 neighbours of 500, 64 columns fp32 57 -> 96.)
 constexpr int64_t kFewBlocks = 2048, kFewRows = 64;
 constexpr int kScan = kThreads;    // rows a workgroup at the head of the grid looks through,
 // in kPlaces places far apart, so that neighbouring long rows (a sorted graph, a block of dense rows) get workgroups
 // of their own: with 256 neighbours a workgroup one had them all.  fp32, 64 columns, rows of 4 entries and among them 256
-// neighbours of 500: 1 M rows 4930 -> 255 us, 200 000 rows 1330 -> 58; power-law rows in descending order, 200 000: 4840 -> 340.
+// neighbours of 500: 1 M rows 4930 -> 255 us, 200 000 rows 1330 -> 57; power-law rows in descending order, 200 000: 4840 -> 330.
 // (A row by itself each: a line of row pointers a row, 1 M rows of 12 entries 242 -> 248 us at 16 columns.)
 constexpr int kPlaces = 32;
 constexpr int kDrawRows = 4;       // rows of a workgroup per group: enough to draw from, few enough that the
@@ -105,11 +112,11 @@ template <int G, typename T> __device__ __forceinline__ T group_total(T v) {
     return v;
 }
 
-template <typename T, int V, int G, typename IDX, bool PERM, bool DOT>
+template <typename T, int V, int G, typename IDX, bool PERM, bool DOT, int BATCH = (G >= 32 ? 4 : 8)>
 struct Walker {
     static constexpr int kGroups = kThreads / G, kRows = kGroups * kDrawRows;
     // rows of the dense operand in flight at once: with 16 too few wavefronts fit (936 against 650 us)
-    static constexpr int kBatch = G >= 32 ? 4 : 8;
+    static constexpr int kBatch = BATCH;
     static constexpr int kHeld = G < kChunk ? kChunk / G : 1;   // entries of a chunk a lane holds
     static constexpr int kWidth = V;
     static constexpr bool kDot = DOT;
@@ -149,9 +156,11 @@ struct Walker {
         for (int h = 0; h < kHeld; ++h) {
             const int e = h * G + l;
             const int64_t k = kc + (e < cnt ? e : cnt - 1);
-            c.col[h] = (uint32_t)nm::stream_load(a.idx + k);
-            if constexpr (PERM) c.pos[h] = nm::stream_load(a.perm + k);
-            if constexpr (!PERM) c.val[h] = nm::stream_load(a.data + k);
+            // (kept in the caches: the rows of other groups lie in the same lines.  Streamed past them: 30 000 rows of 140,
+            // 16 columns fp32 48 instead of 32 us, 100 000 rows of 35, 24 columns 90 instead of 75)
+            c.col[h] = (uint32_t)a.idx[k];
+            if constexpr (PERM) c.pos[h] = a.perm[k];
+            if constexpr (!PERM) c.val[h] = a.data[k];
         }
         if constexpr (PERM) {
 #pragma unroll
@@ -281,7 +290,7 @@ __global__ __launch_bounds__(kThreads, 5) void groups_kernel(const Args<T, IDX> 
         // (sums alone: a workgroup takes 128 bytes of the row's result, so that wide operands have
         // more workgroups and more entries at once on a row; a dot product wants the whole row)
         constexpr int GS = SLICED ? kSliceLanes : G, kGroups = kThreads / GS;
-        using WS = Walker<T, V, GS, IDX, PERM, DOT>;
+        using WS = Walker<T, V, GS, IDX, PERM, DOT, SLICED ? kSliceBatch : W::kBatch>;
         using Chunk = typename WS::Chunk;
         constexpr int kBatch = WS::kBatch;
         const int slices = SLICED ? (a.n + GS * V - 1) / (GS * V) : 1;
@@ -508,13 +517,13 @@ template <typename T> bool takes(int64_t indexed, int64_t ld, int64_t n, int64_t
 template <typename T, int V, int G, typename IDX, bool PERM, bool DOT>
 int launch_shape(Args<T, IDX> a, hipStream_t s) {
     constexpr int64_t rows = (int64_t)(kThreads / G) * kDrawRows;
-    // rows a workgroup at the head of the grid looks through: few where the matrix has few, since it takes
-    // the long ones that it finds one after the other
-    a.scan_rows = kScan;
-    while (a.scan_rows > 16 && nm::ceil_div(a.rows, a.scan_rows) < kFewBlocks) a.scan_rows /= 2;
     constexpr bool kMaySlice = !DOT && G > kSliceLanes;
     const bool sliced = kMaySlice && nm::ceil_div(a.rows, kFewRows) < kFewBlocks;
     const int64_t slices = sliced ? nm::ceil_div(a.n, kSliceLanes * V) : 1;
+    // rows a workgroup at the head of the grid looks through: few where the matrix has few, since it takes
+    // the long ones that it finds one after the other
+    a.scan_rows = kScan;
+    while (a.scan_rows > 16 && nm::ceil_div(a.rows, a.scan_rows) * slices < kFewBlocks) a.scan_rows /= 2;
     a.scan_sets = nm::ceil_div(a.rows, a.scan_rows);
     a.stripe = 0;
     while ((kPlaces << a.stripe) < a.scan_rows) ++a.stripe;
