@@ -69,7 +69,10 @@ constexpr int kScan = kThreads;    // rows a workgroup at the head of the grid l
 // (A row by itself each: a line of row pointers a row, 1 M rows of 12 entries 242 -> 248 us at 16 columns.)
 constexpr int kPlaces = 32;
 constexpr int kDrawRows = 4;       // rows of a workgroup per group: enough to draw from, few enough that the
-                                   // rows of `own` (16 KB) leave room for eight workgroups a compute unit
+                                   // rows of `own` (16 KB) leave room for eight workgroups a compute unit.
+// Fewer, down to one, where a matrix has too few for kFewBlocks workgroups: four rows one after the other took 10 000 rows
+// of 60, both gradients of 16 columns, fp32 84 us (157 workgroups on 256 compute units; lane = column 63) and take 25 side by side;
+// 30 000 rows of 20, 33 columns 41 -> 33, 100 000 rows of 20, 16 columns 76 -> 68.
 
 // V consecutive elements at an address that need only suit one of them
 template <typename T, int V> struct Vec { typedef T type __attribute__((ext_vector_type(V), aligned(sizeof(T)))); };
@@ -98,6 +101,7 @@ template <typename T, typename IDX> struct Args {
     int64_t scan_sets;        // parts the rows are dealt into for that
     unsigned scan_blocks;     // workgroups that look for long rows, a multiple of nm::kXcds
     unsigned tiles;           // workgroups that walk rows, the same
+    int tile_rows;            // rows each of these walks
 };
 
 // Sum over the G lanes of a group, in every one of them and with the same bits in each (every step adds
@@ -420,9 +424,9 @@ __global__ __launch_bounds__(kThreads, 5) void groups_kernel(const Args<T, IDX> 
     // ---- all other rows, drawn by the groups one at a time ----
     W w(a);
     const int g = t / G;
-    const int64_t r0 = nm::xcd_tile(blockIdx.x - a.scan_blocks, a.tiles) * kRows;
+    const int64_t r0 = nm::xcd_tile(blockIdx.x - a.scan_blocks, a.tiles) * a.tile_rows;
     if (r0 >= a.rows) return;
-    const int nr = (int)(a.rows - r0 < kRows ? a.rows - r0 : kRows);
+    const int nr = (int)(a.rows - r0 < a.tile_rows ? a.rows - r0 : a.tile_rows);
     for (int i = t; i <= nr; i += kThreads) s_ptr[i] = (int64_t)a.ptr[r0 + i];
     if constexpr (DOT) {
         for (int i = g; i < nr; i += kGroups) s_own[i * G + w.l] = w.own_row(r0 + i);
@@ -516,7 +520,9 @@ template <typename T> bool takes(int64_t indexed, int64_t ld, int64_t n, int64_t
 
 template <typename T, int V, int G, typename IDX, bool PERM, bool DOT>
 int launch_shape(Args<T, IDX> a, hipStream_t s) {
-    constexpr int64_t rows = (int64_t)(kThreads / G) * kDrawRows;
+    constexpr int kGroups = kThreads / G;
+    a.tile_rows = kGroups * kDrawRows;
+    while (a.tile_rows > kGroups && nm::ceil_div(a.rows, a.tile_rows) < kFewBlocks) a.tile_rows /= 2;
     constexpr bool kMaySlice = !DOT && G > kSliceLanes;
     const bool sliced = kMaySlice && nm::ceil_div(a.rows, kFewRows) < kFewBlocks;
     const int64_t slices = sliced ? nm::ceil_div(a.n, kSliceLanes * V) : 1;
@@ -527,7 +533,7 @@ int launch_shape(Args<T, IDX> a, hipStream_t s) {
     a.scan_sets = nm::ceil_div(a.rows, a.scan_rows);
     a.stripe = 0;
     while ((kPlaces << a.stripe) < a.scan_rows) ++a.stripe;
-    const int64_t scan = nm::xcd_padded(a.scan_sets * slices), tiles = nm::xcd_padded(nm::ceil_div(a.rows, rows));
+    const int64_t scan = nm::xcd_padded(a.scan_sets * slices), tiles = nm::xcd_padded(nm::ceil_div(a.rows, a.tile_rows));
     NM_REQUIRE(scan + tiles <= 0x7fffffff, "too many rows");
     a.scan_blocks = (unsigned)scan;
     a.tiles = (unsigned)tiles;

@@ -78,10 +78,11 @@ def test_long_columns_and_rows_off_alignment(dev, dtype):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
-@pytest.mark.parametrize("rows", [1, 15, 16, 17, 33, 2500, 40_000, 140_000, 300_001])
+@pytest.mark.parametrize("rows", [1, 15, 16, 17, 33, 2500, 40_000, 140_000, 300_001, 600_001])
 def test_long_rows_side_by_side(dev, dtype, rows, mode):
     """Blocks of long rows among short ones, where the rows are dealt to few and to many workgroups, singly and two and four
-    neighbours at a time; in the small ones a workgroup has so many of them that its groups take one each."""
+    neighbours at a time; in the small ones a workgroup has so many of them that its groups take one each.  (The groups of a
+    workgroup have one row each in the small matrices, two from 131 073 rows of four columns on, four from 262 145.)"""
     rng = np.random.default_rng(rows)
     lengths = rng.integers(0, 3, rows)
     for at in (0, rows // 2, rows - 20):
