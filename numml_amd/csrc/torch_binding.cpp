@@ -919,6 +919,21 @@ Tensor spgemv_forward(int A_rows, int A_cols, Tensor A_data, Tensor A_col_ind, T
 // paid within some twenty steps.
 constexpr int64_t kStagedBoth = 950 << 10, kStagedOne = 3 << 20;
 
+// Whether there are rows enough for that.  A walk by column has one open line of values a row, and g: of few rows both
+// stay in the caches, and the entries are scattered in the sense of the plan's count only.  Random columns, on the plan's
+// kernel -> through the order, us (5 M entries; 5 a column of the first three, 50 of the others):
+//             1000 rows                8000 rows                32 000 rows
+//   both      fp32 71 -> 76            114 -> 77                171 -> 77
+//             fp64 109 -> 135          144 -> 132               183 -> 132
+//   grad_x    fp32 40 -> 49            53 -> 49                 64 -> 49
+//             fp64 48 -> 76            60 -> 76                 68 -> 76 (64 000 rows: 79 -> 80)
+//   both      fp32 124 -> 68   fp64 166 -> 98                   grad_x fp32 50 -> 54   fp64 57 -> 78
+// and 15 M, 150 a column, of 1000 rows: grad_x fp32 151 -> 122, fp64 226 -> 196.
+bool rows_scatter(bool both, int64_t value_bytes, int64_t rows, int64_t cols, int64_t nnz) {
+    if (both) return rows >= 8192 || (rows >= 128 && nnz >= 10 * cols);
+    return rows >= (value_bytes == 4 ? 4096 : 32768) || (rows >= 1024 && nnz >= 100 * cols);
+}
+
 std::vector<Tensor> spgemv_backward(Tensor grad_z, int A_rows, int A_cols, Tensor A_data, Tensor A_col_ind,
                                     Tensor A_rowptr, Tensor x) {
     check_csr("spgemv_backward", A_rows, A_cols, A_data, A_col_ind, A_rowptr);
@@ -941,7 +956,8 @@ std::vector<Tensor> spgemv_backward(Tensor grad_z, int A_rows, int A_cols, Tenso
         // most blocks of 256 columns have a staging list: the instantiation that stages g and x in LDS
         const int32_t *info = plan_info(*plan, A_rows, x.size(0), A_data.numel(), dev);
         const bool lists = 2 * (int64_t)info[5] >= ((int64_t)x.size(0) + 255) / 256;
-        auto staged = want.second && !lists ? permute_plan(plan, A_col_ind, A_rowptr, A_rows, x.size(0),
+        auto staged = want.second && !lists && rows_scatter(want.first, A_data.element_size(), A_rows, x.size(0), A_data.numel())
+                          ? permute_plan(plan, A_col_ind, A_rowptr, A_rows, x.size(0),
                                                            want.first ? kStagedBoth : kStagedOne, dev)
                                             : nullptr;
         if (staged) {

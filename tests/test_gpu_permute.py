@@ -96,3 +96,37 @@ def test_default_mode_takes_it_at_the_third_backward(dev):
     finally:
         ops.set_backward_mode(old)
         ops.clear_plan_cache()
+
+
+@pytest.mark.skipif(_binding.name != "compiled", reason="the plan policy lives in the compiled binding")
+@pytest.mark.parametrize("dtype,both,rows,cols,nnz,want", [
+    (np.float32, True, 8191, 200_000, 1_200_000, False), (np.float32, True, 8192, 200_000, 1_200_000, True),
+    (np.float64, True, 4000, 120_001, 1_200_000, False), (np.float64, True, 4000, 120_000, 1_200_000, True),
+    (np.float32, True, 127, 30_000, 1_200_000, False), (np.float32, True, 128, 30_000, 1_200_000, True),
+    (np.float32, False, 4095, 500_000, 3_200_000, False), (np.float32, False, 4096, 500_000, 3_200_000, True),
+    (np.float64, False, 32767, 500_000, 3_200_000, False), (np.float64, False, 32768, 500_000, 3_200_000, True),
+    (np.float64, False, 1023, 32_000, 3_200_000, False), (np.float64, False, 1024, 32_000, 3_200_000, True)])
+def test_vectors_go_through_the_order_where_there_are_rows_enough(dev, dtype, both, rows, cols, nnz, want):
+    ops = _binding.ops
+    D, I, P = _matrix(rows, cols, nnz, dtype, dev)
+    x, g = torch.randn(cols, device=dev, dtype=D.dtype), torch.randn(rows, device=dev, dtype=D.dtype)
+    old = ops.backward_mode()
+    ops.set_backward_mode("planned")
+    ops.clear_plan_cache()
+    X = x if both else x.clone().requires_grad_(True)
+    size, got = [], []
+    for _ in range(4):
+        got = ops.spgemv_backward(g, rows, cols, D, I, P, X)
+        size.append(ops.plan_cache_size())
+    ops.set_backward_mode(old)
+    ops.clear_plan_cache()
+    assert size == [0, 1, 2, 2] if want else size == [0, 1, 1, 1], size
+    row = torch.repeat_interleave(torch.arange(rows, device=dev), P[1:] - P[:-1])
+    terms = g[row].double() * D.double()
+    ref = torch.zeros(cols, dtype=torch.float64, device=dev).index_add_(0, I, terms)
+    size_of = torch.zeros(cols, dtype=torch.float64, device=dev).index_add_(0, I, terms.abs())
+    count = torch.bincount(I, minlength=cols)
+    # sums of n terms in any order: 2 n eps times the sum of their sizes
+    assert ((got[1].double() - ref).abs() <= 2 * torch.finfo(D.dtype).eps * (count + 1) * size_of).all()
+    if both:
+        assert torch.equal(got[0], g[row] * x[I])
