@@ -1404,16 +1404,25 @@ int launch_fwd(int64_t rows, int64_t nnz, const T *data, const IDX *indices, con
     // of 512 rows a tile -> 512 -> 1024 tiles: 200 000 rows of 7 entries on average 26.2 -> 23.9 -> 19.4 us, 130 000 of 5 14.6 ->
     // 8.4 -> 8.1), and below 65 536 rows, where every column fits 16 bits, on any without lists (20 000 rows of 3 12.7 ->
     // 5.6, 10 000 of 7 10.8 -> 5.0; grids the same).
+    // Long rows on a plan whose columns are packed (a band: neighbouring rows name the same part of x) want more a tile, from
+    // 65 536 rows on, where packed means that: 1024 -> 3072 products, 400 000 rows of 35 fp64 54 -> 40 us, of 1 to 70 72 -> 55,
+    // 1 M rows of 20 61 -> 53, fp32 41 -> 35 (2048: 43, 54, 55, 35); 100 000 rows of 16 fp64 7.2 -> 8.6.
     const bool long_rows = nnz > 8 * rows;
+    constexpr bool kByPacking = sizeof(IDX) == 4 && !LISTS;
+    auto at_least_512 = [&](int r) {
+        while (r > 16 && rows < (int64_t)r * 512) r /= 2;
+        return r;
+    };
     int rt = block_rows(rows, nnz, R, long_rows ? (sizeof(T) == 8 && sizeof(IDX) == 8 ? 1280 : 1024) : CAP);
-    if (long_rows || sizeof(IDX) == 8)
-        while (rt > 16 && rows < (int64_t)rt * 512) rt /= 2;
+    if (long_rows || sizeof(IDX) == 8) rt = at_least_512(rt);
     int narrow = rt;
-    if (sizeof(IDX) == 4 && !LISTS && !long_rows)
+    if (kByPacking && long_rows) rt = at_least_512(block_rows(rows, nnz, R, 3072));
+    if (kByPacking && !long_rows)
         while (narrow > 16 && rows < (int64_t)narrow * 1024) narrow /= 2;
+    narrow = std::min(narrow, rt);
     int64_t grid = nm::xcd_padded(nm::ceil_div(rows, narrow));
     if (grid > nm::kMaxGrid) grid = nm::kMaxGrid;
-    if (sizeof(IDX) == 4 && !LISTS) rt = (rows < (1 << 16) ? narrow : rt) | narrow << 16;
+    if (kByPacking) rt = (rows < (1 << 16) ? narrow : rt) | narrow << 16;
     hipLaunchKernelGGL((spmv_fwd_kernel<T, kFwdBlock, R, CAP, false, IDX, LISTS>), dim3((unsigned)grid), dim3(kFwdBlock), 0, s,
                        rows, rt, data, indices, indptr, x, y, off16, flags, f_desc);
     NM_LAUNCH_CHECK("spmv_fwd_kernel");

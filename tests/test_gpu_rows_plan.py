@@ -43,9 +43,19 @@ def _band_with_long_rows(dtype):
     return randn(5, p[-1], dtype), i.astype(np.int64), p, (3072, 3072)
 
 
+def _mixed(rows, width, dtype):
+    """Rows of 1 to 40 entries, 20 on average, somewhere in `width` columns that move along the diagonal."""
+    rng = np.random.default_rng(width)
+    lens = rng.integers(1, 41, rows)
+    p = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    i = np.repeat(np.arange(rows) * (rows - width) // rows, lens) + rng.integers(0, width, p[-1])
+    return randn(6, p[-1], dtype), i.astype(np.int64), p, (rows, rows)
+
+
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("case", ["band with long rows", "grid", "wide band", "scattered", "ragged", "one row", "511 rows", "513 rows", "65536 rows",
-                                  "65535 rows, some long", "70000 rows, some long"])
+                                  "65535 rows, some long", "70000 rows, some long", "65535 rows of 1 to 40", "65536 rows of 1 to 40",
+                                  "65536 rows of 1 to 40, all columns"])
 def test_the_bits_of_the_plain_kernel(dev, dtype, case):
     d, i, p, (rows, cols) = {
         "band with long rows": lambda: _band_with_long_rows(dtype),
@@ -59,6 +69,9 @@ def test_the_bits_of_the_plain_kernel(dev, dtype, case):
         "65536 rows": lambda: G.poisson2d(256, dtype, jitter_seed=1),
         "65535 rows, some long": lambda: _some_long(65535, dtype),
         "70000 rows, some long": lambda: _some_long(70000, dtype),
+        "65535 rows of 1 to 40": lambda: _mixed(65535, 500, dtype),
+        "65536 rows of 1 to 40": lambda: _mixed(65536, 500, dtype),
+        "65536 rows of 1 to 40, all columns": lambda: _mixed(65536, 65536, dtype),
     }[case]()
     nnz = d.size
     x = randn(4, cols, dtype)
