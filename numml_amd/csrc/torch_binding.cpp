@@ -586,13 +586,18 @@ std::shared_ptr<Plan> backward_plan(const Tensor &indices, const Tensor &indptr,
 // The plan that brings A's values into column-major order and back (nm_permute_plan_build), where that pays, or
 // nullptr.  It pays where neighbouring entries of a column lie further apart among the values than a cache holds
 // (of every 64th entry the plan of the transposed structure counts those that do; an eighth of them suffices) and
-// the entries are `fewest` at least (products with vectors: kStagedBoth, kStagedOne; with dense matrices values of
-// kScatteredBytes).  Graphs with random columns, a step with gradients on either side of the latter line,
-// without -> with: 0.94 M fp32 entries 147 -> 146 us at 64 dense columns and 137 -> 113 at 16; 0.51 M fp64 112 -> 116;
-// 1.0 M fp32 129 -> 130 at 64; 1.5 M fp32 173 -> 135 at 16; 15.6 M fp32 1597 -> 1373 at 64, 1060 -> 770 at 16, fp64
-// 1602 -> 1425 at 32.  In the default mode the plan is noted at the pattern's first backward on the transposed
-// structure and built at the next (15.6 M entries: 1.4 ms, seven steps' gain).
-constexpr int64_t kScatteredBytes = (int64_t)4 << 20;
+// the entries are `fewest` at least (products with vectors: kStagedBoth, kStagedOne; with dense matrices
+// kStagedDense).  Graphs with random columns, backward with both gradients, without -> with:
+//   fp32  0.90 M  4 columns 34 -> 36 us, 64 65 -> 62    1.0 M  16 49 -> 41, 64 76 -> 69    1.5 M  16 72 -> 53, 64 109 -> 93
+//   fp64  0.48 M  4 columns 25 -> 34, 32 41 -> 49       0.90 M 4 42 -> 42, 32 68 -> 68     1.0 M  4 48 -> 45, 32 79 -> 76
+//   15.0 M  fp32 16 774 -> 510, 64 1031 -> 811, fp64 32 1223 -> 916
+// In the default mode the plan is noted at the pattern's first backward on the transposed
+// structure and built at the next (15.6 M entries: 1.1 ms, five steps' gain).
+constexpr int64_t kStagedDense = 1 << 20;
+// Of few rows the open lines of values stay in the caches (rows_scatter has the case of vectors).  5 M entries, a million
+// columns, both gradients, of 8000 -> 32 000 rows: 16 columns fp32 107 / 126 -> 191 / 129 us, 4 columns fp64 111 / 160 -> 161 / 159;
+// of 1000 rows 94 / 125 and 98 / 157.
+constexpr int64_t kStagedDenseRows = 16384;
 std::shared_ptr<Plan> permute_plan(const std::shared_ptr<Plan> &transposed, const Tensor &indices, const Tensor &indptr,
                                    int64_t rows, int64_t cols, int64_t fewest, const c10::Device &dev) {
     const int64_t nnz = indices.numel();
@@ -1333,8 +1338,8 @@ std::vector<Tensor> spdmm_backward(int A_rows, int A_cols, Tensor A_data, Tensor
         if (heavy * (want.first && !grouped ? 1000 : 100) > A_data.numel()) plan = nullptr;
     }
     g_last_spdmm_backward.store(plan ? kOnTransposedPlan : kStateless, std::memory_order_relaxed);
-    auto staged = plan && grouped
-                      ? permute_plan(plan, A_indices, A_indptr, A_rows, B.size(0), kScatteredBytes / value_bytes, dev)
+    auto staged = plan && grouped && A_rows >= kStagedDenseRows
+                      ? permute_plan(plan, A_indices, A_indptr, A_rows, B.size(0), kStagedDense, dev)
                       : nullptr;
     if (staged) {
         size_t bytes = 0;

@@ -130,3 +130,25 @@ def test_vectors_go_through_the_order_where_there_are_rows_enough(dev, dtype, bo
     assert ((got[1].double() - ref).abs() <= 2 * torch.finfo(D.dtype).eps * (count + 1) * size_of).all()
     if both:
         assert torch.equal(got[0], g[row] * x[I])
+
+
+@pytest.mark.skipif(_binding.name != "compiled", reason="the plan policy lives in the compiled binding")
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("rows,nnz,want", [(16_383, 1 << 20, False), (16_384, 1 << 20, True), (16_384, (1 << 20) - 1, False)])
+def test_dense_operands_go_through_the_order_where_there_are_rows_and_entries_enough(dev, dtype, rows, nnz, want):
+    ops, cols, n = _binding.ops, 150_000, 3
+    D, I, P = _matrix(rows, cols, nnz, dtype, dev)
+    B, g = torch.randn(cols, n, device=dev, dtype=D.dtype), torch.randn(rows, n, device=dev, dtype=D.dtype)
+    old = ops.backward_mode()
+    ops.set_backward_mode("planned")
+    ops.clear_plan_cache()
+    size, got = [], []
+    for _ in range(4):
+        got.append(ops.spdmm_backward(rows, cols, D, I, P, B, g))
+        size.append(ops.plan_cache_size())
+    ops.set_backward_mode(old)
+    ops.clear_plan_cache()
+    assert size == [0, 1, 2, 2] if want else size == [0, 1, 1, 1], size
+    assert torch.equal(got[1][0], got[3][0]) and torch.equal(got[1][1], got[3][1])
+    assert_close(host(got[0][0]), host(got[3][0]), "grad_A against the stateless kernels")
+    assert_close(host(got[0][1]), host(got[3][1]), "grad_B against the stateless kernels")
