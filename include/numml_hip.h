@@ -52,8 +52,9 @@ int nm_stream_probe(const void *src, size_t read_bytes, void *dst, size_t write_
 /* ------------------------------------------------------------------ SpMV
  * y = A x.  Stands in for spgemv_forward (cpp/sparse_csr.hpp:32-36,
  * cpp/sparse_csr_cpu.cpp:11-39; CUDA launch site cpp/sparse_csr_cuda.cu:42-67).
- * x has `cols` entries, y `rows`.  Rows whose stored entries fit the
- * workgroup's LDS tile are summed in storage order, exactly like the CPU loop.
+ * x has `cols` entries, y `rows`.  Rows of fewer than 32 entries are summed in
+ * storage order, exactly like the CPU loop; longer ones in 64 parts, term k in
+ * part k % 64, which are added pairwise: the same bits on every entry point.
  */
 int nm_spgemv_forward(nm_dtype dt, int64_t rows, int64_t cols, int64_t nnz,
                       const void *data, const int64_t *indices, const int64_t *indptr,
@@ -170,11 +171,8 @@ int nm_spgemv_forward_planned(nm_dtype dt, int64_t rows, int64_t cols, int64_t n
  * entries' factors looked up there, where nm_spgemv_forward_planned gathers them
  * one by one through the plan's 32-bit columns.  It reserves LDS for those
  * segments, which costs resident workgroups on blocks without a list: for plans
- * most of whose blocks have one.  Rows of fewer than 32 entries are summed by one
- * lane in storage order in both, the same bits; a longer row is shared by a
- * wavefront where its block exceeds the tile, and in fp64 this build's tile
- * holds 4096 products against 3072, so such rows can differ in rounding between
- * the two.  No counterpart in the reference. */
+ * most of whose blocks have one.  Both give the same bits.  No counterpart in the
+ * reference. */
 int nm_spgemv_forward_planned_lists(nm_dtype dt, int64_t rows, int64_t cols, int64_t nnz,
                                     const void *data, const void *plan_mem,
                                     const void *x, void *y, nm_stream stream);
@@ -724,8 +722,8 @@ int nm_csr_to_dense_backward(nm_dtype dt, int64_t rows, int64_t cols, int64_t nn
                              const int64_t *indices, const int64_t *indptr,
                              void *grad_A, nm_stream stream);
 
-/* x[i] = sum of the stored values of row i, added in storage order for rows that
- * fit the workgroup's LDS tile (csr_row_sum_forward, cpp/sparse_csr_cpu.cpp:1106-1131);
+/* x[i] = sum of the stored values of row i, added in the order of nm_spgemv_forward
+ * (csr_row_sum_forward, cpp/sparse_csr_cpu.cpp:1106-1131);
  * backward grad_A[k] = g[row(k)] (csr_row_sum_backward, :1133-1156). */
 int nm_csr_row_sum_forward(nm_dtype dt, int64_t rows, int64_t nnz,
                            const void *data, const int64_t *indptr, void *x, nm_stream stream);

@@ -15,7 +15,8 @@
 // Patches are drawn from a counter in an order in which none waits for a later one: whatever part of
 // the launch is on the chip gets on.  Waits are bounded all the same (NaN throughout, as elsewhere).
 //
-// A pass over the whole chip (28.5 us of 1 M rows, as fast as its bytes) first puts the call's values where the
+// A pass over the whole chip (28.5 us of 1 M rows, 92 MB: half the rate of a copy, since lanes next to each other read rows of
+// different lines) first puts the call's values where the
 // wavefronts read them: entry (p, lane) of a patch holds the row that the lane is at in the steps t = p (mod
 // length), so the arrays are as long as the matrix has rows, and a step reads 40 or 48 bytes a lane, coalesced.
 //
