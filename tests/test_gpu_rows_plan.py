@@ -201,10 +201,18 @@ def test_no_memory_for_the_plan(dev):
     ops.clear_plan_cache()
     want = [ops.spgemv_forward(rows, cols, D, I, P, X) for _ in range(2)][0]
     out = torch.empty_like(want)
+    room = torch.empty(20 << 20, dtype=torch.uint8, device=dev)        # for the products
     torch.cuda.synchronize()
     torch.cuda.empty_cache()
+    taken = []
     try:
-        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (8 << 20)) / torch.cuda.get_device_properties(0).total_memory)
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (2 << 20)) / torch.cuda.get_device_properties(0).total_memory)
+        try:
+            while len(taken) < 4096:        # what earlier work has left free inside its blocks
+                taken.append(torch.empty(24 << 20, dtype=torch.uint8, device=dev))
+        except torch.cuda.OutOfMemoryError:
+            pass
+        del room
         for _ in range(3):
             out.copy_(ops.spgemv_forward(rows, cols, D, I, P, X))
         assert ops.plan_cache_size() == 0
